@@ -87,6 +87,9 @@ extern "C" {
                                 31; with bit 1, klog >= 7) */
 #define TO_OP_ROOT_STORE 11  /* descs: to_root_desc[count]: one instance's root -> its accumulator */
 #define TO_OP_BATCH_BEGIN 12 /* aux2: to_accum[iaux0] zeroed; aux3: int64 start time (device clock) */
+#define TO_OP_FOLD 14 /* descs: to_fold_desc[count]; variant TO_FOLD_ANY: one output per thread,
+                         any bit layout; else TO_FOLD_VEC | y mode << 4 | nreg: the 16-byte form,
+                         every descriptor of the launch with that y mode and nreg */
 #define TO_OP_LEAF_BUILD 13  /* descs: to_leaf_build_desc[count]: leaf tables written from their
                                 compact descriptions (OR / variable leaves) */
 
@@ -204,8 +207,44 @@ typedef struct to_gemm_desc {
                                   (batch << (mlog + nlog)) | (m << nlog) | n, for a
                                   TO_OP_JOIN_FINISH launch (fx = mlog, fy = nlog, nsplit =
                                   2^lsplit) to add up into C */
-    int32_t pad1;
+    int32_t hlog;              /* batch items come in groups of 2^hlog that share one scale
+                                  record (record batch >> hlog; 0: one record per item) */
 } to_gemm_desc;
+
+/* A folded join: C[o] = sum_k X[x(o, k)] * Y[y(o, k)], where every tensor is indexed by
+ * *variables* (bits) and a variable may be in X, in Y or in both, summed (a k bit) or kept
+ * (an o bit) either way.  Edges that COPY (variable) tensors force equal
+ * (src/tensor_network/tensor_network.pyx:470-489) are one variable here, so the entries a
+ * tensordot would store and multiply as structural zeros do not exist.  The offsets are sums
+ * over the set bits of (o, k): entry i of bx / by / bc is what bit i adds to the X, Y and C
+ * offset, in elements (0: the tensor does not have that variable; several positions at once
+ * for a leaf that has it on several axes).  No two entries of one array overlap.  Bits are
+ * listed by the role a kernel gives them:
+ *   TO_FOLD_ANY: [0, 8) thread bits (lo of them o bits, then lk k bits, the rest 0);
+ *     [8, 8 + ntile) o bits of the tile index; then nloop k bits walked by each thread and
+ *     lsplit k bits across blocks.  lk > 0 only when ntile == 0 or lo == 8 - lk.
+ *     With lsplit > 0 the double partial sums go to partial[(batch << (lo + ntile) | c) <<
+ *     lsplit | sp], c the C offset, for a TO_OP_JOIN_FINISH launch (fx = lo + ntile).
+ *   TO_FOLD_VEC: [0, 2) the o bits of 4 consecutive outputs, also the lowest 2 bits of X;
+ *     [2, 10) o bits of the thread index; [10, 10 + ntile) tile; nloop k bits; nreg (<= 3) o
+ *     bits that only Y has, all 2^nreg of whose outputs a thread holds at once.
+ *     y mode: 0 Y has neither of the bits [0, 2); 1 both, as its lowest two; 2 otherwise.
+ *     C, X (and Y in mode 1) and their batch strides aligned to 4 elements. */
+#define TO_FOLD_ANY 0
+#define TO_FOLD_VEC 0x100
+#define TO_FOLD_BITS 40
+typedef struct to_fold_desc {
+    uint64_t x, y, c;
+    int64_t xb, yb, cb;        /* batch strides in elements (0 = broadcast) */
+    uint64_t xs, ys, cs;       /* to_scale_rec* per batch item (TO_F32S), else 0 */
+    int64_t xsb, ysb;          /* scale-record batch strides (0 or 1) */
+    uint64_t partial;
+    int32_t nbatch;
+    int32_t block0, nblocks;
+    int32_t lo, lk, ntile, nloop, lsplit, nreg;
+    int32_t pad;
+    uint32_t bx[TO_FOLD_BITS], by[TO_FOLD_BITS], bc[TO_FOLD_BITS];
+} to_fold_desc;
 
 /* The root scalar of one instance of a batch: stored into its accumulator as
  * (mantissa, exponent), with the device clock at that moment in accum.pad. */
@@ -227,7 +266,7 @@ typedef struct to_launch {
     uint64_t descs; /* device pointer to the descriptor array */
     uint64_t aux0, aux1, aux2, aux3; /* per op; for the descriptor-table ops (LEAF_GATHER,
                                         JOIN_STREAM, JOIN_SPLITK, JOIN_FINISH, PERMUTE, GEMM,
-                                        LEAF_BUILD) aux1 is 0 or a device int32[grid] map of
+                                        FOLD, LEAF_BUILD) aux1 is 0 or a device int32[grid] map of
                                         each block to its descriptor (the last one whose
                                         block0 is at or below the block), read instead of a
                                         binary search over block0 (TO_STREAM_WAVE launches
@@ -248,6 +287,9 @@ int to_version(void);
 int to_struct_sizes(int64_t* join_desc, int64_t* leaf_desc, int64_t* scale_rec,
                      int64_t* accum, int64_t* launch, int64_t* perm_desc, int64_t* gemm_desc,
                      int64_t* root_desc, int64_t* leaf_build_desc);
+
+/* Size in bytes of to_fold_desc, for the same check. */
+int to_fold_desc_size(void);
 
 /* Last error message of the calling thread ("" when none). */
 const char* to_last_error(void);

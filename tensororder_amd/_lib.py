@@ -26,7 +26,8 @@ TO_F64, TO_F32S = 0, 1
     TO_OP_ROOT_STORE,
     TO_OP_BATCH_BEGIN,
     TO_OP_LEAF_BUILD,
-) = range(1, 14)
+    TO_OP_FOLD,
+) = range(1, 15)
 TO_LEAF_VAR, TO_LEAF_OR = 0, 1  # leaf build kinds
 TO_STREAM_VEC = 0x100  # stream variant bit: the 16-byte form
 TO_STREAM_ROWS = 0x200  # stream variant: the row form
@@ -34,8 +35,11 @@ TO_STREAM_ANY = 0x400  # stream launch variant: mixed joins, each by its descrip
 TO_STREAM_WAVE = 0x800  # stream launch variant: one wave per (small) join, four per block
 TO_LAUNCH_SIDE = 0x1  # Launch.flags: captured on the side stream
 TO_LAUNCH_JOIN = 0x2  # Launch.flags: join the side stream into the main one and fork it again first
+TO_FOLD_ANY = 0  # fold launch variants: any bit layout
+TO_FOLD_VEC = 0x100  # the 16-byte form; | y mode << 4 | nreg
 MAX_BITS = 32
-ABI_VERSION = 6
+FOLD_BITS = 40
+ABI_VERSION = 7
 
 c_i8x32 = ctypes.c_int8 * MAX_BITS
 
@@ -109,7 +113,24 @@ class GemmDesc(ctypes.Structure):
         ("asb", ctypes.c_int64), ("bsb", ctypes.c_int64),
         ("mlog", ctypes.c_int32), ("nlog", ctypes.c_int32), ("klog", ctypes.c_int32),
         ("nbatch", ctypes.c_int32), ("block0", ctypes.c_int32), ("nblocks", ctypes.c_int32),
-        ("lsplit", ctypes.c_int32), ("pad1", ctypes.c_int32),
+        ("lsplit", ctypes.c_int32), ("hlog", ctypes.c_int32),
+    ]
+
+
+c_u32xF = ctypes.c_uint32 * FOLD_BITS
+
+
+class FoldDesc(ctypes.Structure):
+    _fields_ = [
+        ("x", ctypes.c_uint64), ("y", ctypes.c_uint64), ("c", ctypes.c_uint64),
+        ("xb", ctypes.c_int64), ("yb", ctypes.c_int64), ("cb", ctypes.c_int64),
+        ("xs", ctypes.c_uint64), ("ys", ctypes.c_uint64), ("cs", ctypes.c_uint64),
+        ("xsb", ctypes.c_int64), ("ysb", ctypes.c_int64),
+        ("partial", ctypes.c_uint64),
+        ("nbatch", ctypes.c_int32), ("block0", ctypes.c_int32), ("nblocks", ctypes.c_int32),
+        ("lo", ctypes.c_int32), ("lk", ctypes.c_int32), ("ntile", ctypes.c_int32), ("nloop", ctypes.c_int32),
+        ("lsplit", ctypes.c_int32), ("nreg", ctypes.c_int32), ("pad", ctypes.c_int32),
+        ("bx", c_u32xF), ("by", c_u32xF), ("bc", c_u32xF),
     ]
 
 
@@ -133,7 +154,7 @@ EXPORTED = [
     "to_version", "to_struct_sizes", "to_last_error", "to_device_count", "to_set_device",
     "to_run", "to_run_timed", "to_graph_create", "to_graph_launch", "to_graph_destroy", "to_permute",
     "to_wall_clock_khz", "to_synchronize", "to_mlp_forward", "to_mlp_backward", "to_mlp_adam",
-    "to_tensordot_workspace", "to_tensordot", "to_tensordot_noalloc",
+    "to_tensordot_workspace", "to_tensordot", "to_tensordot_noalloc", "to_fold_desc_size",
 ]
 MLP_IN, MLP_H1, MLP_H2, MLP_OUT = 16, 64, 64, 2
 MLP_NPARAMS = 64 * 16 + 64 + 64 * 64 + 64 + 2 * 64 + 2
@@ -183,7 +204,7 @@ def load(path=LIB_PATH):
     lib.to_struct_sizes(*[ctypes.byref(s) for s in sizes])
     want = [ctypes.sizeof(t) for t in (JoinDesc, LeafDesc, ScaleRec, Accum, Launch, PermDesc, GemmDesc, RootDesc,
                                        LeafBuildDesc)]
-    if [s.value for s in sizes] != want:
+    if [s.value for s in sizes] != want or lib.to_fold_desc_size() != ctypes.sizeof(FoldDesc):
         raise ImportError("record layout mismatch between library and binding: %s vs %s"
                           % ([s.value for s in sizes], want))
     _lib = lib

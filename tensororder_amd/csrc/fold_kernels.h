@@ -1,0 +1,283 @@
+// Folded joins (to_fold_desc): part of tensororder_hip.hip, inside its anonymous namespace.
+//
+// A join over variables: edges forced equal by COPY tensors are one index bit, which may be
+// in both operands and in the result at once, so no structural zero is stored, moved or
+// multiplied.  On the 70-variable 4096-slice formula that is 2^26 instead of 2^34 products
+// and 2^25 instead of 2^27 entries per slice (the plan the learned model picks), so nearly
+// every join reads a large tensor once, multiplies it by a small one and writes it once:
+// bound by HBM, not by the matrix cores.
+
+// Offsets of a deposit: bit i of v adds row entry first + i (held by lane first + i).  The
+// entries of one row never overlap, so sums are ors.
+__device__ __forceinline__ uint32_t fold_dep(uint32_t v, uint32_t row, int first, int n) {
+    uint32_t r = 0;
+    for (int i = 0; i < n; ++i) r |= (0u - ((v >> i) & 1u)) & (uint32_t)__builtin_amdgcn_readlane((int)row, first + i);
+    return r;
+}
+
+struct FoldRows {
+    uint32_t x, y, c;
+};
+
+// lane i < TO_FOLD_BITS holds the bit entries i (one load per lane and tensor)
+__device__ __forceinline__ FoldRows fold_rows(const to_fold_desc* __restrict__ d) {
+    const int lane = threadIdx.x & 63;
+    const int i = lane < TO_FOLD_BITS ? lane : TO_FOLD_BITS - 1;
+    return FoldRows{d->bx[i], d->by[i], d->bc[i]};
+}
+
+// Walk 2^nloop shared indices in Gray-code order, so each step of KU indices changes one bit
+// above them: f(dx, dy) gets the KU x / y offsets of a step (inside it the low bits follow
+// Gray order too, so the walk is a bijection).
+template <int KU, typename F>
+__device__ __forceinline__ void fold_walk(uint32_t xk, uint32_t yk, const FoldRows& row, int first, int nloop, F f) {
+    constexpr int LKU = KU == 4 ? 2 : (KU == 2 ? 1 : 0);
+    uint32_t dx[KU], dy[KU];
+    dx[0] = dy[0] = 0;
+    if constexpr (KU >= 2) {
+        dx[1] = (uint32_t)__builtin_amdgcn_readlane((int)row.x, first);
+        dy[1] = (uint32_t)__builtin_amdgcn_readlane((int)row.y, first);
+    }
+    if constexpr (KU == 4) {
+        const uint32_t bx = (uint32_t)__builtin_amdgcn_readlane((int)row.x, first + 1);
+        const uint32_t by = (uint32_t)__builtin_amdgcn_readlane((int)row.y, first + 1);
+        dx[2] = dx[1] | bx;
+        dx[3] = bx;
+        dy[2] = dy[1] | by;
+        dy[3] = by;
+    }
+    const uint32_t steps = 1u << (nloop - LKU);
+    for (uint32_t k = 1;; ++k) {
+        uint32_t ox[KU], oy[KU];
+#pragma unroll
+        for (int j = 0; j < KU; ++j) {
+            ox[j] = xk ^ dx[j];
+            oy[j] = yk ^ dy[j];
+        }
+        f(ox, oy);
+        if (k == steps) break;
+        const int b = first + LKU + __builtin_ctz(k);
+        xk ^= (uint32_t)__builtin_amdgcn_readlane((int)row.x, b);
+        yk ^= (uint32_t)__builtin_amdgcn_readlane((int)row.y, b);
+    }
+}
+
+// Scale of a batch item's result: the operands' power-of-two factors (applied to the sums,
+// which are in double, so exactly) and the exponent they carry.
+struct FoldScale {
+    double f;
+    int64_t e;
+};
+
+template <bool SCALED>
+__device__ __forceinline__ FoldScale fold_scale(const to_fold_desc* __restrict__ d, int64_t batch) {
+    if (!SCALED) return FoldScale{1.0, 0};
+    const OpScale a = op_scale(d->xs, d->xsb, batch), b = op_scale(d->ys, d->ysb, batch);
+    return FoldScale{(double)a.f * (double)b.f, a.e + b.e};
+}
+
+// Sum over thread bits [lo, lo + lk) of a 256-thread block: shuffles inside a wave, LDS
+// across waves, both in a fixed order.  The sums are valid where those bits are zero.
+__device__ __forceinline__ double fold_reduce(double v, int lo, int lk, double* red) {
+    const int tid = threadIdx.x;
+    const int hi = lo + lk;
+    for (int b = lo; b < hi && b < 6; ++b) v += __shfl_xor(v, 1 << b, 64);
+    if (hi > 6) {
+        __syncthreads();
+        red[tid] = v;
+        __syncthreads();
+        const int w0 = lo > 6 ? lo : 6;
+        double s = 0.0;
+        for (int j = 0; j < (1 << (hi - w0)); ++j) s += red[(tid & ~(((1 << (hi - w0)) - 1) << w0)) | (j << w0)];
+        v = s;
+    }
+    return v;
+}
+
+// General form: one output per thread, or one share of an output's shared range (lk thread
+// bits), any bit layout.  Products of floats are exact in the double sums, which are rounded
+// once, when stored.
+template <typename T, bool SCALED>
+__device__ __forceinline__ void fold_any_body(const to_fold_desc* __restrict__ d, const int local, double* red) {
+    const int tid = threadIdx.x;
+    const FoldRows row = fold_rows(d);
+    const int lo = d->lo, lk = d->lk, ntile = d->ntile, nloop = d->nloop, lsplit = d->lsplit;
+    const int nthr = lo + lk;
+    const TO_GLOBAL T* __restrict__ X = gptr<const T>(d->x);
+    const TO_GLOBAL T* __restrict__ Y = gptr<const T>(d->y);
+    TO_GLOBAL T* __restrict__ C = gptr<T>(d->c);
+    const int kb = 8 + ntile;
+    const uint32_t xl = fold_dep(tid, row.x, 0, nthr), yl = fold_dep(tid, row.y, 0, nthr);
+    const uint32_t cl = fold_dep(tid, row.c, 0, lo);
+    const bool active = tid < (1 << nthr);
+    const bool writer = tid < (1 << lo);
+    const int64_t n = (int64_t)d->nbatch << (ntile + lsplit);
+    const int64_t t0 = n * local / d->nblocks, t1 = n * (local + 1) / d->nblocks;
+    int64_t cur = -1;
+    FoldScale sc{1.0, 0};
+    float mrun = 0.0f;
+    for (int64_t t = t0; t < t1; ++t) {
+        const uint32_t sp = (uint32_t)t & ((1u << lsplit) - 1);
+        const uint32_t tile = (uint32_t)(t >> lsplit) & ((1u << ntile) - 1);
+        const int64_t batch = t >> (lsplit + ntile);
+        if (SCALED && batch != cur) {
+            if (cur >= 0 && lsplit == 0) {
+                const float w = wave_max(mrun);
+                if ((tid & 63) == 0) note_max(d->cs, cur, w);
+                mrun = 0.0f;
+            }
+            sc = fold_scale<SCALED>(d, batch);
+            cur = batch;
+        }
+        const uint32_t xt = fold_dep(tile, row.x, 8, ntile) | fold_dep(sp, row.x, kb + nloop, lsplit);
+        const uint32_t yt = fold_dep(tile, row.y, 8, ntile) | fold_dep(sp, row.y, kb + nloop, lsplit);
+        const uint32_t co = fold_dep(tile, row.c, 8, ntile) | cl;
+        double acc = 0.0;
+        if (active) {
+            const TO_GLOBAL T* Xp = X + batch * d->xb + xl;
+            const TO_GLOBAL T* Yp = Y + batch * d->yb + yl;
+            auto walk = [&](auto ku) {
+                constexpr int KU = decltype(ku)::value;
+                fold_walk<KU>(xt, yt, row, kb, nloop, [&](const uint32_t* ox, const uint32_t* oy) {
+                    T xv[KU], yv[KU];
+#pragma unroll
+                    for (int j = 0; j < KU; ++j) {
+                        xv[j] = Xp[ox[j]];
+                        yv[j] = Yp[oy[j]];
+                    }
+#pragma unroll
+                    for (int j = 0; j < KU; ++j) acc = fma((double)xv[j], (double)yv[j], acc);
+                });
+            };
+            if (nloop >= 2) walk(std::integral_constant<int, 4>{});
+            else if (nloop == 1) walk(std::integral_constant<int, 2>{});
+            else walk(std::integral_constant<int, 1>{});
+        }
+        if (lk > 0) acc = fold_reduce(acc, lo, lk, red);
+        if (writer) {
+            if (lsplit > 0) {
+                gptr<double>(d->partial)[((((uint64_t)batch << (lo + ntile)) | co) << lsplit) | sp] = SCALED ? acc * sc.f : acc;
+            } else {
+                const T v = (T)(SCALED ? acc * sc.f : acc);
+                C[batch * d->cb + co] = v;
+                if (SCALED) {
+                    mrun = fmaxf(mrun, (float)absval(v));
+                    if (tid == 0 && tile == 0) note_exp(d->cs, batch, sc.e);
+                }
+            }
+        }
+    }
+    if (SCALED && cur >= 0 && lsplit == 0) {
+        const float w = wave_max(mrun);
+        if ((tid & 63) == 0) note_max(d->cs, cur, w);
+    }
+}
+
+template <typename T, bool SCALED>
+__global__ __launch_bounds__(kBlock) void k_fold_any(const to_fold_desc* __restrict__ descs, int ndesc, const int32_t* __restrict__ bmap) {
+    __shared__ double red[kBlock];
+    const to_fold_desc* d = descs + find_desc(descs, ndesc, blockIdx.x, bmap);
+    fold_any_body<T, SCALED>(d, blockIdx.x - d->block0, red);
+}
+
+// 16-byte form for the large joins: a thread owns 4 consecutive outputs times the 2^RY
+// outputs of the register bits (variables only Y has), so an X entry is loaded once for all
+// of them, 16 bytes at a time; Y, the small operand, is read through L1.  Bound by the HBM
+// bytes of X and C.
+template <typename T, bool SCALED, int RY, int YM>
+__global__ __launch_bounds__(kBlock) void k_fold_vec(const to_fold_desc* __restrict__ descs, int ndesc, const int32_t* __restrict__ bmap) {
+    constexpr int R = 1 << RY;
+    constexpr int KMAX = RY >= 2 ? 2 : 4;  // shared indices in flight
+    typedef T V4 __attribute__((ext_vector_type(4)));
+    const to_fold_desc* d = descs + find_desc(descs, ndesc, blockIdx.x, bmap);
+    const int local = blockIdx.x - d->block0;
+    const int tid = threadIdx.x;
+    const FoldRows row = fold_rows(d);
+    const int ntile = d->ntile, nloop = d->nloop;
+    const int kb = 10 + ntile, rb = kb + nloop;
+    const TO_GLOBAL T* __restrict__ X = gptr<const T>(d->x);
+    const TO_GLOBAL T* __restrict__ Y = gptr<const T>(d->y);
+    TO_GLOBAL T* __restrict__ C = gptr<T>(d->c);
+    const uint32_t xl = fold_dep(tid, row.x, 2, 8), yl = fold_dep(tid, row.y, 2, 8), cl = fold_dep(tid, row.c, 2, 8);
+    uint32_t ry[R], rc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        ry[r] = fold_dep(r, row.y, rb, RY);
+        rc[r] = fold_dep(r, row.c, rb, RY);
+    }
+    const uint32_t y1 = (uint32_t)__builtin_amdgcn_readlane((int)row.y, 0);
+    const uint32_t y2 = (uint32_t)__builtin_amdgcn_readlane((int)row.y, 1);
+    const int64_t n = (int64_t)d->nbatch << ntile;
+    const int64_t t0 = n * local / d->nblocks, t1 = n * (local + 1) / d->nblocks;
+    int64_t cur = -1;
+    FoldScale sc{1.0, 0};
+    float mrun = 0.0f;
+    for (int64_t t = t0; t < t1; ++t) {
+        const uint32_t tile = (uint32_t)t & ((1u << ntile) - 1);
+        const int64_t batch = t >> ntile;
+        if (SCALED && batch != cur) {
+            if (cur >= 0) {
+                const float w = wave_max(mrun);
+                if ((tid & 63) == 0) note_max(d->cs, cur, w);
+                mrun = 0.0f;
+            }
+            sc = fold_scale<SCALED>(d, batch);
+            cur = batch;
+        }
+        const TO_GLOBAL T* Xp = X + batch * d->xb + xl;
+        const TO_GLOBAL T* Yp = Y + batch * d->yb + yl;
+        const uint32_t xt = fold_dep(tile, row.x, 10, ntile), yt = fold_dep(tile, row.y, 10, ntile);
+        TO_GLOBAL T* Cp = C + batch * d->cb + (fold_dep(tile, row.c, 10, ntile) | cl);
+        double acc[R][4];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[r][v] = 0.0;
+        auto walk = [&](auto ku) {
+            constexpr int KU = decltype(ku)::value;
+            fold_walk<KU>(xt, yt, row, kb, nloop, [&](const uint32_t* ox, const uint32_t* oy) {
+                V4 xv[KU];
+#pragma unroll
+                for (int j = 0; j < KU; ++j) xv[j] = *reinterpret_cast<const TO_GLOBAL V4*>(Xp + ox[j]);
+#pragma unroll
+                for (int j = 0; j < KU; ++j) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        const TO_GLOBAL T* p = Yp + (oy[j] | ry[r]);
+                        if constexpr (YM == 0) {
+                            const double y = (double)*p;
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) acc[r][v] = fma((double)xv[j][v], y, acc[r][v]);
+                        } else if constexpr (YM == 1) {
+                            const V4 y = *reinterpret_cast<const TO_GLOBAL V4*>(p);
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) acc[r][v] = fma((double)xv[j][v], (double)y[v], acc[r][v]);
+                        } else {
+                            const T y[4] = {p[0], p[y1], p[y2], p[y1 | y2]};
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) acc[r][v] = fma((double)xv[j][v], (double)y[v], acc[r][v]);
+                        }
+                    }
+                }
+            });
+        };
+        if (KMAX == 4 && nloop >= 2) walk(std::integral_constant<int, KMAX>{});
+        else if (nloop >= 1) walk(std::integral_constant<int, 2>{});
+        else walk(std::integral_constant<int, 1>{});
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            V4 o;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                o[v] = (T)(SCALED ? acc[r][v] * sc.f : acc[r][v]);
+                if (SCALED) mrun = fmaxf(mrun, (float)absval(o[v]));
+            }
+            *reinterpret_cast<TO_GLOBAL V4*>(Cp + rc[r]) = o;
+        }
+        if (SCALED && tid == 0 && tile == 0) note_exp(d->cs, batch, sc.e);
+    }
+    if (SCALED && cur >= 0) {
+        const float w = wave_max(mrun);
+        if ((tid & 63) == 0) note_max(d->cs, cur, w);
+    }
+}

@@ -25,7 +25,7 @@
 
 #include "tensororder_hip.h"
 
-#define TO_ABI_VERSION 6
+#define TO_ABI_VERSION 7
 
 namespace {
 
@@ -1685,13 +1685,14 @@ __global__ __launch_bounds__(kBlock) void k_gemm(const to_gemm_desc* __restrict_
         const int64_t rem = (t >> lsplit) - batch * per_batch;
         int64_t tm, tn;
         grouped_tile(rem, tiles_m, tiles_n, tm, tn);
-        if (SCALED && lsplit == 0) publish_max_on_change(d->cs, mx_batch, batch, mx, lane);
+        const int64_t rec = batch >> d->hlog;  // batch item of the scale records
+        if (SCALED && lsplit == 0) publish_max_on_change(d->cs, mx_batch, rec, mx, lane);
         const TO_GLOBAL T* A = gptr<const T>(d->a) + batch * d->ab + (tm * BM + lrow) * K + sp * KS + lk;
         const TO_GLOBAL T* B = gptr<const T>(d->b) + batch * d->bb + (tn * BN + lrow) * K + sp * KS + lk;
         T sa = T(1), sb = T(1);
         int64_t ea = 0, eb = 0;
         if (SCALED) {
-            const OpScale x = op_scale(d->as, d->asb, batch), y = op_scale(d->bs, d->bsb, batch);
+            const OpScale x = op_scale(d->as, d->asb, rec), y = op_scale(d->bs, d->bsb, rec);
             sa = T(x.f); ea = x.e; sb = T(y.f); eb = y.e;
         }
         V acc[2][2];
@@ -1773,7 +1774,7 @@ __global__ __launch_bounds__(kBlock) void k_gemm(const to_gemm_desc* __restrict_
                 }
             }
         }
-        if (SCALED && tid == 0 && tm == 0 && tn == 0) note_exp(d->cs, batch, ea + eb);
+        if (SCALED && tid == 0 && tm == 0 && tn == 0 && batch == rec << d->hlog) note_exp(d->cs, rec, ea + eb);
     }
     if (SCALED) publish_max_on_change(d->cs, mx_batch, -1, mx, lane);
 }
@@ -1822,13 +1823,14 @@ __device__ __forceinline__ void gemm128_body(const to_gemm_desc* __restrict__ de
         const int64_t rem = t - batch * per_batch;
         int64_t tm, tn;
         grouped_tile(rem, tiles_m, tiles_n, tm, tn);
-        if (SCALED) publish_max_on_change(d->cs, mx_batch, batch, mx, lane);
+        const int64_t rec = batch >> d->hlog;  // batch item of the scale records
+        if (SCALED) publish_max_on_change(d->cs, mx_batch, rec, mx, lane);
         const TO_GLOBAL T* A = gptr<const T>(d->a) + batch * d->ab + tm * BM * K;
         const TO_GLOBAL T* B = gptr<const T>(d->b) + batch * d->bb + tn * BN * K;
         T sa = T(1), sb = T(1);
         int64_t ea = 0, eb = 0;
         if (SCALED) {
-            const OpScale x = op_scale(d->as, d->asb, batch), y = op_scale(d->bs, d->bsb, batch);
+            const OpScale x = op_scale(d->as, d->asb, rec), y = op_scale(d->bs, d->bsb, rec);
             sa = T(x.f); ea = x.e; sb = T(y.f); eb = y.e;
         }
         V acc[4][NJ];
@@ -1938,7 +1940,7 @@ __device__ __forceinline__ void gemm128_body(const to_gemm_desc* __restrict__ de
                 }
             }
         }
-        if (SCALED && tid == 0 && tm == 0 && tn == 0) note_exp(d->cs, batch, ea + eb);
+        if (SCALED && tid == 0 && tm == 0 && tn == 0 && batch == rec << d->hlog) note_exp(d->cs, rec, ea + eb);
     }
     if (SCALED) publish_max_on_change(d->cs, mx_batch, -1, mx, lane);
 }
@@ -2083,13 +2085,14 @@ __device__ __forceinline__ void gemm_x6_body(const to_gemm_desc* __restrict__ de
         const int64_t rem = t - batch * per_batch;
         int64_t tm, tn;
         grouped_tile(rem, tiles_m, tiles_n, tm, tn);
-        if (SCALED) publish_max_on_change(d->cs, mx_batch, batch, mx, lane);
+        const int64_t rec = batch >> d->hlog;  // batch item of the scale records
+        if (SCALED) publish_max_on_change(d->cs, mx_batch, rec, mx, lane);
         const TO_GLOBAL float* A = gptr<const float>(d->a) + batch * d->ab + tm * BM * K;
         const TO_GLOBAL float* B = gptr<const float>(d->b) + batch * d->bb + tn * BN * K;
         float sa = 1.0f, sb = 1.0f;
         int64_t ea = 0, eb = 0;
         if (SCALED) {
-            const OpScale x = op_scale(d->as, d->asb, batch), y = op_scale(d->bs, d->bsb, batch);
+            const OpScale x = op_scale(d->as, d->asb, rec), y = op_scale(d->bs, d->bsb, rec);
             sa = x.f; ea = x.e; sb = y.f; eb = y.e;
         }
         V acc[4][TJ];
@@ -2257,7 +2260,7 @@ __device__ __forceinline__ void gemm_x6_body(const to_gemm_desc* __restrict__ de
                 }
             }
         }
-        if (SCALED && tid == 0 && tm == 0 && tn == 0) note_exp(d->cs, batch, ea + eb);
+        if (SCALED && tid == 0 && tm == 0 && tn == 0 && batch == rec << d->hlog) note_exp(d->cs, rec, ea + eb);
     }
     if (SCALED) publish_max_on_change(d->cs, mx_batch, -1, mx, lane);
 }
@@ -2267,6 +2270,8 @@ template <bool SCALED, bool WIDE, bool TR, int BM>
 __global__ __launch_bounds__(64 * x6_waves<WIDE>(), 1) void k_gemm_x6(const to_gemm_desc* __restrict__ descs, int ndesc, const int32_t* __restrict__ bmap) {
     gemm_x6_body<SCALED, WIDE, TR, BM>(descs, ndesc, bmap);
 }
+
+#include "fold_kernels.h"
 
 // ---------------------------------------------------------------------------------
 // host dispatch
@@ -2435,6 +2440,30 @@ int launch_one(const to_launch& L, hipStream_t st) {
             hipLaunchKernelGGL((k_root_store<T, SCALED>), grid, block, 0, st,
                                reinterpret_cast<const to_root_desc*>(L.descs), L.count);
             break;
+        case TO_OP_FOLD: {
+            if (!L.descs || L.count <= 0) return TO_ERR_INVALID;
+            const to_fold_desc* fd = reinterpret_cast<const to_fold_desc*>(L.descs);
+            switch (L.variant) {
+                case TO_FOLD_ANY:
+                    hipLaunchKernelGGL((k_fold_any<T, SCALED>), grid, block, 0, st, fd, L.count, bmap);
+                    break;
+#define TO_FOLD_CASE(RY, YM)                                                                         \
+    case TO_FOLD_VEC | YM << 4 | RY:                                                                 \
+        hipLaunchKernelGGL((k_fold_vec<T, SCALED, RY, YM>), grid, block, 0, st, fd, L.count, bmap); \
+        break;
+#define TO_FOLD_CASES(RY) TO_FOLD_CASE(RY, 0) TO_FOLD_CASE(RY, 1) TO_FOLD_CASE(RY, 2)
+                TO_FOLD_CASES(0)
+                TO_FOLD_CASES(1)
+                TO_FOLD_CASES(2)
+                TO_FOLD_CASES(3)
+#undef TO_FOLD_CASES
+#undef TO_FOLD_CASE
+                default:
+                    set_err("fold: unknown variant");
+                    return TO_ERR_INVALID;
+            }
+            break;
+        }
         case TO_OP_LEAF_BUILD:
             if (!L.descs || L.count <= 0) return TO_ERR_INVALID;
             hipLaunchKernelGGL((k_leaf_build<T>), grid, block, 0, st,
@@ -2506,6 +2535,8 @@ int to_struct_sizes(int64_t* join_desc, int64_t* leaf_desc, int64_t* scale_rec, 
     if (launch) *launch = sizeof(to_launch);
     return TO_OK;
 }
+
+int to_fold_desc_size(void) { return (int)sizeof(to_fold_desc); }
 
 const char* to_last_error(void) { return g_err; }
 

@@ -1,0 +1,703 @@
+"""Folded plans: a contraction tree whose COPY tensors are index identities.
+
+A CNF network holds one COPY (variable) tensor per variable, split into pieces by the
+planners, and every COPY tensor forces its edges equal
+(``tensor_network_constructions.py:122-159``; the reference's own equivalence sets are
+``find_equivalent_edges``, ``tensor_network.pyx:470-489``).  A tensordot walk stores one axis
+per *edge*, so an intermediate that holds several edges of one variable is zero wherever they
+differ.  Here such edges are one *variable* of the schedule:
+
+* a tensor is indexed by the distinct variables of its free edges; a join may share a variable
+  with its result (kept), sum it, or take it from one operand (``to_fold_desc``);
+* a variable is summed at the lowest join that covers every leaf holding it;
+* an unweighted COPY piece is a vector of ones and is dropped; a weight vector multiplies one
+  leaf that holds its variable, wherever the tree had placed it;
+* chains in which a large tensor absorbs small ones are reassociated by the bytes and products
+  they cost, as in ``schedule.regroup_absorptions``.
+
+Every tensor's bits are ordered by how late their variable is summed, the latest lowest.  The
+order is one order for the whole plan, so the operands and the result of a join agree on it:
+kept variables run along the lanes in all three, and the summed ones are the highest bits.
+Dense joins (free ranges of >= 2^6 on both sides) go to the MFMA products, with the kept
+shared variables as batch items.
+
+The value is the same contraction; only structural zeros are left out.
+"""
+
+import math
+import struct
+
+import numpy as np
+
+from . import _lib, schedule
+from ._lib import LeafDesc, Launch
+
+ALIGN = schedule.ALIGN
+
+# Cost of a join for the reassociation (seconds): bytes at the rate of a large copy, products
+# at the rate the folded kernels multiply and add (measured on the 4096-slice workload).
+BYTES_PER_S = 5e12
+PRODUCTS_PER_S = 8e12
+GEMM_PRODUCTS_PER_S = 5e13
+# operands of at most this many variables may be combined before a large tensor absorbs them
+SMALL_RANK = 12
+BIG_RANK = 10
+# share of the cost of a join that runs once per slice, against one that runs once
+BATCH_WEIGHT = 64.0
+# threads a general-form launch should have before its shared range is left to one thread
+ANY_MIN_THREADS_LOG = 17
+MAX_ANY_BLOCKS = 8192
+MAX_VEC_BLOCKS = 4096
+MAX_REG_BITS = 3
+
+_HEAD = struct.Struct("<QQQqqqQQQqqQ10i")
+_BITS = struct.Struct("<%dI" % (3 * _lib.FOLD_BITS))
+
+
+class FoldDesc:
+    """A to_fold_desc under construction (``block0`` is set when a launch groups it)."""
+
+    __slots__ = ("ptrs", "strides", "recs", "rec_strides", "partial", "nbatch", "block0", "nblocks", "roles", "bits")
+
+    def __bytes__(self):
+        lo, lk, ntile, nloop, lsplit, nreg = self.roles
+        return _HEAD.pack(*self.ptrs, *self.strides, *self.recs, *self.rec_strides, self.partial, self.nbatch,
+                          self.block0, self.nblocks, lo, lk, ntile, nloop, lsplit, nreg, 0) + _BITS.pack(*self.bits)
+
+
+class FNode:
+    """A node of a folded plan.  ``order`` lists its variables from the lowest bit up and
+    ``off`` maps each to the element offset it adds (several bits at once for a leaf that
+    holds it on several axes); 2^rank entries are stored."""
+
+    __slots__ = ("idx", "is_leaf", "tensor", "rank", "order", "order0", "off", "batched", "left", "right", "parent", "ksum",
+                 "geom", "buf", "ptr", "bstride", "rec", "rec_stride")
+
+    def __init__(self, idx):
+        self.idx = idx
+        self.parent = -1
+        self.buf = None
+        self.rec = None
+        self.rec_stride = 0
+
+
+class _T:
+    """A subtree while the tree is built: ``open`` maps its unsummed variables to the number
+    of leaves below that hold them, ``union`` counts the variables its join touches."""
+
+    __slots__ = ("leaf", "open", "left", "right", "batched", "union", "cost")
+
+    def __init__(self, leaf, open_, left=None, right=None, batched=False, union=0, cost=0.0):
+        self.leaf, self.open, self.left, self.right = leaf, open_, left, right
+        self.batched, self.union, self.cost = batched, union, cost
+
+
+def has_copies(tables):
+    """Whether a plan's leaves include COPY tensors (the plan can be folded)."""
+    return any(t.copy is not None for t in tables.values())
+
+
+def _join_cost(left, right, union, out, batched, esize):
+    lx, ly = len(left.open), len(right.open)
+    c = esize * ((1 << lx) + (1 << ly) + (1 << out)) / BYTES_PER_S
+    # free range of each side: what the MFMA products need
+    dense = union - lx >= 6 and union - ly >= 6 and union - out >= 4
+    c += (1 << union) / (GEMM_PRODUCTS_PER_S if dense else PRODUCTS_PER_S)
+    return c * (BATCH_WEIGHT if batched else 1.0)
+
+
+def analyse(tree, tables, esize, regroup=True):
+    """(post-order FNode list, number of variables no remaining leaf holds -- each doubles the
+    count) of a plan, or None when no leaf would remain."""
+    flat = schedule.flatten_tree(tree)
+    if flat[-1].rank != 0:
+        raise ValueError("the tree's root has free edges; only full contractions are supported")
+    root = {}
+
+    def find(e):
+        while root.setdefault(e, e) != e:
+            e = root[e]
+        return e
+
+    for n in flat:
+        if not n.is_leaf:
+            continue
+        t = tables[n.tensor]
+        if t.rank != n.rank:
+            raise ValueError("leaf %d: table rank %d != tree rank %d" % (n.tensor, t.rank, n.rank))
+        if t.copy is not None:
+            for e in n.free:
+                root[find(e)] = find(n.free[0])
+        else:
+            for e in n.free:
+                find(e)
+
+    # leaves: variable -> offset mask in the leaf's own table
+    offs, weights, hosts = {}, [], []
+    seen = set()
+    for n in flat:
+        if not n.is_leaf:
+            continue
+        off = {}
+        for a, e in enumerate(n.free):
+            v = find(e)
+            off[v] = off.get(v, 0) | 1 << (n.rank - 1 - a)
+        seen.update(off)
+        t = tables[n.tensor]
+        if t.copy is not None and t.copy[2] and t.copy[0] == 1 and t.copy[1] == 1:
+            continue  # a vector of ones
+        offs[n.idx] = off
+        (weights if len(off) <= 1 else hosts).append(n.idx)
+    # weight vectors (and scalars) multiply one leaf that holds their variable: an unsliced
+    # one where possible, so that the product is not repeated per slice
+    attach, placed = {}, set()
+
+    def host_key(i):
+        return (len(offs[i]), i)
+
+    by_var = {}
+    for h in hosts:
+        for v in offs[h]:
+            by_var.setdefault(v, []).append(h)
+    for w in weights:
+        bw = tables[flat[w].tensor].batched
+        cand = by_var.get(next(iter(offs[w])), []) if offs[w] else hosts
+        if cand:
+            h = min(cand, key=lambda i: (tables[flat[i].tensor].batched != bw, host_key(i)))
+            attach.setdefault(h, []).append(w)
+            placed.add(w)
+
+    total = {}
+    for off in offs.values():
+        for v in off:
+            total[v] = total.get(v, 0) + 1
+    missing = len(seen) - len(total)
+
+    def join(left, right):
+        m = dict(left.open)
+        for v, c in right.open.items():
+            m[v] = m.get(v, 0) + c
+        batched = left.batched or right.batched
+        union = len(m)
+        out = {v: c for v, c in m.items() if c != total[v]}
+        return _T(None, out, left, right, batched, union, _join_cost(left, right, union, len(out), batched, esize))
+
+    def leaf(i):
+        return _T(i, {v: 1 for v in offs[i]}, batched=tables[flat[i].tensor].batched)
+
+    stack = []
+    for n in flat:
+        if n.is_leaf:
+            if n.idx not in offs or n.idx in placed:
+                stack.append(None)
+                continue
+            t = leaf(n.idx)
+            for w in sorted(attach.get(n.idx, []), key=lambda i: (tables[flat[i].tensor].batched, i)):
+                t = join(t, leaf(w))
+            stack.append(t)
+            continue
+        right, left = stack.pop(), stack.pop()
+        if left is None or right is None:
+            stack.append(left or right)
+            continue
+        t = join(left, right)
+        while regroup:
+            big, small = (t.left, t.right) if len(t.left.open) >= len(t.right.open) else (t.right, t.left)
+            if big.leaf is not None or len(small.open) > SMALL_RANK:
+                break
+            ib, ism = (big.left, big.right) if len(big.left.open) >= len(big.right.open) else (big.right, big.left)
+            if len(ib.open) < BIG_RANK or len(ism.open) > SMALL_RANK:
+                break
+            m = join(ism, small)
+            if len(m.open) > SMALL_RANK:
+                break
+            nt = join(ib, m)
+            if nt.cost + m.cost >= t.cost + big.cost:
+                break
+            t = nt
+        stack.append(t)
+    top = stack[0]
+    if top is None:
+        return None
+
+    # post-order nodes; a lone leaf is summed by a join with the constant one (no right child)
+    nodes, index, todo = [], {}, [(top, False)]
+    while todo:
+        t, expanded = todo.pop()
+        if t.leaf is None and not expanded:
+            todo += [(t, True), (t.right, False), (t.left, False)]
+            continue
+        n = FNode(len(nodes))
+        n.is_leaf = t.leaf is not None
+        n.batched = t.batched
+        n.left = n.right = -1
+        if n.is_leaf:
+            n.tensor = flat[t.leaf].tensor
+            n.rank = flat[t.leaf].rank
+            n.off = offs[t.leaf]
+        else:
+            n.left, n.right = index[id(t.left)], index[id(t.right)]
+            nodes[n.left].parent = nodes[n.right].parent = n.idx
+            n.rank = len(t.open)
+        n.order = list(t.open)
+        index[id(t)] = n.idx
+        nodes.append(n)
+    if nodes[-1].is_leaf:
+        leaf_node = nodes[-1]
+        n = FNode(len(nodes))
+        n.is_leaf, n.batched, n.left, n.right, n.rank, n.order = False, leaf_node.batched, leaf_node.idx, -1, 0, []
+        leaf_node.parent = n.idx
+        nodes.append(n)
+    # the plan's one bit order: variables summed later are lower bits
+    when = {}
+    for n in nodes:
+        if n.is_leaf:
+            continue
+        kept = set(n.order)
+        held = set(nodes[n.left].order)
+        if n.right >= 0:
+            held |= set(nodes[n.right].order)
+        n.ksum = held - kept
+        for v in n.ksum:
+            when[v] = n.idx
+    for n in nodes:
+        n.order.sort(key=lambda v: (-when[v], v))
+        n.order0 = n.order
+    return nodes, missing
+
+
+def _reordered(n, order):
+    n.order = order
+    n.off = {v: 1 << i for i, v in enumerate(order)}
+
+
+def _canonical(node, want):
+    """True when a stored tensor's bits are the variables ``want`` in order."""
+    return node.rank == len(want) and all(node.off.get(v) == 1 << i for i, v in enumerate(want))
+
+
+def choose(n, nodes, W, esize):
+    """Kernel form and launch shape of one folded join for W slices (``n.geom``).  A dense
+    join also fixes its result's bit order ([kept shared][X][Y])."""
+    A = nodes[n.left]
+    B = nodes[n.right] if n.right >= 0 else None
+    nb = W if n.batched else 1
+    _reordered(n, list(n.order0))
+    if B is None:
+        X, Y = A, None
+    else:
+        X, Y = (A, B) if (A.rank, A.batched) >= (B.rank, B.batched) else (B, A)
+    xoff = X.off
+    yoff = Y.off if Y is not None else {}
+    # shared range in X's memory order, lowest first
+    ks = sorted(n.ksum, key=lambda v: (xoff.get(v, 1 << 40), yoff.get(v, 0), v))
+    s = len(ks)
+    if Y is not None and all(v in xoff and v in yoff for v in ks):
+        kept = [v for v in n.order if v in xoff and v in yoff]
+        xo = [v for v in n.order if v in xoff and v not in yoff]
+        yo = [v for v in n.order if v in yoff and v not in xoff]
+        plain = X.rank == len(xoff) and Y.rank == len(yoff)
+        if len(xo) >= schedule.GEMM_MIN_FREE and len(yo) >= schedule.GEMM_MIN_FREE and \
+                s >= schedule.GEMM_MIN_SHARED and plain and \
+                (not kept or nb == 1 or (X.batched and Y.batched)):
+            if len(yo) > len(xo):
+                X, Y, xo, yo = Y, X, yo, xo
+            h = len(kept)
+            _reordered(n, yo + xo + kept)
+            g = dict(fx=len(xo), fy=len(yo), s=s, shf=len(yo), shy=0, xf=list(range(s, s + len(xo))),
+                     xs=list(range(s)), yf=list(range(s, s + len(yo))), ys=list(range(s)), x_is_left=X is A)
+            v = schedule.choose_variant(g, nb << h, esize)
+            want_x, want_y = ks + xo + kept, ks + yo + kept
+            v.update(perm_x=not _canonical(X, want_x), perm_y=not _canonical(Y, want_y), hlog=h, want_x=want_x,
+                     want_y=want_y)
+            g.update(var=v, X=X.idx, Y=Y.idx)
+            n.geom = g
+            return
+    out = n.order
+    nc = len(out)
+    yonly = [v for v in out if v not in xoff]
+    g = dict(fx=nc - len(yonly), fy=len(yonly), s=s, X=X.idx, Y=Y.idx if Y is not None else -1)
+    lognb = int(math.log2(nb))
+    reg = yonly[:MAX_REG_BITS]
+    body = [v for v in out if v not in reg] if reg else out
+    if Y is not None and len(body) >= 10 and xoff.get(body[0]) == 1 and xoff.get(body[1]) == 2 and \
+            n.off[body[0]] == 1 and n.off[body[1]] == 2 and X.rank >= 2 and \
+            (lognb + len(body) >= 18 or s <= 4) and len(body) + s + len(reg) <= _lib.FOLD_BITS:
+        y0, y1 = yoff.get(body[0], 0), yoff.get(body[1], 0)
+        ym = 0 if y0 == 0 and y1 == 0 else 1 if (y0, y1) == (1, 2) and Y.rank >= 2 else 2
+        ntile = len(body) - 10
+        tiles = nb << ntile
+        g["var"] = dict(kind="fold", variant=_lib.TO_FOLD_VEC | ym << 4 | len(reg), bits=body + ks + reg,
+                        roles=(10, 0, ntile, s, 0, len(reg)), nblocks=int(min(tiles, MAX_VEC_BLOCKS)), lsplit=0,
+                        vec=True, yc=1 << len(reg))
+        n.geom = g
+        return
+    # general form: thread bits go to outputs, then to the shared range while the launch
+    # would have few threads; long shared ranges with few outputs are split over blocks
+    lk = 0
+    if lognb + nc < ANY_MIN_THREADS_LOG and s > 0:
+        lk = min(s, 8, max(8 - nc, min(s - 3, ANY_MIN_THREADS_LOG - lognb - nc)))
+        lk = max(lk, 0)
+    lo = min(nc, 8 - lk)
+    rest = s - lk
+    lsplit = 0
+    if rest > 6:
+        lsplit = max(0, min(rest - 4, ANY_MIN_THREADS_LOG + 3 - lognb - nc - lk))
+    ntile = nc - lo
+    pad = [None] * (8 - lo - lk)
+    g["var"] = dict(kind="fold", variant=_lib.TO_FOLD_ANY, bits=out[:lo] + ks[:lk] + pad + out[lo:] + ks[lk:],
+                    roles=(lo, lk, ntile, rest - lsplit, lsplit, 0),
+                    nblocks=int(min(nb << (ntile + lsplit), MAX_ANY_BLOCKS)), lsplit=lsplit, nout=nb << nc,
+                    nsplit=1 << lsplit, vec=False, yc=1)
+    if len(g["var"]["bits"]) > _lib.FOLD_BITS:
+        raise ValueError("folded join over more than %d variables" % _lib.FOLD_BITS)
+    n.geom = g
+
+
+def choose_all(nodes, W, esize):
+    for n in nodes:
+        if not n.is_leaf:
+            choose(n, nodes, W, esize)
+
+
+def _scratch(arena, n, nodes, nb, esize, table):
+    """Scratch a join needs while it runs: split sums, permuted operands of a product."""
+    v = n.geom["var"]
+    blocks = {}
+    if v["kind"] == "fold" and v["lsplit"]:
+        blocks["partial"] = arena.alloc(v["nout"] * v["nsplit"] * 8)
+    if v["kind"] == "gemm":
+        for key, i in (("perm_x", n.geom["X"]), ("perm_y", n.geom["Y"])):
+            if v[key]:
+                blocks[key] = arena.alloc((nb if nodes[i].batched else 1) * (1 << nodes[i].rank) * esize)
+    table[n.idx] = blocks
+    return list(blocks.values())
+
+
+def join_levels(nodes, batched):
+    """Joins of one phase by level, as ``schedule.join_levels``."""
+    level, out = {}, []
+    for n in nodes:
+        if n.is_leaf or n.batched != batched:
+            continue
+        lv = 1 + max(level.get(n.left, 0), level.get(n.right, 0))
+        level[n.idx] = lv
+        while len(out) < lv:
+            out.append([])
+        out[lv - 1].append(n.idx)
+    return out
+
+
+def plan_memory(nodes, W, esize, order):
+    """(arena peak, scratch placements), as ``schedule.plan_memory``."""
+    arena = schedule._Arena()
+    scratch = {}
+
+    def run(group, nb, release):
+        temps = []
+        for i in group:
+            n = nodes[i]
+            n.buf = arena.alloc(nb * (1 << n.rank) * esize)
+            temps += _scratch(arena, n, nodes, nb, esize, scratch)
+        for blk in temps:
+            arena.release(blk)
+        for i in group:
+            for c in (nodes[i].left, nodes[i].right):
+                if c >= 0 and release(nodes[c]):
+                    arena.release(nodes[c].buf)
+
+    def groups(batched):
+        if order == "level":
+            return join_levels(nodes, batched)
+        return [[n.idx] for n in nodes if not n.is_leaf and n.batched == batched]
+
+    for grp in groups(False):
+        run(grp, 1, lambda c: not c.is_leaf and not c.batched)
+    for n in nodes:
+        if n.is_leaf and n.batched:
+            n.buf = arena.alloc(W * (1 << n.rank) * esize)
+    for grp in groups(True):
+        run(grp, W, lambda c: c.batched)
+    return arena.peak, scratch
+
+
+def choose_order(nodes, W, esize):
+    post, _ = plan_memory(nodes, W, esize, "post")
+    level, _ = plan_memory(nodes, W, esize, "level")
+    if level <= schedule.LEVEL_PEAK_FACTOR * post:
+        return "level", level
+    return "post", post
+
+
+def peak_bytes(nodes, W, esize):
+    choose_all(nodes, W, esize)
+    return choose_order(nodes, W, esize)[1]
+
+
+def join_records(n, nodes, W, esize, scaled, abase, scratch, recp, one):
+    """Descriptor records of one join in execution order, as ``schedule.join_records``:
+    [(kind, op, variant, lds, descriptor, blocks)]; ``one``: (address, record address) of a
+    stored 1.0, the second operand of a lone leaf's sum."""
+    g, v = n.geom, n.geom["var"]
+    nb = W if n.batched else 1
+    X = nodes[g["X"]]
+    Y = nodes[g["Y"]] if g["Y"] >= 0 else None
+    out = []
+    if v["kind"] == "gemm":
+        ops = []
+        for key, op, want in (("perm_x", X, v["want_x"]), ("perm_y", Y, v["want_y"])):
+            stride = (1 << op.rank) if (n.batched and op.batched) else 0
+            if v[key]:
+                dst = abase + scratch[key][0]
+                out_pos = [0] * op.rank
+                for i, var in enumerate(want):
+                    out_pos[op.off[var].bit_length() - 1] = i
+                pd, grid, lds, pvar = schedule.perm_desc(op.ptr, dst, op.rank, out_pos,
+                                                         W if (n.batched and op.batched) else 1, 1 << op.rank, esize)
+                out.append(("permute", _lib.TO_OP_PERMUTE, pvar, lds, pd, grid))
+                ops.append((dst, stride))
+            else:
+                ops.append((op.ptr, stride))
+        gd = _lib.GemmDesc()
+        h = v["hlog"]
+        gd.a, gd.b, gd.c = ops[0][0], ops[1][0], n.ptr
+        gd.mlog, gd.nlog, gd.klog = g["fx"], g["fy"], g["s"]
+        gd.hlog = h
+        gd.ldcm, gd.ldcn = 1 << g["shf"], 1 << g["shy"]
+        if scaled:
+            gd.as_, gd.bs, gd.cs = recp(X), recp(Y), recp(n)
+            gd.asb = X.rec_stride if n.batched else 0
+            gd.bsb = Y.rec_stride if n.batched else 0
+        gd.block0, gd.nblocks = 0, v["nblocks"]
+        # batch items are (slice, kept shared variables); an operand without slices would
+        # repeat its 2^h items per slice, which one batch stride cannot say (see ``choose``)
+        gd.ab = 1 << (g["fx"] + g["s"]) if (ops[0][1] or h) else 0
+        gd.bb = 1 << (g["fy"] + g["s"]) if (ops[1][1] or h) else 0
+        gd.cb = 1 << (g["fx"] + g["fy"])
+        gd.nbatch = nb << h
+        out.append(("gemm", _lib.TO_OP_GEMM, v["tile"], 0, gd, v["nblocks"]))
+        return out
+    d = FoldDesc()
+    yptr, yrec, ystride, yrecs = one[0], one[1], 0, 0
+    if Y is not None:
+        yptr, yrec = Y.ptr, recp(Y)
+        ystride = Y.bstride if n.batched else 0
+        yrecs = Y.rec_stride if n.batched else 0
+    partial = abase + scratch["partial"][0] if v["lsplit"] else 0
+    d.ptrs = (X.ptr, yptr, n.ptr)
+    d.strides = (X.bstride if n.batched else 0, ystride, n.bstride)
+    d.recs = (recp(X), yrec, recp(n)) if scaled else (0, 0, 0)
+    d.rec_strides = (X.rec_stride if n.batched else 0, yrecs)
+    d.partial = partial
+    d.nbatch, d.block0, d.nblocks, d.roles = nb, 0, v["nblocks"], v["roles"]
+    yoff = Y.off if Y is not None else {}
+    fill = [0] * (_lib.FOLD_BITS - len(v["bits"]))
+    d.bits = [X.off.get(b, 0) for b in v["bits"]] + fill + [yoff.get(b, 0) for b in v["bits"]] + fill \
+        + [n.off.get(b, 0) for b in v["bits"]] + fill
+    out.append(("fold", _lib.TO_OP_FOLD, v["variant"], 0, d, v["nblocks"]))
+    if v["lsplit"]:
+        f = _lib.JoinDesc()
+        f.c, f.cb, f.partial, f.nsplit = n.ptr, n.bstride, partial, v["nsplit"]
+        if scaled:
+            f.xs, f.ys, f.cs = d.recs
+            f.xsb, f.ysb = d.rec_strides
+        f.fx, f.nbatch = n.rank, nb
+        wide = v["nsplit"] >= 32
+        f.nblocks = int(min(v["nout"] if wide else -(-v["nout"] // 256), schedule.MAX_STREAM_BLOCKS))
+        out.append(("finish", _lib.TO_OP_JOIN_FINISH, 1 if wide else 0, 0, f, f.nblocks))
+    return out
+
+
+def join_traffic(n, nodes, W, esize):
+    """Algorithmic (bytes, flops) of one folded join."""
+    nb = W if n.batched else 1
+    total = (1 << n.rank) * nb
+    held = set(n.ksum) | set(n.order)
+    for c in (n.left, n.right):
+        if c >= 0:
+            total += (1 << len(nodes[c].order)) * (nb if nodes[c].batched else 1)
+    return total * esize, 2 * nb << len(held)
+
+
+def block_cost(st):
+    if isinstance(st, FoldDesc):
+        lo, lk, ntile, nloop, lsplit, nreg = st.roles
+        return (1 << (nloop + nreg)) * max(1, (st.nbatch << (ntile + lsplit)) // max(1, st.nblocks))
+    return schedule.block_cost(st)
+
+
+def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, group_levels=True):
+    """Build a ``schedule.Program`` of a folded plan (``folded``: what ``analyse`` returned)
+    for W slices."""
+    nodes, missing = folded
+    esize = 8 if entry_type == _lib.TO_F64 else 4
+    scaled = entry_type == _lib.TO_F32S
+    prog = schedule.Program()
+    prog.nbatch, prog.nodes = W, nodes
+    choose_all(nodes, W, esize)
+    order = choose_order(nodes, W, esize)[0] if group_levels else "post"
+    peak, scratch = plan_memory(nodes, W, esize, order)
+    prog.arena_bytes, prog.order = peak, order
+
+    image = schedule.leaf_image(nodes, tables, num_groups, scaled, np.float64 if esize == 8 else np.float32)
+    mant, exp = image.factor
+    prog.leaf_factor = (mant, exp + missing)  # a variable no leaf holds counts twice
+    one = len(image.host)  # a stored 1.0, after the tables
+    image.host = np.concatenate([image.host, np.ones(1, image.host.dtype)])
+
+    # scale records: [constant leaves, the constant one][constant joins][wave tensors]
+    nrec, rec_init = 0, []
+    if scaled:
+        for n in nodes:
+            if n.is_leaf and not n.batched:
+                n.rec, n.rec_stride = nrec, 0
+                rec_init.append((nrec, image.exp0[n.tensor]))
+                nrec += 1
+        one_rec = nrec
+        rec_init.append((nrec, 0))
+        nrec += 1
+        pro_rec0 = nrec
+        for n in nodes:
+            if not n.is_leaf and not n.batched:
+                n.rec, n.rec_stride = nrec, 0
+                nrec += 1
+        wave_rec0 = nrec
+        for n in nodes:
+            if n.batched:
+                n.rec, n.rec_stride = nrec, 1
+                nrec += W
+        prog.rec_ranges = (pro_rec0, wave_rec0, nrec)
+
+    prog.table = device_alloc(image.host.nbytes)
+    prog.coef = device_alloc(image.coef_host.nbytes)
+    prog.arena = device_alloc(max(ALIGN, peak))
+    prog.recs = device_alloc(max(1, nrec) * 16)
+    prog.params = device_alloc(4 * 8)
+    prog.accum = device_alloc(32)
+    prog.table_host, prog.coef_host, prog.rec_init = image.host, image.coef_host, rec_init
+    tbase, abase, rbase = prog.table.data_ptr(), prog.arena.data_ptr(), prog.recs.data_ptr()
+    wave_params = prog.params.data_ptr()
+    one_at = (tbase + one * esize, rbase + one_rec * 16 if scaled else 0)
+    for n in nodes:
+        if n.is_leaf and not n.batched:
+            n.ptr, n.bstride = tbase + image.off[n.tensor] * esize, 0
+        else:
+            n.ptr = abase + n.buf[0]
+            n.bstride = (1 << n.rank) if n.batched else 0
+
+    def recp(n):
+        return rbase + n.rec * 16 if scaled else 0
+
+    blob = bytearray()
+
+    def put(structs):
+        nonlocal blob
+        start = (len(blob) + ALIGN - 1) // ALIGN * ALIGN
+        blob += b"\0" * (start - len(blob))
+        for st in structs:
+            blob += bytes(st)
+        return start
+
+    prog.build = []
+    if image.builds:
+        bdescs, block0 = [], 0
+        for t, v0, v1 in image.builds:
+            bd = tables[t].spec.desc(tbase + image.off[t] * esize, v0, v1)
+            bd.block0 = block0
+            block0 += bd.nblocks
+            bdescs.append(bd)
+        prog.build.append((Launch(op=_lib.TO_OP_LEAF_BUILD, count=len(bdescs), grid=block0), put(bdescs)))
+
+    def group_launches(group, phase):
+        """The joins of one group as one launch per kernel variant; permutes before products,
+        split sums before their finishing."""
+        keyed = {}
+        for i in group:
+            n = nodes[i]
+            for kind, op, variant, lds, st, nblk in join_records(n, nodes, W, esize, scaled, abase,
+                                                                 scratch.get(i, {}), recp, one_at):
+                if kind == "permute":
+                    work = (2 * esize * (int(st.nbatch) << int(st.rank)), 0)
+                elif kind in ("fold", "gemm"):
+                    work = join_traffic(n, nodes, W, esize)
+                else:
+                    work = (0, 0)
+                keyed.setdefault((schedule.KIND_ORDER[kind], op, variant), []).append((kind, st, nblk, lds, i, work))
+        for key in sorted(keyed):
+            grp = sorted(keyed[key], key=lambda r: -block_cost(r[1]))
+            block0, lds, wb, wf = 0, 0, 0, 0
+            for kind, st, nblk, l, i, work in grp:
+                st.block0 = block0
+                block0 += nblk
+                lds = max(lds, l)
+                wb += work[0]
+                wf += work[1]
+            off = put([r[1] for r in grp])
+            phase.append((grp[0][0], Launch(op=key[1], variant=key[2], count=len(grp), grid=block0, lds=lds), off,
+                          grp[0][4] if len(grp) == 1 else None, (wb, wf)))
+
+    def phase_groups(batched):
+        if order == "level":
+            return join_levels(nodes, batched)
+        return [[n.idx] for n in nodes if not n.is_leaf and n.batched == batched]
+
+    def clear(a, b):
+        return ("clear", Launch(op=_lib.TO_OP_SCALE_CLEAR, grid=max(1, min(1024, -(-(b - a) // 256))),
+                                aux0=rbase + a * 16, iaux0=b - a), None, None, (0, 0))
+
+    pro, wave = [], []
+    if scaled and prog.rec_ranges[1] > prog.rec_ranges[0]:
+        pro.append(clear(*prog.rec_ranges[:2]))
+    for grp in phase_groups(False):
+        group_launches(grp, pro)
+    root = nodes[-1]
+    prog.root_const = not root.batched
+    if scaled and prog.rec_ranges[2] > prog.rec_ranges[1]:
+        wave.append(clear(*prog.rec_ranges[1:]))
+    leaf_descs, block0 = [], 0
+    for n in nodes:
+        if n.is_leaf and n.batched:
+            ld = LeafDesc(src=tbase + image.off[n.tensor] * esize, dst=n.ptr,
+                          coef=prog.coef.data_ptr() + image.coef_off[n.tensor] * 8, rec=recp(n),
+                          exp0=image.exp0.get(n.tensor, 0), rank=n.rank, ngroups=num_groups, nbatch=W, block0=block0,
+                          nblocks=int(min(1024, -(-(W << n.rank) // 256))))
+            block0 += ld.nblocks
+            leaf_descs.append(ld)
+    if leaf_descs:
+        wave.append(("leaf", Launch(op=_lib.TO_OP_LEAF_GATHER, count=len(leaf_descs), grid=block0, aux3=wave_params),
+                     put(leaf_descs), None, (sum(esize * (W << ld.rank) for ld in leaf_descs), 0)))
+    for grp in phase_groups(True):
+        group_launches(grp, wave)
+    root_launch = Launch(op=_lib.TO_OP_ROOT_REDUCE, grid=1, aux0=root.ptr, aux1=recp(root),
+                         aux2=prog.accum.data_ptr(), aux3=wave_params + (16 if prog.root_const else 0),
+                         iaux0=1 if prog.root_const else W)
+    (pro if prog.root_const else wave).append(("root", root_launch, None, None, (0, 0)))
+    if not prog.root_const:
+        wave.append(("advance", Launch(op=_lib.TO_OP_WAVE_ADVANCE, grid=1, aux3=wave_params, iaux0=W), None, None,
+                     (0, 0)))
+
+    prog.blob_host = np.frombuffer(bytes(blob) or b"\0", dtype=np.uint8).copy()
+    prog.blob = device_alloc(prog.blob_host.nbytes)
+    bbase = prog.blob.data_ptr()
+    for L, off in prog.build:
+        L.descs = bbase + off
+    prog.build = [L for L, _ in prog.build]
+    prog.prologue_info, prog.wave_info, prog.prologue_work, prog.wave_work = [], [], [], []
+    for lst, out, info, work in ((pro, prog.prologue, prog.prologue_info, prog.prologue_work),
+                                 (wave, prog.wave, prog.wave_info, prog.wave_work)):
+        for kind, L, off, nidx, w in lst:
+            if off is not None:
+                L.descs = bbase + off
+            out.append(L)
+            info.append((kind, nidx))
+            work.append(w)
+    joins = [n for n in nodes if not n.is_leaf]
+    prog.stats = dict(
+        nodes=len(nodes), joins=len(joins), batched_joins=sum(1 for n in joins if n.batched),
+        splitk=sum(1 for n in joins if n.geom["var"].get("lsplit")),
+        gemm=sum(1 for n in joins if n.geom["var"]["kind"] == "gemm"),
+        arena_bytes=peak, table_bytes=int(image.host.nbytes),
+        # leaves described for the device (a vector of ones among them needs no table)
+        device_built_leaves=sum(1 for t in tables.values() if t.spec is not None),
+        launches_prologue=len(prog.prologue), launches_wave=len(prog.wave))
+    return prog

@@ -26,7 +26,7 @@ import math
 
 import numpy as np
 
-from . import _lib, schedule
+from . import _lib, fold, schedule
 from .api import BaseTensorAPI, OutOfMemoryError
 from .tree import TreeContext
 
@@ -214,6 +214,13 @@ class BatchExecutable:
         self._graphs = []
 
 
+def copy_weights(tensor):
+    """(w(not x), w(x), whether it has axes) of a COPY tensor, else None."""
+    from .network import VariableTensor
+
+    return tensor.weights + (tensor.rank > 0,) if isinstance(tensor, VariableTensor) else None
+
+
 def leaf_spec_table(tensor, lookup, ngroups):
     """The LeafTable of an OR or variable leaf whose table the device writes, with its axes
     reordered and its row lookup exactly as ``SliceSequence.reordered_tensor`` gives them
@@ -236,7 +243,7 @@ def leaf_spec_table(tensor, lookup, ngroups):
         coef[lookup[i]] += offset
         offset *= 2
     spec = schedule.LeafSpec(kind, rank, sliced + unsliced, **kw)
-    return schedule.LeafTable(None, coef, len(unsliced), spec)
+    return schedule.LeafTable(None, coef, len(unsliced), spec, copy=copy_weights(tensor))
 
 
 class HipAPI(BaseTensorAPI):
@@ -349,6 +356,20 @@ class HipAPI(BaseTensorAPI):
 
     # -- compiled execution ---------------------------------------------------------
 
+    def choose_folded_batch(self, folded, tree, tables, total_slices):
+        """Largest slice batch W of a folded plan whose arena fits the device budget.  A plan
+        is refused where its tensors, one axis per edge, would not fit one slice at a time:
+        whether a caller has to slice more does not depend on how the plan is executed."""
+        budget = self._budget()
+        nodes, _ = folded
+        fixed = sum(t.size for t in tables.values()) * self._esize
+        if fixed + schedule.peak_bound(tree, self._esize) > budget:
+            self.choose_batch(schedule.analyse(tree, tables, self._regroup), tables, 1)
+        W = max(1, min(self._max_batch, total_slices))
+        while W > 1 and fold.peak_bytes(nodes, W, self._esize) + fixed > budget:
+            W = max(1, W // 2)
+        return W
+
     def choose_batch(self, nodes, tables, total_slices):
         """Largest slice batch W (<= max_batch) whose arena fits the device budget; raises
         OutOfMemoryError when even one slice does not fit."""
@@ -366,6 +387,11 @@ class HipAPI(BaseTensorAPI):
     def _compile(self, tree, tables, num_groups, total_slices, group_levels=True):
         """Compile and upload a plan; returns an ``Executable``.  ``group_levels=False``
         keeps one launch per join (per-join timing)."""
+        folded = fold.analyse(tree, tables, self._esize, self._regroup) if fold.has_copies(tables) else None
+        if folded is not None:
+            W = self.choose_folded_batch(folded, tree, tables, total_slices)
+            prog = fold.compile_program(folded, tables, num_groups, self._entry_type, W, self._alloc, group_levels)
+            return self._resident(prog, total_slices)
         nodes = schedule.analyse(tree, tables, self._regroup)
         W = self.choose_batch(nodes, tables, total_slices)
         if self._autotune:
@@ -375,6 +401,10 @@ class HipAPI(BaseTensorAPI):
                 autotune.save(schedule.TUNED)
         prog = schedule.compile_program(tree, tables, num_groups, self._entry_type, W, self._alloc,
                                         regroup=self._regroup, group_levels=group_levels)
+        return self._resident(prog, total_slices)
+
+    def _resident(self, prog, total_slices):
+        """Upload a compiled plan; returns its ``Executable``."""
         self._upload(prog.table, prog.table_host.tobytes())
         self._upload(prog.coef, prog.coef_host.tobytes())
         self._upload(prog.blob, prog.blob_host.tobytes())
@@ -422,7 +452,8 @@ class HipAPI(BaseTensorAPI):
                     continue
                 reordered, lookup, shape = seq.reordered_tensor(self)
                 reordered = np.asarray(reordered, dtype=np.float64)
-                tables[t] = schedule.LeafTable(reordered.reshape(reordered.shape[0], -1), lookup, len(shape))
+                tables[t] = schedule.LeafTable(reordered.reshape(reordered.shape[0], -1), lookup, len(shape),
+                                               copy=copy_weights(network[t]))
         if num_slice_limit is not None:
             total = min(total, int(num_slice_limit))
         return total, tree, tables, len(groups)

@@ -28,7 +28,7 @@ from ._lib import JoinDesc, LeafDesc, Launch
 ALIGN = 256
 STREAM_MAX_S = 12
 # order of a join's launches inside a group: operand permutes, products, split-K finishing
-KIND_ORDER = {"permute": 0, "stream": 1, "splitk": 1, "gemm": 1, "finish": 2}
+KIND_ORDER = {"permute": 0, "stream": 1, "splitk": 1, "fold": 1, "gemm": 1, "finish": 2}
 LDS_LIMIT = 64 * 1024
 MAX_STREAM_BLOCKS = 4096
 # one-wave streamed joins (many-instance batch): at most this many products per lane
@@ -481,11 +481,13 @@ class LeafSpec:
 class LeafTable:
     """Per-tensor slice rows: ``rows`` (float64 [nrows, 2^rank]) -- or, for a leaf written
     on the device, its ``spec`` -- and ``coef`` (one integer per slice group:
-    row = sum_g coef[g] * assignment[g])."""
+    row = sum_g coef[g] * assignment[g]).  ``copy`` is (w(not x), w(x), whether the whole
+    tensor has axes) of a COPY tensor, else None."""
 
-    __slots__ = ("rows", "coef", "rank", "spec", "nrows")
+    __slots__ = ("rows", "coef", "rank", "spec", "nrows", "copy")
 
-    def __init__(self, rows, coef, rank, spec=None):
+    def __init__(self, rows, coef, rank, spec=None, copy=None):
+        self.copy = copy
         self.coef = [int(c) for c in coef]
         self.rank = rank
         self.spec = spec
@@ -755,6 +757,18 @@ def analyse(tree, tables, regroup=True):
     return nodes
 
 
+def peak_bound(tree, esize):
+    """An upper bound of the arena peak of one slice: every tensor and every join's scratch
+    (permuted operands, partial sums) at once."""
+    total = 0
+    for t in tree.iterate_postorder():
+        # the tensor itself and, as an operand, its permuted copy
+        total += 2 * max(ALIGN, esize << len(t.free_edges))
+        if not t.is_leaf:  # partial sums: at most 4096, or one per output
+            total += 8 * max(4096, 1 << len(t.free_edges))
+    return total
+
+
 def peak_bytes(nodes, tables, W, entry_type):
     esize = 8 if entry_type == _lib.TO_F64 else 4
     for n in nodes:
@@ -870,6 +884,56 @@ def block_cost(st):
     return 0
 
 
+class LeafImage:
+    """The leaf tables of a compiled plan in one buffer (``leaf_image``)."""
+
+    __slots__ = ("off", "exp0", "factor", "builds", "host", "coef_host", "coef_off")
+
+
+def leaf_image(nodes, tables, num_groups, scaled, fdtype):
+    """Place the tables of every leaf tensor of ``nodes`` in one buffer (``host``; offsets in
+    entries, ``off``), with the slice-row coefficients (``coef_host``, ``coef_off``), the
+    tables that the device writes (``builds``: tensor, val0, val1), and, in the scaled
+    executor, each tensor's exponent and the product of the leaf factors."""
+    im = LeafImage()
+    esize = np.dtype(fdtype).itemsize
+    leaf_ids = sorted({n.tensor for n in nodes if n.is_leaf})
+    im.off, im.exp0, im.builds, im.coef_off = {}, {}, [], {}
+    chunks, factor_of, off = [], {}, 0
+    for t in leaf_ids:
+        tab = tables[t]
+        if tab.spec is not None:  # written on the device by the leaf build launch
+            v0, v1, F, e = tab.spec.stored(scaled)
+            im.builds.append((t, v0, v1))
+            size = tab.size
+        else:
+            rows = tab.rows
+            if scaled:
+                rows, F, e = leaf_encoding(rows)
+            arr = np.ascontiguousarray(rows, dtype=fdtype).ravel()
+            chunks.append((t, arr))
+            size = arr.size
+        if scaled:
+            im.exp0[t] = e
+            factor_of[t] = F
+        im.off[t] = off
+        off += (size * esize + ALIGN - 1) // ALIGN * ALIGN // esize
+    im.host = np.zeros(max(off, 1), dtype=fdtype)
+    for t, arr in chunks:
+        im.host[im.off[t]:im.off[t] + arr.size] = arr
+    # one factor per leaf *occurrence*: a tree may hold one tensor at several leaves (the
+    # line planner joins a rank-0 tensor at its first bag and again at the top,
+    # line_graph_method.py:16-35 and contraction_tree.pyx:302-310), and each occurrence
+    # multiplies the count by that tensor's values
+    im.factor = factor_product([factor_of[n.tensor] for n in nodes if n.is_leaf] if scaled else [])
+    im.coef_host = np.zeros(max(1, len(leaf_ids) * max(1, num_groups)), dtype=np.int64)
+    for i, t in enumerate(leaf_ids):
+        c = tables[t].coef
+        im.coef_off[t] = i * max(1, num_groups)
+        im.coef_host[im.coef_off[t]:im.coef_off[t] + len(c)] = c
+    return im
+
+
 def compile_program(tree, tables, num_groups, entry_type, W, device_alloc, regroup=True, group_levels=True):
     """Build a Program for batch size W.
 
@@ -899,41 +963,10 @@ def compile_program(tree, tables, num_groups, entry_type, W, device_alloc, regro
 
     # ---- leaf tables (host) -> one device buffer; the scaled executor's leaf factors
     # multiply the count (prog.leaf_factor, mantissa and exponent)
-    leaf_ids = sorted({n.tensor for n in nodes if n.is_leaf})
-    table_off, chunks, exp0, factor_of, builds = {}, [], {}, {}, []
-    off = 0
-    for t in leaf_ids:
-        tab = tables[t]
-        if tab.spec is not None:  # written on the device by the leaf build launch
-            v0, v1, F, e = tab.spec.stored(scaled)
-            builds.append((t, v0, v1))
-            size = tab.size
-        else:
-            rows = tab.rows
-            if scaled:
-                rows, F, e = leaf_encoding(rows)
-            arr = np.ascontiguousarray(rows, dtype=fdtype).ravel()
-            chunks.append((t, arr))
-            size = arr.size
-        if scaled:
-            exp0[t] = e
-            factor_of[t] = F
-        table_off[t] = off
-        off += (size * esize + ALIGN - 1) // ALIGN * ALIGN // esize
-    table_host = np.zeros(max(off, 1), dtype=fdtype)
-    for t, arr in chunks:
-        table_host[table_off[t]:table_off[t] + arr.size] = arr
-    # one factor per leaf *occurrence*: a tree may hold one tensor at several leaves (the
-    # line planner joins a rank-0 tensor at its first bag and again at the top,
-    # line_graph_method.py:16-35 and contraction_tree.pyx:302-310), and each occurrence
-    # multiplies the count by that tensor's values
-    prog.leaf_factor = factor_product([factor_of[n.tensor] for n in nodes if n.is_leaf] if scaled else [])
-    coef_host = np.zeros(max(1, len(leaf_ids) * max(1, num_groups)), dtype=np.int64)
-    coef_off = {}
-    for i, t in enumerate(leaf_ids):
-        c = tables[t].coef
-        coef_off[t] = i * max(1, num_groups)
-        coef_host[coef_off[t]:coef_off[t] + len(c)] = c
+    image = leaf_image(nodes, tables, num_groups, scaled, fdtype)
+    table_off, exp0, builds = image.off, image.exp0, image.builds
+    table_host, coef_host, coef_off = image.host, image.coef_host, image.coef_off
+    prog.leaf_factor = image.factor
 
     # ---- scale records: [constant leaves][constant joins][wave tensors]
     nrec = 0

@@ -1,0 +1,395 @@
+"""Folded plans (COPY tensors as index identities): the compiled records, executed by a numpy
+emulator of to_fold_desc, reproduce the oracle over plans, slicings, entry types and batch
+sizes; the kernels match float64 sums over every form, on the GPU."""
+
+import ctypes
+import json
+import math
+import os
+import types
+
+import numpy as np
+import pytest
+from fixtures import plan_fixture_paths
+
+import emulator
+from oracle import numpy_oracle
+from tensororder_amd import _lib, fold, hip_api, network, plan_io, planners, schedule
+from tensororder_amd.formula import parse_dimacs_text
+from tensororder_amd.instances import random_3cnf, vertex_cover_cnf
+from tensororder_amd.plan import ALL_SLICERS
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+SMALL = [f for f in plan_fixture_paths() if json.load(open(f))["meta"]["maxrank"] <= 16]
+
+
+def _say(*args):
+    print(*args, flush=True)
+
+
+def _spread(entries, lo, n):
+    """What each value of bits [lo, lo + n) of a descriptor adds to an offset."""
+    out = np.zeros(1, dtype=np.int64)
+    for i in range(lo, lo + n):
+        out = np.concatenate([out, out + int(entries[i])])
+    return out
+
+
+class FoldEmulator(emulator.Emulator):
+    def __init__(self, heap, entry_type):
+        super().__init__(heap, entry_type)
+        self.forms = set()
+
+    def op_14(self, L):
+        size = ctypes.sizeof(_lib.FoldDesc)
+        for i in range(L.count):
+            d = self.heap.read_struct(_lib.FoldDesc, L.descs + i * size)
+            vec = L.variant & _lib.TO_FOLD_VEC
+            self.forms.add(L.variant)
+            if vec:
+                assert d.nreg == (L.variant & 15) and d.lo == 10 and d.lk == 0 and d.lsplit == 0
+                assert list(d.bx[:2]) == [1, 2] and list(d.bc[:2]) == [1, 2]
+                ym = {(0, 0): 0, (1, 2): 1}.get(tuple(d.by[:2]), 2)
+                assert ym == (L.variant >> 4) & 15
+                # 4-element alignment of everything the 16-byte form loads or stores at once
+                for ptr, stride, arr, used in ((d.x, d.xb, d.bx, True), (d.c, d.cb, d.bc, True),
+                                               (d.y, d.yb, d.by, ym == 1)):
+                    if used:
+                        assert ptr % (4 * self.dt().itemsize) == 0 and stride % 4 == 0
+                        assert all(int(e) % 4 == 0 for e in list(arr)[2:])
+                thr, tile0 = (0, 10), 10
+            else:
+                assert d.nreg == 0 and d.lo + d.lk <= 8 and all(int(e) == 0 for e in list(d.bc)[d.lo:8])
+                thr, tile0 = (0, d.lo), 8
+            k0 = tile0 + d.ntile
+            r0 = k0 + d.nloop + d.lsplit
+            assert r0 + d.nreg <= _lib.FOLD_BITS
+            offs = []
+            for arr in (d.bx, d.by, d.bc):
+                o = (_spread(arr, *thr)[None, None, :] + _spread(arr, tile0, d.ntile)[None, :, None]
+                     + _spread(arr, r0, d.nreg)[:, None, None]).ravel()
+                k = (_spread(arr, d.lo, 0 if vec else d.lk)[None, :]
+                     + _spread(arr, k0, d.nloop + d.lsplit)[:, None]).ravel()
+                offs.append((o, k))
+            co = offs[2][0]
+            assert np.array_equal(np.sort(co), np.arange(co.size))  # every output once
+            assert not np.any(offs[2][1])
+            esz = self.dt().itemsize
+            for b in range(d.nbatch):
+                xo = offs[0][0][:, None] + offs[0][1][None, :]
+                yo = offs[1][0][:, None] + offs[1][1][None, :]
+                X = self.heap.view(d.x + b * d.xb * esz, self.dt, int(xo.max()) + 1).astype(np.float64)
+                Y = self.heap.view(d.y + b * d.yb * esz, self.dt, int(yo.max()) + 1).astype(np.float64)
+                e = 0
+                f = 1.0
+                if self.scaled:
+                    for rec in (self.get_rec(d.xs, b * d.xsb), self.get_rec(d.ys, b * d.ysb)):
+                        e += rec[0] + emulator._scale_exp(rec[1])
+                        f *= 2.0 ** -emulator._scale_exp(rec[1])
+                prod = X[xo] * Y[yo]
+                if d.lsplit:
+                    S = 1 << d.lsplit
+                    P = self.heap.view(d.partial, np.float64, (d.nbatch * co.size) << d.lsplit)
+                    # shared index = (split, loop, thread bits)
+                    parts = prod.reshape(co.size, S, -1).sum(axis=2) * f
+                    for sp in range(S):
+                        P[((b * co.size + co) << d.lsplit) | sp] = parts[:, sp]
+                    self.gemm_partials.add(d.partial)
+                    continue
+                val = (prod.sum(axis=1) * f).astype(self.dt)
+                self.heap.view(d.c + b * d.cb * esz, self.dt, co.size)[co] = val
+                if self.scaled:
+                    m = np.float32(np.max(np.abs(val)))
+                    self.set_rec(d.cs, b, exp=e, maxbits=int(m.view(np.uint32)))
+
+    def op_10(self, L):
+        # products whose batch items share scale records in groups of 2^hlog
+        for i in range(L.count):
+            d = self.heap.read_struct(_lib.GemmDesc, L.descs + i * ctypes.sizeof(_lib.GemmDesc))
+            M, N, K = 1 << d.mlog, 1 << d.nlog, 1 << d.klog
+            esz = self.dt().itemsize
+            cidx = np.arange(M)[:, None] * d.ldcm + np.arange(N)[None, :] * d.ldcn
+            for b in range(d.nbatch):
+                A = self.heap.view(d.a + b * d.ab * esz, self.dt, M * K).reshape(M, K).astype(np.float64)
+                B = self.heap.view(d.b + b * d.bb * esz, self.dt, N * K).reshape(N, K).astype(np.float64)
+                e, f, r = 0, 1.0, b >> d.hlog
+                if self.scaled:
+                    for rec in (self.get_rec(d.as_, r * d.asb), self.get_rec(d.bs, r * d.bsb)):
+                        e += rec[0] + emulator._scale_exp(rec[1])
+                        f *= 2.0 ** -emulator._scale_exp(rec[1])
+                Cm = ((A @ B.T) * f).astype(self.dt)
+                self.heap.view(d.c + b * d.cb * esz, self.dt, M * N)[cidx] = Cm
+                if self.scaled:
+                    m = np.float32(np.max(np.abs(Cm)))
+                    self.set_rec(d.cs, r, exp=e, maxbits=int(m.view(np.uint32)))
+
+
+class _Host:
+    """What ``HipAPI._plan_inputs`` needs of an API, without a device."""
+
+    def __init__(self, device_leaves=True):
+        self._device_leaves = device_leaves
+
+    def create_tensor(self, shape, default_value=None):
+        return np.empty(shape) if default_value is None else np.full(shape, default_value, dtype=np.float64)
+
+    reshape = staticmethod(np.reshape)
+
+    @staticmethod
+    def transpose(t, perm):
+        return np.transpose(t, axes=perm)
+
+
+def plan_inputs(plan, device_leaves=True):
+    return hip_api.HipAPI._plan_inputs(_Host(device_leaves), plan, None)
+
+
+def emulate(plan, et, W, device_leaves=True, group_levels=True, **kw):
+    total, tree, tables, G = plan_inputs(plan, device_leaves)
+    folded = fold.analyse(tree, tables, 8 if et == _lib.TO_F64 else 4, **kw)
+    heap = emulator.Heap()
+    prog = fold.compile_program(folded, tables, G, et, W, heap.alloc, group_levels)
+    for buf, data in ((prog.table, prog.table_host), (prog.coef, prog.coef_host), (prog.blob, prog.blob_host)):
+        heap.write(buf, data.tobytes())
+    if et == _lib.TO_F32S:
+        heap.write(prog.recs, schedule.rec_init_bytes(prog))
+    heap.write(prog.params, np.array([0, total, 0, 1], dtype=np.int64).tobytes())
+    heap.write(prog.accum, bytes(_lib.Accum()))
+    emu = FoldEmulator(heap, et)
+    emu.run(prog.build)
+    emu.run(prog.prologue)
+    if not prog.root_const:
+        for _ in range(-(-total // W)):
+            emu.run(prog.wave)
+    acc = heap.read_struct(_lib.Accum, prog.accum.data_ptr())
+    fm, fe = prog.leaf_factor
+    return math.ldexp(acc.mant * fm, acc.exp + fe), prog, emu
+
+
+@pytest.mark.parametrize("path", SMALL, ids=[os.path.basename(p)[:-5] for p in SMALL])
+@pytest.mark.parametrize("et,tol", [(_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)])
+def test_fixture_folded(path, et, tol):
+    doc = json.load(open(path))
+    plan = plan_io.plan_from_dict(doc)
+    want = numpy_oracle.contract_sliced(doc)
+    total = 1 << len(plan.groups_to_slice)
+    for W in sorted({1, 3, total}):
+        got, prog, _ = emulate(plan, et, W)
+        assert got == pytest.approx(want, rel=tol)
+    got, _, _ = emulate(plan, et, total, device_leaves=False, group_levels=False, regroup=False)
+    assert got == pytest.approx(want, rel=tol)
+
+
+def _formula_plan(kind, n, seed, slices):
+    text = vertex_cover_cnf(n, seed, True) if kind == "vc" else random_3cnf(n, int(1.9 * n), seed, True)
+    net = network.cnf_count(parse_dimacs_text(text, "cachet"))
+    plan = planners.best_plan(net, "line" if kind == "vc" else "factor", solver=None, seed=seed)
+    ALL_SLICERS["greedy_mem"].slice_until(plan, slices=slices)
+    return plan
+
+
+@pytest.mark.parametrize("kind,n,slices", [("vc", 14, 0), ("vc", 26, 2), ("cnf", 12, 0), ("cnf", 18, 3), ("cnf", 25, 1)])
+@pytest.mark.parametrize("et,tol", [(_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)])
+def test_random_formulas_folded(kind, n, slices, et, tol):
+    for seed in range(3):
+        plan = _formula_plan(kind, n, seed, slices)
+        want = numpy_oracle.contract_sliced(plan_io.plan_to_dict(plan))
+        got, prog, _ = emulate(plan, et, 1 << slices)
+        assert got == pytest.approx(want, rel=tol)
+
+
+def test_unused_variables_and_repeated_leaves_folded():
+    from test_emulator import unused_variable_plans
+
+    for name, plan in unused_variable_plans():
+        want = numpy_oracle.contract_sliced(plan_io.plan_to_dict(plan))
+        for et, tol in ((_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)):
+            assert emulate(plan, et, 1)[0] == pytest.approx(want, rel=tol), name
+
+
+def test_early_contracted_plan_folded():
+    from test_emulator import early_contracted_plan
+
+    plan, want = early_contracted_plan(4)
+    for et, tol in ((_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)):
+        assert emulate(plan, et, 8)[0] == pytest.approx(want, rel=tol)
+
+
+def test_folded_tensors_hold_each_variable_once():
+    # rank by rank: a folded tensor never holds more variables than the walk's tensor has
+    # axes, and the large formula's plan shrinks as its COPY structure says
+    doc = json.load(open(os.path.join(HERE, "golden", "cnf70_factor_s12.json")))
+    plan = plan_io.plan_from_dict(doc)
+    _, tree, tables, _ = plan_inputs(plan)
+    nodes, missing = fold.analyse(tree, tables, 4)
+    assert missing == 0
+    assert max(n.rank for n in nodes) <= 22 < doc["meta"]["maxrank"]
+    assert sum(fold.join_traffic(n, nodes, 1, 4)[1] for n in nodes if not n.is_leaf) < 2 ** 28
+
+
+# (X-only, Y-only, kept shared, summed shared, X-only summed, slices, X sliced, Y sliced,
+#  shuffled): the general form below and above 256 outputs, with shared thread bits and with
+#  blocks sharing a sum; the 16-byte form with 0..3 (and more) register bits, Y holding none,
+#  both or one of the lowest two variables; odd slice counts
+JOINS = [(0, 0, 0, 0, 0, 1, 1, 1, 0), (2, 1, 1, 1, 0, 3, 1, 1, 1), (3, 2, 2, 2, 1, 5, 1, 0, 1), (0, 0, 3, 9, 0, 2, 1, 1, 0),
+         (0, 0, 0, 16, 0, 1, 1, 1, 0), (1, 0, 1, 14, 0, 3, 1, 1, 1), (4, 5, 1, 6, 0, 1, 1, 1, 1), (10, 0, 0, 0, 0, 1, 1, 1, 0),
+         (11, 0, 2, 1, 0, 2, 1, 0, 0), (9, 1, 4, 2, 0, 3, 1, 1, 0), (10, 2, 2, 3, 0, 1, 1, 1, 0), (8, 3, 3, 1, 0, 7, 1, 0, 0),
+         (9, 5, 3, 2, 0, 2, 1, 1, 0), (0, 0, 13, 1, 0, 3, 1, 1, 0), (1, 0, 12, 2, 0, 2, 1, 1, 0), (12, 1, 1, 4, 0, 3, 1, 1, 0)]
+
+
+def _join(case, et, alloc, write, rng):
+    """One folded join compiled by ``fold.choose``: (records, node list, data, result)."""
+    xo, yo, kept, s, xs, W, xw, yw, shuffled = case
+    esize = 8 if et == _lib.TO_F64 else 4
+    dt = np.float64 if esize == 8 else np.float32
+    names = ["x%d" % i for i in range(xo)] + ["h%d" % i for i in range(kept)]
+    if kept and not shuffled and rng.integers(2):  # kept variables lowest: Y's lowest too
+        names = names[xo:] + names[:xo]
+    xv = names + ["k%d" % i for i in range(s)] + ["q%d" % i for i in range(xs)]
+    yv = [v for v in xv if v[0] in "hk"] + ["y%d" % i for i in range(yo)]
+    out = names + ["y%d" % i for i in range(yo)]
+    if shuffled:
+        for v in (xv, yv, out):
+            rng.shuffle(v)
+    nodes = []
+    for i, (vs, batched) in enumerate(((xv, xw), (yv, yw), (out, xw or yw))):
+        n = fold.FNode(i)
+        n.is_leaf, n.batched, n.order = i < 2, bool(batched), list(vs)
+        n.order0, n.rank, n.left, n.right = n.order, len(vs), 0, 1
+        n.off = {v: 1 << j for j, v in enumerate(vs)}
+        nodes.append(n)
+    X, Y, C = nodes
+    C.ksum = set(xv + yv) - set(out)
+    fold.choose(C, nodes, W, esize)
+    data, recs = {}, {}
+    for n in (X, Y, C):
+        items = W if n.batched else 1
+        n.bstride = (1 << n.rank) if n.batched else 0
+        n.rec_stride = 1 if n.batched else 0
+        n.ptr = alloc(items * esize << n.rank)
+        recs[n.idx] = alloc(16 * items)
+        if n is not C:
+            data[n.idx] = rng.uniform(0.25, 1.0, (items, 1 << n.rank)).astype(dt)
+            write(n.ptr, data[n.idx].tobytes())
+            write(recs[n.idx], b"".join(
+                bytes(_lib.ScaleRec(exp=3 - b, maxbits=int(np.abs(data[n.idx][b]).max().astype(np.float32).view(np.uint32))))
+                for b in range(items)))
+        else:
+            write(recs[n.idx], bytes(16 * items))
+    v = C.geom["var"]
+    scratch = {"partial": (alloc(v["nout"] * v["nsplit"] * 8), 0)} if v.get("lsplit") else {}
+    records = fold.join_records(C, nodes, W, esize, esize == 4, 0, scratch, lambda n: recs[n.idx], (0, 0))
+    # float64 result, indexed by C's own bits
+    def off(n, vs):
+        o = np.zeros(1, dtype=np.int64)
+        for u in vs:
+            o = np.concatenate([o, o + n.off.get(u, 0)])
+        return o
+    ks = sorted(C.ksum)
+    ox, oy = (off(n, C.order)[:, None] + off(n, ks)[None, :] for n in (X, Y))
+    want = []
+    for b in range(W if C.batched else 1):
+        x, y = (data[n.idx][b if n.batched else 0].astype(np.float64) for n in (X, Y))
+        want.append((x[ox] * y[oy]).sum(axis=1) * 2.0 ** (sum(3 - (b if n.batched else 0) for n in (X, Y)) if esize == 4 else 0))
+    return records, nodes, recs, np.array(want)
+
+
+def _launches(records, alloc, write):
+    out = []
+    for kind, op, variant, lds, st, nblk in records:
+        st.block0 = 0
+        at = alloc(len(bytes(st)))
+        write(at, bytes(st))
+        out.append(_lib.Launch(op=op, variant=variant, count=1, grid=nblk, lds=lds, descs=at))
+    return out
+
+
+def _check(case, et, got, rec, want):
+    # products of floats are exact in the double sums: one rounding, at the store
+    dt = np.float64 if et == _lib.TO_F64 else np.float32
+    for b in range(want.shape[0]):
+        scale = 2.0 ** int(rec[b].exp) if et == _lib.TO_F32S else 1.0
+        np.testing.assert_allclose(got[b].astype(np.float64) * scale, want[b], rtol=1e-13 if dt == np.float64 else 1.2e-7)
+        if et == _lib.TO_F32S:
+            assert rec[b].maxbits == int(np.abs(got[b]).max().view(np.uint32))
+
+
+@pytest.mark.parametrize("et", [_lib.TO_F64, _lib.TO_F32S], ids=["f64", "f32s"])
+def test_every_form_emulated(et):
+    forms = set()
+    for i, case in enumerate(JOINS):
+        heap = emulator.Heap(1 << 27)
+        ptr = {}
+
+        def alloc(n):
+            b = heap.alloc(n)
+            ptr[b.data_ptr()] = b
+            return b.data_ptr()
+
+        def write(at, data):
+            heap.write(ptr[at], data)
+
+        records, nodes, recs, want = _join(case, et, alloc, write, np.random.default_rng(i))
+        emu = FoldEmulator(heap, et)
+        emu.run(_launches(records, alloc, write))
+        forms |= emu.forms
+        if any(r[0] == "finish" for r in records):
+            forms.add("split")
+        C = nodes[2]
+        items = want.shape[0]
+        got = heap.view(C.ptr, emu.dt, items << C.rank).reshape(items, -1)
+        _check(case, et, got, [heap.read_struct(_lib.ScaleRec, recs[2] + 16 * b) for b in range(items)], want)
+    assert {f & 15 for f in forms if f != "split" and f & _lib.TO_FOLD_VEC} == {0, 1, 2, 3}
+    assert {f >> 4 & 15 for f in forms if f != "split" and f & _lib.TO_FOLD_VEC} >= {0, 1}
+    assert "split" in forms and _lib.TO_FOLD_ANY in forms
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("et", [_lib.TO_F64, _lib.TO_F32S], ids=["f64", "f32s"])
+def test_every_form_on_the_device(et):
+    import torch
+
+    api = hip_api.HipAPI() if et == _lib.TO_F64 else hip_api.HipF32API()
+    for i, case in enumerate(JOINS):
+        _say("case folded join", et, case)
+        ptr = {}
+
+        def alloc(n):
+            t = torch.full((n,), 255, dtype=torch.uint8, device="cuda")  # NaN where nothing is written
+            ptr[t.data_ptr()] = t
+            return t.data_ptr()
+
+        def write(at, data):
+            ptr[at][:len(data)] = torch.frombuffer(bytearray(data), dtype=torch.uint8).cuda()
+
+        records, nodes, recs, want = _join(case, et, alloc, write, np.random.default_rng(i))
+        launches = _launches(records, alloc, write)
+        torch.cuda.synchronize()
+        api._run(launches)
+        api.synchronize()
+        items, C = want.shape[0], nodes[2]
+        dt = np.float64 if et == _lib.TO_F64 else np.float32
+        got = ptr[C.ptr].cpu().numpy().view(dt).reshape(items, -1)
+        raw = ptr[recs[2]].cpu().numpy().tobytes()
+        _check(case, et, got, [_lib.ScaleRec.from_buffer_copy(raw[16 * b:16 * b + 16]) for b in range(items)], want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("et,tol", [(_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)], ids=["f64", "f32s"])
+def test_folded_and_edge_walk_agree_on_the_device(et, tol):
+    # the folded executor against the walk over edges (tables without their COPY mark), on
+    # plans with products whose kept variables are batch items
+    api = hip_api.HipAPI() if et == _lib.TO_F64 else hip_api.HipF32API()
+    for kind, n, seed, slices in (("vc", 70, 2, 0), ("cnf", 34, 4, 2), ("cnf", 40, 1, 3)):
+        _say("case folded vs walk", kind, n, slices, et)
+        plan = _formula_plan(kind, n, seed, slices)
+        total, tree, tables, G = api._plan_inputs(plan, None)
+        exe = api._compile(tree, tables, G, total)
+        got = [exe.run().value for _ in range(3)]
+        exe.close()
+        for t in tables.values():
+            t.copy = None
+        exe = api._compile(tree, tables, G, total)
+        want = exe.run().value
+        exe.close()
+        assert got == pytest.approx([want] * 3, rel=tol)
