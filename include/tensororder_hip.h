@@ -90,6 +90,8 @@ extern "C" {
 #define TO_OP_FOLD 14 /* descs: to_fold_desc[count]; variant TO_FOLD_ANY: one output per thread,
                          any bit layout; else TO_FOLD_VEC | y mode << 4 | nreg: the 16-byte form,
                          every descriptor of the launch with that y mode and nreg */
+#define TO_OP_FOLD_TREE 15 /* descs: to_tree_desc[count]; iaux0: waves per block (1 to 16, as many
+                         as each program has streams); lds: the largest of their LDS needs */
 #define TO_OP_LEAF_BUILD 13  /* descs: to_leaf_build_desc[count]: leaf tables written from their
                                 compact descriptions (OR / variable leaves) */
 
@@ -246,6 +248,35 @@ typedef struct to_fold_desc {
     uint32_t bx[TO_FOLD_BITS], by[TO_FOLD_BITS], bc[TO_FOLD_BITS];
 } to_fold_desc;
 
+/* A program of small folded joins that one block runs start to end for one batch item: a
+ * connected part of the tree whose intermediate tensors fit LDS.  A join of a program is a
+ * product of up to 4 tensors, summed over the k bits.  Each wave of the block walks its own
+ * stream of ntask words, tasks[wave * ntask + i]: bits 0-15 the join, bits 16-22 its first
+ * chunk of 64 outputs-times-shares and bits 23-26 log2 of the step to the next one, bit 30:
+ * nothing to do, bit 31: all waves meet after this entry (in the same entries of every
+ * stream).  A join is TO_TREE_WORDS words, ops[join * TO_TREE_WORDS + i]:
+ *   0: lo | lk << 4 | nloop << 8 | nchunk << 12 (numbers of o bits and k bits on the lanes, of
+ *      k bits walked, of o bits of the chunk index; 6 + nloop + nchunk at most 16),
+ *      operands - 1 in bits 16-17, bits 20-24: operand 0-3, result lie in LDS, bits 25-29:
+ *      their global scale record advances with the batch item; 3 or 4 operands only with
+ *      nchunk == 0 and nloop <= 2
+ *   1 + 2 j, 2 + 2 j: address of operand j (result: j = 4), low word first, or its element
+ *      offset in the block's LDS tensors; 11 + j: its batch stride in elements (global);
+ *      16 + j: its scale record: an LDS slot for an LDS tensor, else an index into recs
+ *   32-47: what each bit adds to the result's offset, 64 + 16 j + i: to operand j's (as in
+ *      to_fold_desc): 6 lane bits (lo o bits, lk k bits, the rest 0), nchunk, nloop
+ *   128 + 64 j + l: the offset that the lane bits of lane l add to operand j's (result's).
+ * LDS holds nslots 8-byte records, then (16-byte aligned) the tensors. */
+#define TO_TREE_WORDS 448
+#define TO_TREE_IDLE 0x40000000
+#define TO_TREE_MEET 0x80000000
+typedef struct to_tree_desc {
+    uint64_t ops, tasks;       /* uint32 arrays in device memory */
+    uint64_t recs;             /* to_scale_rec* of the program's global tensors (TO_F32S) */
+    int32_t ntask, nslots;
+    int32_t block0, nblocks;   /* one block per batch item */
+} to_tree_desc;
+
 /* The root scalar of one instance of a batch: stored into its accumulator as
  * (mantissa, exponent), with the device clock at that moment in accum.pad. */
 typedef struct to_root_desc {
@@ -266,7 +297,7 @@ typedef struct to_launch {
     uint64_t descs; /* device pointer to the descriptor array */
     uint64_t aux0, aux1, aux2, aux3; /* per op; for the descriptor-table ops (LEAF_GATHER,
                                         JOIN_STREAM, JOIN_SPLITK, JOIN_FINISH, PERMUTE, GEMM,
-                                        FOLD, LEAF_BUILD) aux1 is 0 or a device int32[grid] map of
+                                        FOLD, FOLD_TREE, LEAF_BUILD) aux1 is 0 or a device int32[grid] map of
                                         each block to its descriptor (the last one whose
                                         block0 is at or below the block), read instead of a
                                         binary search over block0 (TO_STREAM_WAVE launches
@@ -288,8 +319,9 @@ int to_struct_sizes(int64_t* join_desc, int64_t* leaf_desc, int64_t* scale_rec,
                      int64_t* accum, int64_t* launch, int64_t* perm_desc, int64_t* gemm_desc,
                      int64_t* root_desc, int64_t* leaf_build_desc);
 
-/* Size in bytes of to_fold_desc, for the same check. */
+/* Size in bytes of to_fold_desc and to_tree_desc, for the same check. */
 int to_fold_desc_size(void);
+int to_tree_desc_size(void);
 
 /* Last error message of the calling thread ("" when none). */
 const char* to_last_error(void);

@@ -27,7 +27,8 @@ TO_F64, TO_F32S = 0, 1
     TO_OP_BATCH_BEGIN,
     TO_OP_LEAF_BUILD,
     TO_OP_FOLD,
-) = range(1, 15)
+    TO_OP_FOLD_TREE,
+) = range(1, 16)
 TO_LEAF_VAR, TO_LEAF_OR = 0, 1  # leaf build kinds
 TO_STREAM_VEC = 0x100  # stream variant bit: the 16-byte form
 TO_STREAM_ROWS = 0x200  # stream variant: the row form
@@ -37,6 +38,8 @@ TO_LAUNCH_SIDE = 0x1  # Launch.flags: captured on the side stream
 TO_LAUNCH_JOIN = 0x2  # Launch.flags: join the side stream into the main one and fork it again first
 TO_FOLD_ANY = 0  # fold launch variants: any bit layout
 TO_FOLD_VEC = 0x100  # the 16-byte form; | y mode << 4 | nreg
+TO_TREE_WORDS = 448  # uint32 words of one join of a fold tree program
+TO_TREE_IDLE, TO_TREE_MEET = 1 << 30, 1 << 31  # fold tree task bits
 MAX_BITS = 32
 FOLD_BITS = 40
 ABI_VERSION = 7
@@ -134,6 +137,12 @@ class FoldDesc(ctypes.Structure):
     ]
 
 
+class TreeDesc(ctypes.Structure):
+    _fields_ = [("ops", ctypes.c_uint64), ("tasks", ctypes.c_uint64), ("recs", ctypes.c_uint64),
+                ("ntask", ctypes.c_int32), ("nslots", ctypes.c_int32),
+                ("block0", ctypes.c_int32), ("nblocks", ctypes.c_int32)]
+
+
 class RootDesc(ctypes.Structure):
     _fields_ = [("root", ctypes.c_uint64), ("rec", ctypes.c_uint64), ("acc", ctypes.c_uint64),
                 ("block0", ctypes.c_int32), ("nblocks", ctypes.c_int32)]
@@ -154,7 +163,7 @@ EXPORTED = [
     "to_version", "to_struct_sizes", "to_last_error", "to_device_count", "to_set_device",
     "to_run", "to_run_timed", "to_graph_create", "to_graph_launch", "to_graph_destroy", "to_permute",
     "to_wall_clock_khz", "to_synchronize", "to_mlp_forward", "to_mlp_backward", "to_mlp_adam",
-    "to_tensordot_workspace", "to_tensordot", "to_tensordot_noalloc", "to_fold_desc_size",
+    "to_tensordot_workspace", "to_tensordot", "to_tensordot_noalloc", "to_fold_desc_size", "to_tree_desc_size",
 ]
 MLP_IN, MLP_H1, MLP_H2, MLP_OUT = 16, 64, 64, 2
 MLP_NPARAMS = 64 * 16 + 64 + 64 * 64 + 64 + 2 * 64 + 2
@@ -204,7 +213,8 @@ def load(path=LIB_PATH):
     lib.to_struct_sizes(*[ctypes.byref(s) for s in sizes])
     want = [ctypes.sizeof(t) for t in (JoinDesc, LeafDesc, ScaleRec, Accum, Launch, PermDesc, GemmDesc, RootDesc,
                                        LeafBuildDesc)]
-    if [s.value for s in sizes] != want or lib.to_fold_desc_size() != ctypes.sizeof(FoldDesc):
+    if [s.value for s in sizes] != want or lib.to_fold_desc_size() != ctypes.sizeof(FoldDesc) \
+            or lib.to_tree_desc_size() != ctypes.sizeof(TreeDesc):
         raise ImportError("record layout mismatch between library and binding: %s vs %s"
                           % ([s.value for s in sizes], want))
     _lib = lib

@@ -26,21 +26,23 @@ __device__ __forceinline__ FoldRows fold_rows(const to_fold_desc* __restrict__ d
     return FoldRows{d->bx[i], d->by[i], d->bc[i]};
 }
 
-// Walk 2^nloop shared indices in Gray-code order, so each step of KU indices changes one bit
+// Walk 2^nloop shared indices (bit entries from lane `first` of row.x and lane ylanes + first
+// of row.y) in Gray-code order, so each step of KU indices changes one bit
 // above them: f(dx, dy) gets the KU x / y offsets of a step (inside it the low bits follow
 // Gray order too, so the walk is a bijection).
 template <int KU, typename F>
-__device__ __forceinline__ void fold_walk(uint32_t xk, uint32_t yk, const FoldRows& row, int first, int nloop, F f) {
+__device__ __forceinline__ void fold_walk(uint32_t xk, uint32_t yk, const FoldRows& row, int first, int ylanes,
+                                          int nloop, F f) {
     constexpr int LKU = KU == 4 ? 2 : (KU == 2 ? 1 : 0);
     uint32_t dx[KU], dy[KU];
     dx[0] = dy[0] = 0;
     if constexpr (KU >= 2) {
         dx[1] = (uint32_t)__builtin_amdgcn_readlane((int)row.x, first);
-        dy[1] = (uint32_t)__builtin_amdgcn_readlane((int)row.y, first);
+        dy[1] = (uint32_t)__builtin_amdgcn_readlane((int)row.y, ylanes + first);
     }
     if constexpr (KU == 4) {
         const uint32_t bx = (uint32_t)__builtin_amdgcn_readlane((int)row.x, first + 1);
-        const uint32_t by = (uint32_t)__builtin_amdgcn_readlane((int)row.y, first + 1);
+        const uint32_t by = (uint32_t)__builtin_amdgcn_readlane((int)row.y, ylanes + first + 1);
         dx[2] = dx[1] | bx;
         dx[3] = bx;
         dy[2] = dy[1] | by;
@@ -58,7 +60,7 @@ __device__ __forceinline__ void fold_walk(uint32_t xk, uint32_t yk, const FoldRo
         if (k == steps) break;
         const int b = first + LKU + __builtin_ctz(k);
         xk ^= (uint32_t)__builtin_amdgcn_readlane((int)row.x, b);
-        yk ^= (uint32_t)__builtin_amdgcn_readlane((int)row.y, b);
+        yk ^= (uint32_t)__builtin_amdgcn_readlane((int)row.y, ylanes + b);
     }
 }
 
@@ -74,6 +76,23 @@ __device__ __forceinline__ FoldScale fold_scale(const to_fold_desc* __restrict__
     if (!SCALED) return FoldScale{1.0, 0};
     const OpScale a = op_scale(d->xs, d->xsb, batch), b = op_scale(d->ys, d->ysb, batch);
     return FoldScale{(double)a.f * (double)b.f, a.e + b.e};
+}
+
+// Largest of the wave's non-negative floats, the same in every lane: row shifts and row
+// broadcasts (VALU only), where shuffles would go through LDS six times
+__device__ __forceinline__ float fold_wave_max(float v) {
+    uint32_t m = __float_as_uint(v);
+    auto step = [&](auto ctrl) {
+        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, decltype(ctrl)::value, 0xf, 0xf, true);
+        m = o > m ? o : m;
+    };
+    step(std::integral_constant<int, 0x111>{});  // row_shr:1, 2, 4, 8
+    step(std::integral_constant<int, 0x112>{});
+    step(std::integral_constant<int, 0x114>{});
+    step(std::integral_constant<int, 0x118>{});
+    step(std::integral_constant<int, 0x142>{});  // row_bcast:15, 31
+    step(std::integral_constant<int, 0x143>{});
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)m, 63));
 }
 
 // Sum over thread bits [lo, lo + lk) of a 256-thread block: shuffles inside a wave, LDS
@@ -122,7 +141,7 @@ __device__ __forceinline__ void fold_any_body(const to_fold_desc* __restrict__ d
         const int64_t batch = t >> (lsplit + ntile);
         if (SCALED && batch != cur) {
             if (cur >= 0 && lsplit == 0) {
-                const float w = wave_max(mrun);
+                const float w = fold_wave_max(mrun);
                 if ((tid & 63) == 0) note_max(d->cs, cur, w);
                 mrun = 0.0f;
             }
@@ -138,7 +157,7 @@ __device__ __forceinline__ void fold_any_body(const to_fold_desc* __restrict__ d
             const TO_GLOBAL T* Yp = Y + batch * d->yb + yl;
             auto walk = [&](auto ku) {
                 constexpr int KU = decltype(ku)::value;
-                fold_walk<KU>(xt, yt, row, kb, nloop, [&](const uint32_t* ox, const uint32_t* oy) {
+                fold_walk<KU>(xt, yt, row, kb, 0, nloop, [&](const uint32_t* ox, const uint32_t* oy) {
                     T xv[KU], yv[KU];
 #pragma unroll
                     for (int j = 0; j < KU; ++j) {
@@ -168,7 +187,7 @@ __device__ __forceinline__ void fold_any_body(const to_fold_desc* __restrict__ d
         }
     }
     if (SCALED && cur >= 0 && lsplit == 0) {
-        const float w = wave_max(mrun);
+        const float w = fold_wave_max(mrun);
         if ((tid & 63) == 0) note_max(d->cs, cur, w);
     }
 }
@@ -217,7 +236,7 @@ __global__ __launch_bounds__(kBlock) void k_fold_vec(const to_fold_desc* __restr
         const int64_t batch = t >> ntile;
         if (SCALED && batch != cur) {
             if (cur >= 0) {
-                const float w = wave_max(mrun);
+                const float w = fold_wave_max(mrun);
                 if ((tid & 63) == 0) note_max(d->cs, cur, w);
                 mrun = 0.0f;
             }
@@ -235,7 +254,7 @@ __global__ __launch_bounds__(kBlock) void k_fold_vec(const to_fold_desc* __restr
             for (int v = 0; v < 4; ++v) acc[r][v] = 0.0;
         auto walk = [&](auto ku) {
             constexpr int KU = decltype(ku)::value;
-            fold_walk<KU>(xt, yt, row, kb, nloop, [&](const uint32_t* ox, const uint32_t* oy) {
+            fold_walk<KU>(xt, yt, row, kb, 0, nloop, [&](const uint32_t* ox, const uint32_t* oy) {
                 V4 xv[KU];
 #pragma unroll
                 for (int j = 0; j < KU; ++j) xv[j] = *reinterpret_cast<const TO_GLOBAL V4*>(Xp + ox[j]);
@@ -277,7 +296,221 @@ __global__ __launch_bounds__(kBlock) void k_fold_vec(const to_fold_desc* __restr
         if (SCALED && tid == 0 && tile == 0) note_exp(d->cs, batch, sc.e);
     }
     if (SCALED && cur >= 0) {
-        const float w = wave_max(mrun);
+        const float w = fold_wave_max(mrun);
         if ((tid & 63) == 0) note_max(d->cs, cur, w);
+    }
+}
+
+// ---------------------------------------------------------------------------------
+// Programs of small joins, one block per batch item (to_tree_desc): the intermediate tensors
+// stay in LDS and the levels meet at block barriers, where a launch per level costs 3-5 us.
+// Bound by the latency of a level: a wave issues one instruction per 4-5 cycles, so what counts
+// is how few a join takes.  Its whole description, the offset of every lane included, is
+// fetched while the wave works on the join before it, and the joins that need no more than one
+// round of four products per lane (nearly all) run straight through: 0.7 us per level in
+// float64, 1.1 us scaled (a chain of 64 joins; 1.2 and 1.6 us at 2^10 outputs), against 3-5 us
+// for a launch.  The n = 90 vertex cover's 224 joins are 10 levels of one block, 32 us where
+// their launches took 450.  Tried: deposits computed per join instead of fetched lane offsets
+// (twice the time of a level), one generic-pointer loop for every sum (long sums 1.6x), the
+// maximum by LDS atomics of all lanes (+2 us per level of 64 outputs).
+
+constexpr int kTreeMaxLds = 128 * 1024;
+
+struct TreeRec {
+    int32_t exp;
+    uint32_t maxbits;
+};
+
+struct TreeWords {
+    uint32_t head, bits, off[5];  // words 0-63, 64-127, and this lane's offsets (result: 4)
+};
+
+__device__ __forceinline__ TreeWords tree_words(const TO_GLOBAL uint32_t* ops, uint32_t task) {
+    const TO_GLOBAL uint32_t* p = ops + (task & 0xffff) * TO_TREE_WORDS;
+    return TreeWords{p[0], p[64], {p[128], p[192], p[256], p[320], p[384]}};
+}
+
+// power of two that brings a tensor of this maximum to at most 1 (any nearby one would do)
+__device__ __forceinline__ int tree_exp(uint32_t maxbits) {
+    return maxbits ? (int)(maxbits >> 23) - 126 : 0;
+}
+
+template <typename T, bool SCALED>
+__global__ __launch_bounds__(1024) void k_fold_tree(const to_tree_desc* __restrict__ descs, int ndesc,
+                                                    const int32_t* __restrict__ bmap) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const to_tree_desc* d = descs + find_desc(descs, ndesc, blockIdx.x, bmap);
+    const int64_t batch = blockIdx.x - d->block0;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ntask = d->ntask, nslots = d->nslots;
+    TreeRec* recs = reinterpret_cast<TreeRec*>(smem);
+    T* data = reinterpret_cast<T*>(smem + ((nslots * sizeof(TreeRec) + 15) & ~(size_t)15));
+    const TO_GLOBAL uint32_t* tasks = gptr<const uint32_t>(d->tasks) + (int64_t)wave * ntask;
+    const TO_GLOBAL uint32_t* ops = gptr<const uint32_t>(d->ops) + lane;
+    const uint64_t grecs = d->recs;
+    uint32_t task = tasks[0];
+    TreeWords w = tree_words(ops, task);
+    if (SCALED) {
+        for (int i = threadIdx.x; i < nslots; i += blockDim.x) recs[i] = TreeRec{0, 0u};
+        __syncthreads();
+    }
+    for (int i = 0; i < ntask; ++i) {
+        const uint32_t next = tasks[i + 1 < ntask ? i + 1 : i];
+        const TreeWords wn = tree_words(ops, next);
+        if (!(task & TO_TREE_IDLE)) {
+            auto word = [&](int j) { return (uint32_t)__builtin_amdgcn_readlane((int)w.head, j); };
+            auto wide = [&](int j) { return (uint64_t)word(j) | (uint64_t)word(j + 1) << 32; };
+            const uint32_t h = word(0);
+            const int lo = h & 15, lk = (h >> 4) & 15, nloop = (h >> 8) & 15, nchunk = (h >> 12) & 15;
+            const int nops = ((h >> 16) & 3) + 1;
+            const bool active = lane < (1 << (lo + lk)), writer = lane < (1 << lo);
+            const bool cl = (h >> 24) & 1;
+            const uint32_t slot = word(20);
+            const int kb = 6 + nchunk;
+            double f = 1.0;
+            int64_t e = 0;
+            if (SCALED) {
+                int x = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (j < nops) {
+                        const uint32_t s = word(16 + j);
+                        if ((h >> (20 + j)) & 1) {
+                            const TreeRec r = recs[s];
+                            x += tree_exp(r.maxbits);
+                            e += r.exp;
+                        } else {
+                            const TO_GLOBAL to_scale_rec* r =
+                                gptr<const to_scale_rec>(grecs) + ((int64_t)s + (((h >> (25 + j)) & 1) ? batch : 0));
+                            x += tree_exp(r->maxbits);
+                            e += r->exp;
+                        }
+                    }
+                }
+                e += x;
+                f = __longlong_as_double((long long)(1023 - x) << 52);
+            }
+            // entry b of operand j's bits (the result: j = 4)
+            auto entry = [&](int j, int b) {
+                return (uint32_t)__builtin_amdgcn_readlane(j < 4 ? (int)w.bits : (int)w.head, (j < 4 ? 16 * j : 32) + b);
+            };
+            const uint32_t first = (task >> 16) & 127;
+            const int lstep = (task >> 23) & 15;
+            float mrun = 0.0f;
+            auto finish = [&](double acc, uint32_t co) {
+                for (int b = lo; b < lo + lk; ++b) acc += __shfl_xor(acc, 1 << b, 64);
+                const T v = (T)(SCALED ? acc * f : acc);
+                if (writer) {
+                    if (cl) data[word(9) + co] = v;
+                    else gptr<T>(wide(9))[batch * (int64_t)word(15) + co] = v;
+                    if (SCALED) mrun = fmaxf(mrun, (float)absval(v));
+                }
+            };
+            if (nchunk == 0 && nloop <= 2) {
+                // one round: up to 4 operands through generic pointers (LDS or global), the up
+                // to 4 shared indices at once
+                T v[4][4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (j < nops) {
+                        const T* q = (((h >> (20 + j)) & 1)
+                                          ? data + word(1 + 2 * j)
+                                          : reinterpret_cast<const T*>(wide(1 + 2 * j)) + batch * (int64_t)word(11 + j)) +
+                                     w.off[j];
+                        const uint32_t b0 = entry(j, 6), b1 = entry(j, 7);
+                        if (active) {
+                            v[j][0] = q[0];
+                            if (nloop >= 1) v[j][1] = q[b0];
+                            if (nloop >= 2) {
+                                v[j][2] = q[b1];
+                                v[j][3] = q[b0 | b1];
+                            }
+                        }
+                    }
+                }
+                double acc = 0.0;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    if (u < (1 << nloop)) {
+                        double t = (double)v[0][u];
+#pragma unroll
+                        for (int j = 1; j < 4; ++j)
+                            if (j < nops) t *= (double)v[j][u];
+                        acc += t;
+                    }
+                }
+                finish(active ? acc : 0.0, w.off[4]);
+            } else {
+                // The task's chunks, each a walk of the shared range four indices at a time.  Both
+                // go in Gray order, so a step changes one bit of the offsets (entries do not
+                // overlap: xor).
+                uint32_t xo = w.off[0], yo = w.off[1], co = w.off[4];
+                for (int b = 0; b < lstep; ++b)
+                    if ((first >> b) & 1) {
+                        xo |= entry(0, 6 + b);
+                        yo |= entry(1, 6 + b);
+                        co |= entry(4, 6 + b);
+                    }
+                const uint32_t chunks = 1u << (nchunk - lstep);
+                auto run = [&](auto X, auto Y) {
+                    for (uint32_t c = 1;; ++c) {
+                        double acc = 0.0;
+                        auto walk = [&](auto ku) {
+                            constexpr int KU = decltype(ku)::value;
+                            fold_walk<KU>(xo, yo, FoldRows{w.bits, w.bits, 0u}, kb, 16, nloop,
+                                          [&](const uint32_t* ox, const uint32_t* oy) {
+                                if (active) {
+                                    T xv[KU], yv[KU];
+#pragma unroll
+                                    for (int j = 0; j < KU; ++j) {
+                                        xv[j] = X[ox[j]];
+                                        yv[j] = Y[oy[j]];
+                                    }
+#pragma unroll
+                                    for (int j = 0; j < KU; ++j) acc = fma((double)xv[j], (double)yv[j], acc);
+                                }
+                            });
+                        };
+                        if (nloop >= 2) walk(std::integral_constant<int, 4>{});
+                        else if (nloop == 1) walk(std::integral_constant<int, 2>{});
+                        else walk(std::integral_constant<int, 1>{});
+                        finish(acc, co);
+                        if (c == chunks) break;
+                        const int b = 6 + lstep + __builtin_ctz(c);
+                        xo ^= entry(0, b);
+                        yo ^= entry(1, b);
+                        co ^= entry(4, b);
+                    }
+                };
+                const T* Xl = data + word(1);
+                const T* Yl = data + word(3);
+                const TO_GLOBAL T* Xg = gptr<const T>(wide(1)) + batch * (int64_t)word(11);
+                const TO_GLOBAL T* Yg = gptr<const T>(wide(3)) + batch * (int64_t)word(12);
+                const bool xl = (h >> 20) & 1, yl = (h >> 21) & 1;
+                if (xl && yl) run(Xl, Yl);
+                else if (xl) run(Xl, Yg);
+                else if (yl) run(Xg, Yl);
+                else run(Xg, Yg);
+            }
+            if (SCALED) {
+                const float m = fold_wave_max(mrun);
+                if (cl) {
+                    if (lane == 0) {
+                        atomicMax(&recs[slot].maxbits, __float_as_uint(m));
+                        if (first == 0) recs[slot].exp = (int32_t)e;
+                    }
+                } else {
+                    const int64_t r = (int64_t)slot + (((h >> 29) & 1) ? batch : 0);
+                    if (lane == 0) {
+                        note_max(grecs, r, m);
+                        if (first == 0) note_exp(grecs, r, e);
+                    }
+                }
+            }
+        }
+        if (task & TO_TREE_MEET) __syncthreads();
+        task = next;
+        w = wn;
     }
 }

@@ -2440,6 +2440,19 @@ int launch_one(const to_launch& L, hipStream_t st) {
             hipLaunchKernelGGL((k_root_store<T, SCALED>), grid, block, 0, st,
                                reinterpret_cast<const to_root_desc*>(L.descs), L.count);
             break;
+        case TO_OP_FOLD_TREE: {
+            if (!L.descs || L.count <= 0 || L.iaux0 < 1 || L.iaux0 > 16) return TO_ERR_INVALID;
+            if (L.lds > 64 * 1024) {
+                // more than the default limit of dynamic LDS
+                const hipError_t raised = hipFuncSetAttribute(
+                    reinterpret_cast<const void*>(&k_fold_tree<T, SCALED>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                    kTreeMaxLds);
+                if (raised != hipSuccess) return hip_fail(raised, "fold tree: LDS limit");
+            }
+            hipLaunchKernelGGL((k_fold_tree<T, SCALED>), grid, dim3(64 * (unsigned)L.iaux0), L.lds, st,
+                               reinterpret_cast<const to_tree_desc*>(L.descs), L.count, bmap);
+            break;
+        }
         case TO_OP_FOLD: {
             if (!L.descs || L.count <= 0) return TO_ERR_INVALID;
             const to_fold_desc* fd = reinterpret_cast<const to_fold_desc*>(L.descs);
@@ -2535,6 +2548,8 @@ int to_struct_sizes(int64_t* join_desc, int64_t* leaf_desc, int64_t* scale_rec, 
     if (launch) *launch = sizeof(to_launch);
     return TO_OK;
 }
+
+int to_tree_desc_size(void) { return (int)sizeof(to_tree_desc); }
 
 int to_fold_desc_size(void) { return (int)sizeof(to_fold_desc); }
 

@@ -24,6 +24,7 @@ shared variables as batch items.
 The value is the same contraction; only structural zeros are left out.
 """
 
+import ctypes
 import math
 import struct
 
@@ -49,7 +50,29 @@ ANY_MIN_THREADS_LOG = 17
 MAX_ANY_BLOCKS = 8192
 MAX_VEC_BLOCKS = 4096
 MAX_REG_BITS = 3
+# programs run by one block per slice: joins over at most 2^TREE_BITS index values with
+# results of at most 2^TREE_RANK entries, the intermediates in TREE_LDS bytes of LDS -- or
+# TREE_LDS_MANY with TREE_WAVES_MANY waves, so that blocks share a CU, when there are enough
+# slices to fill the chip
+TREE_BITS = 16
+TREE_RANK = 13
+TREE_FAR_RANK = 9
+TREE_FAR_BITS = 13
+TREE_WAVES = 16
+TREE_WAVES_MANY = 8
+TREE_LDS = 120 * 1024
+TREE_LDS_MANY = 40 * 1024
+TREE_MANY = 512
+# a program of one join only up to this many index values (a launch of many blocks above)
+TREE_LONE_BITS = 12
+# joins of a program merged into one product: at most 4 operands, 64 outputs and 2^MERGE_LOOP
+# products per output (each merge saves a level)
+MERGE_LOOP = 2
+# level launches are kept whatever they cost in memory up to this arena size
+LEVEL_FREE_BYTES = 256 << 20
 
+# bit b of lane l
+_LANE_BITS = ((np.arange(64)[None, :] >> np.arange(6)[:, None]) & 1).astype(np.uint32)
 _HEAD = struct.Struct("<QQQqqqQQQqqQ10i")
 _BITS = struct.Struct("<%dI" % (3 * _lib.FOLD_BITS))
 
@@ -374,56 +397,238 @@ def _scratch(arena, n, nodes, nb, esize, table):
     return list(blocks.values())
 
 
-def join_levels(nodes, batched):
-    """Joins of one phase by level, as ``schedule.join_levels``."""
+class TreeProgram:
+    """A connected part of the tree, of small joins, that a block runs for one slice: its
+    joins by level as (node, operands), what each sums, the LDS element offsets and record
+    slots of their results (the root's goes to the arena) and the LDS bytes."""
+
+    __slots__ = ("root", "members", "levels", "sums", "at", "slot", "lds", "batched", "outside")
+
+
+def _merge(nodes, members):
+    """Operands and summed variables of the joins of a program after small joins are merged
+    into the products they feed ({join: operands}, {join: variables})."""
+    ops, sums, level = {}, {}, {}
+    for i in sorted(members):
+        n = nodes[i]
+        mine, ks = [c for c in (n.left, n.right) if c >= 0], set(n.ksum)
+        while True:
+            best = None
+            for c in mine:
+                if c not in ops or len(mine) - 1 + len(ops[c]) > 4 or len(ks) + len(sums[c]) > MERGE_LOOP \
+                        or n.rank > 6:
+                    continue
+                if best is None or level[c] > level[best]:
+                    best = c
+            if best is None:
+                break
+            mine = [c for c in mine if c != best] + ops.pop(best)
+            ks |= sums.pop(best)
+        ops[i], sums[i] = mine, ks
+        level[i] = 1 + max((level[c] for c in mine if c in ops), default=0)
+    return ops, sums, level
+
+
+def _program(nodes, root, stage, esize, scaled):
+    p = TreeProgram()
+    p.root, p.batched = root, nodes[root].batched
+    todo, p.members = [root], set()
+    while todo:
+        i = todo.pop()
+        p.members.add(i)
+        todo += [c for c in (nodes[i].left, nodes[i].right) if stage.get(c) == stage[root]]
+    ops, p.sums, level = _merge(nodes, p.members)
+    p.levels = [[] for _ in range(level[root])]
+    for i in ops:
+        p.levels[level[i] - 1].append((i, ops[i]))
+    arena, p.at, live = schedule._Arena(align=16), {}, {}
+    for lv in p.levels:
+        for i, _ in lv:
+            if i != root:
+                live[i] = arena.alloc(esize << nodes[i].rank)
+                p.at[i] = live[i][0] // esize
+        for _, mine in lv:
+            for c in mine:
+                if c in live:
+                    arena.release(live.pop(c))
+    p.slot = {i: k for k, i in enumerate(p.at)}
+    p.lds = arena.peak + ((8 * len(p.slot) + 15) & ~15 if scaled else 0)
+    # tensors of the same phase that other launches make
+    p.outside = [c for _, mine in ((i, m) for lv in p.levels for i, m in lv) for c in mine
+                 if c not in p.at and not nodes[c].is_leaf and nodes[c].batched == p.batched]
+    return p
+
+
+def tree_programs(nodes, W, esize, scaled):
+    """The programs of a plan whose joins carry their forms: maximal connected parts of small
+    joins of one phase whose intermediates fit LDS."""
+    # a small join's stage: its phase and the number of large joins on the longest path below
+    # it; programs are the connected joins of one stage, so none waits for more than it reads
+    stage, depth = {}, {}
+    for n in nodes:
+        if n.is_leaf:
+            continue
+        # a block reads a large tensor of another launch at the latency of L2: fewer products
+        far = any(c >= 0 and nodes[c].rank > TREE_FAR_RANK and (c not in stage or nodes[c].batched != n.batched)
+                  for c in (n.left, n.right))
+        small = n.geom["var"]["kind"] == "fold" and n.rank <= TREE_RANK and \
+            len(n.ksum) + n.rank <= (TREE_FAR_BITS if far else TREE_BITS)
+        depth[n.idx] = max([depth[c] for c in (n.left, n.right)
+                            if c in depth and nodes[c].batched == n.batched], default=0) + (not small)
+        if small:
+            stage[n.idx] = (n.batched, depth[n.idx])
+    out = []
+    todo = [i for i in stage if stage.get(nodes[i].parent) != stage[i]]
+    while todo:
+        i = todo.pop()
+        p = _program(nodes, i, stage, esize, scaled)
+        if p.lds > (TREE_LDS_MANY if p.batched and W >= TREE_MANY else TREE_LDS):
+            # its root runs as a launch of its own, what is below as programs
+            todo += [c for c in (nodes[i].left, nodes[i].right) if stage.get(c) == stage[i]]
+            del stage[i]
+        elif len(p.members) > 1 or len(nodes[i].ksum) + nodes[i].rank <= TREE_LONE_BITS:
+            out.append(p)
+    return sorted(out, key=lambda p: p.root)
+
+
+def _tree_task(n, ksum, operands):
+    """(lo, lk, nloop, nchunk), variables in bit order, of a join inside a program.  Short
+    sums are walked by one lane; longer ones are shared by the lanes the outputs leave."""
+    def key(v):
+        return tuple(t.off.get(v, 1 << 40) for t in operands) + (v,)
+
+    ks = sorted(ksum, key=key)
+    nc, s = n.rank, len(ks)
+    lo = min(nc, 6)
+    lk = max(0, min(s - 2, 6 - lo))
+    bits = n.order[:lo] + ks[:lk] + [None] * (6 - lo - lk) + n.order[lo:] + ks[lk:]
+    return (lo, lk, s - lk, nc - lo), bits
+
+
+def tree_words(p, nodes, waves, rec_index, one):
+    """(uint32 joins [n, 128], uint32 task streams [waves, ntask]) of a program.  ``one``:
+    (address, record index) of the stored 1.0."""
+    words = np.zeros((sum(len(lv) for lv in p.levels), _lib.TO_TREE_WORDS), dtype=np.uint32)
+    streams = [[] for _ in range(waves)]
+    k = 0
+    for lv in p.levels:
+        costs, tasks = [], []
+        for i, mine in lv:
+            n = nodes[i]
+            # the walk of two operands takes the one with more variables first
+            mine = sorted(mine, key=lambda c: -len(nodes[c].order))
+            if len(mine) == 1:
+                mine = mine + [-1]
+            (lo, lk, nloop, nchunk), bits = _tree_task(n, p.sums[i], [nodes[c] for c in mine if c >= 0])
+            row = [0] * 128
+            head = lo | lk << 4 | nloop << 8 | nchunk << 12 | (len(mine) - 1) << 16
+            for j, t in list(enumerate(mine)) + [(4, i)]:
+                if t in p.at:
+                    head |= 1 << (20 + j)
+                    row[1 + 2 * j], row[16 + j] = p.at[t], p.slot[t]
+                else:
+                    addr, rec, stride, advances = (one[0], one[1], 0, 0) if t < 0 else (
+                        nodes[t].ptr, rec_index(nodes[t]), nodes[t].bstride if p.batched else 0,
+                        nodes[t].rec_stride if p.batched else 0)
+                    row[1 + 2 * j], row[2 + 2 * j] = addr & 0xffffffff, addr >> 32
+                    row[11 + j], row[16 + j] = stride, rec
+                    head |= (1 << (25 + j)) if advances else 0
+                off = nodes[t].off if t >= 0 else {}
+                at = 64 + 16 * j if j < 4 else 32
+                for b, v in enumerate(bits):
+                    if v is not None:
+                        row[at + b] = off.get(v, 0)
+            row[0] = head
+            words[k, :128] = row
+            # rough wave cycles: setting up, then per chunk its loads
+            costs.append((300, (1 << nchunk) * (100 + (30 * len(mine) << nloop) // 2), nchunk, k))
+            k += 1
+        share = sum(c[1] for c in costs) / waves
+        for setup, work, nchunk, j in costs:
+            lstep = 0
+            while lstep < nchunk and (1 << lstep) < waves and work / (1 << lstep) > max(share, 2 * setup):
+                lstep += 1
+            tasks += [(setup + work / (1 << lstep), j | c << 16 | lstep << 23) for c in range(1 << lstep)]
+        tasks.sort(key=lambda t: -t[0])
+        load, mine = [0.0] * waves, [[] for _ in range(waves)]
+        for cost, word in tasks:
+            w = load.index(min(load))
+            load[w] += cost
+            mine[w].append(word)
+        rounds = max(len(m) for m in mine)
+        for w in range(waves):
+            m = mine[w] + [_lib.TO_TREE_IDLE] * (rounds - len(mine[w]))
+            m[-1] |= _lib.TO_TREE_MEET
+            streams[w] += m
+    # every lane's offset: the sum of the entries of its bits, for operands 0-3 and the result
+    entries = words[:, [64 + 16 * j + b for j in range(4) for b in range(6)] + [32 + b for b in range(6)]]
+    words[:, 128:] = (entries.reshape(-1, 5, 6) @ _LANE_BITS).reshape(-1, 5 * 64)
+    return words, np.array(streams, dtype=np.uint32)
+
+
+def phase_groups(nodes, batched, order, programs):
+    """Groups of one phase in execution order, each (programs, joins) that may run together.
+    ``order`` "level": every unit (a program, or a join outside all of them) one level above
+    the highest of what it reads; "post": the programs that read nothing of the phase first,
+    then unit by unit."""
+    mine = [p for p in programs if p.batched == batched]
+    unit = {i: p for p in mine for i in p.members}
     level, out = {}, []
+    first = []
     for n in nodes:
         if n.is_leaf or n.batched != batched:
             continue
-        lv = 1 + max(level.get(n.left, 0), level.get(n.right, 0))
+        p = unit.get(n.idx)
+        if p is not None and p.root != n.idx:
+            continue
+        lv = 1 + max((level.get(c, 0) for c in (p.outside if p is not None else (n.left, n.right))), default=0)
         level[n.idx] = lv
-        while len(out) < lv:
-            out.append([])
-        out[lv - 1].append(n.idx)
-    return out
+        if order == "level":
+            while len(out) < lv:
+                out.append(([], []))
+            (out[lv - 1][0] if p is not None else out[lv - 1][1]).append(p if p is not None else n.idx)
+        elif p is not None and lv == 1:
+            first.append(p)
+        else:
+            out.append(([p], []) if p is not None else ([], [n.idx]))
+    return ([(first, [])] if first else []) + out
 
 
-def plan_memory(nodes, W, esize, order):
-    """(arena peak, scratch placements), as ``schedule.plan_memory``."""
+def plan_memory(nodes, W, esize, order, programs=()):
+    """(arena peak, scratch placements), as ``schedule.plan_memory``; what a program keeps in
+    LDS has no place in the arena."""
     arena = schedule._Arena()
     scratch = {}
 
     def run(group, nb, release):
         temps = []
-        for i in group:
-            n = nodes[i]
-            n.buf = arena.alloc(nb * (1 << n.rank) * esize)
-            temps += _scratch(arena, n, nodes, nb, esize, scratch)
+        for i in [p.root for p in group[0]] + group[1]:
+            nodes[i].buf = arena.alloc(nb * (1 << nodes[i].rank) * esize)
+        for i in group[1]:
+            temps += _scratch(arena, nodes[i], nodes, nb, esize, scratch)
         for blk in temps:
             arena.release(blk)
-        for i in group:
-            for c in (nodes[i].left, nodes[i].right):
-                if c >= 0 and release(nodes[c]):
-                    arena.release(nodes[c].buf)
+        read = [c for p in group[0] for lv in p.levels for _, mine in lv for c in mine if c not in p.at]
+        read += [c for i in group[1] for c in (nodes[i].left, nodes[i].right)]
+        for c in read:
+            if c >= 0 and release(nodes[c]):
+                arena.release(nodes[c].buf)
 
-    def groups(batched):
-        if order == "level":
-            return join_levels(nodes, batched)
-        return [[n.idx] for n in nodes if not n.is_leaf and n.batched == batched]
-
-    for grp in groups(False):
+    for grp in phase_groups(nodes, False, order, programs):
         run(grp, 1, lambda c: not c.is_leaf and not c.batched)
     for n in nodes:
         if n.is_leaf and n.batched:
             n.buf = arena.alloc(W * (1 << n.rank) * esize)
-    for grp in groups(True):
+    for grp in phase_groups(nodes, True, order, programs):
         run(grp, W, lambda c: c.batched)
     return arena.peak, scratch
 
 
-def choose_order(nodes, W, esize):
-    post, _ = plan_memory(nodes, W, esize, "post")
-    level, _ = plan_memory(nodes, W, esize, "level")
+def choose_order(nodes, W, esize, programs=()):
+    level, _ = plan_memory(nodes, W, esize, "level", programs)
+    if level <= LEVEL_FREE_BYTES:
+        return "level", level
+    post, _ = plan_memory(nodes, W, esize, "post", programs)
     if level <= schedule.LEVEL_PEAK_FACTOR * post:
         return "level", level
     return "post", post
@@ -431,7 +636,7 @@ def choose_order(nodes, W, esize):
 
 def peak_bytes(nodes, W, esize):
     choose_all(nodes, W, esize)
-    return choose_order(nodes, W, esize)[1]
+    return choose_order(nodes, W, esize, tree_programs(nodes, W, esize, esize == 4))[1]
 
 
 def join_records(n, nodes, W, esize, scaled, abase, scratch, recp, one):
@@ -535,8 +740,11 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
     prog = schedule.Program()
     prog.nbatch, prog.nodes = W, nodes
     choose_all(nodes, W, esize)
-    order = choose_order(nodes, W, esize)[0] if group_levels else "post"
-    peak, scratch = plan_memory(nodes, W, esize, order)
+    programs = tree_programs(nodes, W, esize, scaled) if group_levels else []
+    order = choose_order(nodes, W, esize, programs)[0] if group_levels else "post"
+    peak, scratch = plan_memory(nodes, W, esize, order, programs)
+    prog.programs = programs
+    in_lds = {i for p in programs for i in p.members if i != p.root}
     prog.arena_bytes, prog.order = peak, order
 
     image = schedule.leaf_image(nodes, tables, num_groups, scaled, np.float64 if esize == 8 else np.float32)
@@ -558,12 +766,12 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
         nrec += 1
         pro_rec0 = nrec
         for n in nodes:
-            if not n.is_leaf and not n.batched:
+            if not n.is_leaf and not n.batched and n.idx not in in_lds:
                 n.rec, n.rec_stride = nrec, 0
                 nrec += 1
         wave_rec0 = nrec
         for n in nodes:
-            if n.batched:
+            if n.batched and n.idx not in in_lds:
                 n.rec, n.rec_stride = nrec, 1
                 nrec += W
         prog.rec_ranges = (pro_rec0, wave_rec0, nrec)
@@ -579,6 +787,8 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
     wave_params = prog.params.data_ptr()
     one_at = (tbase + one * esize, rbase + one_rec * 16 if scaled else 0)
     for n in nodes:
+        if n.idx in in_lds:
+            continue
         if n.is_leaf and not n.batched:
             n.ptr, n.bstride = tbase + image.off[n.tensor] * esize, 0
         else:
@@ -636,10 +846,40 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
             phase.append((grp[0][0], Launch(op=key[1], variant=key[2], count=len(grp), grid=block0, lds=lds), off,
                           grp[0][4] if len(grp) == 1 else None, (wb, wf)))
 
-    def phase_groups(batched):
-        if order == "level":
-            return join_levels(nodes, batched)
-        return [[n.idx] for n in nodes if not n.is_leaf and n.batched == batched]
+    def put_raw(data):
+        nonlocal blob
+        start = (len(blob) + ALIGN - 1) // ALIGN * ALIGN
+        blob += b"\0" * (start - len(blob)) + data
+        return start
+
+    def run_phase(batched, phase):
+        for programs_, joins in phase_groups(nodes, batched, order, programs):
+            if programs_:
+                tree_launch(programs_, phase, batched)
+            if joins:
+                group_launches(joins, phase)
+
+    def tree_launch(mine, phase, batched):
+        """One launch of programs, the longest streams first."""
+        block0, wb, wf, built, descs = 0, 0, 0, [], []
+        waves = TREE_WAVES_MANY if batched and W >= TREE_MANY else TREE_WAVES
+        for p in mine:
+            built.append(tree_words(p, nodes, waves, lambda n: n.rec if scaled else 0,
+                                    (one_at[0], one_rec if scaled else 0)) + (p,))
+            for i in p.members:
+                b, f = join_traffic(nodes[i], nodes, W, esize)
+                wb, wf = wb + b, wf + f
+        for words, streams, p in sorted(built, key=lambda b: -b[1].shape[1]):
+            td = _lib.TreeDesc(ntask=streams.shape[1], nslots=len(p.slot) if scaled else 0, block0=block0,
+                               nblocks=W if batched else 1)
+            block0 += td.nblocks
+            descs.append((td, put_raw(words.tobytes()), put_raw(streams.tobytes())))
+        at = put_raw(bytes(ctypes.sizeof(_lib.TreeDesc) * len(descs)))
+        tree_places.append((at, descs))
+        phase.append(("tree", Launch(op=_lib.TO_OP_FOLD_TREE, count=len(descs), grid=block0, iaux0=waves,
+                                     lds=max(16, max(p.lds for p in mine))), at, None, (wb, wf)))
+
+    tree_places = []
 
     def clear(a, b):
         return ("clear", Launch(op=_lib.TO_OP_SCALE_CLEAR, grid=max(1, min(1024, -(-(b - a) // 256))),
@@ -648,8 +888,7 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
     pro, wave = [], []
     if scaled and prog.rec_ranges[1] > prog.rec_ranges[0]:
         pro.append(clear(*prog.rec_ranges[:2]))
-    for grp in phase_groups(False):
-        group_launches(grp, pro)
+    run_phase(False, pro)
     root = nodes[-1]
     prog.root_const = not root.batched
     if scaled and prog.rec_ranges[2] > prog.rec_ranges[1]:
@@ -666,8 +905,7 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
     if leaf_descs:
         wave.append(("leaf", Launch(op=_lib.TO_OP_LEAF_GATHER, count=len(leaf_descs), grid=block0, aux3=wave_params),
                      put(leaf_descs), None, (sum(esize * (W << ld.rank) for ld in leaf_descs), 0)))
-    for grp in phase_groups(True):
-        group_launches(grp, wave)
+    run_phase(True, wave)
     root_launch = Launch(op=_lib.TO_OP_ROOT_REDUCE, grid=1, aux0=root.ptr, aux1=recp(root),
                          aux2=prog.accum.data_ptr(), aux3=wave_params + (16 if prog.root_const else 0),
                          iaux0=1 if prog.root_const else W)
@@ -676,9 +914,14 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
         wave.append(("advance", Launch(op=_lib.TO_OP_WAVE_ADVANCE, grid=1, aux3=wave_params, iaux0=W), None, None,
                      (0, 0)))
 
-    prog.blob_host = np.frombuffer(bytes(blob) or b"\0", dtype=np.uint8).copy()
-    prog.blob = device_alloc(prog.blob_host.nbytes)
+    prog.blob = device_alloc(max(1, len(blob)))
     bbase = prog.blob.data_ptr()
+    for at, descs in tree_places:
+        for td, ops_at, tasks_at in descs:
+            td.ops, td.tasks, td.recs = bbase + ops_at, bbase + tasks_at, rbase
+        raw = b"".join(bytes(td) for td, _, _ in descs)
+        blob[at:at + len(raw)] = raw
+    prog.blob_host = np.frombuffer(bytes(blob) or b"\0", dtype=np.uint8).copy()
     for L, off in prog.build:
         L.descs = bbase + off
     prog.build = [L for L, _ in prog.build]
@@ -696,6 +939,7 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
         nodes=len(nodes), joins=len(joins), batched_joins=sum(1 for n in joins if n.batched),
         splitk=sum(1 for n in joins if n.geom["var"].get("lsplit")),
         gemm=sum(1 for n in joins if n.geom["var"]["kind"] == "gemm"),
+        tree_joins=sum(len(p.members) for p in programs),
         arena_bytes=peak, table_bytes=int(image.host.nbytes),
         # leaves described for the device (a vector of ones among them needs no table)
         device_built_leaves=sum(1 for t in tables.values() if t.spec is not None),

@@ -46,12 +46,13 @@ ROWS_MIN_BITS_BATCH = 20
 class _Arena:
     """First-fit placement of buffers in one linear address space (bytes)."""
 
-    def __init__(self):
+    def __init__(self, align=ALIGN):
         self.free = [(0, 1 << 62)]
         self.peak = 0
+        self.align = align
 
     def alloc(self, nbytes):
-        nbytes = max(ALIGN, (nbytes + ALIGN - 1) // ALIGN * ALIGN)
+        nbytes = max(self.align, (nbytes + self.align - 1) // self.align * self.align)
         for i, (start, size) in enumerate(self.free):
             if size >= nbytes:
                 if size == nbytes:

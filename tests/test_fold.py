@@ -102,6 +102,89 @@ class FoldEmulator(emulator.Emulator):
                     m = np.float32(np.max(np.abs(val)))
                     self.set_rec(d.cs, b, exp=e, maxbits=int(m.view(np.uint32)))
 
+    def op_15(self, L):
+        # block by block: the streams' tasks level by level; LDS starts as NaN, every tensor
+        # is read only after its level, and every wave meets the same barriers
+        esz, waves = self.dt().itemsize, int(L.iaux0)
+        for i in range(L.count):
+            d = self.heap.read_struct(_lib.TreeDesc, L.descs + i * ctypes.sizeof(_lib.TreeDesc))
+            st = self.heap.view(d.tasks, np.uint32, waves * d.ntask).reshape(waves, -1).astype(np.int64)
+            bar = st >> 31
+            assert np.all(bar == bar[0]) and np.all(bar[:, -1] == 1)
+            ops = self.heap.view(d.ops, np.uint32, _lib.TO_TREE_WORDS * (1 + int((st & 0xffff).max())))
+            ops = ops.reshape(-1, _lib.TO_TREE_WORDS)
+            ops = ops.astype(np.int64)
+            for batch in range(d.nblocks):
+                data = np.full((L.lds - (8 * d.nslots + 15) // 16 * 16) // esz, np.nan, dtype=self.dt)
+                recs = [[0, 0.0] for _ in range(d.nslots)]
+                pending, done = [], set()
+                for col in range(d.ntask):
+                    for t in st[:, col]:
+                        if t & _lib.TO_TREE_IDLE:
+                            continue
+                        k, c, step = int(t & 0xffff), int(t >> 16 & 127), 1 << int(t >> 23 & 15)
+                        for chunk in range(c, 1 << int(ops[k][0] >> 12 & 15), step):
+                            assert (k, chunk) not in done
+                            done.add((k, chunk))
+                            self._tree_task(d, ops[k], chunk, batch, data, recs, pending)
+                    if bar[0, col]:
+                        for write in pending:
+                            write()
+                        pending = []
+                assert not pending
+                assert len(done) == sum(1 << int(o[0] >> 12 & 15) for o in ops)
+                self.operands = getattr(self, "operands", set()) | {int(o[0] >> 16 & 3) + 1 for o in ops}
+
+    def _tree_task(self, d, op, chunk, batch, data, recs, pending):
+        head = int(op[0])
+        lo, lk, nloop, nchunk = head & 15, head >> 4 & 15, head >> 8 & 15, head >> 12 & 15
+        nops = (head >> 16 & 3) + 1
+        assert lo + lk <= 6 and 6 + nchunk + nloop <= 16
+        assert nops <= 2 or (nchunk == 0 and nloop <= 2)
+        assert nops >= 2
+        esz = self.dt().itemsize
+        prod, e, f = 1.0, 0, 1.0
+        for j in list(range(nops)) + [4]:
+            bits = op[64 + 16 * j:80 + 16 * j] if j < 4 else op[32:48]
+            assert not np.any(bits[lo + lk:6])
+            assert np.array_equal(op[128 + 64 * j:192 + 64 * j], _spread(bits, 0, 6))
+            o = _spread(bits, 0, lo) + sum(int(bits[6 + b]) for b in range(nchunk) if chunk >> b & 1)
+            k = (_spread(bits, lo, lk)[:, None] + _spread(bits, 6 + nchunk, nloop)[None, :]).ravel()
+            if j == 4:
+                break
+            idx = o[:, None] + k[None, :]
+            addr = int(op[1 + 2 * j]) | int(op[2 + 2 * j]) << 32
+            slot = int(op[16 + j])
+            if head >> (20 + j) & 1:
+                prod = prod * data[addr + idx].astype(np.float64)
+                exp, bits_ = (recs[slot][0], int(np.float32(recs[slot][1]).view(np.uint32))) if self.scaled else (0, 0)
+            else:
+                src = self.heap.view(addr + batch * int(op[11 + j]) * esz, self.dt, int(idx.max()) + 1)
+                prod = prod * src[idx].astype(np.float64)
+                exp, bits_ = self.get_rec(d.recs, slot + (batch if head >> (25 + j) & 1 else 0)) if self.scaled else (0, 0)
+            if self.scaled:
+                e += exp + emulator._scale_exp(bits_)
+                f *= 2.0 ** -emulator._scale_exp(bits_)
+        assert not np.any(k)
+        v = (prod.sum(axis=1) * f).astype(self.dt)
+        assert np.all(np.isfinite(v))
+        addr, slot = int(op[9]) | int(op[10]) << 32, int(op[20])
+
+        def write():
+            m = float(np.max(np.abs(v)))
+            if head >> 24 & 1:
+                data[addr + o] = v
+                if self.scaled:
+                    recs[slot][1] = max(recs[slot][1], m)
+                    if chunk == 0:
+                        recs[slot][0] = e
+            else:
+                self.heap.view(addr + batch * int(op[15]) * esz, self.dt, int(o.max()) + 1)[o] = v
+                if self.scaled:
+                    r = slot + (batch if head >> 29 & 1 else 0)
+                    self.set_rec(d.recs, r, exp=e if chunk == 0 else None, maxbits=int(np.float32(m).view(np.uint32)))
+        pending.append(write)
+
     def op_10(self, L):
         # products whose batch items share scale records in groups of 2^hlog
         for i in range(L.count):
@@ -174,8 +257,10 @@ def test_fixture_folded(path, et, tol):
     want = numpy_oracle.contract_sliced(doc)
     total = 1 << len(plan.groups_to_slice)
     for W in sorted({1, 3, total}):
-        got, prog, _ = emulate(plan, et, W)
+        got, prog, emu = emulate(plan, et, W)
         assert got == pytest.approx(want, rel=tol)
+        assert emu.operands >= {2, 3, 4}
+        assert prog.stats["tree_joins"] > prog.stats["joins"] // 2
     got, _, _ = emulate(plan, et, total, device_leaves=False, group_levels=False, regroup=False)
     assert got == pytest.approx(want, rel=tol)
 
