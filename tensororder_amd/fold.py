@@ -299,9 +299,11 @@ def _canonical(node, want):
     return node.rank == len(want) and all(node.off.get(v) == 1 << i for i, v in enumerate(want))
 
 
-def choose(n, nodes, W, esize):
+def choose(n, nodes, W, esize, launch_bound=False):
     """Kernel form and launch shape of one folded join for W slices (``n.geom``).  A dense
-    join also fixes its result's bit order ([kept shared][X][Y])."""
+    join also fixes its result's bit order ([kept shared][X][Y]).  ``launch_bound`` (the
+    many-instance batch): every product in the 64x64 form, so that those of a step share a
+    launch."""
     A = nodes[n.left]
     B = nodes[n.right] if n.right >= 0 else None
     nb = W if n.batched else 1
@@ -329,7 +331,10 @@ def choose(n, nodes, W, esize):
             _reordered(n, yo + xo + kept)
             g = dict(fx=len(xo), fy=len(yo), s=s, shf=len(yo), shy=0, xf=list(range(s, s + len(xo))),
                      xs=list(range(s)), yf=list(range(s, s + len(yo))), ys=list(range(s)), x_is_left=X is A)
-            v = schedule.choose_variant(g, nb << h, esize)
+            v = schedule.choose_variant(g, nb << h, esize, launch_bound=launch_bound)
+            if h and v.get("lsplit"):  # the finishing launch has one record per batch item
+                del v["lsplit"], v["nsplit"], v["nout"], v["fin_blocks"]
+                v["nblocks"] = int(min((nb << h) << (len(xo) + len(yo) - 12), schedule.MAX_GEMM_BLOCKS))
             want_x, want_y = ks + xo + kept, ks + yo + kept
             v.update(perm_x=not _canonical(X, want_x), perm_y=not _canonical(Y, want_y), hlog=h, want_x=want_x,
                      want_y=want_y)
@@ -377,17 +382,17 @@ def choose(n, nodes, W, esize):
     n.geom = g
 
 
-def choose_all(nodes, W, esize):
+def choose_all(nodes, W, esize, launch_bound=False):
     for n in nodes:
         if not n.is_leaf:
-            choose(n, nodes, W, esize)
+            choose(n, nodes, W, esize, launch_bound)
 
 
 def _scratch(arena, n, nodes, nb, esize, table):
     """Scratch a join needs while it runs: split sums, permuted operands of a product."""
     v = n.geom["var"]
     blocks = {}
-    if v["kind"] == "fold" and v["lsplit"]:
+    if v.get("lsplit"):
         blocks["partial"] = arena.alloc(v["nout"] * v["nsplit"] * 8)
     if v["kind"] == "gemm":
         for key, i in (("perm_x", n.geom["X"]), ("perm_y", n.geom["Y"])):
@@ -459,9 +464,9 @@ def _program(nodes, root, stage, esize, scaled):
     return p
 
 
-def tree_programs(nodes, W, esize, scaled):
+def tree_programs(nodes, W, esize, scaled, lds=None):
     """The programs of a plan whose joins carry their forms: maximal connected parts of small
-    joins of one phase whose intermediates fit LDS."""
+    joins of one phase whose intermediates fit ``lds`` bytes."""
     # a small join's stage: its phase and the number of large joins on the longest path below
     # it; programs are the connected joins of one stage, so none waits for more than it reads
     stage, depth = {}, {}
@@ -482,7 +487,7 @@ def tree_programs(nodes, W, esize, scaled):
     while todo:
         i = todo.pop()
         p = _program(nodes, i, stage, esize, scaled)
-        if p.lds > (TREE_LDS_MANY if p.batched and W >= TREE_MANY else TREE_LDS):
+        if p.lds > (lds or (TREE_LDS_MANY if p.batched and W >= TREE_MANY else TREE_LDS)):
             # its root runs as a launch of its own, what is below as programs
             todo += [c for c in (nodes[i].left, nodes[i].right) if stage.get(c) == stage[i]]
             del stage[i]
@@ -681,6 +686,15 @@ def join_records(n, nodes, W, esize, scaled, abase, scratch, recp, one):
         gd.cb = 1 << (g["fx"] + g["fy"])
         gd.nbatch = nb << h
         out.append(("gemm", _lib.TO_OP_GEMM, v["tile"], 0, gd, v["nblocks"]))
+        if v.get("lsplit"):
+            # split K: the parts' partial sums go to scratch, a finishing launch writes C
+            f = _lib.JoinDesc()
+            f.c, f.cb, f.nsplit = n.ptr, n.bstride, v["nsplit"]
+            gd.c = f.partial = abase + scratch["partial"][0]
+            gd.lsplit = v["lsplit"]
+            f.xs, f.ys, f.cs, f.xsb, f.ysb = gd.as_, gd.bs, gd.cs, gd.asb, gd.bsb
+            f.fx, f.fy, f.shf, f.shy, f.nbatch, f.nblocks = g["fx"], g["fy"], g["shf"], 0, nb, v["fin_blocks"]
+            out.append(("finish", _lib.TO_OP_JOIN_FINISH, 0, 0, f, f.nblocks))
         return out
     d = FoldDesc()
     yptr, yrec, ystride, yrecs = one[0], one[1], 0, 0
@@ -944,4 +958,196 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
         # leaves described for the device (a vector of ones among them needs no table)
         device_built_leaves=sum(1 for t in tables.values() if t.spec is not None),
         launches_prologue=len(prog.prologue), launches_wave=len(prog.wave))
+    return prog
+
+
+# many-instance batches: programs keep to this much LDS, so that two blocks of 16 waves share
+# a CU
+TREE_LDS_BATCH = 64 * 1024
+
+
+def analyse_batch(instances, esize, regroup=True):
+    """Per (tree, tables) of unsliced plans: its folded nodes with their forms, programs,
+    memory plan and arena region; None when a plan cannot be folded."""
+    per = []
+    for tree, tables in instances:
+        folded = analyse(tree, tables, esize, regroup) if has_copies(tables) else None
+        if folded is None:
+            return None
+        nodes, missing = folded
+        if any(n.batched for n in nodes):
+            raise ValueError("batched instances must be unsliced plans")
+        choose_all(nodes, 1, esize, launch_bound=True)
+        programs = tree_programs(nodes, 1, esize, esize == 4, TREE_LDS_BATCH)
+        peak, scratch = plan_memory(nodes, 1, esize, "level", programs)
+        words = sum(len(p.members) for p in programs) * 4 * _lib.TO_TREE_WORDS
+        per.append(dict(nodes=nodes, missing=missing, tables=tables, programs=programs, scratch=scratch,
+                        region=(max(peak, ALIGN) + ALIGN - 1) // ALIGN * ALIGN,
+                        fixed=sum(t.size for t in tables.values()) * esize + 1024 * len(nodes) + words))
+    return per
+
+
+def compile_batch(per, entry_type, device_alloc, arena):
+    """One grouped schedule (``batch.BatchProgram``) of analysed instances: step k runs the
+    k-th group of every instance -- its programs in one launch, its other joins in one launch
+    per kernel form -- through the given arena, every instance in its own region; an
+    instance's root goes to its accumulator right after its last step."""
+    from .batch import MAP_MIN_DESCS, BatchProgram
+
+    esize = 8 if entry_type == _lib.TO_F64 else 4
+    scaled = entry_type == _lib.TO_F32S
+    fdtype = np.float64 if esize == 8 else np.float32
+    prog = BatchProgram()
+    prog.count, prog.per, prog.arena = len(per), per, arena
+    # leaf tables of all instances in one buffer, a stored 1.0 last
+    chunks, top, bases = [], 0, []
+    prog.leaf_factors = []
+    for inst in per:
+        inst["image"] = im = schedule.leaf_image(inst["nodes"], inst["tables"], 0, scaled, fdtype)
+        bases.append(top)
+        chunks.append(im.host)
+        top += im.host.size
+        prog.leaf_factors.append((im.factor[0], im.factor[1] + inst["missing"]))
+    chunks.append(np.ones(1, fdtype))
+    prog.table_host = np.concatenate(chunks)
+    one = top
+    # scale records: constant leaves and the 1.0, then what the launches write
+    nrec, prog.rec_init = 1, [(0, 0)]
+    for inst in per:
+        for n in inst["nodes"]:
+            if n.is_leaf:
+                n.rec, n.rec_stride = nrec, 0
+                if scaled:
+                    prog.rec_init.append((nrec, inst["image"].exp0[n.tensor]))
+                nrec += 1
+    join_rec0 = nrec
+    for inst in per:
+        inst["in_lds"] = {i for p in inst["programs"] for i in p.members if i != p.root}
+        for n in inst["nodes"]:
+            if not n.is_leaf and n.idx not in inst["in_lds"]:
+                n.rec, n.rec_stride = nrec, 0
+                nrec += 1
+    prog.rec_count = nrec if scaled else 0
+    prog.table = device_alloc(prog.table_host.nbytes)
+    prog.recs = device_alloc(max(1, nrec) * 16)
+    prog.accum = device_alloc(len(per) * ctypes.sizeof(_lib.Accum))
+    prog.start = device_alloc(64)
+    tbase, rbase, abase = prog.table.data_ptr(), prog.recs.data_ptr(), arena.data_ptr()
+    one_at = (tbase + one * esize, rbase if scaled else 0)
+
+    def recp(n):
+        return rbase + n.rec * 16 if scaled else 0
+
+    blob = bytearray()
+
+    def put(data):
+        nonlocal blob
+        start = (len(blob) + ALIGN - 1) // ALIGN * ALIGN
+        blob += b"\0" * (start - len(blob)) + data
+        return start
+
+    base, builds, steps, roots = 0, [], [], {}
+    for k, inst in enumerate(per):
+        nodes = inst["nodes"]
+        at, im = bases[k], inst["image"]
+        for n in nodes:
+            n.bstride = 0
+            if n.is_leaf:
+                n.ptr = tbase + (at + im.off[n.tensor]) * esize
+            elif n.idx not in inst["in_lds"]:
+                n.ptr = abase + base + n.buf[0]
+        for t, v0, v1 in im.builds:
+            bd = inst["tables"][t].spec.desc(tbase + (at + im.off[t]) * esize, v0, v1)
+            bd.block0 = builds[-1].block0 + builds[-1].nblocks if builds else 0
+            builds.append(bd)
+        groups = phase_groups(nodes, False, "level", inst["programs"])
+        for i, grp in enumerate(groups):
+            while len(steps) <= i:
+                steps.append(([], {}))
+            for p in grp[0]:
+                steps[i][0].append((p, nodes))
+            for j in grp[1]:
+                scratch = {key: (base + blk[0], blk[1]) for key, blk in inst["scratch"].get(j, {}).items()}
+                for kind, op, variant, lds, st, nblk in join_records(nodes[j], nodes, 1, esize, scaled, abase, scratch,
+                                                                     recp, one_at):
+                    work = join_traffic(nodes[j], nodes, 1, esize) if kind in ("fold", "gemm") else (0, 0)
+                    if kind == "permute":
+                        work = (2 * esize << int(st.rank), 0)
+                    steps[i][1].setdefault((schedule.KIND_ORDER[kind], op, variant), []).append((kind, st, nblk, lds, work))
+        root = nodes[-1]
+        rd = _lib.RootDesc(root=root.ptr, rec=recp(root), acc=prog.accum.data_ptr() + k * ctypes.sizeof(_lib.Accum))
+        roots.setdefault(len(groups) - 1, []).append(rd)
+        base += inst["region"]
+
+    build_at = put(b"".join(bytes(b) for b in builds)) if builds else None
+    pending = [(Launch(op=_lib.TO_OP_BATCH_BEGIN, grid=max(1, min(64, -(-len(per) // 256))), aux2=prog.accum.data_ptr(),
+                       aux3=prog.start.data_ptr(), iaux0=len(per)), None, None, ("begin", -1), (0, 0))]
+    if scaled and nrec > join_rec0:
+        pending.append((Launch(op=_lib.TO_OP_SCALE_CLEAR, grid=max(1, min(1024, -(-(nrec - join_rec0) // 256))),
+                               aux0=rbase + join_rec0 * 16, iaux0=nrec - join_rec0), None, None, ("clear", -1), (0, 0)))
+    tree_places = []
+
+    def bmap(blocks):
+        return put(np.repeat(np.arange(len(blocks), dtype=np.int32), blocks).tobytes()) \
+            if len(blocks) >= MAP_MIN_DESCS else None
+
+    for i, (trees, keyed) in enumerate(steps):
+        if trees:
+            waves = TREE_WAVES_MANY if len(trees) >= TREE_MANY else TREE_WAVES
+            built, wb, wf = [], 0, 0
+            for p, nodes in trees:
+                built.append(tree_words(p, nodes, waves, lambda n: n.rec if scaled else 0, (one_at[0], 0)) + (p,))
+                for j in p.members:
+                    b, f = join_traffic(nodes[j], nodes, 1, esize)
+                    wb, wf = wb + b, wf + f
+            built.sort(key=lambda b: -b[1].shape[1])  # the longest streams start first
+            descs = []
+            for j, (words, streams, p) in enumerate(built):
+                td = _lib.TreeDesc(ntask=streams.shape[1], nslots=len(p.slot) if scaled else 0, block0=j, nblocks=1)
+                descs.append((td, put(words.tobytes()), put(streams.tobytes())))
+            at = put(bytes(ctypes.sizeof(_lib.TreeDesc) * len(descs)))
+            tree_places.append((at, descs))
+            pending.append((Launch(op=_lib.TO_OP_FOLD_TREE, count=len(descs), grid=len(descs), iaux0=waves,
+                                   lds=max(16, max(b[2].lds for b in built))), at, bmap([1] * len(descs)), ("tree", i),
+                            (wb, wf)))
+        for key in sorted(keyed):
+            grp = sorted(keyed[key], key=lambda r: -block_cost(r[1]))
+            block0 = 0
+            for _, st, nblk, _, _ in grp:
+                st.block0 = block0
+                block0 += nblk
+            at = put(b"".join(bytes(r[1]) for r in grp))
+            pending.append((Launch(op=key[1], variant=key[2], count=len(grp), grid=block0, lds=max(r[3] for r in grp)),
+                            at, bmap([r[2] for r in grp]), (grp[0][0], i),
+                            (sum(r[4][0] for r in grp), sum(r[4][1] for r in grp))))
+        if i in roots:
+            at = put(b"".join(bytes(r) for r in roots[i]))
+            pending.append((Launch(op=_lib.TO_OP_ROOT_STORE, count=len(roots[i]), grid=max(1, -(-len(roots[i]) // 256))),
+                            at, None, ("root", i), (0, 0)))
+    prog.blob = device_alloc(max(1, len(blob)))
+    bbase = prog.blob.data_ptr()
+    for at, descs in tree_places:
+        for td, ops_at, tasks_at in descs:
+            td.ops, td.tasks, td.recs = bbase + ops_at, bbase + tasks_at, rbase
+        raw = b"".join(bytes(td) for td, _, _ in descs)
+        blob[at:at + len(raw)] = raw
+    prog.blob_host = np.frombuffer(bytes(blob) or b"\0", dtype=np.uint8).copy()
+    prog.build = [] if build_at is None else [
+        Launch(op=_lib.TO_OP_LEAF_BUILD, count=len(builds), grid=builds[-1].block0 + builds[-1].nblocks,
+               descs=bbase + build_at)]
+    prog.work = []
+    for L, at, mat, info, work in pending:
+        if at is not None:
+            L.descs = bbase + at
+        if mat is not None:
+            L.aux1 = bbase + mat
+        prog.launches.append(L)
+        prog.info.append(info)
+        prog.work.append(work)
+    kinds = {}
+    for kind, _ in prog.info:
+        kinds[kind] = kinds.get(kind, 0) + 1
+    prog.stats = dict(instances=len(per), steps=len(steps), launches=len(prog.launches),
+                      joins=sum(1 for inst in per for n in inst["nodes"] if not n.is_leaf),
+                      arena_bytes=base, launches_per_kind=kinds)
     return prog

@@ -471,15 +471,34 @@ class HipAPI(BaseTensorAPI):
             if groups:
                 raise ValueError("prepare_batch takes unsliced plans")
             instances.append((tree, tables))
-        per = batch.analyse_batch(instances, self._entry_type, regroup=self._regroup)
-        waves = batch.admission_waves(per, self._budget())
+        budget = self._budget()
+        per = fold.analyse_batch(instances, self._esize, self._regroup)
+        folded = per is not None
+        # instances are admitted by what their tensors take with one axis per edge, folded or
+        # not (see choose_folded_batch); the analysis that gives it is needed only where all
+        # of it at once might not fit
+        bound = sum(schedule.peak_bound(tree, self._esize) + sum(t.size for t in tables.values()) * self._esize +
+                    2048 * len(tables) for tree, tables in instances) if folded else None
+        if folded and max(bound, sum(p["region"] + p["fixed"] for p in per)) <= budget:
+            waves = [list(range(len(per)))] if per else []
+        else:
+            walk = batch.analyse_batch(instances, self._entry_type, regroup=self._regroup)
+            if folded:
+                for p, q in zip(per, walk):
+                    q["region"] = max(q["region"], p["region"] + p["fixed"] - q["fixed"])
+            else:
+                per = walk
+            waves = batch.admission_waves(walk, budget)
         if waves is None:
             raise OutOfMemoryError
         arena = self._alloc(max(max(batch.wave_arena_bytes(per, w) for w in waves), schedule.ALIGN))
         progs = []
         for w in waves:
-            prog = batch.compile_batch(None, self._entry_type, self._alloc, regroup=self._regroup,
-                                       per=[per[i] for i in w], arena=arena)
+            if folded:
+                prog = fold.compile_batch([per[i] for i in w], self._entry_type, self._alloc, arena)
+            else:
+                prog = batch.compile_batch(None, self._entry_type, self._alloc, regroup=self._regroup,
+                                           per=[per[i] for i in w], arena=arena)
             self._upload(prog.table, prog.table_host.tobytes())
             self._upload(prog.blob, prog.blob_host.tobytes())
             self._run(prog.build)  # OR / variable leaf tables written on the device

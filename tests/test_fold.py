@@ -36,6 +36,8 @@ def _spread(entries, lo, n):
 
 
 class FoldEmulator(emulator.Emulator):
+    TABLE_DESCS = {**emulator.Emulator.TABLE_DESCS, _lib.TO_OP_FOLD: "FoldDesc", _lib.TO_OP_FOLD_TREE: "TreeDesc"}
+
     def __init__(self, heap, entry_type):
         super().__init__(heap, entry_type)
         self.forms = set()
@@ -189,6 +191,10 @@ class FoldEmulator(emulator.Emulator):
         # products whose batch items share scale records in groups of 2^hlog
         for i in range(L.count):
             d = self.heap.read_struct(_lib.GemmDesc, L.descs + i * ctypes.sizeof(_lib.GemmDesc))
+            if d.lsplit:
+                assert d.hlog == 0 and L.count == 1
+                super().op_10(L)
+                continue
             M, N, K = 1 << d.mlog, 1 << d.nlog, 1 << d.klog
             esz = self.dt().itemsize
             cidx = np.arange(M)[:, None] * d.ldcm + np.arange(N)[None, :] * d.ldcn
@@ -263,6 +269,41 @@ def test_fixture_folded(path, et, tol):
         assert prog.stats["tree_joins"] > prog.stats["joins"] // 2
     got, _, _ = emulate(plan, et, total, device_leaves=False, group_levels=False, regroup=False)
     assert got == pytest.approx(want, rel=tol)
+
+
+@pytest.mark.parametrize("et,tol", [(_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)])
+def test_batch_folded(et, tol):
+    # uneven instances in one grouped schedule: programs, and joins outside them (LDS for the
+    # programs is kept so small that many are), grouped launches with block maps
+    esize = 8 if et == _lib.TO_F64 else 4
+    plans = [_formula_plan("vc", n, seed, 0) for seed, n in enumerate([10, 16, 24, 40, 30, 20, 18, 56])]
+    wants = [numpy_oracle.contract_sliced(plan_io.plan_to_dict(p)) for p in plans]
+    for lds, bits in ((64 * 1024, 16), (256, 5)):
+        saved = fold.TREE_LDS_BATCH, fold.TREE_BITS
+        fold.TREE_LDS_BATCH, fold.TREE_BITS = lds, bits
+        try:
+            per = fold.analyse_batch([plan_inputs(p)[1:3] for p in plans], esize)
+        finally:
+            fold.TREE_LDS_BATCH, fold.TREE_BITS = saved
+        heap = emulator.Heap()
+        arena = heap.alloc(sum(p["region"] for p in per))
+        prog = fold.compile_batch(per, et, heap.alloc, arena)
+        for buf, data in ((prog.table, prog.table_host), (prog.blob, prog.blob_host)):
+            heap.write(buf, data.tobytes())
+        if et == _lib.TO_F32S:
+            from tensororder_amd import batch
+
+            heap.write(prog.recs, batch.rec_init_bytes(prog))
+        emu = FoldEmulator(heap, et)
+        emu.run(prog.build)
+        for _ in range(2):  # replays
+            emu.run(prog.launches)
+            for i, want in enumerate(wants):
+                acc = heap.read_struct(_lib.Accum, prog.accum.data_ptr() + i * ctypes.sizeof(_lib.Accum))
+                fm, fe = prog.leaf_factors[i]
+                assert math.ldexp(acc.mant * fm, acc.exp + fe) == pytest.approx(want, rel=tol)
+        assert emu.maps_checked > 0
+        assert (prog.stats["steps"] > 4) == (bits == 5)
 
 
 def _formula_plan(kind, n, seed, slices):
