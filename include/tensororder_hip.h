@@ -66,7 +66,11 @@ extern "C" {
                                 one block per output (for nsplit >= 32) */
 #define TO_OP_SCALE_CLEAR 5  /* aux0: to_scale_rec*, iaux0: record count */
 #define TO_OP_ROOT_REDUCE 6  /* aux0: root values, aux1: to_scale_rec* (F32S) or 0,
-                                aux2: to_accum*, aux3: wave params (int64[2]) */
+                                aux2: to_accum*, aux3: wave params (int64[2]); variant 1: the
+                                wave at params[0] == 0 starts the sum anew, and params[0] then
+                                advances by iaux0, back to 0 after the last wave; iaux1: 0, or
+                                the address of a to_accum in host memory that the device can
+                                write, which gets a copy of the sum */
 #define TO_OP_WAVE_ADVANCE 7 /* aux3: wave params; adds iaux0 to params[0] */
 #define TO_OP_STEP_BEGIN 8   /* aux2: to_accum* (zeroed), aux3: wave params (params[0] = 0) */
 #define TO_OP_PERMUTE 9      /* descs: to_perm_desc[count]; variant 1: 16-byte chunk kernel,
@@ -92,6 +96,10 @@ extern "C" {
                          every descriptor of the launch with that y mode and nreg */
 #define TO_OP_FOLD_TREE 15 /* descs: to_tree_desc[count]; iaux0: waves per block (1 to 16, as many
                          as each program has streams); lds: the largest of their LDS needs */
+#define TO_OP_WAVE_BEGIN 16 /* TO_OP_LEAF_GATHER on the first iaux1 blocks of the grid and
+                               TO_OP_SCALE_CLEAR (aux0, iaux0) on the others, in one launch:
+                               descs: to_leaf_desc[count], whose records are not among those
+                               cleared; aux3: wave params */
 #define TO_OP_LEAF_BUILD 13  /* descs: to_leaf_build_desc[count]: leaf tables written from their
                                 compact descriptions (OR / variable leaves) */
 

@@ -28,7 +28,8 @@ TO_F64, TO_F32S = 0, 1
     TO_OP_LEAF_BUILD,
     TO_OP_FOLD,
     TO_OP_FOLD_TREE,
-) = range(1, 16)
+    TO_OP_WAVE_BEGIN,
+) = range(1, 17)
 TO_LEAF_VAR, TO_LEAF_OR = 0, 1  # leaf build kinds
 TO_STREAM_VEC = 0x100  # stream variant bit: the 16-byte form
 TO_STREAM_ROWS = 0x200  # stream variant: the row form

@@ -195,9 +195,8 @@ using Acc = double;
 // leaf gather: per batch item, copy row sum_g coef[g]*bit_g(slice) of each leaf table
 
 template <typename T, bool SCALED>
-__global__ __launch_bounds__(kBlock) void k_leaf_gather(const to_leaf_desc* __restrict__ descs,
-                                                        int ndesc, const int32_t* __restrict__ bmap,
-                                                        const int64_t* __restrict__ wave) {
+__device__ __forceinline__ void leaf_gather_body(const to_leaf_desc* __restrict__ descs, int ndesc,
+                                                 const int32_t* __restrict__ bmap, const int64_t* __restrict__ wave) {
     const to_leaf_desc* d = descs + find_desc(descs, ndesc, blockIdx.x, bmap);
     const int rank = d->rank;
     const int64_t E = 1ll << rank;
@@ -221,6 +220,13 @@ __global__ __launch_bounds__(kBlock) void k_leaf_gather(const to_leaf_desc* __re
             r->maxbits = __float_as_uint(1.0f);
         }
     }
+}
+
+template <typename T, bool SCALED>
+__global__ __launch_bounds__(kBlock) void k_leaf_gather(const to_leaf_desc* __restrict__ descs, int ndesc,
+                                                        const int32_t* __restrict__ bmap,
+                                                        const int64_t* __restrict__ wave) {
+    leaf_gather_body<T, SCALED>(descs, ndesc, bmap, wave);
 }
 
 // ---------------------------------------------------------------------------------
@@ -699,6 +705,22 @@ __global__ __launch_bounds__(kBlock) void k_scale_clear(to_scale_rec* recs, int6
     }
 }
 
+// The start of a wave in one launch: blocks below ngather gather the leaves, the others clear
+// the scale records of the wave's joins (a launch costs a small wave 3-5 us).
+template <typename T, bool SCALED>
+__global__ __launch_bounds__(kBlock) void k_wave_begin(const to_leaf_desc* __restrict__ descs, int ndesc,
+                                                       const int32_t* __restrict__ bmap,
+                                                       const int64_t* __restrict__ wave, int ngather,
+                                                       to_scale_rec* recs, int64_t n) {
+    if ((int)blockIdx.x < ngather) {
+        leaf_gather_body<T, SCALED>(descs, ndesc, bmap, wave);
+        return;
+    }
+    const int64_t stride = (int64_t)(gridDim.x - ngather) * kBlock;
+    for (int64_t i = (int64_t)(blockIdx.x - ngather) * kBlock + threadIdx.x; i < n; i += stride)
+        recs[i] = to_scale_rec{0, 0u, 0u};
+}
+
 __global__ void k_wave_advance(int64_t* wave, int64_t step) {
     if (threadIdx.x == 0 && blockIdx.x == 0) wave[0] += step;
 }
@@ -745,8 +767,8 @@ __global__ void k_step_begin(to_accum* acc, int64_t* wave) {
 template <typename T, bool SCALED>
 __global__ __launch_bounds__(kBlock) void k_root_reduce(const T* __restrict__ roots,
                                                         const to_scale_rec* __restrict__ recs,
-                                                        to_accum* acc, const int64_t* __restrict__ wave,
-                                                        int nbatch) {
+                                                        to_accum* acc, int64_t* wave, int nbatch, int self,
+                                                        to_accum* host) {
     __shared__ int64_t emax_s[kBlock / 64];
     __shared__ double red[kBlock / 64];
     const int tid = threadIdx.x;
@@ -786,8 +808,9 @@ __global__ __launch_bounds__(kBlock) void k_root_reduce(const T* __restrict__ ro
     }
     const double total = block_sum(part, red);
     if (tid == 0) {
-        double am = acc->mant;
-        int64_t ae = acc->exp;
+        const bool fresh = self && begin == 0;  // the first wave starts the sum anew
+        double am = fresh ? 0.0 : acc->mant;
+        int64_t ae = fresh ? 0 : acc->exp;
         if (emax != INT64_MIN && total != 0.0) {
             if (am == 0.0) {
                 am = total;
@@ -805,9 +828,12 @@ __global__ __launch_bounds__(kBlock) void k_root_reduce(const T* __restrict__ ro
             am = m2;
             ae += e2;
         }
+        const int64_t count = (fresh ? 0 : acc->count) + nvalid;
         acc->mant = am;
         acc->exp = am == 0.0 ? 0 : ae;
-        acc->count += nvalid;
+        acc->count = count;
+        if (self) wave[0] = begin + nbatch < end ? begin + nbatch : 0;
+        if (host) *host = to_accum{am, am == 0.0 ? 0 : ae, count, 0};
     }
 }
 
@@ -2293,6 +2319,15 @@ int launch_one(const to_launch& L, hipStream_t st) {
                                reinterpret_cast<const to_leaf_desc*>(L.descs), L.count, bmap,
                                reinterpret_cast<const int64_t*>(L.aux3));
             break;
+        case TO_OP_WAVE_BEGIN:
+            if (L.iaux1 < 0 || L.iaux1 > L.grid || (L.iaux1 > 0 && (!L.descs || L.count <= 0)) || L.iaux0 < 0 ||
+                (L.iaux0 > 0 && (!L.aux0 || L.iaux1 == L.grid)))
+                return TO_ERR_INVALID;
+            hipLaunchKernelGGL((k_wave_begin<T, SCALED>), grid, block, 0, st,
+                               reinterpret_cast<const to_leaf_desc*>(L.descs), L.count, bmap,
+                               reinterpret_cast<const int64_t*>(L.aux3), (int)L.iaux1,
+                               reinterpret_cast<to_scale_rec*>(L.aux0), L.iaux0);
+            break;
         case TO_OP_JOIN_STREAM: {
             if (!L.descs || L.count <= 0) return TO_ERR_INVALID;
             const to_join_desc* d = reinterpret_cast<const to_join_desc*>(L.descs);
@@ -2354,8 +2389,8 @@ int launch_one(const to_launch& L, hipStream_t st) {
             hipLaunchKernelGGL((k_root_reduce<T, SCALED>), dim3(1), block, 0, st,
                                reinterpret_cast<const T*>(L.aux0),
                                reinterpret_cast<const to_scale_rec*>(L.aux1),
-                               reinterpret_cast<to_accum*>(L.aux2), reinterpret_cast<const int64_t*>(L.aux3),
-                               (int)L.iaux0);
+                               reinterpret_cast<to_accum*>(L.aux2), reinterpret_cast<int64_t*>(L.aux3),
+                               (int)L.iaux0, (int)(L.variant == 1), reinterpret_cast<to_accum*>(L.iaux1));
             break;
         case TO_OP_WAVE_ADVANCE:
             if (!L.aux3) return TO_ERR_INVALID;

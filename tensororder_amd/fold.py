@@ -745,9 +745,11 @@ def block_cost(st):
     return schedule.block_cost(st)
 
 
-def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, group_levels=True):
+def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, group_levels=True, host_alloc=None):
     """Build a ``schedule.Program`` of a folded plan (``folded``: what ``analyse`` returned)
-    for W slices."""
+    for W slices.  The program starts its own sum (TO_OP_ROOT_REDUCE, variant 1), so a run is
+    its prologue and waves alone; with ``host_alloc`` (host memory that the device writes)
+    the sum also lands there."""
     nodes, missing = folded
     esize = 8 if entry_type == _lib.TO_F64 else 4
     scaled = entry_type == _lib.TO_F32S
@@ -784,10 +786,13 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
                 n.rec, n.rec_stride = nrec, 0
                 nrec += 1
         wave_rec0 = nrec
-        for n in nodes:
-            if n.batched and n.idx not in in_lds:
-                n.rec, n.rec_stride = nrec, 1
-                nrec += W
+        for leaves in (True, False):  # the gather writes the leaves' records, the rest is cleared
+            for n in nodes:
+                if n.batched and n.is_leaf == leaves and n.idx not in in_lds:
+                    n.rec, n.rec_stride = nrec, 1
+                    nrec += W
+            if leaves:
+                clear_rec0 = nrec
         prog.rec_ranges = (pro_rec0, wave_rec0, nrec)
 
     prog.table = device_alloc(image.host.nbytes)
@@ -796,6 +801,7 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
     prog.recs = device_alloc(max(1, nrec) * 16)
     prog.params = device_alloc(4 * 8)
     prog.accum = device_alloc(32)
+    prog.host_accum = host_alloc(32) if host_alloc is not None else None
     prog.table_host, prog.coef_host, prog.rec_init = image.host, image.coef_host, rec_init
     tbase, abase, rbase = prog.table.data_ptr(), prog.arena.data_ptr(), prog.recs.data_ptr()
     wave_params = prog.params.data_ptr()
@@ -895,6 +901,8 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
 
     tree_places = []
 
+    prog.self_start = True
+
     def clear(a, b):
         return ("clear", Launch(op=_lib.TO_OP_SCALE_CLEAR, grid=max(1, min(1024, -(-(b - a) // 256))),
                                 aux0=rbase + a * 16, iaux0=b - a), None, None, (0, 0))
@@ -905,8 +913,6 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
     run_phase(False, pro)
     root = nodes[-1]
     prog.root_const = not root.batched
-    if scaled and prog.rec_ranges[2] > prog.rec_ranges[1]:
-        wave.append(clear(*prog.rec_ranges[1:]))
     leaf_descs, block0 = [], 0
     for n in nodes:
         if n.is_leaf and n.batched:
@@ -916,17 +922,18 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
                           nblocks=int(min(1024, -(-(W << n.rank) // 256))))
             block0 += ld.nblocks
             leaf_descs.append(ld)
-    if leaf_descs:
-        wave.append(("leaf", Launch(op=_lib.TO_OP_LEAF_GATHER, count=len(leaf_descs), grid=block0, aux3=wave_params),
+    nclear = nrec - clear_rec0 if scaled else 0
+    if leaf_descs or nclear:
+        clear_blocks = min(1024, -(-nclear // 256))
+        wave.append(("leaf", Launch(op=_lib.TO_OP_WAVE_BEGIN, count=len(leaf_descs), grid=block0 + clear_blocks,
+                                    aux0=rbase + clear_rec0 * 16 if nclear else 0, iaux0=nclear, iaux1=block0,
+                                    aux3=wave_params),
                      put(leaf_descs), None, (sum(esize * (W << ld.rank) for ld in leaf_descs), 0)))
     run_phase(True, wave)
-    root_launch = Launch(op=_lib.TO_OP_ROOT_REDUCE, grid=1, aux0=root.ptr, aux1=recp(root),
-                         aux2=prog.accum.data_ptr(), aux3=wave_params + (16 if prog.root_const else 0),
+    root_launch = Launch(op=_lib.TO_OP_ROOT_REDUCE, variant=1, grid=1, aux0=root.ptr, aux1=recp(root),
+                         iaux1=prog.host_accum.data_ptr() if prog.host_accum is not None else 0, aux2=prog.accum.data_ptr(), aux3=wave_params + (16 if prog.root_const else 0),
                          iaux0=1 if prog.root_const else W)
     (pro if prog.root_const else wave).append(("root", root_launch, None, None, (0, 0)))
-    if not prog.root_const:
-        wave.append(("advance", Launch(op=_lib.TO_OP_WAVE_ADVANCE, grid=1, aux3=wave_params, iaux0=W), None, None,
-                     (0, 0)))
 
     prog.blob = device_alloc(max(1, len(blob)))
     bbase = prog.blob.data_ptr()
@@ -987,11 +994,12 @@ def analyse_batch(instances, esize, regroup=True):
     return per
 
 
-def compile_batch(per, entry_type, device_alloc, arena):
+def compile_batch(per, entry_type, device_alloc, arena, host_alloc):
     """One grouped schedule (``batch.BatchProgram``) of analysed instances: step k runs the
     k-th group of every instance -- its programs in one launch, its other joins in one launch
     per kernel form -- through the given arena, every instance in its own region; an
-    instance's root goes to its accumulator right after its last step."""
+    instance's root goes to its accumulator right after its last step.  The accumulators and
+    the start time lie in host memory that the device writes (``host_alloc``)."""
     from .batch import MAP_MIN_DESCS, BatchProgram
 
     esize = 8 if entry_type == _lib.TO_F64 else 4
@@ -1030,8 +1038,8 @@ def compile_batch(per, entry_type, device_alloc, arena):
     prog.rec_count = nrec if scaled else 0
     prog.table = device_alloc(prog.table_host.nbytes)
     prog.recs = device_alloc(max(1, nrec) * 16)
-    prog.accum = device_alloc(len(per) * ctypes.sizeof(_lib.Accum))
-    prog.start = device_alloc(64)
+    prog.accum = host_alloc(len(per) * ctypes.sizeof(_lib.Accum))
+    prog.start = host_alloc(64)
     tbase, rbase, abase = prog.table.data_ptr(), prog.recs.data_ptr(), arena.data_ptr()
     one_at = (tbase + one * esize, rbase if scaled else 0)
 

@@ -81,7 +81,11 @@ class Executable:
     the accumulator, prologue (slice-invariant subtrees), then every wave of slices,
     replayed from HIP graphs when the API's ``graph`` option is on."""
 
-    def __init__(self, api, prog, total_slices):
+    # a run of at most this many launches is one graph: between graphs the device waits for
+    # the host
+    ONE_GRAPH_LAUNCHES = 512
+
+    def __init__(self, api, prog, total_slices, once=False):
         self.api = api
         self.prog = prog
         self.total = total_slices
@@ -91,12 +95,19 @@ class Executable:
         self.step_launches = [begin] + list(prog.prologue)
         self.wave_launches = list(prog.wave)
         self._graphs = []
-        self._pro_graph = None
-        self._wave_graph = None
-        if api._use_graph:
-            self._pro_graph = self._capture(self.step_launches)
-            if self.nwaves > 1:
-                self._wave_graph = self._capture(self.wave_launches)
+        # what a run replays, in order: graphs, or launch lists run one by one
+        first = list(prog.prologue) if prog.self_start else self.step_launches
+        runs = [first] + [self.wave_launches] * self.nwaves
+        if sum(len(r) for r in runs) <= self.ONE_GRAPH_LAUNCHES:
+            runs = [sum(runs, [])]
+        # a plan that runs once only pays for capturing waves that repeat
+        captured = {}
+        self._runs = []
+        for r in runs:
+            if id(r) not in captured:
+                use = api._use_graph and r and (not once or (r is self.wave_launches and self.nwaves > 2))
+                captured[id(r)] = (self._capture(r) if use else None, r)
+            self._runs.append(captured[id(r)])
 
     def _capture(self, launches):
         arr = _lib.launch_array(launches)
@@ -113,23 +124,22 @@ class Executable:
 
     def enqueue(self):
         """Queue one full contraction on the API's stream (no synchronisation)."""
-        if self._pro_graph is not None:
-            self._launch_graph(self._pro_graph)
-        else:
-            self.api._run(self.step_launches)
-        for _ in range(self.nwaves):
-            if self._wave_graph is not None:
-                self._launch_graph(self._wave_graph)
+        for graph, launches in self._runs:
+            if graph is not None:
+                self._launch_graph(graph)
             else:
-                self.api._run(self.wave_launches)
+                self.api._run(launches)
 
     def result(self):
         """Synchronise and read the (mantissa, exponent) slice sum."""
         api = self.api
         api.synchronize()
-        with api._torch.cuda.stream(api._stream):
-            acc_bytes = self.prog.accum[: ctypes.sizeof(_lib.Accum)].cpu().numpy().tobytes()
-        acc = _lib.Accum.from_buffer_copy(acc_bytes)
+        if self.prog.host_accum is not None:
+            acc = _lib.Accum.from_address(self.prog.host_accum.data_ptr())
+        else:
+            with api._torch.cuda.stream(api._stream):
+                acc_bytes = self.prog.accum[: ctypes.sizeof(_lib.Accum)].cpu().numpy().tobytes()
+            acc = _lib.Accum.from_buffer_copy(acc_bytes)
         fm, fe = getattr(self.prog, "leaf_factor", (1.0, 0))
         res = Result(acc.mant * fm, acc.exp + fe, acc.count)
         api.last_result = res
@@ -144,7 +154,7 @@ class Executable:
         for g in self._graphs:
             self.api._lib.to_graph_destroy(g)
         self._graphs = []
-        self._pro_graph = self._wave_graph = None
+        self._runs = [(None, launches) for _, launches in self._runs]
 
 
 class BatchExecutable:
@@ -194,6 +204,7 @@ class BatchExecutable:
         api.synchronize()
         size = ctypes.sizeof(_lib.Accum)
         res, ends = [], []
+        # (no copies where the accumulators lie in host memory)
         with api._torch.cuda.stream(api._stream):
             start = int(self.progs[0].start[:8].cpu().numpy().view(np.int64)[0])
             for prog in self.progs:
@@ -327,6 +338,10 @@ class HipAPI(BaseTensorAPI):
         except self._torch.OutOfMemoryError:
             raise OutOfMemoryError
 
+    def _alloc_host(self, nbytes):
+        """Host memory that the device writes (pinned)."""
+        return self._torch.empty(max(1, int(nbytes)), dtype=self._torch.uint8, pin_memory=True)
+
     def _upload(self, dst, host_bytes):
         src = self._torch.from_numpy(np.frombuffer(host_bytes, dtype=np.uint8).copy())
         with self._torch.cuda.stream(self._stream):
@@ -384,14 +399,15 @@ class HipAPI(BaseTensorAPI):
                 raise OutOfMemoryError
             W = max(1, W // 2)
 
-    def _compile(self, tree, tables, num_groups, total_slices, group_levels=True):
+    def _compile(self, tree, tables, num_groups, total_slices, group_levels=True, once=False):
         """Compile and upload a plan; returns an ``Executable``.  ``group_levels=False``
-        keeps one launch per join (per-join timing)."""
+        keeps one launch per join (per-join timing); ``once``: the plan runs a single time."""
         folded = fold.analyse(tree, tables, self._esize, self._regroup) if fold.has_copies(tables) else None
         if folded is not None:
             W = self.choose_folded_batch(folded, tree, tables, total_slices)
-            prog = fold.compile_program(folded, tables, num_groups, self._entry_type, W, self._alloc, group_levels)
-            return self._resident(prog, total_slices)
+            prog = fold.compile_program(folded, tables, num_groups, self._entry_type, W, self._alloc, group_levels,
+                                        self._alloc_host)
+            return self._resident(prog, total_slices, once)
         nodes = schedule.analyse(tree, tables, self._regroup)
         W = self.choose_batch(nodes, tables, total_slices)
         if self._autotune:
@@ -401,9 +417,9 @@ class HipAPI(BaseTensorAPI):
                 autotune.save(schedule.TUNED)
         prog = schedule.compile_program(tree, tables, num_groups, self._entry_type, W, self._alloc,
                                         regroup=self._regroup, group_levels=group_levels)
-        return self._resident(prog, total_slices)
+        return self._resident(prog, total_slices, once)
 
-    def _resident(self, prog, total_slices):
+    def _resident(self, prog, total_slices, once):
         """Upload a compiled plan; returns its ``Executable``."""
         self._upload(prog.table, prog.table_host.tobytes())
         self._upload(prog.coef, prog.coef_host.tobytes())
@@ -413,10 +429,10 @@ class HipAPI(BaseTensorAPI):
             self._upload(prog.recs, schedule.rec_init_bytes(prog))
         self._upload(prog.params, np.array([0, total_slices, 0, 1], dtype=np.int64).tobytes())
         self._upload(prog.accum, bytes(_lib.Accum()))
-        return Executable(self, prog, total_slices)
+        return Executable(self, prog, total_slices, once)
 
     def _execute(self, tree, tables, num_groups, total_slices):
-        exe = self._compile(tree, tables, num_groups, total_slices)
+        exe = self._compile(tree, tables, num_groups, total_slices, once=True)
         try:
             return exe.run()
         finally:
@@ -495,7 +511,7 @@ class HipAPI(BaseTensorAPI):
         progs = []
         for w in waves:
             if folded:
-                prog = fold.compile_batch([per[i] for i in w], self._entry_type, self._alloc, arena)
+                prog = fold.compile_batch([per[i] for i in w], self._entry_type, self._alloc, arena, self._alloc_host)
             else:
                 prog = batch.compile_batch(None, self._entry_type, self._alloc, regroup=self._regroup,
                                            per=[per[i] for i in w], arena=arena)

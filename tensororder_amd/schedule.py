@@ -517,6 +517,8 @@ class Program:
         self.arena_bytes = 0
         self.nbatch = 1
         self.root_const = False
+        self.self_start = False  # whether the first wave starts the sum anew by itself
+        self.host_accum = None   # host copy of the sum, written by the device
         self.stats = {}
 
 

@@ -42,6 +42,32 @@ class FoldEmulator(emulator.Emulator):
         super().__init__(heap, entry_type)
         self.forms = set()
 
+    def op_16(self, L):
+        # leaf gather and record clearing in one launch: whatever the order, neither touches
+        # what the other writes
+        gathered = [self.heap.read_struct(_lib.LeafDesc, L.descs + i * ctypes.sizeof(_lib.LeafDesc))
+                    for i in range(L.count)]
+        assert sum(d.nblocks for d in gathered) == L.iaux1 <= L.grid
+        for d in gathered:
+            assert not L.iaux0 or d.rec + 16 * d.nbatch <= L.aux0 or d.rec >= L.aux0 + 16 * L.iaux0
+        self.op_1(L)
+        if L.iaux0:
+            assert L.grid > L.iaux1
+            self.op_5(L)
+
+    def op_6(self, L):
+        assert L.variant == 1
+        params = self.heap.view(L.aux3, np.int64, 2)
+        if params[0] == 0:
+            off = L.aux2 - emulator.HEAP_BASE
+            self.heap.mem[off:off + ctypes.sizeof(_lib.Accum)] = 0
+        super().op_6(L)
+        params[0] = params[0] + L.iaux0 if params[0] + L.iaux0 < params[1] else 0
+        acc = bytes(self.heap.read_struct(_lib.Accum, L.aux2))
+        if L.iaux1:
+            off = L.iaux1 - emulator.HEAP_BASE
+            self.heap.mem[off:off + len(acc)] = np.frombuffer(acc, np.uint8)
+
     def op_14(self, L):
         size = ctypes.sizeof(_lib.FoldDesc)
         for i in range(L.count):
@@ -237,7 +263,7 @@ def emulate(plan, et, W, device_leaves=True, group_levels=True, **kw):
     total, tree, tables, G = plan_inputs(plan, device_leaves)
     folded = fold.analyse(tree, tables, 8 if et == _lib.TO_F64 else 4, **kw)
     heap = emulator.Heap()
-    prog = fold.compile_program(folded, tables, G, et, W, heap.alloc, group_levels)
+    prog = fold.compile_program(folded, tables, G, et, W, heap.alloc, group_levels, heap.alloc)
     for buf, data in ((prog.table, prog.table_host), (prog.coef, prog.coef_host), (prog.blob, prog.blob_host)):
         heap.write(buf, data.tobytes())
     if et == _lib.TO_F32S:
@@ -246,11 +272,13 @@ def emulate(plan, et, W, device_leaves=True, group_levels=True, **kw):
     heap.write(prog.accum, bytes(_lib.Accum()))
     emu = FoldEmulator(heap, et)
     emu.run(prog.build)
-    emu.run(prog.prologue)
-    if not prog.root_const:
-        for _ in range(-(-total // W)):
-            emu.run(prog.wave)
-    acc = heap.read_struct(_lib.Accum, prog.accum.data_ptr())
+    for run in range(2):  # a second run starts its sum anew
+        emu.run(prog.prologue)
+        if not prog.root_const:
+            for _ in range(-(-total // W)):
+                emu.run(prog.wave)
+        acc = heap.read_struct(_lib.Accum, prog.host_accum.data_ptr())
+        assert bytes(acc) == bytes(heap.read_struct(_lib.Accum, prog.accum.data_ptr())) and acc.count == total
     fm, fe = prog.leaf_factor
     return math.ldexp(acc.mant * fm, acc.exp + fe), prog, emu
 
@@ -287,7 +315,7 @@ def test_batch_folded(et, tol):
             fold.TREE_LDS_BATCH, fold.TREE_BITS = saved
         heap = emulator.Heap()
         arena = heap.alloc(sum(p["region"] for p in per))
-        prog = fold.compile_batch(per, et, heap.alloc, arena)
+        prog = fold.compile_batch(per, et, heap.alloc, arena, heap.alloc)
         for buf, data in ((prog.table, prog.table_host), (prog.blob, prog.blob_host)):
             heap.write(buf, data.tobytes())
         if et == _lib.TO_F32S:
