@@ -127,6 +127,8 @@ class CostModel:
         self.m = torch.zeros_like(self.params)
         self.v = torch.zeros_like(self.params)
         self.grad = torch.zeros_like(self.params)
+        # the loss of a step, in host memory that the device writes
+        self.loss = torch.zeros(1, dtype=torch.float32, pin_memory=True)
         self.step = 0
         self.x_mean = np.zeros(16, np.float32)
         self.x_std = np.ones(16, np.float32)
@@ -149,9 +151,8 @@ class CostModel:
         """Device forward pass on normalised inputs; returns (h1, h2, y) tensors."""
         n = xdev.shape[0]
         h1, h2, y = self._buffers(n)
-        with self.torch.cuda.stream(self.api._stream):
-            rc = self.lib.to_mlp_forward(self._ptr(self.params), self._ptr(xdev), n, self._ptr(h1), self._ptr(h2),
-                                         self._ptr(y), self._stream())
+        rc = self.lib.to_mlp_forward(self._ptr(self.params), self._ptr(xdev), n, self._ptr(h1), self._ptr(h2),
+                                     self._ptr(y), self._stream())
         _lib.check(rc, "to_mlp_forward")
         return h1, h2, y
 
@@ -160,13 +161,13 @@ class CostModel:
         n = xdev.shape[0]
         h1, h2, y = self.forward_raw(xdev)
         dh1, dh2, dy = self._buffers(n)
-        loss = self.torch.zeros(1, dtype=self.torch.float32, device=self.api._device)
+        loss = self.loss
         rc = self.lib.to_mlp_backward(self._ptr(self.params), self._ptr(xdev), self._ptr(h1), self._ptr(h2),
                                       self._ptr(y), self._ptr(tdev), n, self._ptr(dy), self._ptr(dh2),
                                       self._ptr(dh1), self._ptr(self.grad), self._ptr(loss), self._stream())
         _lib.check(rc, "to_mlp_backward")
         self.api.synchronize()
-        return float(loss.cpu()[0]), self.grad
+        return float(loss[0]), self.grad
 
     def adam_step(self, lr=3e-3, b1=0.9, b2=0.999, eps=1e-8):
         self.step += 1

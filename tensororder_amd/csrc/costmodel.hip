@@ -1,9 +1,8 @@
 // Training and inference kernels of the plan-cost MLP (include/tensororder_costmodel.h).
 //
-// The network is tiny (5378 parameters) and the data are ~1e5 rows, so the kernels are
-// written for clarity and determinism: one thread per activation for the forward pass and
-// for activation gradients, one block per parameter for the weight gradients (a fixed-order
-// reduction over the rows), elementwise Adam.
+// The network is tiny (5378 parameters) and a training step has a few thousand rows, so a step
+// is four launches: the forward pass and the activation gradients with a wave per few rows and
+// the weights in LDS, all weight gradients (a fixed-order reduction over the rows), Adam.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -26,85 +25,188 @@ constexpr int OFF_W3 = OFF_B2 + TO_MLP_H2;
 constexpr int OFF_B3 = OFF_W3 + TO_MLP_OUT * TO_MLP_H2;
 static_assert(OFF_B3 + TO_MLP_OUT == TO_MLP_NPARAMS, "parameter layout");
 
-// out[i][j] = act(b[j] + sum_k in[i][k] * W[j][k])
-template <bool RELU>
-__global__ __launch_bounds__(kBlock) void k_dense(const float* __restrict__ in, int64_t n, int din,
-                                                  const float* __restrict__ W, const float* __restrict__ b,
-                                                  int dout, float* __restrict__ out) {
-    const int64_t total = n * dout;
-    for (int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x; t < total; t += (int64_t)gridDim.x * kBlock) {
-        const int64_t i = t / dout;
-        const int j = (int)(t - i * dout);
-        float acc = b[j];
-        for (int k = 0; k < din; ++k) acc += in[i * din + k] * W[j * din + k];
-        out[t] = RELU ? fmaxf(acc, 0.0f) : acc;
-    }
+constexpr int kRows = 4;                       // rows per wave
+constexpr int kRowsPerBlock = kRows * (kBlock / 64);
+
+// h[l] of every lane's value, as a scalar
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// dy[i][o] = 2 (y - target) / (n * OUT)
-__global__ __launch_bounds__(kBlock) void k_out_grad(const float* __restrict__ y, const float* __restrict__ t,
-                                                     int64_t n, float* __restrict__ dy) {
-    const int64_t total = n * TO_MLP_OUT;
-    const float scale = 2.0f / (float)total;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < total; i += (int64_t)gridDim.x * kBlock)
-        dy[i] = scale * (y[i] - t[i]);
-}
-
-// g[i][j] = (sum_o gnext[i][o] * W[o][j]) * (h[i][j] > 0), W is [dnext][d]
-__global__ __launch_bounds__(kBlock) void k_back_act(const float* __restrict__ gnext, int dnext,
-                                                     const float* __restrict__ W, const float* __restrict__ h,
-                                                     int64_t n, int d, float* __restrict__ g) {
-    const int64_t total = n * d;
-    for (int64_t t = (int64_t)blockIdx.x * kBlock + threadIdx.x; t < total; t += (int64_t)gridDim.x * kBlock) {
-        const int64_t i = t / d;
-        const int j = (int)(t - i * d);
-        float acc = 0.0f;
-        for (int o = 0; o < dnext; ++o) acc += gnext[i * dnext + o] * W[o * d + j];
-        g[t] = h[t] > 0.0f ? acc : 0.0f;
-    }
-}
-
-__device__ __forceinline__ float block_sum_f(float v) {
-    __shared__ float red[kBlock / 64];
+__device__ __forceinline__ float wave_sum(float v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    float r = 0.0f;
-    if (threadIdx.x == 0)
-        for (int w = 0; w < kBlock / 64; ++w) r += red[w];
-    return r;
+    return v;
 }
 
-// Block p < dout*din: dW[j][k] = sum_i g[i][j] * in[i][k]; block dout*din + j: db[j] = sum_i g[i][j].
-__global__ __launch_bounds__(kBlock) void k_weight_grad(const float* __restrict__ g, int dout,
-                                                        const float* __restrict__ in, int din, int64_t n,
-                                                        float* __restrict__ dW, float* __restrict__ db) {
-    const int p = blockIdx.x;
-    float acc = 0.0f;
-    if (p < dout * din) {
-        const int j = p / din, k = p - (p / din) * din;
-        for (int64_t i = threadIdx.x; i < n; i += kBlock) acc += g[i * dout + j] * in[i * din + k];
-        acc = block_sum_f(acc);
-        if (threadIdx.x == 0) dW[p] = acc;
+// The whole forward pass of kRows rows per wave: lane j owns unit j of both hidden layers, the
+// previous layer's units are read back with v_readlane, the weights come transposed from LDS
+// (pitch 65: no bank conflicts either way).  Bound by latency at the batch sizes of training:
+// one launch of 6 us where one thread per activation took three of 38 us together at 2048 rows.
+__global__ __launch_bounds__(kBlock) void k_forward(const float* __restrict__ params, const float* __restrict__ x,
+                                                    int64_t n, float* __restrict__ h1, float* __restrict__ h2,
+                                                    float* __restrict__ y) {
+    __shared__ float w1[TO_MLP_IN * 65], w2[TO_MLP_H1 * 65];
+    for (int i = threadIdx.x; i < TO_MLP_H1 * TO_MLP_IN; i += kBlock)
+        w1[(i % TO_MLP_IN) * 65 + i / TO_MLP_IN] = params[OFF_W1 + i];
+    for (int i = threadIdx.x; i < TO_MLP_H2 * TO_MLP_H1; i += kBlock)
+        w2[(i % TO_MLP_H1) * 65 + i / TO_MLP_H1] = params[OFF_W2 + i];
+    const int lane = threadIdx.x & 63;
+    const float b1 = params[OFF_B1 + lane], b2 = params[OFF_B2 + lane];
+    const float w30 = params[OFF_W3 + lane], w31 = params[OFF_W3 + TO_MLP_H2 + lane];
+    const float b30 = params[OFF_B3], b31 = params[OFF_B3 + 1];
+    __syncthreads();
+    const int64_t r0 = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6) * kRows;
+    float in[kRows], a[kRows], b[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        in[r] = lane < TO_MLP_IN && r0 + r < n ? x[(r0 + r) * TO_MLP_IN + lane] : 0.0f;
+        a[r] = b1;
+        b[r] = b2;
+    }
+#pragma unroll
+    for (int k = 0; k < TO_MLP_IN; ++k) {
+        const float w = w1[k * 65 + lane];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) a[r] += lane_value(in[r], k) * w;
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        a[r] = fmaxf(a[r], 0.0f);
+        if (r0 + r < n) h1[(r0 + r) * TO_MLP_H1 + lane] = a[r];
+    }
+#pragma unroll 16
+    for (int k = 0; k < TO_MLP_H1; ++k) {
+        const float w = w2[k * 65 + lane];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) b[r] += lane_value(a[r], k) * w;
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        b[r] = fmaxf(b[r], 0.0f);
+        const float s0 = wave_sum(b[r] * w30) + b30, s1 = wave_sum(b[r] * w31) + b31;
+        if (r0 + r < n) {
+            h2[(r0 + r) * TO_MLP_H2 + lane] = b[r];
+            if (lane < TO_MLP_OUT) y[(r0 + r) * TO_MLP_OUT + lane] = lane == 0 ? s0 : s1;
+        }
+    }
+}
+
+// The gradients of the activations, laid out as in k_forward:
+// dy = 2 (y - target) / (n * OUT), dh2 = (dy W3) * (h2 > 0), dh1 = (dh2 W2) * (h1 > 0)
+__global__ __launch_bounds__(kBlock) void k_backward_rows(const float* __restrict__ params, const float* __restrict__ h1,
+                                                          const float* __restrict__ h2, const float* __restrict__ y,
+                                                          const float* __restrict__ t, int64_t n,
+                                                          float* __restrict__ dy, float* __restrict__ dh2,
+                                                          float* __restrict__ dh1) {
+    __shared__ float w2[TO_MLP_H2 * TO_MLP_H1];
+    for (int i = threadIdx.x; i < TO_MLP_H2 * TO_MLP_H1; i += kBlock) w2[i] = params[OFF_W2 + i];
+    const int lane = threadIdx.x & 63;
+    const float w30 = params[OFF_W3 + lane], w31 = params[OFF_W3 + TO_MLP_H2 + lane];
+    const float scale = 2.0f / (float)(n * TO_MLP_OUT);
+    __syncthreads();
+    const int64_t r0 = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6) * kRows;
+    float g[kRows], a[kRows];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r) {
+        const int64_t i = r0 + r < n ? r0 + r : n - 1;
+        const float d0 = scale * (y[i * TO_MLP_OUT] - t[i * TO_MLP_OUT]);
+        const float d1 = scale * (y[i * TO_MLP_OUT + 1] - t[i * TO_MLP_OUT + 1]);
+        g[r] = h2[i * TO_MLP_H2 + lane] > 0.0f ? d0 * w30 + d1 * w31 : 0.0f;
+        a[r] = 0.0f;
+        if (r0 + r < n) {
+            dh2[i * TO_MLP_H2 + lane] = g[r];
+            if (lane < TO_MLP_OUT) dy[i * TO_MLP_OUT + lane] = lane == 0 ? d0 : d1;
+        }
+    }
+#pragma unroll 16
+    for (int o = 0; o < TO_MLP_H2; ++o) {
+        const float w = w2[o * TO_MLP_H1 + lane];
+#pragma unroll
+        for (int r = 0; r < kRows; ++r) a[r] += lane_value(g[r], o) * w;
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; ++r)
+        if (r0 + r < n) dh1[(r0 + r) * TO_MLP_H1 + lane] = h1[(r0 + r) * TO_MLP_H1 + lane] > 0.0f ? a[r] : 0.0f;
+}
+
+// Every weight gradient dW[j][k] = sum_i g[i][j] in[i][k], bias gradient db[j] = sum_i g[i][j]
+// and the loss in one launch: a block owns an 8 x 8 tile (2 x 8 of the output layer), its 512
+// threads are 64 row groups of 8 columns, each summing its rows in double, then the groups are
+// added in a fixed order.  64 + 16 + 8 tiles and one block for the loss.  Rows are read whole
+// (32 bytes of g, 32 of in per group of 8 lanes); one block per parameter, which read them 4
+// bytes apart, took 83 us of a 180 us step at 2048 rows, this takes 8.
+constexpr int kGradThreads = 512;
+constexpr int kTiles2 = 64, kTiles1 = 16, kTiles3 = 8;
+
+__global__ __launch_bounds__(kGradThreads) void k_weight_grads(
+    const float* __restrict__ x, const float* __restrict__ h1, const float* __restrict__ h2,
+    const float* __restrict__ dy, const float* __restrict__ dh2, const float* __restrict__ dh1,
+    const float* __restrict__ y, const float* __restrict__ t, int64_t n, float* __restrict__ grad,
+    float* __restrict__ loss) {
+    __shared__ double red[kGradThreads / 64][9][8];
+    const int tid = threadIdx.x, wave = tid >> 6;
+    int b = blockIdx.x;
+    if (b == kTiles2 + kTiles1 + kTiles3) {  // the loss
+        double acc = 0.0;
+        for (int64_t i = tid; i < n * TO_MLP_OUT; i += kGradThreads) {
+            const float e = y[i] - t[i];
+            acc += (double)e * (double)e;
+        }
+        for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+        if ((tid & 63) == 0) red[wave][0][0] = acc;
+        __syncthreads();
+        if (tid == 0 && loss) {
+            acc = 0.0;
+            for (int w = 0; w < kGradThreads / 64; ++w) acc += red[w][0][0];
+            loss[0] = (float)(acc / (double)(n * TO_MLP_OUT));
+        }
+        return;
+    }
+    const float *g, *in;
+    float *dW, *db;
+    int dout, din;
+    if (b < kTiles2) {
+        g = dh2, in = h1, dW = grad + OFF_W2, db = grad + OFF_B2, dout = TO_MLP_H2, din = TO_MLP_H1;
+    } else if (b < kTiles2 + kTiles1) {
+        b -= kTiles2;
+        g = dh1, in = x, dW = grad + OFF_W1, db = grad + OFF_B1, dout = TO_MLP_H1, din = TO_MLP_IN;
     } else {
-        const int j = p - dout * din;
-        for (int64_t i = threadIdx.x; i < n; i += kBlock) acc += g[i * dout + j];
-        acc = block_sum_f(acc);
-        if (threadIdx.x == 0) db[j] = acc;
+        b -= kTiles2 + kTiles1;
+        g = dy, in = h2, dW = grad + OFF_W3, db = grad + OFF_B3, dout = TO_MLP_OUT, din = TO_MLP_H2;
     }
-}
-
-__global__ __launch_bounds__(kBlock) void k_loss(const float* __restrict__ y, const float* __restrict__ t,
-                                                 int64_t n, float* __restrict__ loss) {
-    const int64_t total = n * TO_MLP_OUT;
-    float acc = 0.0f;
-    for (int64_t i = threadIdx.x; i < total; i += kBlock) {
-        const float e = y[i] - t[i];
-        acc += e * e;
+    const int kt = din / 8;
+    const int j0 = (b / kt) * 8, k0 = (b % kt) * 8;
+    const int nj = dout < 8 ? dout : 8;
+    const int c = tid & 7, group = tid >> 3;
+    double acc[8], bias = 0.0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = 0.0;
+    for (int64_t i = group; i < n; i += kGradThreads / 8) {
+        const double v = (double)in[i * din + k0 + c];
+        const float* gi = g + i * dout + j0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (j < nj) acc[j] = fma((double)gi[j], v, acc[j]);
+        if (k0 == 0 && c < nj) bias += (double)gi[c];
     }
-    acc = block_sum_f(acc);
-    if (threadIdx.x == 0) loss[0] = acc / (float)total;
+    // lanes 8 apart are the wave's row groups
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        for (int off = 8; off < 64; off <<= 1) acc[j] += __shfl_xor(acc[j], off, 64);
+    for (int off = 8; off < 64; off <<= 1) bias += __shfl_xor(bias, off, 64);
+    if ((tid & 63) < 8) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) red[wave][j][c] = acc[j];
+        red[wave][8][c] = bias;
+    }
+    __syncthreads();
+    if (tid < 72) {
+        const int j = tid >> 3;
+        double s = 0.0;
+        for (int w = 0; w < kGradThreads / 64; ++w) s += red[w][j][c];
+        if (j < nj) dW[(j0 + j) * din + k0 + c] = (float)s;
+        else if (j == 8 && k0 == 0 && c < nj) db[j0 + c] = (float)s;
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_adam(float* __restrict__ p, const float* __restrict__ g,
@@ -137,12 +239,9 @@ extern "C" {
 int to_mlp_forward(const float* params, const float* x, int64_t n, float* h1, float* h2, float* y, void* stream) {
     if (!params || !x || !h1 || !h2 || !y || n <= 0) return TO_ERR_INVALID;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_dense<true>, dim3(grid_for(n * TO_MLP_H1)), dim3(kBlock), 0, st, x, n, TO_MLP_IN,
-                       params + OFF_W1, params + OFF_B1, TO_MLP_H1, h1);
-    hipLaunchKernelGGL(k_dense<true>, dim3(grid_for(n * TO_MLP_H2)), dim3(kBlock), 0, st, h1, n, TO_MLP_H1,
-                       params + OFF_W2, params + OFF_B2, TO_MLP_H2, h2);
-    hipLaunchKernelGGL(k_dense<false>, dim3(grid_for(n * TO_MLP_OUT)), dim3(kBlock), 0, st, h2, n, TO_MLP_H2,
-                       params + OFF_W3, params + OFF_B3, TO_MLP_OUT, y);
+    if (n > (int64_t)INT32_MAX * kRowsPerBlock) return TO_ERR_INVALID;
+    hipLaunchKernelGGL(k_forward, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st, params,
+                       x, n, h1, h2, y);
     return status("to_mlp_forward");
 }
 
@@ -152,18 +251,11 @@ int to_mlp_backward(const float* params, const float* x, const float* h1, const 
     if (!params || !x || !h1 || !h2 || !y || !target || !dy || !dh2 || !dh1 || !grad || n <= 0)
         return TO_ERR_INVALID;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_out_grad, dim3(grid_for(n * TO_MLP_OUT)), dim3(kBlock), 0, st, y, target, n, dy);
-    hipLaunchKernelGGL(k_back_act, dim3(grid_for(n * TO_MLP_H2)), dim3(kBlock), 0, st, dy, TO_MLP_OUT,
-                       params + OFF_W3, h2, n, TO_MLP_H2, dh2);
-    hipLaunchKernelGGL(k_back_act, dim3(grid_for(n * TO_MLP_H1)), dim3(kBlock), 0, st, dh2, TO_MLP_H2,
-                       params + OFF_W2, h1, n, TO_MLP_H1, dh1);
-    hipLaunchKernelGGL(k_weight_grad, dim3(TO_MLP_OUT * TO_MLP_H2 + TO_MLP_OUT), dim3(kBlock), 0, st, dy,
-                       TO_MLP_OUT, h2, TO_MLP_H2, n, grad + OFF_W3, grad + OFF_B3);
-    hipLaunchKernelGGL(k_weight_grad, dim3(TO_MLP_H2 * TO_MLP_H1 + TO_MLP_H2), dim3(kBlock), 0, st, dh2,
-                       TO_MLP_H2, h1, TO_MLP_H1, n, grad + OFF_W2, grad + OFF_B2);
-    hipLaunchKernelGGL(k_weight_grad, dim3(TO_MLP_H1 * TO_MLP_IN + TO_MLP_H1), dim3(kBlock), 0, st, dh1,
-                       TO_MLP_H1, x, TO_MLP_IN, n, grad + OFF_W1, grad + OFF_B1);
-    if (loss) hipLaunchKernelGGL(k_loss, dim3(1), dim3(kBlock), 0, st, y, target, n, loss);
+    if (n > (int64_t)INT32_MAX * kRowsPerBlock) return TO_ERR_INVALID;
+    hipLaunchKernelGGL(k_backward_rows, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st,
+                       params, h1, h2, y, target, n, dy, dh2, dh1);
+    hipLaunchKernelGGL(k_weight_grads, dim3(kTiles2 + kTiles1 + kTiles3 + 1), dim3(kGradThreads), 0, st, x, h1, h2, dy,
+                       dh2, dh1, y, target, n, grad, loss);
     return status("to_mlp_backward");
 }
 
