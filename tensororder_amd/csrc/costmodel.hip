@@ -130,19 +130,20 @@ __global__ __launch_bounds__(kBlock) void k_backward_rows(const float* __restric
 }
 
 // Every weight gradient dW[j][k] = sum_i g[i][j] in[i][k], bias gradient db[j] = sum_i g[i][j]
-// and the loss in one launch: a block owns an 8 x 8 tile (2 x 8 of the output layer), its 512
-// threads are 64 row groups of 8 columns, each summing its rows in double, then the groups are
+// and the loss in one launch: a block owns an 8 x 8 tile (2 x 8 of the output layer), its 1024
+// threads are 128 row groups of 8 columns, each summing its rows in double, then the groups are
 // added in a fixed order.  64 + 16 + 8 tiles and one block for the loss.  Rows are read whole
-// (32 bytes of g, 32 of in per group of 8 lanes); one block per parameter, which read them 4
-// bytes apart, took 83 us of a 180 us step at 2048 rows, this takes 8.
-constexpr int kGradThreads = 512;
+// (32 bytes of g, 32 of in per group of 8 lanes), four in flight per thread; bound by the
+// latency of those reads.  One block per parameter, which read them 4 bytes apart, took 83 us
+// of a 192 us step at 2048 rows; one row in flight 36 us.  wide: g rows are 16-byte aligned.
+constexpr int kGradThreads = 1024;
 constexpr int kTiles2 = 64, kTiles1 = 16, kTiles3 = 8;
 
 __global__ __launch_bounds__(kGradThreads) void k_weight_grads(
     const float* __restrict__ x, const float* __restrict__ h1, const float* __restrict__ h2,
     const float* __restrict__ dy, const float* __restrict__ dh2, const float* __restrict__ dh1,
     const float* __restrict__ y, const float* __restrict__ t, int64_t n, float* __restrict__ grad,
-    float* __restrict__ loss) {
+    float* __restrict__ loss, bool wide) {
     __shared__ double red[kGradThreads / 64][9][8];
     const int tid = threadIdx.x, wave = tid >> 6;
     int b = blockIdx.x;
@@ -181,13 +182,36 @@ __global__ __launch_bounds__(kGradThreads) void k_weight_grads(
     double acc[8], bias = 0.0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = 0.0;
-    for (int64_t i = group; i < n; i += kGradThreads / 8) {
-        const double v = (double)in[i * din + k0 + c];
-        const float* gi = g + i * dout + j0;
+    // four rows in flight per thread: a row's loads take a trip to L2, its sums next to nothing
+    typedef float F4 __attribute__((ext_vector_type(4)));
+    constexpr int kStep = kGradThreads / 8;
+    for (int64_t i = group; i < n; i += 4 * kStep) {
+        float v[4], gv[4][8], gc[4];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            if (j < nj) acc[j] = fma((double)gi[j], v, acc[j]);
-        if (k0 == 0 && c < nj) bias += (double)gi[c];
+        for (int u = 0; u < 4; ++u) {
+            const bool row = i + u * kStep < n;
+            const int64_t r = row ? i + u * kStep : 0;
+            v[u] = in[r * din + k0 + c];
+            if (nj == 8 && wide) {
+                const F4 lo = *reinterpret_cast<const F4*>(g + r * dout + j0), hi = *reinterpret_cast<const F4*>(g + r * dout + j0 + 4);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    gv[u][j] = lo[j];
+                    gv[u][4 + j] = hi[j];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) gv[u][j] = j < nj ? g[r * dout + j0 + j] : 0.0f;
+            }
+            gc[u] = k0 == 0 && c < nj ? g[r * dout + j0 + c] : 0.0f;
+            if (!row) v[u] = gc[u] = 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] = fma((double)gv[u][j], (double)v[u], acc[j]);
+            bias += (double)gc[u];
+        }
     }
     // lanes 8 apart are the wave's row groups
 #pragma unroll
@@ -255,7 +279,8 @@ int to_mlp_backward(const float* params, const float* x, const float* h1, const 
     hipLaunchKernelGGL(k_backward_rows, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st,
                        params, h1, h2, y, target, n, dy, dh2, dh1);
     hipLaunchKernelGGL(k_weight_grads, dim3(kTiles2 + kTiles1 + kTiles3 + 1), dim3(kGradThreads), 0, st, x, h1, h2, dy,
-                       dh2, dh1, y, target, n, grad, loss);
+                       dh2, dh1, y, target, n, grad, loss,
+                       ((reinterpret_cast<uintptr_t>(dh2) | reinterpret_cast<uintptr_t>(dh1)) & 15) == 0);
     return status("to_mlp_backward");
 }
 

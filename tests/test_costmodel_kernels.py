@@ -1,0 +1,51 @@
+"""The plan-cost model's kernels at the edges of their row tiles, and with buffers that are not
+16-byte aligned, against the float64 oracle."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from oracle import mlp_oracle
+from tensororder_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 3, 15, 16, 17, 127, 129, 513, 2050])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_rows_and_alignment(n, shift):
+    import torch
+
+    print("case mlp rows", n, "shift", shift, flush=True)
+    lib = _lib.load()
+    rng = np.random.default_rng(n)
+    p = (rng.standard_normal(_lib.MLP_NPARAMS) * 0.3).astype(np.float32)
+    x = rng.standard_normal((n, 16)).astype(np.float32)
+    t = rng.standard_normal((n, 2)).astype(np.float32)
+
+    def dev(a):  # a device copy, its first entry `shift` floats after an aligned address
+        buf = torch.full((a.size + shift,), float("nan"), dtype=torch.float32, device="cuda")
+        buf[shift:] = torch.from_numpy(np.ascontiguousarray(a, np.float32).ravel()).cuda()
+        return buf
+
+    def ptr(buf):
+        return ctypes.c_void_p(buf.data_ptr() + 4 * shift)
+
+    nan = np.full
+    P, X, T = dev(p), dev(x), dev(t)
+    H1, H2, DH1, DH2 = (dev(nan((n, 64), np.nan)) for _ in range(4))
+    Y, DY = dev(nan((n, 2), np.nan)), dev(nan((n, 2), np.nan))
+    G, L = dev(nan(_lib.MLP_NPARAMS, np.nan)), dev(nan(1, np.nan))
+    torch.cuda.synchronize()
+    _lib.check(lib.to_mlp_forward(ptr(P), ptr(X), n, ptr(H1), ptr(H2), ptr(Y), None), "to_mlp_forward")
+    _lib.check(lib.to_mlp_backward(ptr(P), ptr(X), ptr(H1), ptr(H2), ptr(Y), ptr(T), n, ptr(DY), ptr(DH2), ptr(DH1),
+                                   ptr(G), ptr(L), None), "to_mlp_backward")
+    torch.cuda.synchronize()
+    _, _, want = mlp_oracle.forward(p.astype(np.float64), x)
+    loss, grad = mlp_oracle.loss_and_grad(p.astype(np.float64), x, t)
+    # sums of at most 64 float terms of order 1 per layer, the row sums in double
+    np.testing.assert_allclose(Y[shift:].cpu().numpy().reshape(n, 2), want, rtol=1e-4, atol=1e-5)
+    assert float(L[shift]) == pytest.approx(loss, rel=1e-5)
+    scale = np.abs(grad).max()
+    np.testing.assert_allclose(G[shift:].cpu().numpy(), grad, rtol=1e-3, atol=1e-5 * scale)
