@@ -389,6 +389,12 @@ int to_tensordot(const void* a, const void* b, void* c, int rank_a, int rank_b,
 int to_tensordot_noalloc(const void* a, const void* b, void* c, int rank_a, int rank_b,
                          const int32_t* axes_a, const int32_t* axes_b, int nshared, int entry_type,
                          const void* a_rec, const void* b_rec, void* c_rec, void* stream);
+/* Copy `bytes` (a multiple of 4) of host memory at `src` to 4-byte aligned device memory at
+ * `dst`, in stream order: the data travel in kernel arguments, up to 3 KB a launch, so the host
+ * memory may be reused as soon as the call returns and nothing waits.  For descriptors and
+ * other small records; a copy engine is faster above some 16 KB. */
+int to_upload(void* dst, const void* src, int64_t bytes, void* stream);
+
 /* Frequency of the device clock stamped by TO_OP_ROOT_STORE / TO_OP_BATCH_BEGIN, in kHz. */
 int to_wall_clock_khz(int* khz);
 

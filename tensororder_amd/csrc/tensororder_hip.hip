@@ -855,7 +855,7 @@ struct Vec16<double> {
 // loads 16-byte X chunks and stores its VF * 2^fy outputs as 16-byte chunks; a block walks
 // tiles of 256 * VF consecutive f of one batch item.
 
-template <typename T, bool SCALED, int YC>
+template <typename T, bool SCALED, int YC, typename A = T>
 __device__ __forceinline__ void join_stream_vec_body(const to_join_desc* __restrict__ d, const int local,
                                                      unsigned char* smem) {
     constexpr int VF = 16 / sizeof(T);
@@ -913,13 +913,13 @@ __device__ __forceinline__ void join_stream_vec_body(const to_join_desc* __restr
             staged = batch;
         }
         const auto Xp = X + batch * xb + xhi + xlo;
-        // float accumulators here: the 16-byte form keeps VF * YC sums live, which in
-        // double would cost the occupancy this HBM-bound kernel needs
-        T acc[VF][YC];
+        // accumulators of type A: float in the table launches of float joins, whose VF * YC
+        // live sums in double would cost the occupancy this HBM-bound kernel needs
+        A acc[VF][YC];
 #pragma unroll
         for (int i = 0; i < VF; ++i)
 #pragma unroll
-            for (int y = 0; y < YC; ++y) acc[i][y] = T(0);
+            for (int y = 0; y < YC; ++y) acc[i][y] = A(0);
         for (int k0 = 0; k0 < K; k0 += 4) {
             V xv[4];
 #pragma unroll
@@ -932,7 +932,7 @@ __device__ __forceinline__ void join_stream_vec_body(const to_join_desc* __restr
                     for (int y = 0; y < YC; ++y) {
                         const T yv = ylds[y * K + k0 + kk];
 #pragma unroll
-                        for (int i = 0; i < VF; ++i) acc[i][y] = fma(xv[kk][i], yv, acc[i][y]);
+                        for (int i = 0; i < VF; ++i) acc[i][y] = fma((A)xv[kk][i], (A)yv, acc[i][y]);
                     }
                 }
             }
@@ -959,7 +959,7 @@ __device__ __forceinline__ void join_stream_vec_body(const to_join_desc* __restr
                         V o;
 #pragma unroll
                         for (int c = 0; c < VF; ++c) {
-                            const T v = acc[(j + c) / YC][(j + c) % YC];
+                            const T v = (T)acc[(j + c) / YC][(j + c) % YC];
                             o[c] = v;
                             if (SCALED) m = fmaxf(m, (float)absval(v));
                         }
@@ -986,7 +986,7 @@ __device__ __forceinline__ void join_stream_vec_body(const to_join_desc* __restr
                 V o;
 #pragma unroll
                 for (int c = 0; c < VF; ++c) {
-                    const T v = acc[(j + c) / YC][(j + c) % YC];
+                    const T v = (T)acc[(j + c) / YC][(j + c) % YC];
                     o[c] = v;
                     if (SCALED) m = fmaxf(m, (float)absval(v));
                 }
@@ -1017,6 +1017,13 @@ __global__ __launch_bounds__(kBlock) void k_join_stream_vec(const to_join_desc* 
     extern __shared__ __align__(16) unsigned char smem[];
     const to_join_desc* d = descs + find_desc(descs, ndesc, blockIdx.x, bmap);
     join_stream_vec_body<T, SCALED, YC>(d, blockIdx.x - d->block0, smem);
+}
+
+// One join given by value (to_tensordot), summed in double as its general form does.
+template <typename T, bool SCALED, int YC>
+__global__ __launch_bounds__(kBlock) void k_join_stream_vec_one(const to_join_desc desc) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    join_stream_vec_body<T, SCALED, YC, double>(&desc, blockIdx.x, smem);
 }
 
 // ---------------------------------------------------------------------------------
@@ -2850,12 +2857,25 @@ int to_permute(const void* in, void* out, int rank, const int32_t* perm, int ele
 
 namespace {
 
+// Small host data in kernel arguments (to_upload): no copy engine, no staging buffer and no
+// wait, 4 us of host time where a pageable copy through the runtime took 25-30.
+constexpr int kUploadWords = 768;
+struct UploadWords {
+    uint32_t w[kUploadWords];
+};
+
+__global__ __launch_bounds__(kBlock) void k_upload(uint32_t* dst, const UploadWords data, int n) {
+    for (int i = threadIdx.x; i < n; i += kBlock) dst[i] = data.w[i];
+}
+
 // One tensordot as one join: the bit geometry, the kernel form (streamed join, or split-K
 // with double partial sums and a finishing pass) and the scratch it needs.
 struct DotPlan {
     to_join_desc d;
     bool x_is_left;  // a is the streamed operand X
     bool splitk;
+    bool vec;        // streamed: the 16-byte form, where the tensors are 16-byte aligned
+    int vlds, vgrid; // its LDS bytes and blocks
     int yc, lds, grid, fin_grid;
     bool fin_wide;
     int64_t partial_bytes;
@@ -2943,6 +2963,20 @@ int plan_tensordot(int rank_a, int rank_b, const int32_t* axes_a, const int32_t*
             d.lnych = l;
             d.nsplit = 1;
             d.nblocks = P.grid;
+            // The 16-byte form: X's lowest bits free (16 bytes of consecutive f), all y of one f
+            // adjacent in the output, at least one tile of f; with double sums 64 accumulators
+            // at most.  From 2^20 index values on: a 2^23 by 2^6 float64 join over 2^3 took 43 us
+            // in the general form and takes 24; below, both are one launch's latency.
+            const int lvf = entry_type == TO_F64 ? 1 : 2, esize = entry_type == TO_F64 ? 8 : 4;
+            bool low = fx >= 8 + lvf;
+            for (int t = 0; low && t < lvf; ++t) low = d.xf_pos[t] == t;
+            const int64_t vlds = ((8 * K + 15) & ~15ll) + (K << fy) * esize;
+            const bool run64 = ((16 / esize) << fy) * esize >= 64;
+            P.vec = low && d.shy == 0 && d.shf == fy && fy <= (entry_type == TO_F64 ? 4 : 3) &&
+                    fx + fy + s >= 20 && vlds + (run64 ? 4 * 4096 : 0) <= kDotLdsLimit;
+            P.vlds = (int)(vlds + (run64 ? 4 * 4096 : 0));
+            const int64_t vtiles = 1ll << (fx >= 8 + lvf ? fx - 8 - lvf : 0);
+            P.vgrid = (int)(vtiles < kDotMaxBlocks ? vtiles : kDotMaxBlocks);
             return TO_OK;
         }
     }
@@ -2974,7 +3008,28 @@ template <typename T, bool SCALED>
 int launch_tensordot(DotPlan& P, hipStream_t st) {
     if (SCALED) hipLaunchKernelGGL(k_scale_clear, dim3(1), dim3(kBlock), 0, st, reinterpret_cast<to_scale_rec*>(P.d.cs), (int64_t)1);
     const dim3 block(kBlock);
-    if (!P.splitk) {
+    if (!P.splitk && P.vec && ((P.d.x | P.d.c) & 15) == 0) {
+        P.d.nblocks = P.vgrid;
+        switch (P.yc) {
+#define TO_DOT_CASE(YC)                                                                                    \
+    case YC:                                                                                               \
+        hipLaunchKernelGGL((k_join_stream_vec_one<T, SCALED, YC>), dim3(P.vgrid), block, P.vlds, st, P.d); \
+        break;
+            TO_DOT_CASE(1)
+            TO_DOT_CASE(2)
+            TO_DOT_CASE(4)
+            TO_DOT_CASE(8)
+            case 16:
+                if constexpr (sizeof(T) == 8) {
+                    hipLaunchKernelGGL((k_join_stream_vec_one<T, SCALED, 16>), dim3(P.vgrid), block, P.vlds, st, P.d);
+                    break;
+                }
+#undef TO_DOT_CASE
+            default:
+                set_err("tensordot: bad y chunk");
+                return TO_ERR_INVALID;
+        }
+    } else if (!P.splitk) {
         switch (P.yc) {
 #define TO_DOT_CASE(YC)                                                                                   \
     case YC:                                                                                              \
@@ -3104,6 +3159,27 @@ int to_tensordot(const void* a, const void* b, void* c, int rank_a, int rank_b, 
     }
     return run_tensordot(P, a, b, c, entry_type, a_rec, b_rec, c_rec, workspace,
                          reinterpret_cast<hipStream_t>(stream));
+}
+
+int to_upload(void* dst, const void* src, int64_t bytes, void* stream) {
+    g_err[0] = 0;
+    if (bytes < 0 || (bytes & 3) || (bytes > 0 && (!dst || !src || (reinterpret_cast<uintptr_t>(dst) & 3)))) {
+        set_err("to_upload: invalid argument");
+        return TO_ERR_INVALID;
+    }
+    uint32_t* out = static_cast<uint32_t*>(dst);
+    const unsigned char* in = static_cast<const unsigned char*>(src);
+    for (int64_t left = bytes / 4; left > 0;) {
+        const int n = (int)(left < kUploadWords ? left : kUploadWords);
+        UploadWords data;
+        memcpy(data.w, in, (size_t)n * 4);
+        hipLaunchKernelGGL(k_upload, dim3(1), dim3(kBlock), 0, reinterpret_cast<hipStream_t>(stream), out, data, n);
+        out += n;
+        in += (int64_t)n * 4;
+        left -= n;
+    }
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? TO_OK : hip_fail(e, "to_upload launch");
 }
 
 int to_wall_clock_khz(int* khz) {

@@ -342,7 +342,15 @@ class HipAPI(BaseTensorAPI):
         """Host memory that the device writes (pinned)."""
         return self._torch.empty(max(1, int(nbytes)), dtype=self._torch.uint8, pin_memory=True)
 
+    # larger data go through a copy engine
+    UPLOAD_BYTES = 12 * 1024
+
     def _upload(self, dst, host_bytes):
+        n = len(host_bytes)
+        if n <= self.UPLOAD_BYTES and n % 4 == 0:
+            _lib.check(self._lib.to_upload(ctypes.c_void_p(dst.data_ptr()), ctypes.c_char_p(bytes(host_bytes)), n,
+                                           ctypes.c_void_p(self._stream.cuda_stream)), "to_upload")
+            return
         src = self._torch.from_numpy(np.frombuffer(host_bytes, dtype=np.uint8).copy())
         with self._torch.cuda.stream(self._stream):
             dst[: src.numel()].copy_(src, non_blocking=False)
@@ -603,10 +611,15 @@ class HipAPI(BaseTensorAPI):
         d.xf_pos, d.xs_pos = schedule._pos_array(g["xf"]), schedule._pos_array(g["xs"])
         d.yf_pos, d.ys_pos = schedule._pos_array(g["yf"]), schedule._pos_array(g["ys"])
         v = g["var"]
-        launches = []
+        launches, blob = [], []
         if scaled:
             launches.append(_lib.Launch(op=_lib.TO_OP_SCALE_CLEAR, grid=1, aux0=crec.data_ptr(), iaux0=1))
         keep = [cbuf, crec]
+
+        def launch(desc, **kw):  # a launch of one descriptor; all of them go up together
+            launches.append(_lib.Launch(count=1, **kw))
+            blob.append((launches[-1], bytes(desc)))
+
         if v["kind"] == "gemm":
             ops = []
             for need, T, fpos, spos in ((v["perm_x"], X, g["xf"], g["xs"]), (v["perm_y"], Y, g["yf"], g["ys"])):
@@ -621,11 +634,8 @@ class HipAPI(BaseTensorAPI):
                 dst = self._alloc((1 << T.rank) * self._esize)
                 pd, grid, lds, pvar = schedule.perm_desc(T.data.data_ptr(), dst.data_ptr(), T.rank, out_pos, 1,
                                                          1 << T.rank, self._esize)
-                pblob = self._alloc(ctypes.sizeof(pd))
-                self._upload(pblob, bytes(pd))
-                launches.append(_lib.Launch(op=_lib.TO_OP_PERMUTE, variant=pvar, count=1, grid=grid, lds=lds,
-                                            descs=pblob.data_ptr()))
-                keep += [dst, pblob]
+                launch(pd, op=_lib.TO_OP_PERMUTE, variant=pvar, grid=grid, lds=lds)
+                keep.append(dst)
                 ops.append(dst.data_ptr())
             gd = _lib.GemmDesc()
             gd.a, gd.b, gd.c = ops[0], ops[1], cbuf.data_ptr()
@@ -634,34 +644,28 @@ class HipAPI(BaseTensorAPI):
                 gd.as_, gd.bs, gd.cs = X.rec.data_ptr(), Y.rec.data_ptr(), crec.data_ptr()
             gd.mlog, gd.nlog, gd.klog = g["fx"], g["fy"], g["s"]
             gd.nbatch, gd.block0, gd.nblocks = 1, 0, v["nblocks"]
-            gblob = self._alloc(ctypes.sizeof(gd))
-            self._upload(gblob, bytes(gd))
-            launches.append(_lib.Launch(op=_lib.TO_OP_GEMM, variant=v["tile"], count=1, grid=v["nblocks"],
-                                        descs=gblob.data_ptr()))
-            keep.append(gblob)
+            launch(gd, op=_lib.TO_OP_GEMM, variant=v["tile"], grid=v["nblocks"])
         elif v["kind"] == "stream":
             d.nblocks, d.nych, d.nsplit = v["nblocks"], v["nych"], 1
             d.lnych = v["nych"].bit_length() - 1
             d.stage = int(v["stage"])
-            blob = self._alloc(ctypes.sizeof(d))
-            self._upload(blob, bytes(d))
-            variant = schedule.stream_variant(v, g)
-            launches.append(_lib.Launch(op=_lib.TO_OP_JOIN_STREAM, variant=variant, count=1,
-                                        grid=v["nblocks"], lds=v["lds"], descs=blob.data_ptr()))
-            keep.append(blob)
+            launch(d, op=_lib.TO_OP_JOIN_STREAM, variant=schedule.stream_variant(v, g), grid=v["nblocks"], lds=v["lds"])
         else:
             part = self._alloc(v["nout"] * v["nsplit"] * 8)  # double partial sums
             d.partial = part.data_ptr()
             d.nsplit, d.nblocks = v["nsplit"], v["nblocks"]
             d2 = _lib.JoinDesc.from_buffer_copy(bytes(d))
             d2.nblocks = v["fin_blocks"]
-            blob = self._alloc(2 * ctypes.sizeof(d))
-            self._upload(blob, bytes(d) + bytes(d2))
-            launches.append(_lib.Launch(op=_lib.TO_OP_JOIN_SPLITK, count=1, grid=v["nblocks"],
-                                        descs=blob.data_ptr()))
-            launches.append(_lib.Launch(op=_lib.TO_OP_JOIN_FINISH, variant=v["fin_variant"], count=1,
-                                        grid=v["fin_blocks"], descs=blob.data_ptr() + ctypes.sizeof(d)))
-            keep += [blob, part]
+            launch(d, op=_lib.TO_OP_JOIN_SPLITK, grid=v["nblocks"])
+            launch(d2, op=_lib.TO_OP_JOIN_FINISH, variant=v["fin_variant"], grid=v["fin_blocks"])
+            keep.append(part)
+        table = self._alloc(sum(len(data) for _, data in blob))
+        at = 0
+        for L, data in blob:
+            L.descs = table.data_ptr() + at
+            at += len(data)
+        self._upload(table, b"".join(data for _, data in blob))
+        keep.append(table)
         self._run(launches)
         self.synchronize()
         tdtype = self._torch.float64 if not scaled else self._torch.float32
