@@ -92,8 +92,10 @@ extern "C" {
 #define TO_OP_ROOT_STORE 11  /* descs: to_root_desc[count]: one instance's root -> its accumulator */
 #define TO_OP_BATCH_BEGIN 12 /* aux2: to_accum[iaux0] zeroed; aux3: int64 start time (device clock) */
 #define TO_OP_FOLD 14 /* descs: to_fold_desc[count]; variant TO_FOLD_ANY: one output per thread,
-                         any bit layout; else TO_FOLD_VEC | y mode << 4 | nreg: the 16-byte form,
-                         every descriptor of the launch with that y mode and nreg */
+                         any bit layout; TO_FOLD_DOT: the same, 4 products per load;
+                         TO_FOLD_VEC | y mode << 4 | nreg: the 16-byte form, TO_FOLD_REG | a << 4 |
+                         b: a register tile, every descriptor of the launch with that y mode and
+                         nreg, or those a and b */
 #define TO_OP_FOLD_TREE 15 /* descs: to_tree_desc[count]; iaux0: waves per block (1 to 16, as many
                          as each program has streams); lds: the largest of their LDS needs */
 #define TO_OP_WAVE_BEGIN 16 /* TO_OP_LEAF_GATHER on the first iaux1 blocks of the grid and
@@ -235,6 +237,10 @@ typedef struct to_gemm_desc {
  *     lsplit k bits across blocks.  lk > 0 only when ntile == 0 or lo == 8 - lk.
  *     With lsplit > 0 the double partial sums go to partial[(batch << (lo + ntile) | c) <<
  *     lsplit | sp], c the C offset, for a TO_OP_JOIN_FINISH launch (fx = lo + ntile).
+ *   TO_FOLD_DOT: as TO_FOLD_ANY, with two more k bits, not listed, that add 1 and 2 to the
+ *     offsets of X and of Y (X, Y and their batch strides aligned to 4 elements).
+ *   TO_FOLD_REG: as TO_FOLD_ANY with lo == 8, lk == lsplit == 0; then nreg = a + b o bits, a
+ *     that only X has and b that only Y has ((a, b) one of (1, 1), (2, 2), (2, 3), (2, 0)), all 2^nreg of whose outputs a thread holds at once.
  *   TO_FOLD_VEC: [0, 2) the o bits of 4 consecutive outputs, also the lowest 2 bits of X;
  *     [2, 10) o bits of the thread index; [10, 10 + ntile) tile; nloop k bits; nreg (<= 3) o
  *     bits that only Y has, all 2^nreg of whose outputs a thread holds at once.
@@ -242,6 +248,8 @@ typedef struct to_gemm_desc {
  *     C, X (and Y in mode 1) and their batch strides aligned to 4 elements. */
 #define TO_FOLD_ANY 0
 #define TO_FOLD_VEC 0x100
+#define TO_FOLD_REG 0x200
+#define TO_FOLD_DOT 0x400
 #define TO_FOLD_BITS 40
 typedef struct to_fold_desc {
     uint64_t x, y, c;

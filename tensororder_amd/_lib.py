@@ -39,6 +39,8 @@ TO_LAUNCH_SIDE = 0x1  # Launch.flags: captured on the side stream
 TO_LAUNCH_JOIN = 0x2  # Launch.flags: join the side stream into the main one and fork it again first
 TO_FOLD_ANY = 0  # fold launch variants: any bit layout
 TO_FOLD_VEC = 0x100  # the 16-byte form; | y mode << 4 | nreg
+TO_FOLD_REG = 0x200  # a register tile; | a << 4 | b
+TO_FOLD_DOT = 0x400  # as TO_FOLD_ANY, 4 products per load
 TO_TREE_WORDS = 448  # uint32 words of one join of a fold tree program
 TO_TREE_IDLE, TO_TREE_MEET = 1 << 30, 1 << 31  # fold tree task bits
 MAX_BITS = 32

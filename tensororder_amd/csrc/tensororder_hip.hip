@@ -2500,8 +2500,20 @@ int launch_one(const to_launch& L, hipStream_t st) {
             const to_fold_desc* fd = reinterpret_cast<const to_fold_desc*>(L.descs);
             switch (L.variant) {
                 case TO_FOLD_ANY:
-                    hipLaunchKernelGGL((k_fold_any<T, SCALED>), grid, block, 0, st, fd, L.count, bmap);
+                    hipLaunchKernelGGL((k_fold_any<T, SCALED, false>), grid, block, 0, st, fd, L.count, bmap);
                     break;
+                case TO_FOLD_DOT:
+                    hipLaunchKernelGGL((k_fold_any<T, SCALED, true>), grid, block, 0, st, fd, L.count, bmap);
+                    break;
+#define TO_FOLD_CASE(A, B)                                                                         \
+    case TO_FOLD_REG | A << 4 | B:                                                                 \
+        hipLaunchKernelGGL((k_fold_reg<T, SCALED, A, B>), grid, block, 0, st, fd, L.count, bmap); \
+        break;
+                TO_FOLD_CASE(1, 1)
+                TO_FOLD_CASE(2, 2)
+                TO_FOLD_CASE(2, 3)
+                TO_FOLD_CASE(2, 0)
+#undef TO_FOLD_CASE
 #define TO_FOLD_CASE(RY, YM)                                                                         \
     case TO_FOLD_VEC | YM << 4 | RY:                                                                 \
         hipLaunchKernelGGL((k_fold_vec<T, SCALED, RY, YM>), grid, block, 0, st, fd, L.count, bmap); \

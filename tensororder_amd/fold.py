@@ -50,6 +50,12 @@ ANY_MIN_THREADS_LOG = 17
 MAX_ANY_BLOCKS = 8192
 MAX_VEC_BLOCKS = 4096
 MAX_REG_BITS = 3
+# register tiles (variables only X has, only Y has), the first that a join has; it must leave
+# this many outputs to threads
+REG_TILES = ((2, 3), (2, 2), (1, 1), (2, 0))
+REG_MIN_LOG = 16
+# shared range from which a sum over few outputs takes four consecutive products per load
+DOT_MIN_SHARED = 10
 # programs run by one block per slice: joins over at most 2^TREE_BITS index values with
 # results of at most 2^TREE_RANK entries, the intermediates in TREE_LDS bytes of LDS -- or
 # TREE_LDS_MANY with TREE_WAVES_MANY waves, so that blocks share a CU, when there are enough
@@ -360,8 +366,28 @@ def choose(n, nodes, W, esize, launch_bound=False):
                         vec=True, yc=1 << len(reg))
         n.geom = g
         return
+    # register tile: outputs enough to fill the chip without the tile's bits
+    xonly = [v for v in out if v not in yoff]
+    for na, nbits in REG_TILES if Y is not None else ():
+        if len(xonly) < na or len(yonly) < nbits or nc - na - nbits < 8 or lognb + nc - na - nbits < REG_MIN_LOG:
+            continue
+        # the tile's variables: the highest bits of the result, so that the lanes keep low ones
+        reg = (xonly[len(xonly) - na:] if na else []) + (yonly[len(yonly) - nbits:] if nbits else [])
+        body = [v for v in out if v not in reg]
+        ntile = len(body) - 8
+        g["var"] = dict(kind="fold", variant=_lib.TO_FOLD_REG | na << 4 | nbits, bits=body + ks + reg,
+                        roles=(8, 0, ntile, s, 0, na + nbits), nblocks=int(min(nb << ntile, MAX_ANY_BLOCKS)), lsplit=0,
+                        vec=False, yc=1)
+        if len(g["var"]["bits"]) <= _lib.FOLD_BITS:
+            n.geom = g
+            return
     # general form: thread bits go to outputs, then to the shared range while the launch
     # would have few threads; long shared ranges with few outputs are split over blocks
+    dot = s >= DOT_MIN_SHARED and nc <= 6 and all((xoff.get(v), yoff.get(v)) == (o, o) for v, o in zip(ks, (1, 2))) \
+        and X.rank >= 2 and Y.rank >= 2
+    if dot:  # its four consecutive shared indices go with one load
+        ks = ks[2:]
+        s -= 2
     lk = 0
     if lognb + nc < ANY_MIN_THREADS_LOG and s > 0:
         lk = min(s, 8, max(8 - nc, min(s - 3, ANY_MIN_THREADS_LOG - lognb - nc)))
@@ -373,7 +399,8 @@ def choose(n, nodes, W, esize, launch_bound=False):
         lsplit = max(0, min(rest - 4, ANY_MIN_THREADS_LOG + 3 - lognb - nc - lk))
     ntile = nc - lo
     pad = [None] * (8 - lo - lk)
-    g["var"] = dict(kind="fold", variant=_lib.TO_FOLD_ANY, bits=out[:lo] + ks[:lk] + pad + out[lo:] + ks[lk:],
+    g["var"] = dict(kind="fold", variant=_lib.TO_FOLD_DOT if dot else _lib.TO_FOLD_ANY,
+                    bits=out[:lo] + ks[:lk] + pad + out[lo:] + ks[lk:],
                     roles=(lo, lk, ntile, rest - lsplit, lsplit, 0),
                     nblocks=int(min(nb << (ntile + lsplit), MAX_ANY_BLOCKS)), lsplit=lsplit, nout=nb << nc,
                     nsplit=1 << lsplit, vec=False, yc=1)

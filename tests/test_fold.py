@@ -86,6 +86,12 @@ class FoldEmulator(emulator.Emulator):
                         assert ptr % (4 * self.dt().itemsize) == 0 and stride % 4 == 0
                         assert all(int(e) % 4 == 0 for e in list(arr)[2:])
                 thr, tile0 = (0, 10), 10
+            elif L.variant & _lib.TO_FOLD_REG:
+                na, nb = L.variant >> 4 & 15, L.variant & 15
+                assert d.nreg == na + nb and d.lo == 8 and d.lk == 0 and d.lsplit == 0
+                r0 = 8 + d.ntile + d.nloop
+                assert not any(list(d.by)[r0:r0 + na]) and not any(list(d.bx)[r0 + na:r0 + d.nreg])
+                thr, tile0 = (0, 8), 8
             else:
                 assert d.nreg == 0 and d.lo + d.lk <= 8 and all(int(e) == 0 for e in list(d.bc)[d.lo:8])
                 thr, tile0 = (0, d.lo), 8
@@ -93,11 +99,18 @@ class FoldEmulator(emulator.Emulator):
             r0 = k0 + d.nloop + d.lsplit
             assert r0 + d.nreg <= _lib.FOLD_BITS
             offs = []
-            for arr in (d.bx, d.by, d.bc):
+            bx, by, bc = list(d.bx), list(d.by), list(d.bc)
+            for arr in (bx, by, bc):
                 o = (_spread(arr, *thr)[None, None, :] + _spread(arr, tile0, d.ntile)[None, :, None]
                      + _spread(arr, r0, d.nreg)[:, None, None]).ravel()
                 k = (_spread(arr, d.lo, 0 if vec else d.lk)[None, :]
                      + _spread(arr, k0, d.nloop + d.lsplit)[:, None]).ravel()
+                if L.variant == _lib.TO_FOLD_DOT:
+                    four = np.arange(4) if arr is not bc else np.zeros(4, dtype=np.int64)
+                    if arr is not bc:
+                        assert all(int(e) % 4 == 0 for e in arr) and d.x % 16 == d.y % 16 == 0
+                        assert d.xb % 4 == d.yb % 4 == 0
+                    k = (k[:, None] + four[None, :]).ravel()
                 offs.append((o, k))
             co = offs[2][0]
             assert np.array_equal(np.sort(co), np.arange(co.size))  # every output once
@@ -388,6 +401,8 @@ def test_folded_tensors_hold_each_variable_once():
 JOINS = [(0, 0, 0, 0, 0, 1, 1, 1, 0), (2, 1, 1, 1, 0, 3, 1, 1, 1), (3, 2, 2, 2, 1, 5, 1, 0, 1), (0, 0, 3, 9, 0, 2, 1, 1, 0),
          (0, 0, 0, 16, 0, 1, 1, 1, 0), (1, 0, 1, 14, 0, 3, 1, 1, 1), (4, 5, 1, 6, 0, 1, 1, 1, 1), (10, 0, 0, 0, 0, 1, 1, 1, 0),
          (11, 0, 2, 1, 0, 2, 1, 0, 0), (9, 1, 4, 2, 0, 3, 1, 1, 0), (10, 2, 2, 3, 0, 1, 1, 1, 0), (8, 3, 3, 1, 0, 7, 1, 0, 0),
+         (4, 6, 5, 2, 0, 65, 1, 1, 1), (4, 2, 9, 1, 0, 33, 1, 0, 1), (1, 1, 13, 1, 1, 9, 1, 1, 1),
+         (2, 0, 13, 0, 0, 9, 1, 1, 1), (0, 0, 0, 18, 0, 3, 1, 1, 0), (1, 0, 2, 11, 0, 2, 1, 0, 0),
          (9, 5, 3, 2, 0, 2, 1, 1, 0), (0, 0, 13, 1, 0, 3, 1, 1, 0), (1, 0, 12, 2, 0, 2, 1, 1, 0), (12, 1, 1, 4, 0, 3, 1, 1, 0)]
 
 
@@ -399,7 +414,8 @@ def _join(case, et, alloc, write, rng):
     names = ["x%d" % i for i in range(xo)] + ["h%d" % i for i in range(kept)]
     if kept and not shuffled and rng.integers(2):  # kept variables lowest: Y's lowest too
         names = names[xo:] + names[:xo]
-    xv = names + ["k%d" % i for i in range(s)] + ["q%d" % i for i in range(xs)]
+    ks = ["k%d" % i for i in range(s)] + ["q%d" % i for i in range(xs)]
+    xv = names + ks if s < fold.DOT_MIN_SHARED else ks + names  # long sums: shared lowest
     yv = [v for v in xv if v[0] in "hk"] + ["y%d" % i for i in range(yo)]
     out = names + ["y%d" % i for i in range(yo)]
     if shuffled:
@@ -495,7 +511,9 @@ def test_every_form_emulated(et):
         _check(case, et, got, [heap.read_struct(_lib.ScaleRec, recs[2] + 16 * b) for b in range(items)], want)
     assert {f & 15 for f in forms if f != "split" and f & _lib.TO_FOLD_VEC} == {0, 1, 2, 3}
     assert {f >> 4 & 15 for f in forms if f != "split" and f & _lib.TO_FOLD_VEC} >= {0, 1}
-    assert "split" in forms and _lib.TO_FOLD_ANY in forms
+    assert "split" in forms and _lib.TO_FOLD_ANY in forms and _lib.TO_FOLD_DOT in forms
+    assert {f for f in forms if f != "split" and f & _lib.TO_FOLD_REG} == {
+        _lib.TO_FOLD_REG | a << 4 | b for a, b in fold.REG_TILES}
 
 
 @pytest.mark.gpu
