@@ -163,8 +163,8 @@ def tune_perm(api, rank, nb):
 
 
 def tune_plan(api, nodes, W, cache):
-    """Tune every product and permute shape of an analysed plan missing from ``cache``
-    (joins carry their variants).  Returns the number of shapes tuned."""
+    """Tune every product and permute shape of an analysed plan, folded or not, missing from
+    ``cache`` (joins carry their variants).  Returns the number of shapes tuned."""
     esize = api.get_entry_size()
     tuned = 0
     for n in nodes:
@@ -174,11 +174,15 @@ def tune_plan(api, nodes, W, cache):
         if v["kind"] != "gemm":
             continue
         nb = W if n.batched else 1
-        key = gemm_key(esize, g["fx"], g["fy"], g["s"], nb)
+        items = nb << v.get("hlog", 0)  # a folded product's kept shared variables are items too
+        key = gemm_key(esize, g["fx"], g["fy"], g["s"], items)
         if key not in cache:
-            cache[key], _ = tune_gemm(api, g["fx"], g["fy"], g["s"], nb)
+            cache[key], _ = tune_gemm(api, g["fx"], g["fy"], g["s"], items)
             tuned += 1
-        X, Y = (nodes[n.left], nodes[n.right]) if g["x_is_left"] else (nodes[n.right], nodes[n.left])
+        if "X" in g:
+            X, Y = nodes[g["X"]], nodes[g["Y"]]
+        else:
+            X, Y = (nodes[n.left], nodes[n.right]) if g["x_is_left"] else (nodes[n.right], nodes[n.left])
         for need, op in ((v["perm_x"], X), (v["perm_y"], Y)):
             nbo = W if (n.batched and op.batched) else 1
             pk = perm_key(esize, op.rank, nbo)
@@ -195,7 +199,7 @@ def main():
     and write the cache:  python -m tensororder_amd.autotune FIXTURE.json ... [--out PATH]"""
     import argparse
 
-    from . import plan_io
+    from . import fold, plan_io
     from .hip_api import HipAPI, HipF32API
 
     ap = argparse.ArgumentParser()
@@ -205,6 +209,7 @@ def main():
     cache = load(args.out)
     for cls in (HipF32API, HipAPI):
         api = cls()
+        esize = api.get_entry_size()
         for path in args.fixtures:
             with open(path) as f:
                 doc = json.load(f)
@@ -219,9 +224,15 @@ def main():
             shapes = 0
             for plan in plans:
                 total, tree, tables, groups = api._plan_inputs(plan, None)
-                nodes = schedule.analyse(tree, tables, api._regroup)
-                W = api.choose_batch(nodes, tables, total) if groups else 1
-                schedule.peak_bytes(nodes, tables, W, api._entry_type)
+                W = 0
+                folded = fold.analyse(tree, tables, esize, api._regroup) if fold.has_copies(tables) else None
+                if folded is not None:
+                    W = api.choose_folded_batch(folded, tree, tables, total if groups else 1)
+                    nodes = folded[0]
+                if not W:
+                    nodes = schedule.analyse(tree, tables, api._regroup)
+                    W = api.choose_batch(nodes, tables, total) if groups else 1
+                    schedule.peak_bytes(nodes, tables, W, api._entry_type)
                 shapes += tune_plan(api, nodes, W, cache)
             print("%s %s: %d new shapes, cache %d" % (cls.__name__, os.path.basename(path), shapes, len(cache)),
                   flush=True)

@@ -94,6 +94,10 @@ class FoldDesc:
                           self.block0, self.nblocks, lo, lk, ntile, nloop, lsplit, nreg, 0) + _BITS.pack(*self.bits)
 
 
+class TooWide(ValueError):
+    """A join over more variables than a descriptor holds: the plan runs edge by edge."""
+
+
 class FNode:
     """A node of a folded plan.  ``order`` lists its variables from the lowest bit up and
     ``off`` maps each to the element offset it adds (several bits at once for a leaf that
@@ -405,7 +409,7 @@ def choose(n, nodes, W, esize, launch_bound=False):
                     nblocks=int(min(nb << (ntile + lsplit), MAX_ANY_BLOCKS)), lsplit=lsplit, nout=nb << nc,
                     nsplit=1 << lsplit, vec=False, yc=1)
     if len(g["var"]["bits"]) > _lib.FOLD_BITS:
-        raise ValueError("folded join over more than %d variables" % _lib.FOLD_BITS)
+        raise TooWide("folded join over more than %d variables" % _lib.FOLD_BITS)
     n.geom = g
 
 
@@ -1011,7 +1015,10 @@ def analyse_batch(instances, esize, regroup=True):
         nodes, missing = folded
         if any(n.batched for n in nodes):
             raise ValueError("batched instances must be unsliced plans")
-        choose_all(nodes, 1, esize, launch_bound=True)
+        try:
+            choose_all(nodes, 1, esize, launch_bound=True)
+        except TooWide:
+            return None
         programs = tree_programs(nodes, 1, esize, esize == 4, TREE_LDS_BATCH)
         peak, scratch = plan_memory(nodes, 1, esize, "level", programs)
         words = sum(len(p.members) for p in programs) * 4 * _lib.TO_TREE_WORDS

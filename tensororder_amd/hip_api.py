@@ -380,17 +380,21 @@ class HipAPI(BaseTensorAPI):
     # -- compiled execution ---------------------------------------------------------
 
     def choose_folded_batch(self, folded, tree, tables, total_slices):
-        """Largest slice batch W of a folded plan whose arena fits the device budget.  A plan
-        is refused where its tensors, one axis per edge, would not fit one slice at a time:
-        whether a caller has to slice more does not depend on how the plan is executed."""
+        """Largest slice batch W of a folded plan whose arena fits the device budget (0: it
+        runs edge by edge).  A plan is refused where its tensors, one axis per edge, would not
+        fit one slice at a time: whether a caller has to slice more does not depend on how the
+        plan is executed."""
         budget = self._budget()
         nodes, _ = folded
         fixed = sum(t.size for t in tables.values()) * self._esize
         if fixed + schedule.peak_bound(tree, self._esize) > budget:
             self.choose_batch(schedule.analyse(tree, tables, self._regroup), tables, 1)
         W = max(1, min(self._max_batch, total_slices))
-        while W > 1 and fold.peak_bytes(nodes, W, self._esize) + fixed > budget:
-            W = max(1, W // 2)
+        try:
+            while W and fold.peak_bytes(nodes, W, self._esize) + fixed > budget:
+                W //= 2
+        except fold.TooWide:
+            return 0
         return W
 
     def choose_batch(self, nodes, tables, total_slices):
@@ -411,21 +415,26 @@ class HipAPI(BaseTensorAPI):
         """Compile and upload a plan; returns an ``Executable``.  ``group_levels=False``
         keeps one launch per join (per-join timing); ``once``: the plan runs a single time."""
         folded = fold.analyse(tree, tables, self._esize, self._regroup) if fold.has_copies(tables) else None
-        if folded is not None:
-            W = self.choose_folded_batch(folded, tree, tables, total_slices)
+        W = self.choose_folded_batch(folded, tree, tables, total_slices) if folded is not None else 0
+        if W:
+            self._tune(folded[0], W)
             prog = fold.compile_program(folded, tables, num_groups, self._entry_type, W, self._alloc, group_levels,
                                         self._alloc_host)
             return self._resident(prog, total_slices, once)
         nodes = schedule.analyse(tree, tables, self._regroup)
         W = self.choose_batch(nodes, tables, total_slices)
+        self._tune(nodes, W)
+        prog = schedule.compile_program(tree, tables, num_groups, self._entry_type, W, self._alloc,
+                                        regroup=self._regroup, group_levels=group_levels)
+        return self._resident(prog, total_slices, once)
+
+    def _tune(self, nodes, W):
+        """Time the launch shapes that a plan is the first to need (``autotune`` option)."""
         if self._autotune:
             from . import autotune
 
             if autotune.tune_plan(self, nodes, W, schedule.TUNED):
                 autotune.save(schedule.TUNED)
-        prog = schedule.compile_program(tree, tables, num_groups, self._entry_type, W, self._alloc,
-                                        regroup=self._regroup, group_levels=group_levels)
-        return self._resident(prog, total_slices, once)
 
     def _resident(self, prog, total_slices, once):
         """Upload a compiled plan; returns its ``Executable``."""

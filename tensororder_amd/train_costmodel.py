@@ -40,8 +40,11 @@ def log(*a):
 
 
 def timed_records(api, plan, wave_flops=WAVE_FLOPS):
-    """Records of the first wave of one contraction, the wave capped at ``wave_flops``."""
+    """Records of the first wave of one contraction, the wave capped at ``wave_flops``.  The
+    joins are those of the tree edge by edge, as ``costmodel.predicted_seconds`` lists them."""
     total, tree, tables, groups = api._plan_inputs(plan, None)
+    for t in tables.values():
+        t.copy = None
     nodes = schedule.analyse(tree, tables, api._regroup)
     esize = api.get_entry_size()
     per_slice, _ = costmodel.plan_flops(nodes, tables, esize, api._entry_type)

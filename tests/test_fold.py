@@ -565,3 +565,58 @@ def test_folded_and_edge_walk_agree_on_the_device(et, tol):
         want = exe.run().value
         exe.close()
         assert got == pytest.approx([want] * 3, rel=tol)
+
+
+@pytest.mark.gpu
+def test_options_on_folded_plans(tmp_path, monkeypatch):
+    # the autotune option times the products of a folded plan; the cost model's records are
+    # those of the joins edge by edge
+    from tensororder_amd import autotune, train_costmodel
+
+    monkeypatch.setenv("TENSORORDER_TUNE_CACHE", str(tmp_path / "tune.json"))
+    f = parse_dimacs_text(vertex_cover_cnf(80, 3, True), "cachet")
+    plan = planners.candidate_plans(network.cnf_count(f), "line", [11])[0]
+    api = hip_api.HipF32API()
+    want = api.contract_sliced(plan)
+    saved = dict(schedule.TUNED)
+    try:
+        schedule.TUNED.clear()
+        api.add_argument("autotune", True)
+        got = api.contract_sliced(plan)
+        total, tree, tables, groups = api._plan_inputs(plan, None)
+        nodes, _ = fold.analyse(tree, tables, 4)
+        fold.choose_all(nodes, 1, 4)
+        products = {autotune.gemm_key(4, n.geom["fx"], n.geom["fy"], n.geom["s"], 1 << n.geom["var"]["hlog"])
+                    for n in nodes if not n.is_leaf and n.geom["var"]["kind"] == "gemm"}
+        assert products and products <= set(schedule.TUNED)
+    finally:
+        schedule.TUNED.clear()
+        schedule.TUNED.update(saved)
+    assert got == pytest.approx(want, rel=1e-5)
+    x, y = train_costmodel.timed_records(api, plan)
+    assert x.shape[0] == y.shape[0] > 0 and x.shape[1] == 16 and np.isfinite(x).all() and np.isfinite(y).all()
+
+
+def test_wide_joins_run_edge_by_edge(monkeypatch):
+    # a join over more variables than a descriptor holds, or a plan whose folded arena would
+    # not fit: the batch size says so (0), the unfolded path takes the plan
+    f = parse_dimacs_text(random_3cnf(24, 46, 5, True), "cachet")
+    plan = planners.candidate_plans(network.cnf_count(f), "factor", [11])[0]
+    total, tree, tables = plan_inputs(plan)[:3]
+    folded = fold.analyse(tree, tables, 8)
+
+    class Api:
+        _esize, _regroup, _max_batch, budget = 8, True, 64, 1 << 30
+        choose_batch = None
+
+        def _budget(self):
+            return self.budget
+
+    api = Api()
+    assert hip_api.HipAPI.choose_folded_batch(api, folded, tree, tables, 1) == 1
+    with monkeypatch.context() as m:
+        m.setattr(fold._lib, "FOLD_BITS", 6)
+        assert hip_api.HipAPI.choose_folded_batch(api, folded, tree, tables, 1) == 0
+        assert fold.analyse_batch([(tree, tables)], 8) is None
+    monkeypatch.setattr(fold, "peak_bytes", lambda *a: 2 << 30)
+    assert hip_api.HipAPI.choose_folded_batch(api, folded, tree, tables, 1) == 0
