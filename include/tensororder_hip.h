@@ -70,7 +70,8 @@ extern "C" {
                                 wave at params[0] == 0 starts the sum anew, and params[0] then
                                 advances by iaux0, back to 0 after the last wave; iaux1: 0, or
                                 the address of a to_accum in host memory that the device can
-                                write, which gets a copy of the sum */
+                                write, which gets a copy of the sum and then, in pad, the
+                                number of sums written so far: a word for to_wait */
 #define TO_OP_WAVE_ADVANCE 7 /* aux3: wave params; adds iaux0 to params[0] */
 #define TO_OP_STEP_BEGIN 8   /* aux2: to_accum* (zeroed), aux3: wave params (params[0] = 0) */
 #define TO_OP_PERMUTE 9      /* descs: to_perm_desc[count]; variant 1: 16-byte chunk kernel,
@@ -408,6 +409,13 @@ int to_wall_clock_khz(int* khz);
 
 /* Block until all work on `stream` is done. */
 int to_synchronize(void* stream);
+
+/* Store `value` in the host word *word (host memory that the device writes) once the work now
+ * on `stream` is done; to_wait spins on such a word for up to 2 ms, then blocks as
+ * to_synchronize does, and returns when *word >= value or the stream is idle.  The work of a
+ * stream is then seen to end without the stream's own completion marker. */
+int to_signal(int64_t* word, int64_t value, void* stream);
+int to_wait(const int64_t* word, int64_t value, void* stream);
 
 #ifdef __cplusplus
 }

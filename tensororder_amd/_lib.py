@@ -167,7 +167,7 @@ EXPORTED = [
     "to_run", "to_run_timed", "to_graph_create", "to_graph_launch", "to_graph_destroy", "to_permute",
     "to_wall_clock_khz", "to_synchronize", "to_mlp_forward", "to_mlp_backward", "to_mlp_adam",
     "to_tensordot_workspace", "to_tensordot", "to_tensordot_noalloc", "to_fold_desc_size", "to_tree_desc_size",
-    "to_upload",
+    "to_upload", "to_signal", "to_wait",
 ]
 MLP_IN, MLP_H1, MLP_H2, MLP_OUT = 16, 64, 64, 2
 MLP_NPARAMS = 64 * 16 + 64 + 64 * 64 + 64 + 2 * 64 + 2
@@ -204,6 +204,8 @@ def load(path=LIB_PATH):
     lib.to_graph_destroy.argtypes = [vp]
     lib.to_permute.argtypes = [vp, vp, i32, vp, i32, i64, vp]
     lib.to_synchronize.argtypes = [vp]
+    lib.to_signal.argtypes = [vp, i64, vp]
+    lib.to_wait.argtypes = [vp, i64, vp]
     lib.to_upload.argtypes = [vp, vp, i64, vp]
     lib.to_tensordot_workspace.argtypes = [i32, i32, vp, vp, i32, i32, p64]
     lib.to_tensordot.argtypes = [vp, vp, vp, i32, i32, vp, vp, i32, i32, vp, vp, vp, vp, i64, vp]

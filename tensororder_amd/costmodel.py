@@ -166,7 +166,7 @@ class CostModel:
                                       self._ptr(y), self._ptr(tdev), n, self._ptr(dy), self._ptr(dh2),
                                       self._ptr(dh1), self._ptr(self.grad), self._ptr(loss), self._stream())
         _lib.check(rc, "to_mlp_backward")
-        self.api.synchronize()
+        self.api.finish()
         return float(loss[0]), self.grad
 
     def adam_step(self, lr=3e-3, b1=0.9, b2=0.999, eps=1e-8):

@@ -160,6 +160,7 @@ __global__ __launch_bounds__(kGradThreads) void k_weight_grads(
             acc = 0.0;
             for (int w = 0; w < kGradThreads / 64; ++w) acc += red[w][0][0];
             loss[0] = (float)(acc / (double)(n * TO_MLP_OUT));
+            __threadfence_system();  // it may lie in host memory
         }
         return;
     }

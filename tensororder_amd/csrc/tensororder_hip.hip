@@ -16,6 +16,7 @@
 //  * FP32 mode keeps one power-of-two exponent per tensor and batch item; consumers
 //    rescale on load, producers fold max |entry| into an atomicMax on its float bits.
 #include <hip/hip_runtime.h>
+#include <chrono>
 #include <mutex>
 #include <type_traits>
 
@@ -833,7 +834,15 @@ __global__ __launch_bounds__(kBlock) void k_root_reduce(const T* __restrict__ ro
         acc->exp = am == 0.0 ? 0 : ae;
         acc->count = count;
         if (self) wave[0] = begin + nbatch < end ? begin + nbatch : 0;
-        if (host) *host = to_accum{am, am == 0.0 ? 0 : ae, count, 0};
+        if (host) {
+            host->mant = am;
+            host->exp = am == 0.0 ? 0 : ae;
+            host->count = count;
+            const int64_t sums = acc->pad + 1;
+            acc->pad = sums;
+            __threadfence_system();
+            *reinterpret_cast<volatile int64_t*>(&host->pad) = sums;
+        }
     }
 }
 
@@ -3200,6 +3209,34 @@ int to_wall_clock_khz(int* khz) {
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(khz, hipDeviceAttributeWallClockRate, dev);
     return e == hipSuccess ? TO_OK : hip_fail(e, "hipDeviceGetAttribute(WallClockRate)");
+}
+
+// What a host waits for is a word that the last kernel of a run (k_root_reduce) or this one
+// writes to its memory: the completion marker of a stream takes 11 us after the kernel's end to
+// be seen (hipStreamSynchronize or a spin on hipStreamQuery alike), such a word 1 us, and this
+// launch adds 3.
+__global__ void k_signal(int64_t* word, int64_t value) {
+    __threadfence_system();
+    *reinterpret_cast<volatile int64_t*>(word) = value;
+}
+
+int to_signal(int64_t* word, int64_t value, void* stream) {
+    g_err[0] = 0;
+    if (!word) return TO_ERR_INVALID;
+    hipLaunchKernelGGL(k_signal, dim3(1), dim3(1), 0, reinterpret_cast<hipStream_t>(stream), word, value);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? TO_OK : hip_fail(e, "to_signal launch");
+}
+
+int to_wait(const int64_t* word, int64_t value, void* stream) {
+    g_err[0] = 0;
+    if (!word) return TO_ERR_INVALID;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
+    for (int i = 0;; ++i) {
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) >= value) return TO_OK;
+        if ((i & 63) == 63 && std::chrono::steady_clock::now() > until) break;
+    }
+    return to_synchronize(stream);
 }
 
 int to_synchronize(void* stream) {

@@ -23,6 +23,7 @@ If the library or the GPU is missing, construction raises.
 
 import ctypes
 import math
+import threading
 
 import numpy as np
 
@@ -103,6 +104,9 @@ class Executable:
         # a plan that runs once only pays for capturing waves that repeat
         captured = {}
         self._runs = []
+        # runs queued since the last wait, and the value of the sum's word that ends them
+        self._queued, self._word = 0, 0
+        self._sums = sum(L.op == _lib.TO_OP_ROOT_REDUCE for r in runs for L in r)
         for r in runs:
             if id(r) not in captured:
                 use = api._use_graph and r and (not once or (r is self.wave_launches and self.nwaves > 2))
@@ -124,6 +128,11 @@ class Executable:
 
     def enqueue(self):
         """Queue one full contraction on the API's stream (no synchronisation)."""
+        if self.prog.host_accum is not None:
+            if not self._queued:
+                self._word = self._host_sum().pad
+            self._queued += 1
+            self._word += self._sums
         for graph, launches in self._runs:
             if graph is not None:
                 self._launch_graph(graph)
@@ -133,10 +142,15 @@ class Executable:
     def result(self):
         """Synchronise and read the (mantissa, exponent) slice sum."""
         api = self.api
-        api.synchronize()
         if self.prog.host_accum is not None:
-            acc = _lib.Accum.from_address(self.prog.host_accum.data_ptr())
+            acc = self._host_sum()
+            if self._queued:
+                _lib.check(api._lib.to_wait(ctypes.c_void_p(ctypes.addressof(acc) + _lib.Accum.pad.offset),
+                                            self._word, ctypes.c_void_p(api._stream.cuda_stream)), "to_wait")
+                self._queued = 0
+            acc = _lib.Accum.from_buffer_copy(acc)
         else:
+            api.synchronize()
             with api._torch.cuda.stream(api._stream):
                 acc_bytes = self.prog.accum[: ctypes.sizeof(_lib.Accum)].cpu().numpy().tobytes()
             acc = _lib.Accum.from_buffer_copy(acc_bytes)
@@ -146,11 +160,16 @@ class Executable:
         api.last_stats = dict(self.prog.stats, nbatch=self.prog.nbatch, waves=self.nwaves, slices=self.total)
         return res
 
+    def _host_sum(self):
+        return _lib.Accum.from_address(self.prog.host_accum.data_ptr())
+
     def run(self):
         self.enqueue()
         return self.result()
 
     def close(self):
+        if self._graphs:
+            self.api.synchronize()  # the sum's word is written by a kernel that has yet to end
         for g in self._graphs:
             self.api._lib.to_graph_destroy(g)
         self._graphs = []
@@ -274,6 +293,9 @@ class HipAPI(BaseTensorAPI):
         self._use_graph = True
         self._regroup = True
         self._autotune = False
+        self._signal_lock = threading.Lock()
+        self._signals = 0
+        self._signal_word = torch.zeros(1, dtype=torch.int64, pin_memory=True)  # see ``finish``
         self._device_leaves = True
         # launch shapes tuned on this GPU model (autotune.py), used where a shape is known
         from . import autotune
@@ -368,6 +390,16 @@ class HipAPI(BaseTensorAPI):
     def synchronize(self):
         _lib.check(self._lib.to_synchronize(ctypes.c_void_p(self._stream.cuda_stream)), "to_synchronize")
 
+    def finish(self):
+        """Wait until the work queued so far is done, by a word the device writes at its end."""
+        with self._signal_lock:  # the words' order is the stream's
+            self._signals += 1
+            value = self._signals
+            word = ctypes.c_void_p(self._signal_word.data_ptr())
+            stream = ctypes.c_void_p(self._stream.cuda_stream)
+            _lib.check(self._lib.to_signal(word, value, stream), "to_signal")
+        _lib.check(self._lib.to_wait(word, value, stream), "to_wait")
+
     def _budget(self):
         # free device memory plus what torch's caching allocator holds without using it
         free, _total = self._torch.cuda.mem_get_info(self._device)
@@ -446,6 +478,8 @@ class HipAPI(BaseTensorAPI):
             self._upload(prog.recs, schedule.rec_init_bytes(prog))
         self._upload(prog.params, np.array([0, total_slices, 0, 1], dtype=np.int64).tobytes())
         self._upload(prog.accum, bytes(_lib.Accum()))
+        if prog.host_accum is not None:
+            ctypes.memset(prog.host_accum.data_ptr(), 0, ctypes.sizeof(_lib.Accum))
         return Executable(self, prog, total_slices, once)
 
     def _execute(self, tree, tables, num_groups, total_slices):
@@ -676,7 +710,7 @@ class HipAPI(BaseTensorAPI):
         self._upload(table, b"".join(data for _, data in blob))
         keep.append(table)
         self._run(launches)
-        self.synchronize()
+        self.finish()
         tdtype = self._torch.float64 if not scaled else self._torch.float32
         view = cbuf[: (1 << out_rank) * self._esize].view(tdtype)
         return DeviceTensor(view, out_shape, crec, self)

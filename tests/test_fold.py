@@ -620,3 +620,44 @@ def test_wide_joins_run_edge_by_edge(monkeypatch):
         assert fold.analyse_batch([(tree, tables)], 8) is None
     monkeypatch.setattr(fold, "peak_bytes", lambda *a: 2 << 30)
     assert hip_api.HipAPI.choose_folded_batch(api, folded, tree, tables, 1) == 0
+
+
+@pytest.mark.gpu
+def test_ends_of_runs_on_the_device():
+    # a run's end is seen by a word its sum writes, that of other calls by a signal: runs
+    # queued together, launches run outside the executable between runs, and several threads
+    # waiting on one API
+    import threading
+
+    plan = plan_io.plan_from_dict(json.load(open(os.path.join(HERE, "golden", "cnf20_factor_s4.json"))))
+    want = numpy_oracle.contract_sliced(plan_io.plan_to_dict(plan))
+    for graph in (True, False):
+        api = hip_api.HipAPI()
+        api.add_argument("graph", graph)
+        api.add_argument("max_batch", 4)
+        exe = api.prepare(plan)
+        for queued in (1, 3, 2):
+            for _ in range(queued):
+                exe.enqueue()
+            r = exe.result()
+            assert r.value == pytest.approx(want, rel=1e-12) and r.slices == exe.total
+            api._run(exe.step_launches + exe.wave_launches * exe.nwaves)
+            api.synchronize()
+            assert exe.result().mant == r.mant
+        exe.close()
+    rng = np.random.default_rng(0)
+    pairs = [(rng.random((2,) * 12), rng.random((2,) * 10)) for _ in range(4)]
+    got = [None] * 4
+
+    def work(i):
+        for _ in range(20):
+            got[i] = api.tensordot(*pairs[i], ([0, 1, 2], [2, 1, 0]))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for (a, b), out in zip(pairs, got):
+        out = out.numpy() if hasattr(out, "numpy") else out
+        np.testing.assert_allclose(out, np.tensordot(a, b, ([0, 1, 2], [2, 1, 0])), rtol=1e-12)
