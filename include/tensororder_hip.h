@@ -99,6 +99,10 @@ extern "C" {
                          nreg, or those a and b */
 #define TO_OP_FOLD_TREE 15 /* descs: to_tree_desc[count]; iaux0: waves per block (1 to 16, as many
                          as each program has streams); lds: the largest of their LDS needs */
+#define TO_OP_FOLD_PAIR 17 /* descs: to_pair_desc[count], all with the same nk[0] >= nk[1]; variant:
+                              nk[0] << 4 | nk[1], each at most 2, | TO_PAIR_ONE where no Y has
+                              the lowest two o bits */
+#define TO_PAIR_ONE 0x100
 #define TO_OP_WAVE_BEGIN 16 /* TO_OP_LEAF_GATHER on the first iaux1 blocks of the grid and
                                TO_OP_SCALE_CLEAR (aux0, iaux0) on the others, in one launch:
                                descs: to_leaf_desc[count], whose records are not among those
@@ -265,6 +269,30 @@ typedef struct to_fold_desc {
     uint32_t bx[TO_FOLD_BITS], by[TO_FOLD_BITS], bc[TO_FOLD_BITS];
 } to_fold_desc;
 
+/* The dot product of two folded joins that are not stored: C = sum_o (sum_i X0 Y0) (sum_j X1 Y1),
+ * o over the variables of both joins' results, i and j over what each sums (nk[0], nk[1]
+ * variables).  Entry b of bx[side] / by[side] is what bit b adds to that side's offsets, in
+ * elements.  Bits: [0, 2) o bits that add 1 and 2 to both X; [2, 10) o bits of the thread
+ * index; then nloop o bits walked by each thread, lsplit o bits across blocks, nreg o bits that
+ * X0 lacks (its entries are loaded once for them), nk[0] bits i, nk[1] bits j.  X and its batch strides are aligned to 4
+ * elements.  With lsplit > 0 the double partial sums go to
+ * partial[batch << lsplit | sp] for a TO_OP_JOIN_FINISH launch, and rs[side], where not 0, gets
+ * the exponent of its side (TO_F32S): the records that launch reads in place of the stored
+ * results'. */
+typedef struct to_pair_desc {
+    uint64_t x[2], y[2], c;
+    int64_t xb[2], yb[2], cb;  /* batch strides in elements (0 = broadcast) */
+    uint64_t xs[2], ys[2], cs; /* to_scale_rec* per batch item (TO_F32S), else 0; ys also 0 for a
+                                  Y of ones */
+    int64_t xsb[2], ysb[2];
+    uint64_t rs[2], partial;
+    int32_t nbatch;
+    int32_t block0, nblocks;
+    int32_t nloop, lsplit, nreg;
+    int32_t nk[2];
+    uint32_t bx[2][TO_FOLD_BITS], by[2][TO_FOLD_BITS];
+} to_pair_desc;
+
 /* A program of small folded joins that one block runs start to end for one batch item: a
  * connected part of the tree whose intermediate tensors fit LDS.  A join of a program is a
  * product of up to 4 tensors, summed over the k bits.  Each wave of the block walks its own
@@ -339,6 +367,7 @@ int to_struct_sizes(int64_t* join_desc, int64_t* leaf_desc, int64_t* scale_rec,
 /* Size in bytes of to_fold_desc and to_tree_desc, for the same check. */
 int to_fold_desc_size(void);
 int to_tree_desc_size(void);
+int to_pair_desc_size(void);
 
 /* Last error message of the calling thread ("" when none). */
 const char* to_last_error(void);

@@ -29,7 +29,8 @@ TO_F64, TO_F32S = 0, 1
     TO_OP_FOLD,
     TO_OP_FOLD_TREE,
     TO_OP_WAVE_BEGIN,
-) = range(1, 17)
+    TO_OP_FOLD_PAIR,
+) = range(1, 18)
 TO_LEAF_VAR, TO_LEAF_OR = 0, 1  # leaf build kinds
 TO_STREAM_VEC = 0x100  # stream variant bit: the 16-byte form
 TO_STREAM_ROWS = 0x200  # stream variant: the row form
@@ -45,6 +46,7 @@ TO_TREE_WORDS = 448  # uint32 words of one join of a fold tree program
 TO_TREE_IDLE, TO_TREE_MEET = 1 << 30, 1 << 31  # fold tree task bits
 MAX_BITS = 32
 FOLD_BITS = 40
+TO_PAIR_ONE = 0x100
 ABI_VERSION = 7
 
 c_i8x32 = ctypes.c_int8 * MAX_BITS
@@ -146,6 +148,17 @@ class TreeDesc(ctypes.Structure):
                 ("block0", ctypes.c_int32), ("nblocks", ctypes.c_int32)]
 
 
+class PairDesc(ctypes.Structure):
+    _fields_ = [("x", ctypes.c_uint64 * 2), ("y", ctypes.c_uint64 * 2), ("c", ctypes.c_uint64),
+                ("xb", ctypes.c_int64 * 2), ("yb", ctypes.c_int64 * 2), ("cb", ctypes.c_int64),
+                ("xs", ctypes.c_uint64 * 2), ("ys", ctypes.c_uint64 * 2), ("cs", ctypes.c_uint64),
+                ("xsb", ctypes.c_int64 * 2), ("ysb", ctypes.c_int64 * 2),
+                ("rs", ctypes.c_uint64 * 2), ("partial", ctypes.c_uint64), ("nbatch", ctypes.c_int32),
+                ("block0", ctypes.c_int32), ("nblocks", ctypes.c_int32), ("nloop", ctypes.c_int32),
+                ("lsplit", ctypes.c_int32), ("nreg", ctypes.c_int32), ("nk", ctypes.c_int32 * 2),
+                ("bx", c_u32xF * 2), ("by", c_u32xF * 2)]
+
+
 class RootDesc(ctypes.Structure):
     _fields_ = [("root", ctypes.c_uint64), ("rec", ctypes.c_uint64), ("acc", ctypes.c_uint64),
                 ("block0", ctypes.c_int32), ("nblocks", ctypes.c_int32)]
@@ -167,6 +180,7 @@ EXPORTED = [
     "to_run", "to_run_timed", "to_graph_create", "to_graph_launch", "to_graph_destroy", "to_permute",
     "to_wall_clock_khz", "to_synchronize", "to_mlp_forward", "to_mlp_backward", "to_mlp_adam",
     "to_tensordot_workspace", "to_tensordot", "to_tensordot_noalloc", "to_fold_desc_size", "to_tree_desc_size",
+    "to_pair_desc_size",
     "to_upload", "to_signal", "to_wait",
 ]
 MLP_IN, MLP_H1, MLP_H2, MLP_OUT = 16, 64, 64, 2
@@ -221,7 +235,7 @@ def load(path=LIB_PATH):
     want = [ctypes.sizeof(t) for t in (JoinDesc, LeafDesc, ScaleRec, Accum, Launch, PermDesc, GemmDesc, RootDesc,
                                        LeafBuildDesc)]
     if [s.value for s in sizes] != want or lib.to_fold_desc_size() != ctypes.sizeof(FoldDesc) \
-            or lib.to_tree_desc_size() != ctypes.sizeof(TreeDesc):
+            or lib.to_tree_desc_size() != ctypes.sizeof(TreeDesc) or lib.to_pair_desc_size() != ctypes.sizeof(PairDesc):
         raise ImportError("record layout mismatch between library and binding: %s vs %s"
                           % ([s.value for s in sizes], want))
     _lib = lib

@@ -2491,6 +2491,30 @@ int launch_one(const to_launch& L, hipStream_t st) {
             hipLaunchKernelGGL((k_root_store<T, SCALED>), grid, block, 0, st,
                                reinterpret_cast<const to_root_desc*>(L.descs), L.count);
             break;
+        case TO_OP_FOLD_PAIR: {
+            if (!L.descs || L.count <= 0) return TO_ERR_INVALID;
+            const to_pair_desc* pd = reinterpret_cast<const to_pair_desc*>(L.descs);
+            switch (L.variant) {
+#define TO_PAIR_CASE(A, B)                                                                                 \
+    case A << 4 | B:                                                                                       \
+        hipLaunchKernelGGL((k_fold_pair<T, SCALED, A, B, false>), grid, block, 0, st, pd, L.count, bmap); \
+        break;                                                                                             \
+    case TO_PAIR_ONE | A << 4 | B:                                                                         \
+        hipLaunchKernelGGL((k_fold_pair<T, SCALED, A, B, true>), grid, block, 0, st, pd, L.count, bmap);  \
+        break;
+                TO_PAIR_CASE(0, 0)
+                TO_PAIR_CASE(1, 0)
+                TO_PAIR_CASE(1, 1)
+                TO_PAIR_CASE(2, 0)
+                TO_PAIR_CASE(2, 1)
+                TO_PAIR_CASE(2, 2)
+#undef TO_PAIR_CASE
+                default:
+                    set_err("fold pair: unsupported variant");
+                    return TO_ERR_INVALID;
+            }
+            break;
+        }
         case TO_OP_FOLD_TREE: {
             if (!L.descs || L.count <= 0 || L.iaux0 < 1 || L.iaux0 > 16) return TO_ERR_INVALID;
             if (L.lds > 64 * 1024) {
@@ -2611,6 +2635,8 @@ int to_struct_sizes(int64_t* join_desc, int64_t* leaf_desc, int64_t* scale_rec, 
     if (launch) *launch = sizeof(to_launch);
     return TO_OK;
 }
+
+int to_pair_desc_size(void) { return (int)sizeof(to_pair_desc); }
 
 int to_tree_desc_size(void) { return (int)sizeof(to_tree_desc); }
 

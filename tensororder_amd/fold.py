@@ -50,6 +50,8 @@ ANY_MIN_THREADS_LOG = 17
 MAX_ANY_BLOCKS = 8192
 MAX_VEC_BLOCKS = 4096
 MAX_REG_BITS = 3
+# blocks of a fused dot product (four waves each; a CU holds eight blocks)
+PAIR_MIN_BLOCKS_LOG = 13
 # register tiles (variables only X has, only Y has), the first that a join has; it must leave
 # this many outputs to threads
 REG_TILES = ((2, 3), (2, 2), (1, 1), (2, 0))
@@ -281,8 +283,10 @@ def analyse(tree, tables, esize, regroup=True):
         n.is_leaf, n.batched, n.left, n.right, n.rank, n.order = False, leaf_node.batched, leaf_node.idx, -1, 0, []
         leaf_node.parent = n.idx
         nodes.append(n)
-    # the plan's one bit order: variables summed later are lower bits
-    when = {}
+    # the plan's one bit order: variables summed later are lower bits, of these the ones that
+    # the smaller operands of the larger joins hold less (a wave's loads of such an operand
+    # take fewer lines)
+    when, weight = {}, {}
     for n in nodes:
         if n.is_leaf:
             continue
@@ -293,8 +297,11 @@ def analyse(tree, tables, esize, regroup=True):
         n.ksum = held - kept
         for v in n.ksum:
             when[v] = n.idx
+        if n.right >= 0:
+            for v in min(nodes[n.left].order, nodes[n.right].order, key=len):
+                weight[v] = weight.get(v, 0.0) + 2.0 ** len(held)
     for n in nodes:
-        n.order.sort(key=lambda v: (-when[v], v))
+        n.order.sort(key=lambda v: (-when[v], weight.get(v, 0.0), v))
         n.order0 = n.order
     return nodes, missing
 
@@ -417,6 +424,65 @@ def choose_all(nodes, W, esize, launch_bound=False):
     for n in nodes:
         if not n.is_leaf:
             choose(n, nodes, W, esize, launch_bound)
+    if not launch_bound and not nodes[-1].is_leaf:
+        _fuse(nodes[-1], nodes, W)
+
+
+def _fuse(n, nodes, W):
+    """The dot product at the root with the joins that make its operands, or one of them, run
+    inside it (TO_OP_FOLD_PAIR): each stores and reads back a large tensor otherwise (the
+    2^20-entry operands of 4096 slices: 7.4 + 7.3 ms for the joins and 5.6 for the dot).  Only
+    joins too large for a program, that sum at most two variables: their large operand is then
+    read about once."""
+    if n.geom["var"].get("variant") != _lib.TO_FOLD_DOT or n.rank or n.left < 0:
+        return
+
+    def side(c):
+        f = nodes[c]
+        if f.is_leaf or f.right < 0 or f.batched != n.batched or f.geom["var"]["kind"] != "fold" or \
+                f.rank <= TREE_RANK or len(f.ksum) > 2:
+            return None
+        return nodes[f.geom["X"]], nodes[f.geom["Y"]], sorted(f.ksum), f
+
+    plain = [(nodes[c], None, [], None) for c in (n.geom["X"], n.geom["Y"])]
+    inner = [side(c) for c in (n.geom["X"], n.geom["Y"])]
+    for pair in ((inner[0], inner[1]), (inner[0], plain[1]), (inner[1], plain[0])):
+        if None in pair:
+            continue
+        a, b = sorted(pair, key=lambda p: -len(p[2]))
+        xa, xb = a[0].off, b[0].off
+        order = sorted(n.ksum, key=lambda v: (xa.get(v, 1 << 40), xb.get(v, 1 << 40), v))
+        body = [v for v in order if v in xa]
+        reg = [v for v in order if v not in xa]
+        # the variables only X0 has change fastest (X1's entries come again from a cache)
+        wide = [v for v in body if v in xb][:10]
+        body = wide + [v for v in body if v not in xb] + [v for v in body if v in xb and v not in wide]
+        bits = body + reg + a[2] + b[2]
+        if len(body) < 10 or len(reg) > 4 or len(bits) > _lib.FOLD_BITS or \
+                any(x.get(body[0]) != 1 or x.get(body[1]) != 2 for x in (xa, xb)):
+            continue
+
+        lows = any(y is not None and (v in y.off) for v in body[:2] for y in (a[1], b[1]))
+        nb = W if n.batched else 1
+        lsplit = max(0, min(len(body) - 10, PAIR_MIN_BLOCKS_LOG - int(math.log2(nb))))
+        reads = [t.idx for s in (a, b) for t in s[:2] if t is not None]
+        n.geom.update(reads=reads, var=dict(
+            kind="pair", variant=len(a[2]) << 4 | len(b[2]) | (0 if lows else _lib.TO_PAIR_ONE), sides=(a, b), bits=bits, nreg=len(reg),
+            nloop=len(body) - 10 - lsplit, lsplit=lsplit, nsplit=1 << lsplit, nout=nb,
+            nblocks=int(min(nb << lsplit, MAX_ANY_BLOCKS))))
+        for s in (a, b):
+            if s[3] is not None:
+                s[3].geom["var"] = dict(kind="fused")
+        return
+
+
+def _reads(n):
+    """The tensors a join reads (of a fused one, those its parts read)."""
+    return n.geom.get("reads") or [c for c in (n.left, n.right) if c >= 0]
+
+
+def _fused(n):
+    return not n.is_leaf and n.geom["var"]["kind"] == "fused"
 
 
 def _scratch(arena, n, nodes, nb, esize, table):
@@ -612,12 +678,12 @@ def phase_groups(nodes, batched, order, programs):
     level, out = {}, []
     first = []
     for n in nodes:
-        if n.is_leaf or n.batched != batched:
+        if n.is_leaf or n.batched != batched or _fused(n):
             continue
         p = unit.get(n.idx)
         if p is not None and p.root != n.idx:
             continue
-        lv = 1 + max((level.get(c, 0) for c in (p.outside if p is not None else (n.left, n.right))), default=0)
+        lv = 1 + max((level.get(c, 0) for c in (p.outside if p is not None else _reads(n))), default=0)
         level[n.idx] = lv
         if order == "level":
             while len(out) < lv:
@@ -645,9 +711,9 @@ def plan_memory(nodes, W, esize, order, programs=()):
         for blk in temps:
             arena.release(blk)
         read = [c for p in group[0] for lv in p.levels for _, mine in lv for c in mine if c not in p.at]
-        read += [c for i in group[1] for c in (nodes[i].left, nodes[i].right)]
+        read += [c for i in group[1] for c in _reads(nodes[i])]
         for c in read:
-            if c >= 0 and release(nodes[c]):
+            if release(nodes[c]):
                 arena.release(nodes[c].buf)
 
     for grp in phase_groups(nodes, False, order, programs):
@@ -727,6 +793,8 @@ def join_records(n, nodes, W, esize, scaled, abase, scratch, recp, one):
             f.fx, f.fy, f.shf, f.shy, f.nbatch, f.nblocks = g["fx"], g["fy"], g["shf"], 0, nb, v["fin_blocks"]
             out.append(("finish", _lib.TO_OP_JOIN_FINISH, 0, 0, f, f.nblocks))
         return out
+    if v["kind"] == "pair":
+        return pair_records(n, W, esize, scaled, abase, scratch, recp, one)
     d = FoldDesc()
     yptr, yrec, ystride, yrecs = one[0], one[1], 0, 0
     if Y is not None:
@@ -746,16 +814,49 @@ def join_records(n, nodes, W, esize, scaled, abase, scratch, recp, one):
         + [n.off.get(b, 0) for b in v["bits"]] + fill
     out.append(("fold", _lib.TO_OP_FOLD, v["variant"], 0, d, v["nblocks"]))
     if v["lsplit"]:
-        f = _lib.JoinDesc()
-        f.c, f.cb, f.partial, f.nsplit = n.ptr, n.bstride, partial, v["nsplit"]
-        if scaled:
-            f.xs, f.ys, f.cs = d.recs
-            f.xsb, f.ysb = d.rec_strides
-        f.fx, f.nbatch = n.rank, nb
-        wide = v["nsplit"] >= 32
-        f.nblocks = int(min(v["nout"] if wide else -(-v["nout"] // 256), schedule.MAX_STREAM_BLOCKS))
-        out.append(("finish", _lib.TO_OP_JOIN_FINISH, 1 if wide else 0, 0, f, f.nblocks))
+        out.append(_finish(n, v, partial, nb, list(zip(d.recs, d.rec_strides)) if scaled else [], d.recs[2]))
     return out
+
+
+def pair_records(n, W, esize, scaled, abase, scratch, recp, one):
+    """Descriptor records of a fused dot product (see ``join_records``)."""
+    v = n.geom["var"]
+    nb = W if n.batched else 1
+    d = _lib.PairDesc(c=n.ptr, cb=n.bstride, cs=recp(n) if scaled else 0, nbatch=nb, nblocks=v["nblocks"],
+                      nloop=v["nloop"], lsplit=v["lsplit"], nreg=v["nreg"])
+    nbits = len(v["bits"])
+    ends = []
+    for k, (X, Y, ksum, f) in enumerate(v["sides"]):
+        d.x[k], d.xb[k] = X.ptr, X.bstride if n.batched else 0
+        d.y[k], d.yb[k] = (Y.ptr, Y.bstride if n.batched else 0) if Y is not None else (one[0], 0)
+        d.nk[k] = len(ksum)
+        d.bx[k][:nbits] = [X.off.get(b, 0) for b in v["bits"]]
+        d.by[k][:nbits] = [Y.off.get(b, 0) if Y is not None else 0 for b in v["bits"]]
+        if scaled:
+            d.xs[k], d.xsb[k] = recp(X), X.rec_stride if n.batched else 0
+            if Y is not None:
+                d.ys[k], d.ysb[k] = recp(Y), Y.rec_stride if n.batched else 0
+            if f is not None:
+                d.rs[k] = recp(f)
+            ends.append((recp(f), f.rec_stride if n.batched else 0) if f is not None else (d.xs[k], d.xsb[k]))
+    out = [("pair", _lib.TO_OP_FOLD_PAIR, v["variant"], 0, d, v["nblocks"])]
+    if v["lsplit"]:
+        d.partial = abase + scratch["partial"][0]
+        out.append(_finish(n, v, d.partial, nb, ends, d.cs))
+    return out
+
+
+def _finish(n, v, partial, nb, ends, crec):
+    """The record that adds up a join's partial sums; ``ends``: (record, stride) of the two
+    operands, whose exponents the result carries (scaled only)."""
+    f = _lib.JoinDesc()
+    f.c, f.cb, f.partial, f.nsplit = n.ptr, n.bstride, partial, v["nsplit"]
+    if ends:
+        (f.xs, f.xsb), (f.ys, f.ysb), f.cs = ends[0], ends[1], crec
+    f.fx, f.nbatch = n.rank, nb
+    wide = v["nsplit"] >= 32
+    f.nblocks = int(min(v["nout"] if wide else -(-v["nout"] // 256), schedule.MAX_STREAM_BLOCKS))
+    return "finish", _lib.TO_OP_JOIN_FINISH, 1 if wide else 0, 0, f, f.nblocks
 
 
 def join_traffic(n, nodes, W, esize):
@@ -838,7 +939,7 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
     wave_params = prog.params.data_ptr()
     one_at = (tbase + one * esize, rbase + one_rec * 16 if scaled else 0)
     for n in nodes:
-        if n.idx in in_lds:
+        if n.idx in in_lds or _fused(n):
             continue
         if n.is_leaf and not n.batched:
             n.ptr, n.bstride = tbase + image.off[n.tensor] * esize, 0
@@ -881,6 +982,10 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
                     work = (2 * esize * (int(st.nbatch) << int(st.rank)), 0)
                 elif kind in ("fold", "gemm"):
                     work = join_traffic(n, nodes, W, esize)
+                elif kind == "pair":
+                    work = (sum((1 << nodes[c].rank) * (W if nodes[c].batched else 1) for c in _reads(n)) * esize,
+                            sum(join_traffic(nodes[c], nodes, W, esize)[1]
+                                for c in [i] + [f.idx for *_, f in n.geom["var"]["sides"] if f is not None]))
                 else:
                     work = (0, 0)
                 keyed.setdefault((schedule.KIND_ORDER[kind], op, variant), []).append((kind, st, nblk, lds, i, work))

@@ -28,7 +28,7 @@ from ._lib import JoinDesc, LeafDesc, Launch
 ALIGN = 256
 STREAM_MAX_S = 12
 # order of a join's launches inside a group: operand permutes, products, split-K finishing
-KIND_ORDER = {"permute": 0, "stream": 1, "splitk": 1, "fold": 1, "gemm": 1, "finish": 2}
+KIND_ORDER = {"permute": 0, "stream": 1, "splitk": 1, "fold": 1, "pair": 1, "gemm": 1, "finish": 2}
 LDS_LIMIT = 64 * 1024
 MAX_STREAM_BLOCKS = 4096
 # one-wave streamed joins (many-instance batch): at most this many products per lane

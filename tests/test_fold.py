@@ -36,7 +36,8 @@ def _spread(entries, lo, n):
 
 
 class FoldEmulator(emulator.Emulator):
-    TABLE_DESCS = {**emulator.Emulator.TABLE_DESCS, _lib.TO_OP_FOLD: "FoldDesc", _lib.TO_OP_FOLD_TREE: "TreeDesc"}
+    TABLE_DESCS = {**emulator.Emulator.TABLE_DESCS, _lib.TO_OP_FOLD: "FoldDesc", _lib.TO_OP_FOLD_TREE: "TreeDesc",
+                   _lib.TO_OP_FOLD_PAIR: "PairDesc"}
 
     def __init__(self, heap, entry_type):
         super().__init__(heap, entry_type)
@@ -142,6 +143,45 @@ class FoldEmulator(emulator.Emulator):
                 if self.scaled:
                     m = np.float32(np.max(np.abs(val)))
                     self.set_rec(d.cs, b, exp=e, maxbits=int(m.view(np.uint32)))
+
+    def op_17(self, L):
+        esz = self.dt().itemsize
+        for i in range(L.count):
+            d = self.heap.read_struct(_lib.PairDesc, L.descs + i * ctypes.sizeof(_lib.PairDesc))
+            self.forms.add((_lib.TO_OP_FOLD_PAIR, L.variant))
+            one = 0 if any(list(d.by[0])[:2] + list(d.by[1])[:2]) else _lib.TO_PAIR_ONE
+            assert L.variant == d.nk[0] << 4 | d.nk[1] | one and d.nk[0] >= d.nk[1]
+            ka = 10 + d.nloop + d.lsplit + d.nreg
+            assert ka + sum(d.nk) <= _lib.FOLD_BITS and not any(list(d.bx[0])[ka - d.nreg:ka])
+            for b in range(d.nbatch):
+                side, f, exps = [], 1.0, []
+                for k in range(2):
+                    bx, by = list(d.bx[k]), list(d.by[k])
+                    assert bx[:2] == [1, 2] and all(int(e) % 4 == 0 for e in bx[2:])
+                    assert d.x[k] % (4 * esz) == 0 and d.xb[k] % 4 == 0
+                    first = ka + (d.nk[0] if k else 0)
+                    xo, yo = (_spread(arr, 0, ka)[:, None] + _spread(arr, first, d.nk[k])[None, :] for arr in (bx, by))
+                    X = self.heap.view(d.x[k] + b * d.xb[k] * esz, self.dt, int(xo.max()) + 1).astype(np.float64)
+                    Y = self.heap.view(d.y[k] + b * d.yb[k] * esz, self.dt, int(yo.max()) + 1).astype(np.float64)
+                    side.append((X[xo] * Y[yo]).sum(axis=1))
+                    if self.scaled:
+                        recs = [self.get_rec(at, b * stride)
+                                for at, stride in ((d.xs[k], d.xsb[k]), (d.ys[k], d.ysb[k])) if at]
+                        exps.append(sum(r[0] + emulator._scale_exp(r[1]) for r in recs))
+                        f *= math.prod(2.0 ** -emulator._scale_exp(r[1]) for r in recs)
+                        if d.lsplit and d.rs[k]:
+                            self.set_rec(d.rs[k], b, exp=exps[k], maxbits=0)
+                prod = side[0] * side[1] * f
+                if d.lsplit:
+                    parts = prod.reshape(1 << d.nreg, 1 << d.lsplit, -1).sum(axis=(0, 2))
+                    P = self.heap.view(d.partial, np.float64, d.nbatch << d.lsplit)
+                    P[b << d.lsplit:(b + 1) << d.lsplit] = parts
+                    self.gemm_partials.add(d.partial)
+                    continue
+                val = self.dt(prod.sum())
+                self.heap.view(d.c + b * d.cb * esz, self.dt, 1)[0] = val
+                if self.scaled:
+                    self.set_rec(d.cs, b, exp=sum(exps), maxbits=int(np.abs(val).view(np.uint32)))
 
     def op_15(self, L):
         # block by block: the streams' tasks level by level; LDS starts as NaN, every tensor
@@ -474,12 +514,12 @@ def _launches(records, alloc, write):
     return out
 
 
-def _check(case, et, got, rec, want):
+def _check(case, et, got, rec, want, rtol=1e-13):
     # products of floats are exact in the double sums: one rounding, at the store
     dt = np.float64 if et == _lib.TO_F64 else np.float32
     for b in range(want.shape[0]):
         scale = 2.0 ** int(rec[b].exp) if et == _lib.TO_F32S else 1.0
-        np.testing.assert_allclose(got[b].astype(np.float64) * scale, want[b], rtol=1e-13 if dt == np.float64 else 1.2e-7)
+        np.testing.assert_allclose(got[b].astype(np.float64) * scale, want[b], rtol=rtol if dt == np.float64 else 1.2e-7)
         if et == _lib.TO_F32S:
             assert rec[b].maxbits == int(np.abs(got[b]).max().view(np.uint32))
 
@@ -661,3 +701,203 @@ def test_ends_of_runs_on_the_device():
     for (a, b), out in zip(pairs, got):
         out = out.numpy() if hasattr(out, "numpy") else out
         np.testing.assert_allclose(out, np.tensordot(a, b, ([0, 1, 2], [2, 1, 0])), rtol=1e-12)
+
+
+# dot products with their operands' joins inside (each with the lowest variables in no small
+# operand, and as listed): variables both large operands have, that only
+# the first / only the second has, summed by the joins; slices; whether each operand has them;
+# the lowest two variables in the small operands: none, both lowest, both, first, second
+PAIRS = [(14, 0, 0, 0, 0, 1, "xyzw", "nn"), (15, 0, 1, 1, 0, 3, "xyzw", "vs"), (13, 2, 1, 2, 1, 5, "xyz", "sv"),
+         (12, 1, 3, 1, 1, 2, "xzw", "ss"), (13, 1, 0, 2, 0, 33, "xyzw", "nf"), (13, 3, 1, 2, 2, 2, "xyzw", "bv"),
+         (10, 4, 1, 2, 1, 4097, "xyzw", "sn"), (16, 0, 0, 1, None, 2, "xyz", "s"), (14, 0, 1, 2, None, 3, "xyz", "v")]
+
+
+PAIRS += [case[:7] + ("n" * len(case[7]),) for case in PAIRS] + [(13, 1, 1, 1, 1, 3, "xyzw", "nn"), (14, 1, 0, 2, 2, 1, "xw", "nn"),
+                                                              (14, 0, 0, 0, 0, 2, "yz", "sn")]
+
+
+def _pair(case, et, alloc, write, rng):
+    """A root dot product with its joins compiled by ``fold.choose_all``, as ``_join``."""
+    body, r0, r1, na, nb, W, sliced, lows = case
+    esize = 8 if et == _lib.TO_F64 else 4
+    dt = np.float64 if esize == 8 else np.float32
+    big = ["v%d" % i for i in range(body)]
+    ya_only, yb_only = ["s%d" % i for i in range(r0)], ["t%d" % i for i in range(r1)]
+    sums = [["i%d" % i for i in range(na)], ["j%d" % i for i in range(nb or 0)]]
+    out = big + ya_only + yb_only
+
+    def small(how, own):
+        mid = [str(v) for v in rng.permutation(big[2:])[:3]]
+        low = {"n": [], "v": big[:2], "s": [], "f": [], "b": []}[how]
+        rest = mid + own + {"s": big[1:2], "f": big[:1], "b": big[:2]}.get(how, [])
+        rng.shuffle(rest)
+        return low + rest
+
+    def large(own):
+        rest = big[2:] + own
+        rng.shuffle(rest)
+        return big[:2] + rest
+
+    specs = [(large(yb_only + sums[0]), "x" in sliced), (small(lows[0], ya_only + sums[0]), "y" in sliced)]
+    if nb is not None:
+        specs += [(large(ya_only + sums[1]), "z" in sliced), (small(lows[1], yb_only + sums[1]), "w" in sliced)]
+    else:  # the other operand is stored
+        specs += [(big + yb_only, "z" in sliced)]
+    nodes = []
+
+    def add(order, batched, left=-1, right=-1, ksum=()):
+        n = fold.FNode(len(nodes))
+        n.is_leaf, n.batched, n.order, n.order0 = left < 0, bool(batched), list(order), list(order)
+        n.rank, n.left, n.right, n.ksum = len(order), left, right, set(ksum)
+        n.off = {v: 1 << j for j, v in enumerate(order)}
+        nodes.append(n)
+        return n.idx
+
+    leaves = [add(*sp) for sp in specs]
+    a = add(out, True, leaves[0], leaves[1], sums[0])
+    b = add(out, True, leaves[2], leaves[3], sums[1]) if nb is not None else leaves[2]
+    add([], True, a, b, out)
+    fold.choose_all(nodes, W, esize)
+    data, recs = {}, {}
+    for n in nodes:
+        items = W if n.batched else 1
+        n.bstride = (1 << n.rank) if n.batched else 0
+        n.rec_stride = 1 if n.batched else 0
+        recs[n.idx] = alloc(16 * items)
+        write(recs[n.idx], bytes(16 * items))
+        if n.is_leaf or n is nodes[-1]:
+            n.ptr = alloc(items * esize << n.rank)
+        if n.is_leaf:
+            data[n.idx] = rng.uniform(0.25, 1.0, (items, 1 << n.rank)).astype(dt)
+            write(n.ptr, data[n.idx].tobytes())
+            write(recs[n.idx], b"".join(bytes(_lib.ScaleRec(exp=3 - k % 7, maxbits=int(
+                np.abs(data[n.idx][k]).max().astype(np.float32).view(np.uint32)))) for k in range(items)))
+    root = nodes[-1]
+    v = root.geom["var"]
+    assert v["kind"] == "pair" and nodes[a].geom["var"]["kind"] == "fused"
+    one = alloc(256)
+    write(one, dt(1).tobytes())
+    scratch = {"partial": (alloc(v["nout"] * v["nsplit"] * 8), 0)} if v.get("lsplit") else {}
+    records = fold.join_records(root, nodes, W, esize, esize == 4, 0, scratch, lambda n: recs[n.idx], (one, 0))
+    want = []
+    for k in range(min(W, 5)):
+        terms = [(data[i][k if nodes[i].batched else 0].astype(np.float64).reshape((2,) * nodes[i].rank),
+                  nodes[i].order[::-1]) for i in leaves]
+        number = {u: j for j, u in enumerate(sorted({u for _, vs in terms for u in vs}))}
+        halves = []
+        for part in (terms[:2], terms[2:]):
+            args = [x for t, vs in part for x in (t, [number[u] for u in vs])]
+            halves.append(np.einsum(*args, [number[u] for u in out]))
+        e = sum(3 - (k % 7 if nodes[i].batched else 0) for i in leaves) if esize == 4 else 0
+        want.append([(halves[0] * halves[1]).sum() * 2.0 ** e])
+    return records, nodes, recs, np.array(want)
+
+
+@pytest.mark.parametrize("et", [_lib.TO_F64, _lib.TO_F32S], ids=["f64", "f32s"])
+def test_fused_dot_products_emulated(et):
+    forms = set()
+    for i, case in enumerate(PAIRS):
+        if case[5] > 100:
+            continue  # whole blocks of slices: on the device
+        heap = emulator.Heap(1 << 26)
+        ptr = {}
+
+        def alloc(n):
+            b = heap.alloc(n)
+            ptr[b.data_ptr()] = b
+            return b.data_ptr()
+
+        def write(at, data):
+            heap.write(ptr[at], data)
+
+        records, nodes, recs, want = _pair(case, et, alloc, write, np.random.default_rng(i))
+        emu = FoldEmulator(heap, et)
+        emu.run(_launches(records, alloc, write))
+        forms |= emu.forms
+        got = heap.view(nodes[-1].ptr, emu.dt, case[5]).reshape(-1, 1)[:len(want)]
+        rec = [heap.read_struct(_lib.ScaleRec, recs[nodes[-1].idx] + 16 * b) for b in range(len(want))]
+        _check(case, et, got, rec, want, 1e-12)
+    assert {f[1] for f in forms if isinstance(f, tuple)} == {
+        k | one for k in (0x00, 0x10, 0x11, 0x20, 0x21, 0x22) for one in (0, _lib.TO_PAIR_ONE)}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("et", [_lib.TO_F64, _lib.TO_F32S], ids=["f64", "f32s"])
+def test_fused_dot_products_on_the_device(et):
+    import torch
+
+    api = hip_api.HipAPI() if et == _lib.TO_F64 else hip_api.HipF32API()
+    for i, case in enumerate(PAIRS):
+        _say("case fused dot", et, case)
+        ptr = {}
+
+        def alloc(n):
+            t = torch.full((n,), 255, dtype=torch.uint8, device="cuda")
+            ptr[t.data_ptr()] = t
+            return t.data_ptr()
+
+        def write(at, data):
+            ptr[at][:len(data)] = torch.frombuffer(bytearray(data), dtype=torch.uint8).cuda()
+
+        records, nodes, recs, want = _pair(case, et, alloc, write, np.random.default_rng(i))
+        launches = _launches(records, alloc, write)
+        torch.cuda.synchronize()
+        api._run(launches)
+        api.synchronize()
+        dt = np.float64 if et == _lib.TO_F64 else np.float32
+        got = ptr[nodes[-1].ptr].cpu().numpy().view(dt).reshape(-1, 1)[:len(want)]
+        raw = ptr[recs[nodes[-1].idx]].cpu().numpy().tobytes()
+        rec = [_lib.ScaleRec.from_buffer_copy(raw[16 * b:16 * b + 16]) for b in range(len(want))]
+        _check(case, et, got, rec, want, 1e-12)
+
+
+def _halves_plan(seed, slices):
+    """A plan whose root is the dot product of two halves, each a large tensor absorbing a
+    small one: dense tensors tied by COPY tensors of 12 to 14 variables."""
+    from tensororder_amd.network import BuiltTensor, TensorNetwork, VariableTensor
+    from tensororder_amd.plan import SlicedExecutionPlan
+    from tensororder_amd.tree import TreeContext
+
+    rng = np.random.default_rng(seed)
+    big = ["v%d" % i for i in range(13)]
+    tensors = [big + ["i"], ["i", "s"] + big[3:6], big[:11] + ["s", "j"], ["j"] + big[9:13]]
+    net, ends = TensorNetwork(), {}
+    for vs in tensors:
+        # the first variables are the lowest bits of the large tensors, as the executor orders its own
+        vs = [str(v) for v in rng.permutation(vs[2:])] + vs[1::-1] if len(vs) > 6 else vs
+        for v, end in zip(vs, net.add_node(BuiltTensor(rng.uniform(0.5, 1.0, (2,) * len(vs))))):
+            ends.setdefault(v, []).append(end)
+    copies = {}
+    for v, held in ends.items():
+        at = net.add_node(VariableTensor(len(held), 1, 1 if v != "v5" else 0.5))
+        copies[v] = at[0][0]
+        for (t, ax), end in zip(held, at):
+            net.connect(t, ax, *end)
+    ctx = TreeContext()
+    halves = []
+    for a, b, inner in ((0, 1, "i"), (2, 3, "j")):
+        # (the variable summed inside a half is tied before the small tensor comes)
+        half = ctx.join(ctx.join(ctx.leaf(net, a), ctx.leaf(net, copies[inner])), ctx.leaf(net, b))
+        halves.append(half)
+    for v in copies:
+        if v not in "ij":
+            halves[0] = ctx.join(halves[0], ctx.leaf(net, copies[v]))
+    plan = SlicedExecutionPlan(ctx.get_tree(ctx.join(*halves)), net)
+    ALL_SLICERS["greedy_mem"].slice_until(plan, slices=slices)
+    return plan
+
+
+@pytest.mark.parametrize("et,tol", [(_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)])
+def test_fused_dot_products_in_plans(et, tol, monkeypatch):
+    # whole plans, the rank from which joins are fused lowered
+    monkeypatch.setattr(fold, "TREE_RANK", 9)
+    fused = set()
+    for seed in range(3):
+        for slices in (0, 1, 2):
+            plan = _halves_plan(seed, slices)
+            want = numpy_oracle.contract_sliced(plan_io.plan_to_dict(plan))
+            for W in {1, 1 << slices}:
+                got, prog, emu = emulate(plan, et, W, device_leaves=False)
+                assert got == pytest.approx(want, rel=tol)
+                fused |= {(slices, f[1]) for f in emu.forms if isinstance(f, tuple)}
+    assert {f[0] for f in fused} >= {0, 1} and {f[1] & 0xff for f in fused} == {0x11}
