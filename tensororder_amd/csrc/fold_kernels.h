@@ -310,8 +310,14 @@ __global__ __launch_bounds__(kBlock) void k_fold_reg(const to_fold_desc* __restr
 
 // 16-byte form for the large joins: a thread owns 4 consecutive outputs times the 2^RY
 // outputs of the register bits (variables only Y has), so an X entry is loaded once for all
-// of them, 16 bytes at a time; Y, the small operand, is read through L1.  Bound by the HBM
-// bytes of X and C.
+// of them, 16 bytes at a time; Y is read through L1, with as few loads as the places of the
+// outputs' two lowest variables and of the register variables in it allow (YM).  Bound by the
+// HBM bytes of X and C where few indices are summed: 2^19 by 2^15 over 2 to 2^20, 4096 slices
+// (26 GB), 5.3 ms, the rate of a copy.  2^16 by 2^16 over 2^3 to 2^20 (19 GB) takes 5.7 ms: its
+// stores alone take 3.0, the loads and double products alone 2.7, and the address units are
+// busy for 84 % of the time.  Tried there: loads one step ahead of the products and the stores
+// (6.7 ms, more registers), nontemporal stores (5.7), half the register outputs (6.8), blocks
+// of one XCD on neighbouring tiles (5.8), 4 and 16 times the blocks (5.8, 5.9).
 template <typename T, bool SCALED, int RY, int YM>
 __global__ __launch_bounds__(kBlock) void k_fold_vec(const to_fold_desc* __restrict__ descs, int ndesc, const int32_t* __restrict__ bmap) {
     constexpr int R = 1 << RY;
@@ -367,6 +373,22 @@ __global__ __launch_bounds__(kBlock) void k_fold_vec(const to_fold_desc* __restr
                 V4 xv[KU];
 #pragma unroll
                 for (int j = 0; j < KU; ++j) xv[j] = *reinterpret_cast<const TO_GLOBAL V4*>(Xp + ox[j]);
+                if constexpr (YM == 5) {  // four register outputs' entries lie together
+                    V4 yv[KU][R / 4];
+#pragma unroll
+                    for (int j = 0; j < KU; ++j)
+#pragma unroll
+                        for (int r = 0; r < R / 4; ++r)
+                            yv[j][r] = *reinterpret_cast<const TO_GLOBAL V4*>(Yp + (oy[j] | ry[4 * r]));
+#pragma unroll
+                    for (int j = 0; j < KU; ++j)
+#pragma unroll
+                        for (int r = 0; r < R; ++r)
+#pragma unroll
+                            for (int v = 0; v < 4; ++v)
+                                acc[r][v] = fma((double)xv[j][v], (double)yv[j][r / 4][r & 3], acc[r][v]);
+                    return;
+                }
 #pragma unroll
                 for (int j = 0; j < KU; ++j) {
 #pragma unroll
@@ -380,10 +402,15 @@ __global__ __launch_bounds__(kBlock) void k_fold_vec(const to_fold_desc* __restr
                             const V4 y = *reinterpret_cast<const TO_GLOBAL V4*>(p);
 #pragma unroll
                             for (int v = 0; v < 4; ++v) acc[r][v] = fma((double)xv[j][v], (double)y[v], acc[r][v]);
-                        } else {
+                        } else if constexpr (YM == 2) {
                             const T y[4] = {p[0], p[y1], p[y2], p[y1 | y2]};
 #pragma unroll
                             for (int v = 0; v < 4; ++v) acc[r][v] = fma((double)xv[j][v], (double)y[v], acc[r][v]);
+                        } else {  // Y has one of the outputs' two lowest variables
+                            const double a = (double)p[0], b = (double)p[YM == 3 ? y1 : y2];
+#pragma unroll
+                            for (int v = 0; v < 4; ++v)
+                                acc[r][v] = fma((double)xv[j][v], (YM == 3 ? v & 1 : v >> 1) ? b : a, acc[r][v]);
                         }
                     }
                 }

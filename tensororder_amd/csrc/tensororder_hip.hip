@@ -183,7 +183,8 @@ __device__ __forceinline__ void note_exp(uint64_t recs, int64_t b, int64_t e) {
 
 template <typename T>
 __device__ __forceinline__ T absval(T v) {
-    return v < T(0) ? -v : v;
+    // (a source modifier of the next instruction; a comparison with 0 would be three more)
+    return sizeof(T) == 4 ? (T)__builtin_fabsf((float)v) : (T)__builtin_fabs((double)v);
 }
 
 // The general streaming joins accumulate float operands in double: the products of two
@@ -2551,11 +2552,14 @@ int launch_one(const to_launch& L, hipStream_t st) {
     case TO_FOLD_VEC | YM << 4 | RY:                                                                 \
         hipLaunchKernelGGL((k_fold_vec<T, SCALED, RY, YM>), grid, block, 0, st, fd, L.count, bmap); \
         break;
-#define TO_FOLD_CASES(RY) TO_FOLD_CASE(RY, 0) TO_FOLD_CASE(RY, 1) TO_FOLD_CASE(RY, 2)
+#define TO_FOLD_CASES(RY)                                                                          \
+    TO_FOLD_CASE(RY, 0) TO_FOLD_CASE(RY, 1) TO_FOLD_CASE(RY, 2) TO_FOLD_CASE(RY, 3) TO_FOLD_CASE(RY, 4)
                 TO_FOLD_CASES(0)
                 TO_FOLD_CASES(1)
                 TO_FOLD_CASES(2)
                 TO_FOLD_CASES(3)
+                TO_FOLD_CASE(2, 5)
+                TO_FOLD_CASE(3, 5)
 #undef TO_FOLD_CASES
 #undef TO_FOLD_CASE
                 default:

@@ -78,14 +78,16 @@ class FoldEmulator(emulator.Emulator):
             if vec:
                 assert d.nreg == (L.variant & 15) and d.lo == 10 and d.lk == 0 and d.lsplit == 0
                 assert list(d.bx[:2]) == [1, 2] and list(d.bc[:2]) == [1, 2]
-                ym = {(0, 0): 0, (1, 2): 1}.get(tuple(d.by[:2]), 2)
+                ym = {(0, 0): 0, (1, 2): 1}.get(tuple(d.by[:2]), 2 if d.by[0] and d.by[1] else 3 if d.by[0] else 4)
+                at = 10 + d.ntile + d.nloop
+                ym = 5 if not ym and d.nreg >= 2 and list(d.by[at:at + 2]) == [1, 2] else ym
                 assert ym == (L.variant >> 4) & 15
                 # 4-element alignment of everything the 16-byte form loads or stores at once
-                for ptr, stride, arr, used in ((d.x, d.xb, d.bx, True), (d.c, d.cb, d.bc, True),
-                                               (d.y, d.yb, d.by, ym == 1)):
+                for ptr, stride, arr, used, low in ((d.x, d.xb, d.bx, True, 0), (d.c, d.cb, d.bc, True, 0),
+                                                    (d.y, d.yb, d.by, ym in (1, 5), at if ym == 5 else 0)):
                     if used:
                         assert ptr % (4 * self.dt().itemsize) == 0 and stride % 4 == 0
-                        assert all(int(e) % 4 == 0 for e in list(arr)[2:])
+                        assert all(int(e) % 4 == 0 for i, e in enumerate(arr) if not low <= i < low + 2)
                 thr, tile0 = (0, 10), 10
             elif L.variant & _lib.TO_FOLD_REG:
                 na, nb = L.variant >> 4 & 15, L.variant & 15
@@ -437,13 +439,16 @@ def test_folded_tensors_hold_each_variable_once():
 # (X-only, Y-only, kept shared, summed shared, X-only summed, slices, X sliced, Y sliced,
 #  shuffled): the general form below and above 256 outputs, with shared thread bits and with
 #  blocks sharing a sum; the 16-byte form with 0..3 (and more) register bits, Y holding none,
-#  both or one of the lowest two variables; odd slice counts
+#  both or one of the lowest two variables; the streamed operand the smaller one ("yy", "yh",
+#  "hy": the outputs' lowest variables by kind); odd slice counts
 JOINS = [(0, 0, 0, 0, 0, 1, 1, 1, 0), (2, 1, 1, 1, 0, 3, 1, 1, 1), (3, 2, 2, 2, 1, 5, 1, 0, 1), (0, 0, 3, 9, 0, 2, 1, 1, 0),
          (0, 0, 0, 16, 0, 1, 1, 1, 0), (1, 0, 1, 14, 0, 3, 1, 1, 1), (4, 5, 1, 6, 0, 1, 1, 1, 1), (10, 0, 0, 0, 0, 1, 1, 1, 0),
          (11, 0, 2, 1, 0, 2, 1, 0, 0), (9, 1, 4, 2, 0, 3, 1, 1, 0), (10, 2, 2, 3, 0, 1, 1, 1, 0), (8, 3, 3, 1, 0, 7, 1, 0, 0),
          (4, 6, 5, 2, 0, 65, 1, 1, 1), (4, 2, 9, 1, 0, 33, 1, 0, 1), (1, 1, 13, 1, 1, 9, 1, 1, 1),
          (2, 0, 13, 0, 0, 9, 1, 1, 1), (0, 0, 0, 18, 0, 3, 1, 1, 0), (1, 0, 2, 11, 0, 2, 1, 0, 0),
-         (9, 5, 3, 2, 0, 2, 1, 1, 0), (0, 0, 13, 1, 0, 3, 1, 1, 0), (1, 0, 12, 2, 0, 2, 1, 1, 0), (12, 1, 1, 4, 0, 3, 1, 1, 0)]
+         (9, 5, 3, 2, 0, 2, 1, 1, 0), (0, 0, 13, 1, 0, 3, 1, 1, 0), (1, 0, 12, 2, 0, 2, 1, 1, 0), (12, 1, 1, 4, 0, 3, 1, 1, 0),
+         (6, 5, 4, 3, 0, 5, 1, 1, "yy"), (5, 4, 6, 0, 1, 3, 1, 0, "yh"), (6, 5, 4, 3, 0, 5, 1, 1, "yyxx"), (2, 8, 3, 1, 0, 3, 0, 1, "yyxx"), (3, 2, 8, 1, 0, 65, 1, 1, "hy"),
+         (4, 3, 6, 2, 0, 3, 0, 1, "hx"), (9, 0, 3, 1, 1, 2, 1, 1, "xh"), (2, 2, 9, 2, 0, 9, 1, 1, "hh"), (4, 3, 7, 2, 0, 3, 1, 0, "hhr")]
 
 
 def _join(case, et, alloc, write, rng):
@@ -461,6 +466,12 @@ def _join(case, et, alloc, write, rng):
     if shuffled:
         for v in (xv, yv, out):
             rng.shuffle(v)
+    if isinstance(shuffled, str):  # the lowest two variables by kind, as in the plan's one order
+        low = [u + str(shuffled[:i].count(u)) for i, u in enumerate(shuffled.rstrip("r"))]
+        one = low + [v for v in out if v not in low] + sorted(set(xv + yv) - set(out))
+        xv, yv, out = ([v for v in one if v in vs] for vs in (xv, yv, out))
+        if shuffled.endswith("r"):  # (a leaf's axes lie as they are)
+            yv.reverse()
     nodes = []
     for i, (vs, batched) in enumerate(((xv, xw), (yv, yw), (out, xw or yw))):
         n = fold.FNode(i)
@@ -550,7 +561,7 @@ def test_every_form_emulated(et):
         got = heap.view(C.ptr, emu.dt, items << C.rank).reshape(items, -1)
         _check(case, et, got, [heap.read_struct(_lib.ScaleRec, recs[2] + 16 * b) for b in range(items)], want)
     assert {f & 15 for f in forms if f != "split" and f & _lib.TO_FOLD_VEC} == {0, 1, 2, 3}
-    assert {f >> 4 & 15 for f in forms if f != "split" and f & _lib.TO_FOLD_VEC} >= {0, 1}
+    assert {f >> 4 & 15 for f in forms if f != "split" and f & _lib.TO_FOLD_VEC} == {0, 1, 2, 3, 4, 5}
     assert "split" in forms and _lib.TO_FOLD_ANY in forms and _lib.TO_FOLD_DOT in forms
     assert {f for f in forms if f != "split" and f & _lib.TO_FOLD_REG} == {
         _lib.TO_FOLD_REG | a << 4 | b for a, b in fold.REG_TILES}
