@@ -249,9 +249,10 @@ typedef struct to_gemm_desc {
  *   TO_FOLD_VEC: [0, 2) the o bits of 4 consecutive outputs, also the lowest 2 bits of X;
  *     [2, 10) o bits of the thread index; [10, 10 + ntile) tile; nloop k bits; nreg (<= 3) o
  *     bits that only Y has, all 2^nreg of whose outputs a thread holds at once.
- *     y mode: 0 Y has neither of the bits [0, 2); 1 both, as its lowest two; 2 both in other
- *     places; 3 the first alone; 4 the second alone; 5 neither, and the first two of the
- *     nreg bits (nreg >= 2) are its lowest.  C, X (and Y in modes 1 and 5) and their batch strides aligned to 4 elements. */
+ *     y mode: 0 Y has neither of the bits [0, 2); 1 both, as its lowest two; 2 any of them, in
+ *     any place; 3 the first alone; 4 the second alone; 5 neither, and the first two of the
+ *     nreg bits (nreg >= 2) are its lowest.  C, X (and Y in modes 1 and 5) and their batch
+ *     strides aligned to 4 elements. */
 #define TO_FOLD_ANY 0
 #define TO_FOLD_VEC 0x100
 #define TO_FOLD_REG 0x200

@@ -76,6 +76,10 @@ TREE_LONE_BITS = 12
 # joins of a program merged into one product: at most 4 operands, 64 outputs and 2^MERGE_LOOP
 # products per output (each merge saves a level)
 MERGE_LOOP = 2
+# small operands of a product are stored by the join that makes them as the product reads them,
+# whatever that does to its own stores: the launch that permuted them before the product took
+# 17-19 us on a few tensors of 2^12 entries
+WANT_ENTRIES = 1 << 20
 # level launches are kept whatever they cost in memory up to this arena size
 LEVEL_FREE_BYTES = 256 << 20
 
@@ -105,12 +109,13 @@ class FNode:
     ``off`` maps each to the element offset it adds (several bits at once for a leaf that
     holds it on several axes); 2^rank entries are stored."""
 
-    __slots__ = ("idx", "is_leaf", "tensor", "rank", "order", "order0", "off", "batched", "left", "right", "parent", "ksum",
+    __slots__ = ("idx", "is_leaf", "tensor", "rank", "order", "order0", "want", "off", "batched", "left", "right", "parent", "ksum",
                  "geom", "buf", "ptr", "bstride", "rec", "rec_stride")
 
     def __init__(self, idx):
         self.idx = idx
         self.parent = -1
+        self.want = None  # the order that the product reading it takes, where it is stored so
         self.buf = None
         self.rec = None
         self.rec_stride = 0
@@ -316,7 +321,7 @@ def _canonical(node, want):
     return node.rank == len(want) and all(node.off.get(v) == 1 << i for i, v in enumerate(want))
 
 
-def _vec_form(xoff, yoff, xrank, yrank, out, off, ksum, nb):
+def _vec_form(xoff, yoff, xrank, yrank, out, off, ksum, nb, launch_bound):
     """The 16-byte form of a join that streams the operand of offsets ``xoff``, or None."""
     yonly = [v for v in out if v not in xoff]
     reg = yonly[:MAX_REG_BITS]
@@ -335,6 +340,8 @@ def _vec_form(xoff, yoff, xrank, yrank, out, off, ksum, nb):
             ym = 5
     else:
         ym = 1 if (y0, y1) == (1, 2) and yrank >= 2 else 2
+    if launch_bound:  # fewer launches a step: the forms that the others are cases of
+        ym = {3: 2, 4: 2, 5: 0}.get(ym, ym)
     ntile = len(body) - 10
     return dict(kind="fold", variant=_lib.TO_FOLD_VEC | ym << 4 | len(reg), bits=body + ks + reg, fy=len(yonly),
                 roles=(10, 0, ntile, s, 0, len(reg)), nblocks=int(min(nb << ntile, MAX_VEC_BLOCKS)), lsplit=0,
@@ -349,7 +356,7 @@ def choose(n, nodes, W, esize, launch_bound=False):
     A = nodes[n.left]
     B = nodes[n.right] if n.right >= 0 else None
     nb = W if n.batched else 1
-    _reordered(n, list(n.order0))
+    _reordered(n, list(n.want or n.order0))
     if B is None:
         X, Y = A, None
     else:
@@ -378,6 +385,11 @@ def choose(n, nodes, W, esize, launch_bound=False):
                 del v["lsplit"], v["nsplit"], v["nout"], v["fin_blocks"]
                 v["nblocks"] = int(min((nb << h) << (len(xo) + len(yo) - 12), schedule.MAX_GEMM_BLOCKS))
             want_x, want_y = ks + xo + kept, ks + yo + kept
+            for t, want in ((X, want_x), (Y, want_y)):
+                if not t.is_leaf and not _canonical(t, want) and t.geom["var"]["kind"] == "fold" and \
+                        t.rank <= TREE_RANK and (W if t.batched else 1) << t.rank <= WANT_ENTRIES:
+                    t.want = want
+                    choose(t, nodes, W, esize, launch_bound)
             v.update(perm_x=not _canonical(X, want_x), perm_y=not _canonical(Y, want_y), hlog=h, want_x=want_x,
                      want_y=want_y)
             g.update(var=v, X=X.idx, Y=Y.idx)
@@ -390,7 +402,7 @@ def choose(n, nodes, W, esize, launch_bound=False):
     # own: the larger one, else the other (2^16 by 2^16 over 2^3 to 2^20, 4096 slices: 6.4 ms as
     # a register tile with 4-byte stores, 5.7 here)
     for x, y in ((X, Y), (Y, X)) if Y is not None else ():
-        v = _vec_form(x.off, y.off, x.rank, y.rank, out, n.off, n.ksum, nb)
+        v = _vec_form(x.off, y.off, x.rank, y.rank, out, n.off, n.ksum, nb, launch_bound)
         if v is not None:
             n.geom = dict(fx=nc - v["fy"], fy=v["fy"], s=s, X=x.idx, Y=y.idx, var=v)
             return
@@ -440,6 +452,8 @@ def choose(n, nodes, W, esize, launch_bound=False):
 
 
 def choose_all(nodes, W, esize, launch_bound=False):
+    for n in nodes:
+        n.want = None
     for n in nodes:
         if not n.is_leaf:
             choose(n, nodes, W, esize, launch_bound)
@@ -761,10 +775,11 @@ def peak_bytes(nodes, W, esize):
     return choose_order(nodes, W, esize, tree_programs(nodes, W, esize, esize == 4))[1]
 
 
-def join_records(n, nodes, W, esize, scaled, abase, scratch, recp, one):
+def join_records(n, nodes, W, esize, scaled, abase, scratch, recp, one, launch_bound=False):
     """Descriptor records of one join in execution order, as ``schedule.join_records``:
     [(kind, op, variant, lds, descriptor, blocks)]; ``one``: (address, record address) of a
-    stored 1.0, the second operand of a lone leaf's sum."""
+    stored 1.0, the second operand of a lone leaf's sum; ``launch_bound`` (the many-instance
+    batch): permutes in one form, so that those of a step share a launch."""
     g, v = n.geom, n.geom["var"]
     nb = W if n.batched else 1
     X = nodes[g["X"]]
@@ -780,7 +795,8 @@ def join_records(n, nodes, W, esize, scaled, abase, scratch, recp, one):
                 for i, var in enumerate(want):
                     out_pos[op.off[var].bit_length() - 1] = i
                 pd, grid, lds, pvar = schedule.perm_desc(op.ptr, dst, op.rank, out_pos,
-                                                         W if (n.batched and op.batched) else 1, 1 << op.rank, esize)
+                                                         W if (n.batched and op.batched) else 1, 1 << op.rank, esize,
+                                                         not launch_bound)
                 out.append(("permute", _lib.TO_OP_PERMUTE, pvar, lds, pd, grid))
                 ops.append((dst, stride))
             else:
@@ -1236,7 +1252,7 @@ def compile_batch(per, entry_type, device_alloc, arena, host_alloc):
             for j in grp[1]:
                 scratch = {key: (base + blk[0], blk[1]) for key, blk in inst["scratch"].get(j, {}).items()}
                 for kind, op, variant, lds, st, nblk in join_records(nodes[j], nodes, 1, esize, scaled, abase, scratch,
-                                                                     recp, one_at):
+                                                                     recp, one_at, True):
                     work = join_traffic(nodes[j], nodes, 1, esize) if kind in ("fold", "gemm") else (0, 0)
                     if kind == "permute":
                         work = (2 * esize << int(st.rank), 0)
