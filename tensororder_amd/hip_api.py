@@ -168,12 +168,18 @@ class Executable:
         return self.result()
 
     def close(self):
-        if self._graphs:
+        if self._graphs or self._queued:
             self.api.synchronize()  # the sum's word is written by a kernel that has yet to end
+            self._queued = 0
         for g in self._graphs:
             self.api._lib.to_graph_destroy(g)
         self._graphs = []
         self._runs = [(None, launches) for _, launches in self._runs]
+
+    def __del__(self):
+        # runs that nobody waited for write to this object's host memory until they end
+        if getattr(self, "_queued", 0):
+            self.api.synchronize()
 
 
 class BatchExecutable:
@@ -189,6 +195,7 @@ class BatchExecutable:
         self.arena = arena
         self.count = sum(p.count for p in self.progs)
         self._graphs = []
+        self._queued = False
         if api._use_graph:
             for prog in self.progs:
                 arr = _lib.launch_array(prog.launches)
@@ -210,6 +217,7 @@ class BatchExecutable:
         return [w for prog in self.progs for w in prog.work]
 
     def enqueue(self):
+        self._queued = True
         if self._graphs:
             for graph in self._graphs:
                 _lib.check(self.api._lib.to_graph_launch(graph, ctypes.c_void_p(self.api._stream.cuda_stream)),
@@ -221,6 +229,7 @@ class BatchExecutable:
     def results(self):
         api = self.api
         api.synchronize()
+        self._queued = False
         size = ctypes.sizeof(_lib.Accum)
         res, ends = [], []
         # (no copies where the accumulators lie in host memory)
@@ -239,9 +248,17 @@ class BatchExecutable:
         return self.results()
 
     def close(self):
+        if self._queued:
+            self.api.synchronize()
+            self._queued = False
         for graph in self._graphs:
             self.api._lib.to_graph_destroy(graph)
         self._graphs = []
+
+    def __del__(self):
+        # (see Executable)
+        if getattr(self, "_queued", False):
+            self.api.synchronize()
 
 
 def copy_weights(tensor):

@@ -921,3 +921,24 @@ def test_fused_dot_products_in_plans(et, tol, monkeypatch):
                 assert got == pytest.approx(want, rel=tol)
                 fused |= {(slices, f[1]) for f in emu.forms if isinstance(f, tuple)}
     assert {f[0] for f in fused} >= {0, 1} and {f[1] & 0xff for f in fused} == {0x11}
+
+
+@pytest.mark.parametrize("cls", [hip_api.Executable, hip_api.BatchExecutable])
+def test_dropped_runs_are_waited_for(cls):
+    # the device writes an executable's host memory until its runs end: one that goes away, or
+    # is closed, with a run nobody waited for waits first
+    class Api:
+        waits = 0
+
+        def synchronize(self):
+            Api.waits += 1
+
+    for close in (False, True):
+        exe = object.__new__(cls)
+        exe.api, exe._graphs, exe._runs, exe._queued = Api(), [], [], 1
+        before = Api.waits
+        if close:
+            exe.close()
+            assert Api.waits == before + 1
+        del exe
+        assert Api.waits == before + 1
