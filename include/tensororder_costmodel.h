@@ -39,6 +39,12 @@ int to_mlp_backward(const float* params, const float* x, const float* h1, const 
                     const float* y, const float* target, int64_t n, float* dy, float* dh2,
                     float* dh1, float* grad, float* loss, void* stream);
 
+/* to_mlp_forward and to_mlp_backward in one call: the gradient and the loss with the activations
+ * written on the way. */
+int to_mlp_gradient(const float* params, const float* x, const float* target, int64_t n, float* h1,
+                    float* h2, float* y, float* dy, float* dh2, float* dh1, float* grad, float* loss,
+                    void* stream);
+
 /* One Adam step (bias-corrected, step >= 1) on count parameters. */
 int to_mlp_adam(float* params, const float* grad, float* m, float* v, int64_t count, float lr,
                 float beta1, float beta2, float eps, int64_t step, void* stream);

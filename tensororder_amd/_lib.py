@@ -178,7 +178,7 @@ class Launch(ctypes.Structure):
 EXPORTED = [
     "to_version", "to_struct_sizes", "to_last_error", "to_device_count", "to_set_device",
     "to_run", "to_run_timed", "to_graph_create", "to_graph_launch", "to_graph_destroy", "to_permute",
-    "to_wall_clock_khz", "to_synchronize", "to_mlp_forward", "to_mlp_backward", "to_mlp_adam",
+    "to_wall_clock_khz", "to_synchronize", "to_mlp_forward", "to_mlp_backward", "to_mlp_gradient", "to_mlp_adam",
     "to_tensordot_workspace", "to_tensordot", "to_tensordot_noalloc", "to_fold_desc_size", "to_tree_desc_size",
     "to_pair_desc_size",
     "to_upload", "to_signal", "to_wait",
@@ -226,6 +226,7 @@ def load(path=LIB_PATH):
     lib.to_tensordot_noalloc.argtypes = [vp, vp, vp, i32, i32, vp, vp, i32, i32, vp, vp, vp, vp]
     lib.to_mlp_forward.argtypes = [vp, vp, i64, vp, vp, vp, vp]
     lib.to_mlp_backward.argtypes = [vp, vp, vp, vp, vp, vp, i64, vp, vp, vp, vp, vp, vp]
+    lib.to_mlp_gradient.argtypes = [vp, vp, vp, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp]
     lib.to_mlp_adam.argtypes = [vp, vp, vp, vp, i64, ctypes.c_float, ctypes.c_float, ctypes.c_float,
                                 ctypes.c_float, i64, vp]
     if lib.to_version() != ABI_VERSION:

@@ -159,13 +159,11 @@ class CostModel:
     def gradient(self, xdev, tdev):
         """(loss, gradient) on device data (normalised)."""
         n = xdev.shape[0]
-        h1, h2, y = self.forward_raw(xdev)
-        dh1, dh2, dy = self._buffers(n)
+        (h1, h2, y), (dh1, dh2, dy) = self._buffers(n), self._buffers(n)
         loss = self.loss
-        rc = self.lib.to_mlp_backward(self._ptr(self.params), self._ptr(xdev), self._ptr(h1), self._ptr(h2),
-                                      self._ptr(y), self._ptr(tdev), n, self._ptr(dy), self._ptr(dh2),
-                                      self._ptr(dh1), self._ptr(self.grad), self._ptr(loss), self._stream())
-        _lib.check(rc, "to_mlp_backward")
+        rc = self.lib.to_mlp_gradient(*map(self._ptr, (self.params, xdev, tdev)), n,
+                                      *map(self._ptr, (h1, h2, y, dy, dh2, dh1, self.grad, loss)), self._stream())
+        _lib.check(rc, "to_mlp_gradient")
         self.api.finish()
         return float(loss[0]), self.grad
 

@@ -1,7 +1,7 @@
 // Training and inference kernels of the plan-cost MLP (include/tensororder_costmodel.h).
 //
 // The network is tiny (5378 parameters) and a training step has a few thousand rows, so a step
-// is four launches: the forward pass and the activation gradients with a wave per few rows and
+// is three launches: the forward pass with the activation gradients, a wave per few rows and
 // the weights in LDS, all weight gradients (a fixed-order reduction over the rows), Adam.
 #include <hip/hip_runtime.h>
 
@@ -25,7 +25,9 @@ constexpr int OFF_W3 = OFF_B2 + TO_MLP_H2;
 constexpr int OFF_B3 = OFF_W3 + TO_MLP_OUT * TO_MLP_H2;
 static_assert(OFF_B3 + TO_MLP_OUT == TO_MLP_NPARAMS, "parameter layout");
 
-constexpr int kRows = 4;                       // rows per wave
+// rows per wave: 2048 rows are a block for every CU, and a training step takes 44.9 us (46.7 with 4
+// rows, half the CUs idle; the same from 4096 rows on)
+constexpr int kRows = 2;
 constexpr int kRowsPerBlock = kRows * (kBlock / 64);
 
 // h[l] of every lane's value, as a scalar
@@ -42,9 +44,14 @@ __device__ __forceinline__ float wave_sum(float v) {
 // previous layer's units are read back with v_readlane, the weights come transposed from LDS
 // (pitch 65: no bank conflicts either way).  Bound by latency at the batch sizes of training:
 // one launch of 6 us where one thread per activation took three of 38 us together at 2048 rows.
+// TRAIN: the gradients of the activations too (as k_backward_rows), from the values at hand and
+// the same copy of W2, read along its rows: 14 us where the two launches took 18 (2048 rows).
+template <bool TRAIN>
 __global__ __launch_bounds__(kBlock) void k_forward(const float* __restrict__ params, const float* __restrict__ x,
                                                     int64_t n, float* __restrict__ h1, float* __restrict__ h2,
-                                                    float* __restrict__ y) {
+                                                    float* __restrict__ y, const float* __restrict__ t,
+                                                    float* __restrict__ dy, float* __restrict__ dh2,
+                                                    float* __restrict__ dh1) {
     __shared__ float w1[TO_MLP_IN * 65], w2[TO_MLP_H1 * 65];
     for (int i = threadIdx.x; i < TO_MLP_H1 * TO_MLP_IN; i += kBlock)
         w1[(i % TO_MLP_IN) * 65 + i / TO_MLP_IN] = params[OFF_W1 + i];
@@ -56,9 +63,14 @@ __global__ __launch_bounds__(kBlock) void k_forward(const float* __restrict__ pa
     const float b30 = params[OFF_B3], b31 = params[OFF_B3 + 1];
     __syncthreads();
     const int64_t r0 = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6) * kRows;
-    float in[kRows], a[kRows], b[kRows];
+    float in[kRows], a[kRows], b[kRows], t0[kRows], t1[kRows];
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
+        if constexpr (TRAIN) {
+            const int64_t i = r0 + r < n ? r0 + r : n - 1;
+            t0[r] = t[i * TO_MLP_OUT];
+            t1[r] = t[i * TO_MLP_OUT + 1];
+        }
         in[r] = lane < TO_MLP_IN && r0 + r < n ? x[(r0 + r) * TO_MLP_IN + lane] : 0.0f;
         a[r] = b1;
         b[r] = b2;
@@ -80,6 +92,8 @@ __global__ __launch_bounds__(kBlock) void k_forward(const float* __restrict__ pa
 #pragma unroll
         for (int r = 0; r < kRows; ++r) b[r] += lane_value(a[r], k) * w;
     }
+    const float scale = 2.0f / (float)(n * TO_MLP_OUT);
+    float g[kRows], d[kRows];
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
         b[r] = fmaxf(b[r], 0.0f);
@@ -88,6 +102,26 @@ __global__ __launch_bounds__(kBlock) void k_forward(const float* __restrict__ pa
             h2[(r0 + r) * TO_MLP_H2 + lane] = b[r];
             if (lane < TO_MLP_OUT) y[(r0 + r) * TO_MLP_OUT + lane] = lane == 0 ? s0 : s1;
         }
+        if constexpr (TRAIN) {
+            const float d0 = scale * (s0 - t0[r]), d1 = scale * (s1 - t1[r]);
+            g[r] = b[r] > 0.0f ? d0 * w30 + d1 * w31 : 0.0f;
+            d[r] = 0.0f;
+            if (r0 + r < n) {
+                dh2[(r0 + r) * TO_MLP_H2 + lane] = g[r];
+                if (lane < TO_MLP_OUT) dy[(r0 + r) * TO_MLP_OUT + lane] = lane == 0 ? d0 : d1;
+            }
+        }
+    }
+    if constexpr (TRAIN) {
+#pragma unroll 16
+        for (int o = 0; o < TO_MLP_H2; ++o) {
+            const float w = w2[lane * 65 + o];
+#pragma unroll
+            for (int r = 0; r < kRows; ++r) d[r] += lane_value(g[r], o) * w;
+        }
+#pragma unroll
+        for (int r = 0; r < kRows; ++r)
+            if (r0 + r < n) dh1[(r0 + r) * TO_MLP_H1 + lane] = a[r] > 0.0f ? d[r] : 0.0f;
     }
 }
 
@@ -205,7 +239,11 @@ __global__ __launch_bounds__(kGradThreads) void k_weight_grads(
                 for (int j = 0; j < 8; ++j) gv[u][j] = j < nj ? g[r * dout + j0 + j] : 0.0f;
             }
             gc[u] = k0 == 0 && c < nj ? g[r * dout + j0 + c] : 0.0f;
-            if (!row) v[u] = gc[u] = 0.0f;
+            if (!row) {  // (row 0 in its place may hold what times 0 is no 0)
+                v[u] = gc[u] = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) gv[u][j] = 0.0f;
+            }
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -257,6 +295,13 @@ int status(const char*) {
     return e == hipSuccess ? TO_OK : TO_ERR_HIP;
 }
 
+void launch_weight_grads(const float* x, const float* h1, const float* h2, const float* y, const float* target, int64_t n,
+                         const float* dy, const float* dh2, const float* dh1, float* grad, float* loss, hipStream_t st) {
+    hipLaunchKernelGGL(k_weight_grads, dim3(kTiles2 + kTiles1 + kTiles3 + 1), dim3(kGradThreads), 0, st, x, h1, h2, dy,
+                       dh2, dh1, y, target, n, grad, loss,
+                       ((reinterpret_cast<uintptr_t>(dh2) | reinterpret_cast<uintptr_t>(dh1)) & 15) == 0);
+}
+
 }  // namespace
 
 extern "C" {
@@ -265,8 +310,8 @@ int to_mlp_forward(const float* params, const float* x, int64_t n, float* h1, fl
     if (!params || !x || !h1 || !h2 || !y || n <= 0) return TO_ERR_INVALID;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     if (n > (int64_t)INT32_MAX * kRowsPerBlock) return TO_ERR_INVALID;
-    hipLaunchKernelGGL(k_forward, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st, params,
-                       x, n, h1, h2, y);
+    hipLaunchKernelGGL(k_forward<false>, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st,
+                       params, x, n, h1, h2, y, nullptr, nullptr, nullptr, nullptr);
     return status("to_mlp_forward");
 }
 
@@ -279,10 +324,19 @@ int to_mlp_backward(const float* params, const float* x, const float* h1, const 
     if (n > (int64_t)INT32_MAX * kRowsPerBlock) return TO_ERR_INVALID;
     hipLaunchKernelGGL(k_backward_rows, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st,
                        params, h1, h2, y, target, n, dy, dh2, dh1);
-    hipLaunchKernelGGL(k_weight_grads, dim3(kTiles2 + kTiles1 + kTiles3 + 1), dim3(kGradThreads), 0, st, x, h1, h2, dy,
-                       dh2, dh1, y, target, n, grad, loss,
-                       ((reinterpret_cast<uintptr_t>(dh2) | reinterpret_cast<uintptr_t>(dh1)) & 15) == 0);
+    launch_weight_grads(x, h1, h2, y, target, n, dy, dh2, dh1, grad, loss, st);
     return status("to_mlp_backward");
+}
+
+int to_mlp_gradient(const float* params, const float* x, const float* target, int64_t n, float* h1, float* h2, float* y,
+                    float* dy, float* dh2, float* dh1, float* grad, float* loss, void* stream) {
+    if (!params || !x || !target || !h1 || !h2 || !y || !dy || !dh2 || !dh1 || !grad || n <= 0) return TO_ERR_INVALID;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (n > (int64_t)INT32_MAX * kRowsPerBlock) return TO_ERR_INVALID;
+    hipLaunchKernelGGL(k_forward<true>, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st,
+                       params, x, n, h1, h2, y, target, dy, dh2, dh1);
+    launch_weight_grads(x, h1, h2, y, target, n, dy, dh2, dh1, grad, loss, st);
+    return status("to_mlp_gradient");
 }
 
 int to_mlp_adam(float* params, const float* grad, float* m, float* v, int64_t count, float lr, float beta1,

@@ -49,3 +49,12 @@ def test_rows_and_alignment(n, shift):
     assert float(L[shift]) == pytest.approx(loss, rel=1e-5)
     scale = np.abs(grad).max()
     np.testing.assert_allclose(G[shift:].cpu().numpy(), grad, rtol=1e-3, atol=1e-5 * scale)
+    # both in one call: the same numbers
+    G1, L1 = dev(nan(_lib.MLP_NPARAMS, np.nan)), dev(nan(1, np.nan))
+    outs = [dev(nan((n, w), np.nan)) for w in (64, 64, 2, 2, 64, 64)]
+    torch.cuda.synchronize()
+    _lib.check(lib.to_mlp_gradient(ptr(P), ptr(X), ptr(T), n, *map(ptr, outs), ptr(G1), ptr(L1), None), "to_mlp_gradient")
+    torch.cuda.synchronize()
+    for got, ref in zip(outs + [G1, L1], (H1, H2, Y, DY, DH2, DH1, G, L)):
+        np.testing.assert_allclose(got[shift:].cpu().numpy(), ref[shift:].cpu().numpy(), rtol=1e-5,
+                                   atol=1e-6 * float(ref[shift:].abs().max()))
