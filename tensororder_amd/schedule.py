@@ -452,15 +452,22 @@ class LeafSpec:
             return float(self.w_neg), float(self.w_pos), np.array([0.0, self.w_neg, self.w_pos], dtype=np.float64)
         return 0.0, 1.0, np.array([0.0, 1.0])
 
-    def stored(self, scaled):
+    def stored(self, scaled, known=None):
         """(val0, val1, F, e): the values the device writes and, for the FP32-scaled executor,
         the table's encoding factor and exponent -- those ``leaf_encoding`` gives the whole
-        table, which depend only on its set of values."""
+        table, which depend only on its set of values.  ``known``: a dict of encodings by
+        these values, kept by a caller with many leaves (nearly all of a plan's hold 0 and 1)."""
         v0, v1, vals = self.values()
         if not scaled:
             return v0, v1, 1.0, 0
-        enc, F, e = leaf_encoding(np.concatenate([vals, [v0, v1]]))
-        return float(enc[-2]), float(enc[-1]), F, e
+        key = (len(vals), v0, v1)
+        out = known.get(key) if known is not None else None
+        if out is None:
+            enc, F, e = leaf_encoding(np.concatenate([vals, [v0, v1]]))
+            out = float(enc[-2]), float(enc[-1]), F, e
+            if known is not None:
+                known[key] = out
+        return out
 
     def desc(self, dst, v0, v1):
         """The ``to_leaf_build_desc`` of this leaf's table at device address ``dst``."""
@@ -902,11 +909,11 @@ def leaf_image(nodes, tables, num_groups, scaled, fdtype):
     esize = np.dtype(fdtype).itemsize
     leaf_ids = sorted({n.tensor for n in nodes if n.is_leaf})
     im.off, im.exp0, im.builds, im.coef_off = {}, {}, [], {}
-    chunks, factor_of, off = [], {}, 0
+    chunks, factor_of, off, known = [], {}, 0, {}
     for t in leaf_ids:
         tab = tables[t]
         if tab.spec is not None:  # written on the device by the leaf build launch
-            v0, v1, F, e = tab.spec.stored(scaled)
+            v0, v1, F, e = tab.spec.stored(scaled, known)
             im.builds.append((t, v0, v1))
             size = tab.size
         else:
