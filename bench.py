@@ -89,7 +89,10 @@ def kernel_symbol(L, scaled):
         if v & _lib.TO_FOLD_REG:
             return "k_fold_reg<%s, %s, %d, %d>" % (T, S, v >> 4 & 15, v & 15)
         return "k_fold_any<%s, %s, %s>" % (T, S, "true" if v == _lib.TO_FOLD_DOT else "false")
-    names = {_lib.TO_OP_FOLD_TREE: "k_fold_tree", _lib.TO_OP_FOLD_PAIR: "k_fold_pair", _lib.TO_OP_WAVE_BEGIN: "k_wave_begin", _lib.TO_OP_LEAF_GATHER: "k_leaf_gather", _lib.TO_OP_JOIN_SPLITK: "k_join_splitk",
+    if op == _lib.TO_OP_FOLD_PAIR:
+        return "k_fold_pair<%s, %s, %d, %d, %s>" % (T, S, v >> 4 & 15, v & 15, "true" if v & _lib.TO_PAIR_ONE else "false")
+    names = {_lib.TO_OP_FOLD_TREE: "k_fold_tree", _lib.TO_OP_WAVE_BEGIN: "k_wave_begin",
+             _lib.TO_OP_LEAF_GATHER: "k_leaf_gather", _lib.TO_OP_JOIN_SPLITK: "k_join_splitk",
              _lib.TO_OP_JOIN_FINISH: "k_join_finish", _lib.TO_OP_ROOT_REDUCE: "k_root_reduce",
              _lib.TO_OP_ROOT_STORE: "k_root_store"}
     if op in names:

@@ -313,7 +313,7 @@ __global__ __launch_bounds__(kBlock) void k_fold_reg(const to_fold_desc* __restr
 // of them, 16 bytes at a time; Y is read through L1, with as few loads as the places of the
 // outputs' two lowest variables and of the register variables in it allow (YM).  Bound by the
 // HBM bytes of X and C where few indices are summed: 2^19 by 2^15 over 2 to 2^20, 4096 slices
-// (26 GB), 5.3 ms, the rate of a copy.  2^16 by 2^16 over 2^3 to 2^20 (19 GB) takes 5.7 ms: its
+// (26 GB), 5.3-5.7 ms, the rate of a copy.  2^16 by 2^16 over 2^3 to 2^20 (19 GB) takes 5.7 ms: its
 // stores alone take 3.0, the loads and double products alone 2.7, and the address units are
 // busy for 84 % of the time.  Tried there: loads one step ahead of the products and the stores
 // (6.7 ms, more registers), nontemporal stores (5.7), half the register outputs (6.8), blocks
