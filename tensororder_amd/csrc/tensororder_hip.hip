@@ -3015,8 +3015,9 @@ int plan_tensordot(int rank_a, int rank_b, const int32_t* axes_a, const int32_t*
             d.nsplit = 1;
             d.nblocks = P.grid;
             // The 16-byte form: X's lowest bits free (16 bytes of consecutive f), all y of one f
-            // adjacent in the output, at least one tile of f; with double sums 64 accumulators
-            // at most.  From 2^20 index values on: a 2^23 by 2^6 float64 join over 2^3 took 43 us
+            // adjacent in the output and in one chunk (its kernel walks no chunks, and a long
+            // shared range leaves the general form several), at least one tile of f; with double
+            // sums 64 accumulators at most.  From 2^20 index values on: a 2^23 by 2^6 float64 join over 2^3 took 43 us
             // in the general form and takes 24; below, both are one launch's latency.
             const int lvf = entry_type == TO_F64 ? 1 : 2, esize = entry_type == TO_F64 ? 8 : 4;
             bool low = fx >= 8 + lvf;
@@ -3024,7 +3025,7 @@ int plan_tensordot(int rank_a, int rank_b, const int32_t* axes_a, const int32_t*
             const int64_t vlds = ((8 * K + 15) & ~15ll) + (K << fy) * esize;
             const bool run64 = ((16 / esize) << fy) * esize >= 64;
             P.vec = low && d.shy == 0 && d.shf == fy && fy <= (entry_type == TO_F64 ? 4 : 3) &&
-                    fx + fy + s >= 20 && vlds + (run64 ? 4 * 4096 : 0) <= kDotLdsLimit;
+                    yc == 1 << fy && fx + fy + s >= 20 && vlds + (run64 ? 4 * 4096 : 0) <= kDotLdsLimit;
             P.vlds = (int)(vlds + (run64 ? 4 * 4096 : 0));
             const int64_t vtiles = 1ll << (fx >= 8 + lvf ? fx - 8 - lvf : 0);
             P.vgrid = (int)(vtiles < kDotMaxBlocks ? vtiles : kDotMaxBlocks);

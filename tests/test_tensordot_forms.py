@@ -54,6 +54,17 @@ def test_streamed_forms(et, ra, rb, low, shift):
         assert int(recs[2, 1]) & 0xffffffff == int(np.float32(got.max()).view(np.uint32))
 
 
+# float joins with shared ranges so long that the general form's slab of double y entries holds
+# only a part of the 2^fy of them (2^10 by 8, 2^11 by 4, 2^12 by 2), and the next shorter ones,
+# where it holds all
+LONG = [(24, 13, 10), (25, 13, 11), (26, 13, 12), (24, 12, 9), (25, 12, 10), (26, 12, 11)]
+
+
+@pytest.mark.parametrize("ra,rb,s", LONG)
+def test_long_shared_ranges(ra, rb, s):
+    test_streamed_forms("f32s", ra, rb, list(range(2, 2 + s)), 0)
+
+
 @pytest.mark.parametrize("words", [0, 1, 767, 768, 769, 5000])
 def test_upload(words):
     import torch
