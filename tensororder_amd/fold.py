@@ -133,8 +133,12 @@ class _T:
 
 
 def has_copies(tables):
-    """Whether a plan's leaves include COPY tensors (the plan can be folded)."""
-    return any(t.copy is not None for t in tables.values())
+    """Whether a plan can be folded: its leaves include COPY tensors, each sliced on all of its
+    edges by one group, or on none.  A COPY tensor sliced on a part of them ties what is left
+    to the slice's value (and one sliced by two groups is 0 where these differ), which is no
+    vector of ones and no identity of indices."""
+    copies = [t for t in tables.values() if t.copy is not None]
+    return bool(copies) and not any(t.rank if sum(map(bool, t.coef)) == 1 else t.batched for t in copies)
 
 
 def _join_cost(left, right, union, out, batched, esize):
