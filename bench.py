@@ -78,7 +78,7 @@ def kernel_symbol(L, scaled):
             return "k_join_stream_vec<%s, %s, %d>" % (T, S, v & ~_lib.TO_STREAM_VEC)
         return "k_join_stream<%s, %s, %d>" % (T, S, v)
     if op == _lib.TO_OP_JOIN_FINISH:
-        return "%s<%s, %s>" % ("k_join_finish_wide" if v == 1 else "k_join_finish", T, S)
+        return "k_join_finish%s%s<%s, %s>" % ("_wide" if v & 1 else "", "_norm" if v & _lib.TO_FINISH_NORM else "", T, S)
     if op == _lib.TO_OP_PERMUTE:
         if v in (1, 3):  # chunk tiles of 13 / 14 bits (float), 12 / 13 (double)
             return "k_permute_vec_desc<%s, %d>" % (T, (13 if scaled else 12) + (v == 3))

@@ -63,7 +63,10 @@ extern "C" {
                                 nblocks / kvar unread), no LDS */
 #define TO_OP_JOIN_SPLITK 3  /* descs: to_join_desc[count]; partial sums (double) to d.partial */
 #define TO_OP_JOIN_FINISH 4  /* descs: to_join_desc[count]; sums d.partial into C; variant 1:
-                                one block per output (for nsplit >= 32) */
+                                one block per output (for nsplit >= 32); | TO_FINISH_NORM
+                                (TO_F32S, fx == fy == 0): the result is stored as its mantissa,
+                                its exponent added to the record's */
+#define TO_FINISH_NORM 0x100
 #define TO_OP_SCALE_CLEAR 5  /* aux0: to_scale_rec*, iaux0: record count */
 #define TO_OP_ROOT_REDUCE 6  /* aux0: root values, aux1: to_scale_rec* (F32S) or 0,
                                 aux2: to_accum*, aux3: wave params (int64[2]); variant 1: the
@@ -280,7 +283,8 @@ typedef struct to_fold_desc {
  * elements.  With lsplit > 0 the double partial sums go to
  * partial[batch << lsplit | sp] for a TO_OP_JOIN_FINISH launch, and rs[side], where not 0, gets
  * the exponent of its side (TO_F32S): the records that launch reads in place of the stored
- * results'. */
+ * results'.  The results' maxima are not known: the sum is stored as its mantissa, its exponent
+ * added to the record's (with lsplit > 0 by TO_FINISH_NORM). */
 typedef struct to_pair_desc {
     uint64_t x[2], y[2], c;
     int64_t xb[2], yb[2], cb;  /* batch strides in elements (0 = broadcast) */
@@ -297,8 +301,9 @@ typedef struct to_pair_desc {
 
 /* A program of small folded joins that one block runs start to end for one batch item: a
  * connected part of the tree whose intermediate tensors fit LDS.  A join of a program is a
- * product of up to 4 tensors, summed over the k bits.  Each wave of the block walks its own
- * stream of ntask words, tasks[wave * ntask + i]: bits 0-15 the join, bits 16-22 its first
+ * product of up to 4 tensors, summed over the k bits; one of 3 or 4 is stored scaled by the power
+ * of two that brings its largest entry to [0.5, 1), which its record's exponent carries
+ * (TO_F32S).  Each wave of the block walks its own stream of ntask words, tasks[wave * ntask + i]: bits 0-15 the join, bits 16-22 its first
  * chunk of 64 outputs-times-shares and bits 23-26 log2 of the step to the next one, bit 30:
  * nothing to do, bit 31: all waves meet after this entry (in the same entries of every
  * stream).  A join is TO_TREE_WORDS words, ops[join * TO_TREE_WORDS + i]:

@@ -47,6 +47,7 @@ TO_TREE_IDLE, TO_TREE_MEET = 1 << 30, 1 << 31  # fold tree task bits
 MAX_BITS = 32
 FOLD_BITS = 40
 TO_PAIR_ONE = 0x100
+TO_FINISH_NORM = 0x100  # finish variant bit: one output per item, stored normalised
 ABI_VERSION = 7
 
 c_i8x32 = ctypes.c_int8 * MAX_BITS

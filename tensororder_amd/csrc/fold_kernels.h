@@ -78,10 +78,9 @@ __device__ __forceinline__ FoldScale fold_scale(const to_fold_desc* __restrict__
     return FoldScale{(double)a.f * (double)b.f, a.e + b.e};
 }
 
-// Largest of the wave's non-negative floats, the same in every lane: row shifts and row
-// broadcasts (VALU only), where shuffles would go through LDS six times
-__device__ __forceinline__ float fold_wave_max(float v) {
-    uint32_t m = __float_as_uint(v);
+// Largest of the wave's words, the same in every lane: row shifts and row broadcasts (VALU only),
+// where shuffles would go through LDS six times
+__device__ __forceinline__ uint32_t fold_wave_umax(uint32_t m) {
     auto step = [&](auto ctrl) {
         const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, decltype(ctrl)::value, 0xf, 0xf, true);
         m = o > m ? o : m;
@@ -92,8 +91,11 @@ __device__ __forceinline__ float fold_wave_max(float v) {
     step(std::integral_constant<int, 0x118>{});
     step(std::integral_constant<int, 0x142>{});  // row_bcast:15, 31
     step(std::integral_constant<int, 0x143>{});
-    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)m, 63));
+    return (uint32_t)__builtin_amdgcn_readlane((int)m, 63);
 }
+
+// ... of its non-negative floats, which compare as their bits
+__device__ __forceinline__ float fold_wave_max(float v) { return __uint_as_float(fold_wave_umax(__float_as_uint(v))); }
 
 // Sum over thread bits [lo, lo + lk) of a 256-thread block: shuffles inside a wave, LDS
 // across waves, both in a fixed order.  The sums are valid where those bits are zero.
@@ -553,7 +555,7 @@ __global__ __launch_bounds__(kBlock) void k_fold_pair(const to_pair_desc* __rest
             if (lsplit > 0) {
                 gptr<double>(d->partial)[(uint64_t)batch << lsplit | sp] = SCALED ? sum * s.f : sum;
             } else {
-                const T v = (T)(SCALED ? sum * s.f : sum);
+                const T v = (T)norm_sum<SCALED>(SCALED ? sum * s.f : sum, s.e);
                 gptr<T>(d->c)[batch * d->cb] = v;
                 if (SCALED) {
                     note_max(d->cs, batch, (float)absval(v));
@@ -651,8 +653,10 @@ __global__ __launch_bounds__(1024) void k_fold_tree(const to_tree_desc* __restri
                         }
                     }
                 }
-                e += x;
-                f = __longlong_as_double((long long)(1023 - x) << 52);
+                if (nops <= 2) {
+                    e += x;
+                    f = __longlong_as_double((long long)(1023 - x) << 52);
+                }
             }
             // entry b of operand j's bits (the result: j = 4)
             auto entry = [&](int j, int b) {
@@ -663,11 +667,23 @@ __global__ __launch_bounds__(1024) void k_fold_tree(const to_tree_desc* __restri
             float mrun = 0.0f;
             auto finish = [&](double acc, uint32_t co) {
                 for (int b = lo; b < lo + lk; ++b) acc += __shfl_xor(acc, 1 << b, 64);
+                if (SCALED && nops > 2) {
+                    // A product of 3 or 4 tensors may lie far below the product of their maxima, so
+                    // it is scaled by its own largest entry (to [0.5, 1); all entries are in this
+                    // wave, and double holds any product of four floats), whose high word gives
+                    // an upper bound for the record.  One reduction, as the others need after
+                    // their store.
+                    const uint32_t top = fold_wave_umax((uint32_t)((unsigned long long)__double_as_longlong(acc) >> 32) & 0x7fffffffu);
+                    const int x = top >= 0x00100000u && top < 0x7ff00000u ? (int)(top >> 20) - 1022 : 0;
+                    f = __longlong_as_double((long long)(1023 - x) << 52);
+                    e += x;
+                    mrun = top ? (float)(__longlong_as_double((long long)((unsigned long long)top << 32 | 0xffffffffu)) * f) : 0.0f;
+                }
                 const T v = (T)(SCALED ? acc * f : acc);
                 if (writer) {
                     if (cl) data[word(9) + co] = v;
                     else gptr<T>(wide(9))[batch * (int64_t)word(15) + co] = v;
-                    if (SCALED) mrun = fmaxf(mrun, (float)absval(v));
+                    if (SCALED && nops <= 2) mrun = fmaxf(mrun, (float)absval(v));
                 }
             };
             if (nchunk == 0 && nloop <= 2) {
@@ -757,7 +773,7 @@ __global__ __launch_bounds__(1024) void k_fold_tree(const to_tree_desc* __restri
                 else run(Xg, Yg);
             }
             if (SCALED) {
-                const float m = fold_wave_max(mrun);
+                const float m = nops > 2 ? mrun : fold_wave_max(mrun);
                 if (cl) {
                     if (lane == 0) {
                         atomicMax(&recs[slot].maxbits, __float_as_uint(m));

@@ -16,6 +16,7 @@
 //  * FP32 mode keeps one power-of-two exponent per tensor and batch item; consumers
 //    rescale on load, producers fold max |entry| into an atomicMax on its float bits.
 #include <hip/hip_runtime.h>
+#include <cfloat>
 #include <chrono>
 #include <mutex>
 #include <type_traits>
@@ -590,7 +591,18 @@ __global__ __launch_bounds__(kBlock) void k_join_splitk(const to_join_desc* __re
     join_splitk_body<T, SCALED>(d, blockIdx.x - d->block0);
 }
 
-template <typename T, bool SCALED>
+// A value as mantissa and exponent: NORM stores the mantissa and adds the exponent to the result's
+// record, so that a sum far below the product of its operands' maxima keeps all its bits.
+template <bool NORM>
+__device__ __forceinline__ double norm_sum(double v, int64_t& e) {
+    if (!NORM || !(fabs(v) <= DBL_MAX)) return v;
+    int k;
+    const double m = frexp(v, &k);
+    e += k;
+    return m;
+}
+
+template <typename T, bool SCALED, bool NORM = false>
 __device__ __forceinline__ void join_finish_body(const to_join_desc* __restrict__ d, const int64_t local) {
     const int fx = d->fx, fy = d->fy;
     const int nsplit = d->nsplit;
@@ -609,14 +621,15 @@ __device__ __forceinline__ void join_finish_body(const to_join_desc* __restrict_
         if (valid) {
             double acc = 0.0;
             for (int sp = 0; sp < nsplit; ++sp) acc += partial[o * nsplit + sp];
-            const T sum = (T)acc;
+            int64_t k = 0;
+            const T sum = (T)norm_sum<NORM>(acc, k);
             const int64_t f = (o >> fy) & ((1ll << fx) - 1);
             const int64_t y = o & ((1ll << fy) - 1);
             C[batch * d->cb + ((f << d->shf) | (y << d->shy))] = sum;
             m = (float)absval(sum);
             if (SCALED && f == 0 && y == 0) {
                 const int64_t e = op_scale(d->xs, d->xsb, batch).e + op_scale(d->ys, d->ysb, batch).e;
-                note_exp(d->cs, batch, e);
+                note_exp(d->cs, batch, e + k);
             }
         }
         if (SCALED) {
@@ -637,9 +650,16 @@ __global__ __launch_bounds__(kBlock) void k_join_finish(const to_join_desc* __re
     join_finish_body<T, SCALED>(d, blockIdx.x - d->block0);
 }
 
+// (TO_FINISH_NORM)
+template <typename T, bool SCALED>
+__global__ __launch_bounds__(kBlock) void k_join_finish_norm(const to_join_desc* __restrict__ descs, int ndesc, const int32_t* __restrict__ bmap) {
+    const to_join_desc* d = descs + find_desc(descs, ndesc, blockIdx.x, bmap);
+    join_finish_body<T, SCALED, SCALED>(d, blockIdx.x - d->block0);
+}
+
 // Many partial sums per output (nsplit >= 32, e.g. a dot product of two large tensors):
 // one block per output, its threads sum strided partials and reduce in LDS.
-template <typename T, bool SCALED>
+template <typename T, bool SCALED, bool NORM = false>
 __device__ __forceinline__ void join_finish_wide_body(const to_join_desc* __restrict__ d, const int64_t local) {
     __shared__ double red[kBlock / 64];
     const int fx = d->fx, fy = d->fy;
@@ -652,7 +672,8 @@ __device__ __forceinline__ void join_finish_wide_body(const to_join_desc* __rest
         for (int sp = threadIdx.x; sp < nsplit; sp += kBlock) acc += partial[o * nsplit + sp];
         acc = block_sum(acc, red);
         if (threadIdx.x == 0) {
-            const T sum = (T)acc;
+            int64_t k = 0;
+            const T sum = (T)norm_sum<NORM>(acc, k);
             const int64_t batch = o >> (fx + fy);
             const int64_t f = (o >> fy) & ((1ll << fx) - 1);
             const int64_t y = o & ((1ll << fy) - 1);
@@ -661,7 +682,7 @@ __device__ __forceinline__ void join_finish_wide_body(const to_join_desc* __rest
                 note_max(d->cs, batch, (float)absval(sum));
                 if (f == 0 && y == 0) {
                     const int64_t e = op_scale(d->xs, d->xsb, batch).e + op_scale(d->ys, d->ysb, batch).e;
-                    note_exp(d->cs, batch, e);
+                    note_exp(d->cs, batch, e + k);
                 }
             }
         }
@@ -672,6 +693,13 @@ template <typename T, bool SCALED>
 __global__ __launch_bounds__(kBlock) void k_join_finish_wide(const to_join_desc* __restrict__ descs, int ndesc, const int32_t* __restrict__ bmap) {
     const to_join_desc* d = descs + find_desc(descs, ndesc, blockIdx.x, bmap);
     join_finish_wide_body<T, SCALED>(d, blockIdx.x - d->block0);
+}
+
+// (TO_FINISH_NORM)
+template <typename T, bool SCALED>
+__global__ __launch_bounds__(kBlock) void k_join_finish_wide_norm(const to_join_desc* __restrict__ descs, int ndesc, const int32_t* __restrict__ bmap) {
+    const to_join_desc* d = descs + find_desc(descs, ndesc, blockIdx.x, bmap);
+    join_finish_wide_body<T, SCALED, SCALED>(d, blockIdx.x - d->block0);
 }
 
 // One join given by value (to_tensordot): the kernels above without a descriptor table.
@@ -2388,12 +2416,23 @@ int launch_one(const to_launch& L, hipStream_t st) {
             break;
         case TO_OP_JOIN_FINISH:
             if (!L.descs || L.count <= 0) return TO_ERR_INVALID;
-            if (L.variant == 1)
-                hipLaunchKernelGGL((k_join_finish_wide<T, SCALED>), grid, block, 0, st,
-                                   reinterpret_cast<const to_join_desc*>(L.descs), L.count, bmap);
-            else
-                hipLaunchKernelGGL((k_join_finish<T, SCALED>), grid, block, 0, st,
-                                   reinterpret_cast<const to_join_desc*>(L.descs), L.count, bmap);
+            switch (L.variant) {
+#define TO_FINISH_LAUNCH(KERNEL)                                      \
+    hipLaunchKernelGGL((KERNEL<T, SCALED>), grid, block, 0, st,       \
+                       reinterpret_cast<const to_join_desc*>(L.descs), L.count, bmap);
+                case 1:
+                    TO_FINISH_LAUNCH(k_join_finish_wide)
+                    break;
+                case TO_FINISH_NORM:
+                    TO_FINISH_LAUNCH(k_join_finish_norm)
+                    break;
+                case TO_FINISH_NORM | 1:
+                    TO_FINISH_LAUNCH(k_join_finish_wide_norm)
+                    break;
+                default:
+                    TO_FINISH_LAUNCH(k_join_finish)
+#undef TO_FINISH_LAUNCH
+            }
             break;
         case TO_OP_SCALE_CLEAR:
             if (!L.aux0 || L.iaux0 <= 0) return TO_ERR_INVALID;

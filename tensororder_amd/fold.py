@@ -883,13 +883,14 @@ def pair_records(n, W, esize, scaled, abase, scratch, recp, one):
     out = [("pair", _lib.TO_OP_FOLD_PAIR, v["variant"], 0, d, v["nblocks"])]
     if v["lsplit"]:
         d.partial = abase + scratch["partial"][0]
-        out.append(_finish(n, v, d.partial, nb, ends, d.cs))
+        out.append(_finish(n, v, d.partial, nb, ends, d.cs, _lib.TO_FINISH_NORM if scaled else 0))
     return out
 
 
-def _finish(n, v, partial, nb, ends, crec):
+def _finish(n, v, partial, nb, ends, crec, norm=0):
     """The record that adds up a join's partial sums; ``ends``: (record, stride) of the two
-    operands, whose exponents the result carries (scaled only)."""
+    operands, whose exponents the result carries (scaled only); ``norm``: TO_FINISH_NORM for a
+    sum of products of more than two stored tensors."""
     f = _lib.JoinDesc()
     f.c, f.cb, f.partial, f.nsplit = n.ptr, n.bstride, partial, v["nsplit"]
     if ends:
@@ -897,7 +898,7 @@ def _finish(n, v, partial, nb, ends, crec):
     f.fx, f.nbatch = n.rank, nb
     wide = v["nsplit"] >= 32
     f.nblocks = int(min(v["nout"] if wide else -(-v["nout"] // 256), schedule.MAX_STREAM_BLOCKS))
-    return "finish", _lib.TO_OP_JOIN_FINISH, 1 if wide else 0, 0, f, f.nblocks
+    return "finish", _lib.TO_OP_JOIN_FINISH, norm | wide, 0, f, f.nblocks
 
 
 def join_traffic(n, nodes, W, esize):

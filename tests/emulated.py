@@ -4,10 +4,12 @@ without a GPU.  Launches run as they are queued; ``synchronize`` and ``finish`` 
 
 import contextlib
 import ctypes
+import math
 import types
 
 import emulator
-from test_fold import FoldEmulator
+import numpy as np
+from test_fold import FoldEmulator, _spread
 
 from tensororder_amd import _lib, hip_api
 
@@ -45,8 +47,57 @@ class _Device:
 
 
 class RunEmulator(FoldEmulator):
-    """... with the bookkeeping launches that open a run of the edge walk, and sums that also go
-    to host memory."""
+    """... with the bookkeeping launches that open a run of the edge walk, sums that also go to
+    host memory, and results of more than two operands scaled by their own largest entry."""
+
+    def _tree_task(self, d, op, chunk, batch, data, recs, pending):
+        if not self.scaled or int(op[0]) >> 16 & 3 < 2:
+            return super()._tree_task(d, op, chunk, batch, data, recs, pending)
+        head = int(op[0])
+        lo, lk, nloop = head & 15, head >> 4 & 15, head >> 8 & 15
+        prod, e = 1.0, 0
+        for j in range((head >> 16 & 3) + 1):
+            bits = op[64 + 16 * j:80 + 16 * j]
+            k = (_spread(bits, lo, lk)[:, None] + _spread(bits, 6, nloop)[None, :]).ravel()
+            idx = _spread(bits, 0, lo)[:, None] + k[None, :]
+            addr, slot = int(op[1 + 2 * j]) | int(op[2 + 2 * j]) << 32, int(op[16 + j])
+            if head >> (20 + j) & 1:
+                prod = prod * data[addr + idx].astype(np.float64)
+                e += recs[slot][0]
+            else:
+                src = self.heap.view(addr + batch * int(op[11 + j]) * 4, np.float32, int(idx.max()) + 1)
+                prod = prod * src[idx].astype(np.float64)
+                e += self.get_rec(d.recs, slot + (batch if head >> (25 + j) & 1 else 0))[0]
+        total = prod.sum(axis=1)
+        x = math.frexp(np.abs(total).max())[1]
+        v = np.ldexp(total, -x).astype(np.float32)
+        o, addr, slot = _spread(op[32:48], 0, lo), int(op[9]) | int(op[10]) << 32, int(op[20])
+        self.operands = getattr(self, "operands", set()) | {(head >> 16 & 3) + 1}
+
+        def write():
+            m = np.abs(v).max()
+            if head >> 24 & 1:
+                data[addr + o] = v
+                recs[slot][:] = [e + x, float(m)]
+            else:
+                self.heap.view(addr + batch * int(op[15]) * 4, np.float32, int(o.max()) + 1)[o] = v
+                self.set_rec(d.recs, slot + (batch if head >> 29 & 1 else 0), exp=e + x, maxbits=int(m.view(np.uint32)))
+        pending.append(write)
+
+    def op_4(self, L):
+        if not L.variant & _lib.TO_FINISH_NORM:
+            return super().op_4(L)
+        assert self.scaled
+        for i in range(L.count):
+            d = self.heap.read_struct(_lib.JoinDesc, L.descs + i * ctypes.sizeof(_lib.JoinDesc))
+            assert d.partial in self.gemm_partials and d.fx == d.fy == 0
+            P = self.heap.view(d.partial, np.float64, d.nbatch * d.nsplit).reshape(-1, d.nsplit)
+            for b, total in enumerate(P.sum(axis=1)):
+                m, x = math.frexp(total)
+                e = x + sum(exp + emulator._scale_exp(top) for exp, top in
+                            (self.get_rec(d.xs, b * d.xsb), self.get_rec(d.ys, b * d.ysb)))
+                self.heap.view(d.c + 4 * b * d.cb, np.float32, 1)[0] = m
+                self.set_rec(d.cs, b, exp=e, maxbits=int(np.float32(abs(m)).view(np.uint32)))
 
     def op_6(self, L):
         if L.variant == 0:
