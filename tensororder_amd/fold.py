@@ -71,6 +71,8 @@ TREE_WAVES_MANY = 8
 TREE_LDS = 120 * 1024
 TREE_LDS_MANY = 40 * 1024
 TREE_MANY = 512
+# joins from which a program is fitted to LDS bit by bit as it grows
+TREE_LONG = 256
 # a program of one join only up to this many index values (a launch of many blocks above)
 TREE_LONE_BITS = 12
 # joins of a program merged into one product: at most 4 operands, 64 outputs and 2^MERGE_LOOP
@@ -601,35 +603,80 @@ def _program(nodes, root, stage, esize, scaled):
 
 
 def tree_programs(nodes, W, esize, scaled, lds=None):
-    """The programs of a plan whose joins carry their forms: maximal connected parts of small
-    joins of one phase whose intermediates fit ``lds`` bytes."""
-    # a small join's stage: its phase and the number of large joins on the longest path below
-    # it; programs are the connected joins of one stage, so none waits for more than it reads
+    """The programs of a plan whose joins carry their forms: connected parts of small joins of
+    one phase whose intermediates fit ``lds`` bytes."""
+    # a small join's stage: its phase and the number of large joins -- and of places where a
+    # program ends because LDS holds no more -- on the longest path below it; programs are the
+    # connected joins of one stage, so none waits for more than it reads
+    joins = [n for n in nodes if not n.is_leaf]
+    at = {n.idx: k for k, n in enumerate(joins)}
     stage, depth = {}, {}
-    for n in nodes:
-        if n.is_leaf:
-            continue
-        # a block reads a large tensor of another launch at the latency of L2: fewer products
-        far = any(c >= 0 and nodes[c].rank > TREE_FAR_RANK and (c not in stage or nodes[c].batched != n.batched)
-                  for c in (n.left, n.right))
-        small = n.geom["var"]["kind"] == "fold" and n.rank <= TREE_RANK and \
-            len(n.ksum) + n.rank <= (TREE_FAR_BITS if far else TREE_BITS)
-        depth[n.idx] = max([depth[c] for c in (n.left, n.right)
-                            if c in depth and nodes[c].batched == n.batched], default=0) + (not small)
-        if small:
-            stage[n.idx] = (n.batched, depth[n.idx])
-    out = []
-    todo = [i for i in stage if stage.get(nodes[i].parent) != stage[i]]
-    while todo:
-        i = todo.pop()
+    size = {}  # joins of the program that ends at a small join
+    sure = {}  # ... and how many of them one join below it has been seen to hold
+    full = set()  # joins that do not fit LDS with what is below them
+
+    def fits(i):
         p = _program(nodes, i, stage, esize, scaled)
-        if p.lds > (lds or (TREE_LDS_MANY if p.batched and W >= TREE_MANY else TREE_LDS)):
-            # its root runs as a launch of its own, what is below as programs
-            todo += [c for c in (nodes[i].left, nodes[i].right) if stage.get(c) == stage[i]]
-            del stage[i]
-        elif len(p.members) > 1 or len(nodes[i].ksum) + nodes[i].rank <= TREE_LONE_BITS:
-            out.append(p)
-    return sorted(out, key=lambda p: p.root)
+        ok = p.lds <= (lds or (TREE_LDS_MANY if p.batched and W >= TREE_MANY else TREE_LDS))
+        if ok:
+            sure[i] = size[i]
+        return p if ok else None
+
+    def first_full(i):
+        """The first join of the program ending at ``i``, which does not fit, that is too much."""
+        todo, members = [i], []
+        while todo:
+            members.append(todo.pop())
+            todo += [c for c in (nodes[members[-1]].left, nodes[members[-1]].right) if stage.get(c) == stage[i]]
+        members.sort()
+        lo, hi = 0, len(members)  # of the first lo joins every program fits, of the first hi one does not
+        while hi - lo > 1:
+            mid = (lo + hi) // 2
+            tops = [m for m in members[:mid] if nodes[m].parent > members[mid - 1]]
+            if all(sure[m] == size[m] or fits(m) for m in tops):
+                lo = mid
+            else:
+                hi = mid
+        return members[hi - 1]
+
+    k, out = 0, []
+    while True:
+        while k < len(joins):
+            n = joins[k]
+            i, cut = n.idx, n.idx in full
+            below = [c for c in (n.left, n.right) if c in depth and nodes[c].batched == n.batched]
+            # a block reads a large tensor of another launch at the latency of L2: fewer products
+            far = any(c >= 0 and nodes[c].rank > TREE_FAR_RANK and
+                      (cut or c not in stage or nodes[c].batched != n.batched) for c in (n.left, n.right))
+            small = n.geom["var"]["kind"] == "fold" and n.rank <= TREE_RANK and \
+                len(n.ksum) + n.rank <= (TREE_FAR_BITS if far else TREE_BITS)
+            depth[i] = max([depth[c] for c in below], default=0) + (cut or not small)
+            stage.pop(i, None)
+            k += 1
+            if not small:
+                continue
+            stage[i] = (n.batched, depth[i])
+            mine = [c for c in below if stage.get(c) == stage[i]]
+            size[i] = 1 + sum(size[c] for c in mine)
+            sure[i] = max([sure[c] for c in mine], default=1)
+            # (long ones are checked where they have doubled, so that a join is looked at a few
+            # times in all; the others where they end)
+            if size[i] > max(TREE_LONG, 2 * sure[i]) and fits(i) is None:
+                j = first_full(i)
+                full.add(j)
+                k = at[j]
+        out, again = [], []
+        for i in stage:
+            if stage.get(nodes[i].parent) != stage[i]:
+                p = fits(i)
+                if p is None:
+                    again.append(first_full(i))
+                elif size[i] > 1 or len(nodes[i].ksum) + nodes[i].rank <= TREE_LONE_BITS:
+                    out.append(p)
+        if not again:
+            return sorted(out, key=lambda p: p.root)
+        full.update(again)
+        k = min(at[j] for j in again)
 
 
 def _tree_task(n, ksum, operands):

@@ -1,0 +1,98 @@
+"""How the programs of a plan are cut: to what LDS holds, with work that grows with the plan, and
+to the same count wherever the cuts lie."""
+
+import numpy as np
+import pytest
+import test_fold
+
+from oracle import numpy_oracle
+from tensororder_amd import _lib, fold, network, plan_io, planners, schedule
+from tensororder_amd.formula import parse_dimacs_text
+from tensororder_amd.network import BuiltTensor, TensorNetwork, VariableTensor
+from tensororder_amd.tree import TreeContext
+
+
+def grid_plan(width, length):
+    """The line plan of a vertex cover of a width x length grid."""
+    def v(i, j):
+        return i * width + j + 1
+
+    clauses = [(v(i, j), v(i, j + 1)) for i in range(length) for j in range(width - 1)]
+    clauses += [(v(i, j), v(i + 1, j)) for i in range(length - 1) for j in range(width)]
+    text = "p cnf %d %d\n" % (width * length, len(clauses)) + "".join("%d %d 0\n" % c for c in clauses)
+    return planners.best_plan(network.cnf_count(parse_dimacs_text(text, "cachet")), "line", solver=None, seed=0)
+
+
+def chain(n):
+    """(tree, tables) of a product of n 2 x 2 matrices, COPY tensors between them."""
+    net, order, last = TensorNetwork(), [], None
+    for i in range(n):
+        ends = net.add_node(BuiltTensor(np.ones((2,) * (1 if i in (0, n - 1) else 2))))
+        if last is not None:
+            tie = net.add_node(VariableTensor(2, 1, 1))
+            net.connect(*last, *tie[0])
+            net.connect(*tie[1], *ends[0])
+            order.append(tie[0][0])
+        order.append(ends[0][0])
+        last = ends[-1]
+    ctx, tree, tables = TreeContext(), None, {}
+    for t in order:
+        rank = net[t].rank
+        tables[t] = schedule.LeafTable(np.eye(2).reshape(1, -1) if rank == 2 else np.ones((1, 2)), [], rank,
+                                       copy=(1, 1, True) if isinstance(net[t], VariableTensor) else None)
+        tree = ctx.leaf(net, t) if tree is None else ctx.join(tree, ctx.leaf(net, t))
+    return ctx.get_tree(tree), tables
+
+
+def checked_programs(nodes, W, esize, lds=None):
+    """The programs of a plan, and how many joins were looked at to find them."""
+    seen = []
+    inner = fold._program
+
+    def counted(*args):
+        p = inner(*args)
+        seen.append(len(p.members))
+        return p
+
+    fold._program = counted
+    try:
+        programs = fold.tree_programs(nodes, W, esize, esize == 4, lds)
+    finally:
+        fold._program = inner
+    members = [i for p in programs for i in p.members]
+    assert len(members) == len(set(members))
+    assert all(p.lds <= (lds or fold.TREE_LDS) for p in programs)
+    return programs, sum(seen)
+
+
+@pytest.mark.parametrize("esize", [8, 4])
+@pytest.mark.parametrize("name", ["grid", "chain"])
+def test_long_plans_are_cut_with_little_work(name, esize):
+    if name == "grid":
+        tree, tables = test_fold.plan_inputs(grid_plan(8, 120))[1:3]
+    else:
+        tree, tables = chain(40000 if esize == 4 else 8000)
+    nodes, _ = fold.analyse(tree, tables, esize)
+    fold.choose_all(nodes, 1, esize)
+    programs, seen = checked_programs(nodes, 1, esize)
+    joins = sum(not n.is_leaf for n in nodes)
+    assert joins > 2500 and seen < 16 * joins
+    if name == "chain" and esize == 4:
+        assert 2 < len(programs) < 10  # (the records of a program's tensors fill LDS)
+    # next to all joins are in programs: what does not fit one goes on in another
+    assert sum(len(p.members) for p in programs) > 0.99 * joins
+    assert len(fold.phase_groups(nodes, False, "level", programs)) < 8
+
+
+@pytest.mark.parametrize("lds", [64, 256, 1024, 8192])
+@pytest.mark.parametrize("et,tol", [(_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)])
+def test_counts_wherever_programs_are_cut(lds, et, tol, monkeypatch):
+    monkeypatch.setattr(fold, "TREE_LDS", lds)
+    monkeypatch.setattr(fold, "TREE_LONG", 8)
+    for kind, n, slices in (("vc", 30, 1), ("cnf", 20, 2)):
+        plan = test_fold._formula_plan(kind, n, 3, slices)
+        want = numpy_oracle.contract_sliced(plan_io.plan_to_dict(plan))
+        got, prog, _ = test_fold.emulate(plan, et, 1 << slices)
+        assert got == pytest.approx(want, rel=tol, abs=0)
+        assert len(prog.programs) > 2
+        checked_programs(prog.nodes, 1 << slices, 8 if et == _lib.TO_F64 else 4)
