@@ -71,8 +71,10 @@ TREE_WAVES_MANY = 8
 TREE_LDS = 120 * 1024
 TREE_LDS_MANY = 40 * 1024
 TREE_MANY = 512
-# joins from which a program is fitted to LDS bit by bit as it grows
+# joins from which a program is fitted bit by bit as it grows
 TREE_LONG = 256
+# products of a program (a task word has 16 bits for its product)
+TREE_PRODUCTS = 1 << 16
 # a program of one join only up to this many index values (a launch of many blocks above)
 TREE_LONE_BITS = 12
 # joins of a program merged into one product: at most 4 operands, 64 outputs and 2^MERGE_LOOP
@@ -604,20 +606,21 @@ def _program(nodes, root, stage, esize, scaled):
 
 def tree_programs(nodes, W, esize, scaled, lds=None):
     """The programs of a plan whose joins carry their forms: connected parts of small joins of
-    one phase whose intermediates fit ``lds`` bytes."""
+    one phase whose intermediates fit ``lds`` bytes, of at most TREE_PRODUCTS products."""
     # a small join's stage: its phase and the number of large joins -- and of places where a
-    # program ends because LDS holds no more -- on the longest path below it; programs are the
+    # program ends because it may hold no more -- on the longest path below it; programs are the
     # connected joins of one stage, so none waits for more than it reads
     joins = [n for n in nodes if not n.is_leaf]
     at = {n.idx: k for k, n in enumerate(joins)}
     stage, depth = {}, {}
     size = {}  # joins of the program that ends at a small join
     sure = {}  # ... and how many of them one join below it has been seen to hold
-    full = set()  # joins that do not fit LDS with what is below them
+    full = set()  # joins that do not fit one program with what is below them
 
     def fits(i):
         p = _program(nodes, i, stage, esize, scaled)
-        ok = p.lds <= (lds or (TREE_LDS_MANY if p.batched and W >= TREE_MANY else TREE_LDS))
+        ok = p.lds <= (lds or (TREE_LDS_MANY if p.batched and W >= TREE_MANY else TREE_LDS)) and \
+            sum(map(len, p.levels)) <= TREE_PRODUCTS
         if ok:
             sure[i] = size[i]
         return p if ok else None
@@ -696,7 +699,9 @@ def _tree_task(n, ksum, operands):
 def tree_words(p, nodes, waves, rec_index, one):
     """(uint32 joins [n, 128], uint32 task streams [waves, ntask]) of a program.  ``one``:
     (address, record index) of the stored 1.0."""
-    words = np.zeros((sum(len(lv) for lv in p.levels), _lib.TO_TREE_WORDS), dtype=np.uint32)
+    words = np.zeros((sum(map(len, p.levels)), _lib.TO_TREE_WORDS), dtype=np.uint32)
+    if len(words) > TREE_PRODUCTS:
+        raise ValueError("a program of %d products" % len(words))
     streams = [[] for _ in range(waves)]
     k = 0
     for lv in p.levels:

@@ -96,3 +96,24 @@ def test_counts_wherever_programs_are_cut(lds, et, tol, monkeypatch):
         assert got == pytest.approx(want, rel=tol, abs=0)
         assert len(prog.programs) > 2
         checked_programs(prog.nodes, 1 << slices, 8 if et == _lib.TO_F64 else 4)
+
+
+@pytest.mark.parametrize("most", [1, 3, 40])
+@pytest.mark.parametrize("et,tol", [(_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)])
+def test_programs_hold_no_more_products_than_a_task_names(most, et, tol, monkeypatch):
+    assert fold.TREE_PRODUCTS == 0xffff + 1  # bits 0-15 of a task
+    monkeypatch.setattr(fold, "TREE_PRODUCTS", most)
+    plan = test_fold._formula_plan("vc", 40, 1, 0)
+    want = numpy_oracle.contract_sliced(plan_io.plan_to_dict(plan))
+    got, prog, _ = test_fold.emulate(plan, et, 1)
+    assert got == pytest.approx(want, rel=tol, abs=0)
+    sizes = [sum(map(len, p.levels)) for p in prog.programs]
+    assert max(sizes) <= most and len(sizes) > 1
+    tree, tables = chain(500)
+    nodes, _ = fold.analyse(tree, tables, 8)
+    fold.choose_all(nodes, 1, 8)
+    programs, _ = checked_programs(nodes, 1, 8)
+    assert max(sum(map(len, p.levels)) for p in programs) <= most
+    monkeypatch.setattr(fold, "TREE_PRODUCTS", 0)
+    with pytest.raises(ValueError):
+        fold.tree_words(programs[0], nodes, 16, lambda n: 0, (0, 0))
