@@ -145,12 +145,17 @@ def has_copies(tables):
     return bool(copies) and not any(t.rank if sum(map(bool, t.coef)) == 1 else t.batched for t in copies)
 
 
+def _power(n):
+    """2.0^n, for any number n of variables (a plan far too large is refused for its memory)."""
+    return 2.0 ** min(n, 900)
+
+
 def _join_cost(left, right, union, out, batched, esize):
     lx, ly = len(left.open), len(right.open)
-    c = esize * ((1 << lx) + (1 << ly) + (1 << out)) / BYTES_PER_S
+    c = esize * (_power(lx) + _power(ly) + _power(out)) / BYTES_PER_S
     # free range of each side: what the MFMA products need
     dense = union - lx >= 6 and union - ly >= 6 and union - out >= 4
-    c += (1 << union) / (GEMM_PRODUCTS_PER_S if dense else PRODUCTS_PER_S)
+    c += _power(union) / (GEMM_PRODUCTS_PER_S if dense else PRODUCTS_PER_S)
     return c * (BATCH_WEIGHT if batched else 1.0)
 
 
@@ -312,7 +317,7 @@ def analyse(tree, tables, esize, regroup=True):
             when[v] = n.idx
         if n.right >= 0:
             for v in min(nodes[n.left].order, nodes[n.right].order, key=len):
-                weight[v] = weight.get(v, 0.0) + 2.0 ** len(held)
+                weight[v] = weight.get(v, 0.0) + _power(len(held))
     for n in nodes:
         n.order.sort(key=lambda v: (-when[v], weight.get(v, 0.0), v))
         n.order0 = n.order

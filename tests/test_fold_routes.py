@@ -1,6 +1,7 @@
 """Which plans are folded, and that the others are answered as well: COPY tensors sliced on a
 part of their edges, or by two groups."""
 
+import numpy as np
 import pytest
 from emulated import EmulatedAPI
 
@@ -8,6 +9,9 @@ from oracle import numpy_oracle
 from tensororder_amd import _lib, fold, network, plan_io, planners
 from tensororder_amd.formula import parse_dimacs_text
 from tensororder_amd.instances import random_3cnf
+from tensororder_amd.network import BuiltTensor, TensorNetwork, VariableTensor
+from tensororder_amd.plan import SlicedExecutionPlan
+from tensororder_amd.tree import TreeContext
 
 
 def _plan(n, seed):
@@ -38,3 +42,40 @@ def test_copies_sliced_on_a_part_of_their_edges(seed, et, tol):
         got = plan_io.plan_from_dict(doc)
         assert fold.has_copies(api._plan_inputs(got, None)[2]) == (groups == [whole])
         assert api.contract_sliced(got) == pytest.approx(want, rel=tol)
+
+
+def _star(n):
+    """A plan of dense tensors and COPY tensors that opens 2 n variables before it sums any."""
+    net, first, second = TensorNetwork(), [], []
+    for _ in range(n):
+        a, b, d = (net.add_node(BuiltTensor(np.ones((2, 2)))) for _ in range(3))
+        c = net.add_node(VariableTensor(2, 1, 1))
+        net.connect(*a[0], *c[0])
+        net.connect(*c[1], *b[0])
+        net.connect(*a[1], *d[0])
+        net.connect(*d[1], *b[1])
+        first += [a[0][0], c[0][0], d[0][0]]
+        second.append(b[0][0])
+    ctx, tree = TreeContext(), None
+    for t in first + second:
+        tree = ctx.leaf(net, t) if tree is None else ctx.join(tree, ctx.leaf(net, t))
+    return SlicedExecutionPlan(ctx.get_tree(tree), net)
+
+
+def _answer(call, plan):
+    """What a call answers, with its kind of refusal in place of an answer."""
+    try:
+        return call(plan)
+    except Exception as e:
+        return type(e)
+
+
+@pytest.mark.parametrize("n", [40, 600])
+@pytest.mark.parametrize("et", [_lib.TO_F64, _lib.TO_F32S])
+def test_far_too_large_plans_are_refused_alike(n, et, monkeypatch):
+    # (a join over more variables than a float has exponents)
+    plan, api = _star(n), EmulatedAPI(et)
+    calls = [lambda p: api.contract_sliced(p), lambda p: api.contract_batch([p])]
+    folded = [_answer(call, plan) for call in calls]
+    monkeypatch.setattr(fold, "has_copies", lambda tables: False)
+    assert folded == [_answer(call, plan) for call in calls] == [MemoryError] * 2
