@@ -105,7 +105,11 @@ class FoldDesc:
 
 
 class TooWide(ValueError):
-    """A join over more variables than a descriptor holds: the plan runs edge by edge."""
+    """A join over more variables, or of a larger tensor, than a descriptor holds (offsets are
+    32 bits): the plan runs edge by edge."""
+
+
+OFFSET_BITS = 32
 
 
 class FNode:
@@ -369,6 +373,8 @@ def choose(n, nodes, W, esize, launch_bound=False):
     A = nodes[n.left]
     B = nodes[n.right] if n.right >= 0 else None
     nb = W if n.batched else 1
+    if max(t.rank for t in (A, B, n) if t is not None) > OFFSET_BITS:
+        raise TooWide("folded join of a tensor of more than 2^%d entries" % OFFSET_BITS)
     _reordered(n, list(n.want or n.order0))
     if B is None:
         X, Y = A, None

@@ -6,7 +6,7 @@ import pytest
 from emulated import EmulatedAPI
 
 from oracle import numpy_oracle
-from tensororder_amd import _lib, fold, network, plan_io, planners
+from tensororder_amd import _lib, fold, hip_api, network, plan_io, planners
 from tensororder_amd.formula import parse_dimacs_text
 from tensororder_amd.instances import random_3cnf
 from tensororder_amd.network import BuiltTensor, TensorNetwork, VariableTensor
@@ -79,3 +79,32 @@ def test_far_too_large_plans_are_refused_alike(n, et, monkeypatch):
     folded = [_answer(call, plan) for call in calls]
     monkeypatch.setattr(fold, "has_copies", lambda tables: False)
     assert folded == [_answer(call, plan) for call in calls] == [MemoryError] * 2
+
+
+@pytest.mark.parametrize("esize", [8, 4])
+def test_tensors_beyond_32_bit_offsets_run_edge_by_edge(esize):
+    class Api:
+        _esize, _regroup, _max_batch = esize, True, 64
+
+        def _budget(self):
+            return 1 << 50
+
+    seen = set()
+    for n in range(14, 21):
+        _, tree, tables, _ = EmulatedAPI._plan_inputs(EmulatedAPI(heap_bytes=64), _star(n), None)
+        folded = fold.analyse(tree, tables, esize, regroup=False)
+        rank = max(t.rank for t in folded[0])
+        folds = rank <= 32
+        seen.add(rank)
+        assert hip_api.HipAPI.choose_folded_batch(Api(), folded, tree, tables, 1) == folds
+        assert (fold.analyse_batch([(tree, tables)], esize, regroup=False) is not None) == folds
+        if folds:  # every record of the plan holds its offsets
+            nodes = folded[0]
+            for t in nodes:
+                t.ptr = t.bstride = 0
+            for t in nodes:
+                if not t.is_leaf and t.geom["var"]["kind"] == "fold":
+                    scratch = {"partial": (0, 0)}
+                    for record in fold.join_records(t, nodes, 1, esize, False, 0, scratch, lambda n: 0, (0, 0)):
+                        assert bytes(record[4])
+    assert 32 in seen and max(seen) > 32
