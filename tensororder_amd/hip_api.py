@@ -93,12 +93,11 @@ class Executable:
         self.nwaves = 0 if prog.root_const else -(-total_slices // prog.nbatch)
         begin = _lib.Launch(op=_lib.TO_OP_STEP_BEGIN, grid=1, aux2=prog.accum.data_ptr(),
                             aux3=prog.params.data_ptr())
-        self.step_launches = [begin] + list(prog.prologue)
-        self.wave_launches = list(prog.wave)
+        self._step, self._wave = [begin] + list(prog.prologue), list(prog.wave)
         self._graphs = []
         # what a run replays, in order: graphs, or launch lists run one by one
-        first = list(prog.prologue) if prog.self_start else self.step_launches
-        runs = [first] + [self.wave_launches] * self.nwaves
+        first = list(prog.prologue) if prog.self_start else self._step
+        runs = [first] + [self._wave] * self.nwaves
         if sum(len(r) for r in runs) <= self.ONE_GRAPH_LAUNCHES:
             runs = [sum(runs, [])]
         # a plan that runs once only pays for capturing waves that repeat
@@ -106,10 +105,14 @@ class Executable:
         self._runs = []
         # runs queued since the last wait, and the value of the sum's word that ends them
         self._queued, self._word = 0, 0
+        # whether the device's wave counter stands at the first slice once what is queued is
+        # done: a run leaves it there, one cut short does not
+        self._whole = True
+        self._lent = False  # whether a caller has the launches, and may run them by itself
         self._sums = sum(L.op == _lib.TO_OP_ROOT_REDUCE for r in runs for L in r)
         for r in runs:
             if id(r) not in captured:
-                use = api._use_graph and r and (not once or (r is self.wave_launches and self.nwaves > 2))
+                use = api._use_graph and r and (not once or (r is self._wave and self.nwaves > 2))
                 captured[id(r)] = (self._capture(r) if use else None, r)
             self._runs.append(captured[id(r)])
 
@@ -126,28 +129,61 @@ class Executable:
         _lib.check(self.api._lib.to_graph_launch(graph, ctypes.c_void_p(self.api._stream.cuda_stream)),
                    "to_graph_launch")
 
+    @property
+    def step_launches(self):
+        """The launches that open a run: its start, then the prologue."""
+        self._lent = True
+        return self._step
+
+    @property
+    def wave_launches(self):
+        """The launches of one wave of slices."""
+        self._lent = True
+        return self._wave
+
     def enqueue(self):
         """Queue one full contraction on the API's stream (no synchronisation)."""
-        if self.prog.host_accum is not None:
-            if not self._queued:
-                self._word = self._host_sum().pad
-            self._queued += 1
-            self._word += self._sums
+        own = self.prog.host_accum is not None  # (else the run's first launch resets what it needs)
+        if own and not self._whole:
+            # an earlier run was cut short (a failed launch, an interrupt): nothing of it is
+            # counted, and the device's counter may stand between its waves
+            self.api.synchronize()
+            self._queued = 0
+        if own and (self._lent or not self._whole):
+            self.api._upload(self.prog.params, self.counters(self.total))
+        if own and not self._queued:
+            self._word = self._host_sum().pad
+        self._whole = False
         for graph, launches in self._runs:
             if graph is not None:
                 self._launch_graph(graph)
             else:
                 self.api._run(launches)
+        self._queued += own
+        self._word += self._sums
+        self._whole = True
+
+    @staticmethod
+    def counters(total):
+        """The device's counters: the wave's first slice and the number of slices, and the same
+        of the prologue."""
+        return np.array([0, total, 0, 1], dtype=np.int64).tobytes()
 
     def result(self):
         """Synchronise and read the (mantissa, exponent) slice sum."""
         api = self.api
         if self.prog.host_accum is not None:
+            if not self._whole:
+                raise RuntimeError("the last run was cut short while it was queued")
             acc = self._host_sum()
-            if self._queued:
+            if self._lent:  # (launches that a caller runs count in the word too)
+                api.synchronize()
+            elif self._queued:
                 _lib.check(api._lib.to_wait(ctypes.c_void_p(ctypes.addressof(acc) + _lib.Accum.pad.offset),
                                             self._word, ctypes.c_void_p(api._stream.cuda_stream)), "to_wait")
-                self._queued = 0
+                if acc.pad < self._word:
+                    raise RuntimeError("the device is idle and has not written the sum")
+            self._queued = 0
             acc = _lib.Accum.from_buffer_copy(acc)
         else:
             api.synchronize()
@@ -168,7 +204,7 @@ class Executable:
         return self.result()
 
     def close(self):
-        if self._graphs or self._queued:
+        if self._graphs or self._queued or not getattr(self, "_whole", True):
             self.api.synchronize()  # the sum's word is written by a kernel that has yet to end
             self._queued = 0
         for g in self._graphs:
@@ -178,7 +214,7 @@ class Executable:
 
     def __del__(self):
         # runs that nobody waited for write to this object's host memory until they end
-        if getattr(self, "_queued", 0):
+        if getattr(self, "_queued", 0) or not getattr(self, "_whole", True):
             self.api.synchronize()
 
 
@@ -493,7 +529,7 @@ class HipAPI(BaseTensorAPI):
         self._run(prog.build)  # OR / variable leaf tables written on the device
         if self._entry_type == _lib.TO_F32S:
             self._upload(prog.recs, schedule.rec_init_bytes(prog))
-        self._upload(prog.params, np.array([0, total_slices, 0, 1], dtype=np.int64).tobytes())
+        self._upload(prog.params, Executable.counters(total_slices))
         self._upload(prog.accum, bytes(_lib.Accum()))
         if prog.host_accum is not None:
             ctypes.memset(prog.host_accum.data_ptr(), 0, ctypes.sizeof(_lib.Accum))

@@ -104,15 +104,13 @@ class RunEmulator(FoldEmulator):
             return emulator.Emulator.op_6(self, L)
         device = _lib.Launch.from_buffer_copy(bytes(L))
         device.iaux1 = 0
+        sums = self.heap.read_struct(_lib.Accum, L.aux2).pad  # written so far
         super().op_6(device)
         acc = self.heap.read_struct(_lib.Accum, L.aux2)
-        acc.pad += 1
-        raw = bytes(acc)
-        self.heap.view(L.aux2, "u1", len(raw))[:] = list(raw)
+        acc.pad = sums + bool(L.iaux1)
+        self.heap.view(L.aux2, "u1", ctypes.sizeof(acc))[:] = list(bytes(acc))
         if L.iaux1:
-            ctypes.memmove(L.iaux1, raw, len(raw))
-            if L.variant == 1 and acc.pad:
-                self.sums = getattr(self, "sums", 0) + 1
+            ctypes.memmove(L.iaux1, bytes(acc), ctypes.sizeof(acc))
 
     def op_8(self, L):
         self.heap.view(L.aux2, "u1", ctypes.sizeof(_lib.Accum))[:] = 0
