@@ -21,6 +21,7 @@ Device memory is allocated through PyTorch; the arithmetic runs only in the HIP 
 If the library or the GPU is missing, construction raises.
 """
 
+import contextlib
 import ctypes
 import math
 import threading
@@ -109,6 +110,8 @@ class Executable:
         # done: a run leaves it there, one cut short does not
         self._whole = True
         self._lent = False  # whether a caller has the launches, and may run them by itself
+        # whether the uploads that made the plan resident may still be under way
+        self._fresh = True
         self._sums = sum(L.op == _lib.TO_OP_ROOT_REDUCE for r in runs for L in r)
         for r in runs:
             if id(r) not in captured:
@@ -183,10 +186,12 @@ class Executable:
                                             self._word, ctypes.c_void_p(api._stream.cuda_stream)), "to_wait")
                 if acc.pad < self._word:
                     raise RuntimeError("the device is idle and has not written the sum")
-            self._queued = 0
+            if self._queued or self._lent:
+                self._queued, self._fresh = 0, False
             acc = _lib.Accum.from_buffer_copy(acc)
         else:
             api.synchronize()
+            self._fresh = False
             with api._torch.cuda.stream(api._stream):
                 acc_bytes = self.prog.accum[: ctypes.sizeof(_lib.Accum)].cpu().numpy().tobytes()
             acc = _lib.Accum.from_buffer_copy(acc_bytes)
@@ -203,18 +208,22 @@ class Executable:
         self.enqueue()
         return self.result()
 
+    def _in_flight(self):
+        """Whether the device may still write this object's memory."""
+        return bool(getattr(self, "_queued", 0) or getattr(self, "_fresh", False) or not getattr(self, "_whole", True))
+
     def close(self):
-        if self._graphs or self._queued or not getattr(self, "_whole", True):
+        if self._graphs or self._in_flight():
             self.api.synchronize()  # the sum's word is written by a kernel that has yet to end
-            self._queued = 0
+            self._queued, self._fresh = 0, False
         for g in self._graphs:
             self.api._lib.to_graph_destroy(g)
         self._graphs = []
         self._runs = [(None, launches) for _, launches in self._runs]
 
     def __del__(self):
-        # runs that nobody waited for write to this object's host memory until they end
-        if getattr(self, "_queued", 0) or not getattr(self, "_whole", True):
+        # runs, or uploads, that nobody waited for write to this object's memory until they end
+        if self._in_flight():
             self.api.synchronize()
 
 
@@ -231,7 +240,7 @@ class BatchExecutable:
         self.arena = arena
         self.count = sum(p.count for p in self.progs)
         self._graphs = []
-        self._queued = False
+        self._queued = True  # (the uploads that made the plans resident)
         if api._use_graph:
             for prog in self.progs:
                 arr = _lib.launch_array(prog.launches)
@@ -420,7 +429,17 @@ class HipAPI(BaseTensorAPI):
     # larger data go through a copy engine
     UPLOAD_BYTES = 12 * 1024
 
+    @contextlib.contextmanager
+    def _settled(self):
+        """Queued work is waited for before an exception drops the memory it uses."""
+        try:
+            yield
+        except BaseException:
+            self.synchronize()
+            raise
+
     def _upload(self, dst, host_bytes):
+        """Copy to the device in stream order: small data are still on their way on return."""
         n = len(host_bytes)
         if n <= self.UPLOAD_BYTES and n % 4 == 0:
             _lib.check(self._lib.to_upload(ctypes.c_void_p(dst.data_ptr()), ctypes.c_char_p(bytes(host_bytes)), n,
@@ -518,22 +537,25 @@ class HipAPI(BaseTensorAPI):
         if self._autotune:
             from . import autotune
 
-            if autotune.tune_plan(self, nodes, W, schedule.TUNED):
+            with self._settled():
+                tuned = autotune.tune_plan(self, nodes, W, schedule.TUNED)
+            if tuned:
                 autotune.save(schedule.TUNED)
 
     def _resident(self, prog, total_slices, once):
         """Upload a compiled plan; returns its ``Executable``."""
-        self._upload(prog.table, prog.table_host.tobytes())
-        self._upload(prog.coef, prog.coef_host.tobytes())
-        self._upload(prog.blob, prog.blob_host.tobytes())
-        self._run(prog.build)  # OR / variable leaf tables written on the device
-        if self._entry_type == _lib.TO_F32S:
-            self._upload(prog.recs, schedule.rec_init_bytes(prog))
-        self._upload(prog.params, Executable.counters(total_slices))
-        self._upload(prog.accum, bytes(_lib.Accum()))
-        if prog.host_accum is not None:
-            ctypes.memset(prog.host_accum.data_ptr(), 0, ctypes.sizeof(_lib.Accum))
-        return Executable(self, prog, total_slices, once)
+        with self._settled():
+            self._upload(prog.table, prog.table_host.tobytes())
+            self._upload(prog.coef, prog.coef_host.tobytes())
+            self._upload(prog.blob, prog.blob_host.tobytes())
+            self._run(prog.build)  # OR / variable leaf tables written on the device
+            if self._entry_type == _lib.TO_F32S:
+                self._upload(prog.recs, schedule.rec_init_bytes(prog))
+            self._upload(prog.params, Executable.counters(total_slices))
+            self._upload(prog.accum, bytes(_lib.Accum()))
+            if prog.host_accum is not None:
+                ctypes.memset(prog.host_accum.data_ptr(), 0, ctypes.sizeof(_lib.Accum))
+            return Executable(self, prog, total_slices, once)
 
     def _execute(self, tree, tables, num_groups, total_slices):
         exe = self._compile(tree, tables, num_groups, total_slices, once=True)
@@ -613,19 +635,20 @@ class HipAPI(BaseTensorAPI):
             raise OutOfMemoryError
         arena = self._alloc(max(max(batch.wave_arena_bytes(per, w) for w in waves), schedule.ALIGN))
         progs = []
-        for w in waves:
-            if folded:
-                prog = fold.compile_batch([per[i] for i in w], self._entry_type, self._alloc, arena, self._alloc_host)
-            else:
-                prog = batch.compile_batch(None, self._entry_type, self._alloc, regroup=self._regroup,
-                                           per=[per[i] for i in w], arena=arena)
-            self._upload(prog.table, prog.table_host.tobytes())
-            self._upload(prog.blob, prog.blob_host.tobytes())
-            self._run(prog.build)  # OR / variable leaf tables written on the device
-            if self._entry_type == _lib.TO_F32S:
-                self._upload(prog.recs, batch.rec_init_bytes(prog))
-            progs.append(prog)
-        return BatchExecutable(self, progs, arena)
+        with self._settled():
+            for w in waves:
+                if folded:
+                    prog = fold.compile_batch([per[i] for i in w], self._entry_type, self._alloc, arena, self._alloc_host)
+                else:
+                    prog = batch.compile_batch(None, self._entry_type, self._alloc, regroup=self._regroup,
+                                               per=[per[i] for i in w], arena=arena)
+                self._upload(prog.table, prog.table_host.tobytes())
+                self._upload(prog.blob, prog.blob_host.tobytes())
+                self._run(prog.build)  # OR / variable leaf tables written on the device
+                if self._entry_type == _lib.TO_F32S:
+                    self._upload(prog.recs, batch.rec_init_bytes(prog))
+                progs.append(prog)
+            return BatchExecutable(self, progs, arena)
 
     def contract_batch(self, plans):
         """Counts (floats) of many unsliced plans contracted together."""
@@ -684,11 +707,13 @@ class HipAPI(BaseTensorAPI):
     def tensordot(self, a, b, axes):
         """``numpy.tensordot(a, b, axes)`` on the device; result keeps numpy's axis
         order (left free axes, then right free axes)."""
-        A, B = self._to_device(a), self._to_device(b)
-        lmap, rmap = list(axes[0]), list(axes[1])
-        for (t, m) in ((A, lmap), (B, rmap)):
-            if any(d != 2 for d in t.shape):
+        for t in (a, b):
+            if any(d != 2 for d in (t.shape if isinstance(t, DeviceTensor) else np.shape(t))):
                 raise ValueError("HipAPI tensors must have all dimensions 2")
+        with self._settled():
+            return self._tensordot(self._to_device(a), self._to_device(b), list(axes[0]), list(axes[1]))
+
+    def _tensordot(self, A, B, lmap, rmap):
         g = schedule.join_geometry(A.rank, B.rank, lmap, rmap)
         g["var"] = schedule.choose_variant(g, 1, self._esize)
         out_rank = g["fx"] + g["fy"]
@@ -770,7 +795,10 @@ class HipAPI(BaseTensorAPI):
 
     def permute(self, tensor, perm):
         """Device ``numpy.transpose`` of an all-dimension-2 tensor (returns numpy)."""
-        A = self._to_device(tensor)
+        with self._settled():
+            return self._permute(self._to_device(tensor), perm)
+
+    def _permute(self, A, perm):
         out = self._alloc((1 << A.rank) * self._esize)
         p = (ctypes.c_int32 * max(1, len(perm)))(*perm)
         rc = self._lib.to_permute(ctypes.c_void_p(A.data.data_ptr()), ctypes.c_void_p(out.data_ptr()), A.rank,

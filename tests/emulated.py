@@ -125,7 +125,8 @@ class EmulatedAPI(hip_api.HipAPI):
         self._use_graph, self._regroup, self._autotune, self._device_leaves = False, True, False, True
         self._stream = types.SimpleNamespace(cuda_stream=0)
         self._torch = types.SimpleNamespace(cuda=types.SimpleNamespace(stream=lambda s: contextlib.nullcontext()))
-        self._lib = types.SimpleNamespace(to_wait=lambda *a: _lib.TO_OK)
+        self._lib = types.SimpleNamespace(to_wait=lambda *a: _lib.TO_OK, 
+                                          to_wall_clock_khz=lambda khz: setattr(khz._obj, "value", 1) or _lib.TO_OK)
         self.budget, self.waits, self.fail_at = 1 << 40, 0, None
 
     def _alloc(self, nbytes):
@@ -133,6 +134,13 @@ class EmulatedAPI(hip_api.HipAPI):
 
     def _alloc_host(self, nbytes):
         return _Host(nbytes)
+
+    def prepare_batch(self, plans):
+        self._alloc_host = self._alloc  # (a batch reads its accumulators as tensors)
+        try:
+            return super().prepare_batch(plans)
+        finally:
+            del self._alloc_host
 
     def _upload(self, dst, host_bytes):
         self.heap.write(dst, host_bytes)
