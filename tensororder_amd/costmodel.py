@@ -15,6 +15,7 @@ every candidate is an exact plan of the same network.
 import ctypes
 import math
 import os
+import threading
 
 import numpy as np
 
@@ -127,8 +128,8 @@ class CostModel:
         self.m = torch.zeros_like(self.params)
         self.v = torch.zeros_like(self.params)
         self.grad = torch.zeros_like(self.params)
-        # the loss of a step, in host memory that the device writes
-        self.loss = torch.zeros(1, dtype=torch.float32, pin_memory=True)
+        # the loss of a step, in host memory that the device writes, for each calling thread
+        self.losses = threading.local()
         self.step = 0
         self.x_mean = np.zeros(16, np.float32)
         self.x_std = np.ones(16, np.float32)
@@ -160,7 +161,9 @@ class CostModel:
         """(loss, gradient) on device data (normalised)."""
         n = xdev.shape[0]
         (h1, h2, y), (dh1, dh2, dy) = self._buffers(n), self._buffers(n)
-        loss = self.loss
+        loss = getattr(self.losses, "word", None)
+        if loss is None:
+            loss = self.losses.word = self.torch.zeros(1, dtype=self.torch.float32, pin_memory=True)
         rc = self.lib.to_mlp_gradient(*map(self._ptr, (self.params, xdev, tdev)), n,
                                       *map(self._ptr, (h1, h2, y, dy, dh2, dh1, self.grad, loss)), self._stream())
         _lib.check(rc, "to_mlp_gradient")
