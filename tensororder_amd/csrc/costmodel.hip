@@ -51,7 +51,7 @@ __global__ __launch_bounds__(kBlock) void k_forward(const float* __restrict__ pa
                                                     int64_t n, float* __restrict__ h1, float* __restrict__ h2,
                                                     float* __restrict__ y, const float* __restrict__ t,
                                                     float* __restrict__ dy, float* __restrict__ dh2,
-                                                    float* __restrict__ dh1) {
+                                                    float* __restrict__ dh1, float scale) {
     __shared__ float w1[TO_MLP_IN * 65], w2[TO_MLP_H1 * 65];
     for (int i = threadIdx.x; i < TO_MLP_H1 * TO_MLP_IN; i += kBlock)
         w1[(i % TO_MLP_IN) * 65 + i / TO_MLP_IN] = params[OFF_W1 + i];
@@ -92,7 +92,6 @@ __global__ __launch_bounds__(kBlock) void k_forward(const float* __restrict__ pa
 #pragma unroll
         for (int r = 0; r < kRows; ++r) b[r] += lane_value(a[r], k) * w;
     }
-    const float scale = 2.0f / (float)(n * TO_MLP_OUT);
     float g[kRows], d[kRows];
 #pragma unroll
     for (int r = 0; r < kRows; ++r) {
@@ -131,12 +130,11 @@ __global__ __launch_bounds__(kBlock) void k_backward_rows(const float* __restric
                                                           const float* __restrict__ h2, const float* __restrict__ y,
                                                           const float* __restrict__ t, int64_t n,
                                                           float* __restrict__ dy, float* __restrict__ dh2,
-                                                          float* __restrict__ dh1) {
+                                                          float* __restrict__ dh1, float scale) {
     __shared__ float w2[TO_MLP_H2 * TO_MLP_H1];
     for (int i = threadIdx.x; i < TO_MLP_H2 * TO_MLP_H1; i += kBlock) w2[i] = params[OFF_W2 + i];
     const int lane = threadIdx.x & 63;
     const float w30 = params[OFF_W3 + lane], w31 = params[OFF_W3 + TO_MLP_H2 + lane];
-    const float scale = 2.0f / (float)(n * TO_MLP_OUT);
     __syncthreads();
     const int64_t r0 = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6) * kRows;
     float g[kRows], a[kRows];
@@ -302,6 +300,19 @@ void launch_weight_grads(const float* x, const float* h1, const float* h2, const
                        ((reinterpret_cast<uintptr_t>(dh2) | reinterpret_cast<uintptr_t>(dh1)) & 15) == 0);
 }
 
+// The rows in launches of at most 2^26 (the threads of a launch are counted in 32 bits, 32 a row)
+template <typename F>
+void launch_rows(int64_t n, F launch) {
+    constexpr int64_t kMost = 1ll << 26;
+    for (int64_t r = 0; r < n; r += kMost) {
+        const int64_t m = n - r < kMost ? n - r : kMost;
+        launch(r, m, dim3((unsigned)((m + kRowsPerBlock - 1) / kRowsPerBlock)));
+    }
+}
+
+// dy = scale (y - target)
+float out_scale(int64_t n) { return 2.0f / (float)(n * TO_MLP_OUT); }
+
 }  // namespace
 
 extern "C" {
@@ -309,9 +320,10 @@ extern "C" {
 int to_mlp_forward(const float* params, const float* x, int64_t n, float* h1, float* h2, float* y, void* stream) {
     if (!params || !x || !h1 || !h2 || !y || n <= 0) return TO_ERR_INVALID;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    if (n > (int64_t)INT32_MAX * kRowsPerBlock) return TO_ERR_INVALID;
-    hipLaunchKernelGGL(k_forward<false>, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st,
-                       params, x, n, h1, h2, y, nullptr, nullptr, nullptr, nullptr);
+    launch_rows(n, [&](int64_t r, int64_t m, dim3 grid) {
+        hipLaunchKernelGGL(k_forward<false>, grid, dim3(kBlock), 0, st, params, x + r * TO_MLP_IN, m, h1 + r * TO_MLP_H1,
+                           h2 + r * TO_MLP_H2, y + r * TO_MLP_OUT, nullptr, nullptr, nullptr, nullptr, 0.0f);
+    });
     return status("to_mlp_forward");
 }
 
@@ -321,9 +333,11 @@ int to_mlp_backward(const float* params, const float* x, const float* h1, const 
     if (!params || !x || !h1 || !h2 || !y || !target || !dy || !dh2 || !dh1 || !grad || n <= 0)
         return TO_ERR_INVALID;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    if (n > (int64_t)INT32_MAX * kRowsPerBlock) return TO_ERR_INVALID;
-    hipLaunchKernelGGL(k_backward_rows, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st,
-                       params, h1, h2, y, target, n, dy, dh2, dh1);
+    launch_rows(n, [&](int64_t r, int64_t m, dim3 grid) {
+        hipLaunchKernelGGL(k_backward_rows, grid, dim3(kBlock), 0, st, params, h1 + r * TO_MLP_H1, h2 + r * TO_MLP_H2,
+                           y + r * TO_MLP_OUT, target + r * TO_MLP_OUT, m, dy + r * TO_MLP_OUT, dh2 + r * TO_MLP_H2,
+                           dh1 + r * TO_MLP_H1, out_scale(n));
+    });
     launch_weight_grads(x, h1, h2, y, target, n, dy, dh2, dh1, grad, loss, st);
     return status("to_mlp_backward");
 }
@@ -332,9 +346,11 @@ int to_mlp_gradient(const float* params, const float* x, const float* target, in
                     float* dy, float* dh2, float* dh1, float* grad, float* loss, void* stream) {
     if (!params || !x || !target || !h1 || !h2 || !y || !dy || !dh2 || !dh1 || !grad || n <= 0) return TO_ERR_INVALID;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    if (n > (int64_t)INT32_MAX * kRowsPerBlock) return TO_ERR_INVALID;
-    hipLaunchKernelGGL(k_forward<true>, dim3((unsigned)((n + kRowsPerBlock - 1) / kRowsPerBlock)), dim3(kBlock), 0, st,
-                       params, x, n, h1, h2, y, target, dy, dh2, dh1);
+    launch_rows(n, [&](int64_t r, int64_t m, dim3 grid) {
+        hipLaunchKernelGGL(k_forward<true>, grid, dim3(kBlock), 0, st, params, x + r * TO_MLP_IN, m, h1 + r * TO_MLP_H1,
+                           h2 + r * TO_MLP_H2, y + r * TO_MLP_OUT, target + r * TO_MLP_OUT, dy + r * TO_MLP_OUT,
+                           dh2 + r * TO_MLP_H2, dh1 + r * TO_MLP_H1, out_scale(n));
+    });
     launch_weight_grads(x, h1, h2, y, target, n, dy, dh2, dh1, grad, loss, st);
     return status("to_mlp_gradient");
 }

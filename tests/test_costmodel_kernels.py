@@ -58,3 +58,35 @@ def test_rows_and_alignment(n, shift):
     for got, ref in zip(outs + [G1, L1], (H1, H2, Y, DY, DH2, DH1, G, L)):
         np.testing.assert_allclose(got[shift:].cpu().numpy(), ref[shift:].cpu().numpy(), rtol=1e-5,
                                    atol=1e-6 * float(ref[shift:].abs().max()))
+
+
+def test_rows_beyond_one_launch():
+    # 2^27 rows and some: more threads, at 32 a row, than a launch counts
+    import torch
+
+    n = (1 << 27) + 11
+    free, _ = torch.cuda.mem_get_info()
+    if free < 340 * n + (8 << 30):
+        pytest.skip("needs %d GB of device memory" % (340 * n >> 30))
+    print("case mlp rows", n, flush=True)
+    lib = _lib.load()
+    rng = np.random.default_rng(0)
+    p = (rng.standard_normal(_lib.MLP_NPARAMS) * 0.3).astype(np.float32)
+    few = 64
+    x = rng.standard_normal((few, 16)).astype(np.float32)
+    P, X = torch.from_numpy(p).cuda(), torch.zeros((n, 16), dtype=torch.float32, device="cuda")
+    at = [0, (1 << 26) - few // 2, n - few]  # across the ends of the launches
+    for r in at:
+        X[r:r + few] = torch.from_numpy(x).cuda()
+    H1, H2 = (torch.empty((n, 64), dtype=torch.float32, device="cuda") for _ in range(2))
+    Y = torch.full((n, 2), float("nan"), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    _lib.check(lib.to_mlp_forward(*(ctypes.c_void_p(t.data_ptr()) for t in (P, X)), n,
+                                  *(ctypes.c_void_p(t.data_ptr()) for t in (H1, H2, Y)), None), "to_mlp_forward")
+    torch.cuda.synchronize()
+    _, _, want = mlp_oracle.forward(p.astype(np.float64), x)
+    for r in at:
+        np.testing.assert_allclose(Y[r:r + few].cpu().numpy(), want, rtol=1e-4, atol=1e-5)
+    assert not bool(torch.isnan(Y).any())
+    del X, H1, H2, Y
+    torch.cuda.empty_cache()
