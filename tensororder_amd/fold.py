@@ -89,6 +89,8 @@ LEVEL_FREE_BYTES = 256 << 20
 
 # bit b of lane l
 _LANE_BITS = ((np.arange(64)[None, :] >> np.arange(6)[:, None]) & 1).astype(np.uint32)
+# words of a product that hold the entries of its lane bits: operands 0-3, the result
+_LANE_ENTRIES = np.array([at + b for at in (64, 80, 96, 112, 32) for b in range(6)])
 _HEAD = struct.Struct("<QQQqqqQQQqqQ10i")
 _BITS = struct.Struct("<%dI" % (3 * _lib.FOLD_BITS))
 
@@ -118,7 +120,7 @@ class FNode:
     holds it on several axes); 2^rank entries are stored."""
 
     __slots__ = ("idx", "is_leaf", "tensor", "rank", "order", "order0", "want", "off", "batched", "left", "right", "parent",
-                 "ksum", "geom", "buf", "ptr", "bstride", "rec", "rec_stride")
+                 "ksum", "geom", "buf", "ptr", "bstride", "rec", "rec_stride", "layout")
 
     def __init__(self, idx):
         self.idx = idx
@@ -127,6 +129,7 @@ class FNode:
         self.buf = None
         self.rec = None
         self.rec_stride = 0
+        self.layout = None  # at the root: the plan's layout, while the joins' forms are its own
 
 
 class _T:
@@ -471,6 +474,7 @@ def choose(n, nodes, W, esize, launch_bound=False):
 
 
 def choose_all(nodes, W, esize, launch_bound=False):
+    nodes[-1].layout = None
     for n in nodes:
         n.want = None
     for n in nodes:
@@ -765,8 +769,7 @@ def tree_words(p, nodes, waves, rec_index, one):
             m[-1] |= _lib.TO_TREE_MEET
             streams[w] += m
     # every lane's offset: the sum of the entries of its bits, for operands 0-3 and the result
-    entries = words[:, [64 + 16 * j + b for j in range(4) for b in range(6)] + [32 + b for b in range(6)]]
-    words[:, 128:] = (entries.reshape(-1, 5, 6) @ _LANE_BITS).reshape(-1, 5 * 64)
+    words[:, 128:] = (words[:, _LANE_ENTRIES].reshape(-1, 5, 6) @ _LANE_BITS).reshape(-1, 5 * 64)
     return words, np.array(streams, dtype=np.uint32)
 
 
@@ -829,18 +832,32 @@ def plan_memory(nodes, W, esize, order, programs=()):
 
 
 def choose_order(nodes, W, esize, programs=()):
-    level, _ = plan_memory(nodes, W, esize, "level", programs)
+    """(order, arena peak, scratch placements): level launches unless they take far more
+    memory."""
+    level, scratch = plan_memory(nodes, W, esize, "level", programs)
     if level <= LEVEL_FREE_BYTES:
-        return "level", level
-    post, _ = plan_memory(nodes, W, esize, "post", programs)
+        return "level", level, scratch
+    post, scratch = plan_memory(nodes, W, esize, "post", programs)
     if level <= schedule.LEVEL_PEAK_FACTOR * post:
-        return "level", level
-    return "post", post
+        return "level", *plan_memory(nodes, W, esize, "level", programs)
+    return "post", post, scratch
+
+
+def lay_out(nodes, W, esize, group_levels=True):
+    """Forms, programs and memory plan of a folded plan for W slices: (programs, order, arena
+    peak, scratch placements)."""
+    choose_all(nodes, W, esize)
+    if not group_levels:
+        return [], "post", *plan_memory(nodes, W, esize, "post", [])
+    programs = tree_programs(nodes, W, esize, esize == 4)
+    return programs, *choose_order(nodes, W, esize, programs)
 
 
 def peak_bytes(nodes, W, esize):
-    choose_all(nodes, W, esize)
-    return choose_order(nodes, W, esize, tree_programs(nodes, W, esize, esize == 4))[1]
+    """Arena bytes for W slices; the layout stays with the plan for ``compile_program``."""
+    layout = lay_out(nodes, W, esize)
+    nodes[-1].layout = (W, esize), layout
+    return layout[2]
 
 
 def join_records(n, nodes, W, esize, scaled, abase, scratch, recp, one, launch_bound=False):
@@ -992,10 +1009,12 @@ def compile_program(folded, tables, num_groups, entry_type, W, device_alloc, gro
     scaled = entry_type == _lib.TO_F32S
     prog = schedule.Program()
     prog.nbatch, prog.nodes = W, nodes
-    choose_all(nodes, W, esize)
-    programs = tree_programs(nodes, W, esize, scaled) if group_levels else []
-    order = choose_order(nodes, W, esize, programs)[0] if group_levels else "post"
-    peak, scratch = plan_memory(nodes, W, esize, order, programs)
+    # (the layout that the batch size was accepted with, if the joins' forms are still its own)
+    known, nodes[-1].layout = nodes[-1].layout, None
+    if group_levels and known is not None and known[0] == (W, esize):
+        programs, order, peak, scratch = known[1]
+    else:
+        programs, order, peak, scratch = lay_out(nodes, W, esize, group_levels)
     prog.programs = programs
     in_lds = {i for p in programs for i in p.members if i != p.root}
     prog.arena_bytes, prog.order = peak, order

@@ -521,7 +521,8 @@ class HipAPI(BaseTensorAPI):
         folded = fold.analyse(tree, tables, self._esize, self._regroup) if fold.has_copies(tables) else None
         W = self.choose_folded_batch(folded, tree, tables, total_slices) if folded is not None else 0
         if W:
-            self._tune(folded[0], W)
+            if self._tune(folded[0], W):
+                folded[0][-1].layout = None  # (laid out with the shapes known before)
             prog = fold.compile_program(folded, tables, num_groups, self._entry_type, W, self._alloc, group_levels,
                                         self._alloc_host)
             return self._resident(prog, total_slices, once)
@@ -533,14 +534,17 @@ class HipAPI(BaseTensorAPI):
         return self._resident(prog, total_slices, once)
 
     def _tune(self, nodes, W):
-        """Time the launch shapes that a plan is the first to need (``autotune`` option)."""
-        if self._autotune:
-            from . import autotune
+        """Time the launch shapes that a plan is the first to need (``autotune`` option); returns
+        how many."""
+        if not self._autotune:
+            return 0
+        from . import autotune
 
-            with self._settled():
-                tuned = autotune.tune_plan(self, nodes, W, schedule.TUNED)
-            if tuned:
-                autotune.save(schedule.TUNED)
+        with self._settled():
+            tuned = autotune.tune_plan(self, nodes, W, schedule.TUNED)
+        if tuned:
+            autotune.save(schedule.TUNED)
+        return tuned
 
     def _resident(self, prog, total_slices, once):
         """Upload a compiled plan; returns its ``Executable``."""

@@ -4,6 +4,7 @@ to the same count wherever the cuts lie."""
 import numpy as np
 import pytest
 import test_fold
+from emulated import EmulatedAPI
 
 from oracle import numpy_oracle
 from tensororder_amd import _lib, fold, network, plan_io, planners, schedule
@@ -117,3 +118,34 @@ def test_programs_hold_no_more_products_than_a_task_names(most, et, tol, monkeyp
     monkeypatch.setattr(fold, "TREE_PRODUCTS", 0)
     with pytest.raises(ValueError):
         fold.tree_words(programs[0], nodes, 16, lambda n: 0, (0, 0))
+
+
+@pytest.mark.parametrize("et,tol", [(_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)])
+def test_the_layout_of_the_accepted_batch_is_compiled(et, tol, monkeypatch):
+    # forms and programs are made once for each batch size tried, and are those of the last
+    plan = test_fold._formula_plan("cnf", 16, 1, 6)
+    want = numpy_oracle.contract_sliced(plan_io.plan_to_dict(plan))
+    made, seen = [], set()
+    inner = fold.choose_all
+    monkeypatch.setattr(fold, "choose_all", lambda nodes, W, *a: made.append(W) or inner(nodes, W, *a))
+    for share in (1.0, 0.6, 0.3):
+        api = EmulatedAPI(et)
+        total, tree, tables, groups = api._plan_inputs(plan, None)
+        esize = api._esize
+        nodes = fold.analyse(tree, tables, esize)[0]
+        fixed = sum(t.size for t in tables.values()) * esize
+        one = schedule.peak_bytes(schedule.analyse(tree, tables), tables, 1, et)  # (below, it is refused)
+        api.budget = fixed + max(int(share * fold.peak_bytes(nodes, 64, esize)), one)
+        made.clear()
+        exe = api.prepare(plan)
+        assert made == sorted(made, reverse=True) and len(set(made)) == len(made)
+        assert made[0] == 64 and exe.prog.nbatch == made[-1]
+        seen.add(made[-1])
+        assert exe.run().value == pytest.approx(want, rel=tol, abs=0)
+    assert len(seen) > 1
+    # a shape tuned in between is a new layout
+    api = EmulatedAPI(et)
+    api._tune = lambda nodes, W: 1
+    made.clear()
+    assert api.contract_sliced(plan) == pytest.approx(want, rel=tol, abs=0)
+    assert made == [64, 64]
