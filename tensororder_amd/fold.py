@@ -152,9 +152,12 @@ def has_copies(tables):
     return bool(copies) and not any(t.rank if sum(map(bool, t.coef)) == 1 else t.batched for t in copies)
 
 
+# 2.0^n of n variables (a plan of far more is refused for its memory)
+_POWERS = [2.0 ** n for n in range(900)]
+
+
 def _power(n):
-    """2.0^n, for any number n of variables (a plan far too large is refused for its memory)."""
-    return 2.0 ** min(n, 900)
+    return _POWERS[n if n < 900 else -1]
 
 
 def _join_cost(left, right, union, out, batched, esize):
@@ -169,45 +172,46 @@ def _join_cost(left, right, union, out, batched, esize):
 def analyse(tree, tables, esize, regroup=True):
     """(post-order FNode list, number of variables no remaining leaf holds -- each doubles the
     count) of a plan, or None when no leaf would remain."""
-    flat = schedule.flatten_tree(tree)
-    if flat[-1].rank != 0:
+    # the tree's nodes, children before parents
+    flat, inner, todo = [], tree.context.nodes, [tree.node_id]
+    while todo:  # (each after what is to its right, then turned round)
+        t = inner[todo.pop()]
+        flat.append(t)
+        if not t.is_leaf:
+            todo += (t.left, t.right)
+    flat.reverse()
+    if flat[-1].free_edges:
         raise ValueError("the tree's root has free edges; only full contractions are supported")
+    leaves = [(i, tables[n.tensor_index], n.free_edges) for i, n in enumerate(flat) if n.is_leaf]
     root = {}
 
     def find(e):
         while root.setdefault(e, e) != e:
-            e = root[e]
+            root[e] = e = root[root[e]]
         return e
 
-    for n in flat:
-        if not n.is_leaf:
-            continue
-        t = tables[n.tensor]
-        if t.rank != n.rank:
-            raise ValueError("leaf %d: table rank %d != tree rank %d" % (n.tensor, t.rank, n.rank))
+    for i, t, free in leaves:
+        if t.rank != len(free):
+            raise ValueError("leaf %d: table rank %d != tree rank %d" % (flat[i].tensor_index, t.rank, len(free)))
         if t.copy is not None:
-            for e in n.free:
-                root[find(e)] = find(n.free[0])
-        else:
-            for e in n.free:
-                find(e)
+            for e in free:
+                root[find(e)] = find(free[0])
 
     # leaves: variable -> offset mask in the leaf's own table
     offs, weights, hosts = {}, [], []
-    seen = set()
-    for n in flat:
-        if not n.is_leaf:
-            continue
-        off = {}
-        for a, e in enumerate(n.free):
+    seen, sliced = set(), {}
+    for i, t, free in leaves:
+        off, bit = {}, 1 << len(free)
+        for e in free:
+            bit >>= 1
             v = find(e)
-            off[v] = off.get(v, 0) | 1 << (n.rank - 1 - a)
+            off[v] = off.get(v, 0) | bit
         seen.update(off)
-        t = tables[n.tensor]
         if t.copy is not None and t.copy[2] and t.copy[0] == 1 and t.copy[1] == 1:
             continue  # a vector of ones
-        offs[n.idx] = off
-        (weights if len(off) <= 1 else hosts).append(n.idx)
+        offs[i] = off
+        sliced[i] = t.batched
+        (weights if len(off) <= 1 else hosts).append(i)
     # weight vectors (and scalars) multiply one leaf that holds their variable: an unsliced
     # one where possible, so that the product is not repeated per slice
     attach, placed = {}, set()
@@ -220,10 +224,9 @@ def analyse(tree, tables, esize, regroup=True):
         for v in offs[h]:
             by_var.setdefault(v, []).append(h)
     for w in weights:
-        bw = tables[flat[w].tensor].batched
         cand = by_var.get(next(iter(offs[w])), []) if offs[w] else hosts
         if cand:
-            h = min(cand, key=lambda i: (tables[flat[i].tensor].batched != bw, host_key(i)))
+            h = min(cand, key=lambda i: (sliced[i] != sliced[w], host_key(i)))
             attach.setdefault(h, []).append(w)
             placed.add(w)
 
@@ -243,16 +246,16 @@ def analyse(tree, tables, esize, regroup=True):
         return _T(None, out, left, right, batched, union, _join_cost(left, right, union, len(out), batched, esize))
 
     def leaf(i):
-        return _T(i, {v: 1 for v in offs[i]}, batched=tables[flat[i].tensor].batched)
+        return _T(i, {v: 1 for v in offs[i]}, batched=sliced[i])
 
     stack = []
-    for n in flat:
+    for i, n in enumerate(flat):
         if n.is_leaf:
-            if n.idx not in offs or n.idx in placed:
+            if i not in offs or i in placed:
                 stack.append(None)
                 continue
-            t = leaf(n.idx)
-            for w in sorted(attach.get(n.idx, []), key=lambda i: (tables[flat[i].tensor].batched, i)):
+            t = leaf(i)
+            for w in sorted(attach.get(i, []), key=lambda i: (sliced[i], i)):
                 t = join(t, leaf(w))
             stack.append(t)
             continue
@@ -292,8 +295,8 @@ def analyse(tree, tables, esize, regroup=True):
         n.batched = t.batched
         n.left = n.right = -1
         if n.is_leaf:
-            n.tensor = flat[t.leaf].tensor
-            n.rank = flat[t.leaf].rank
+            n.tensor = flat[t.leaf].tensor_index
+            n.rank = len(flat[t.leaf].free_edges)
             n.off = offs[t.leaf]
         else:
             n.left, n.right = index[id(t.left)], index[id(t.right)]
@@ -325,8 +328,9 @@ def analyse(tree, tables, esize, regroup=True):
         if n.right >= 0:
             for v in min(nodes[n.left].order, nodes[n.right].order, key=len):
                 weight[v] = weight.get(v, 0.0) + _power(len(held))
+    place = {v: i for i, v in enumerate(sorted(when, key=lambda v: (-when[v], weight.get(v, 0.0), v)))}
     for n in nodes:
-        n.order.sort(key=lambda v: (-when[v], weight.get(v, 0.0), v))
+        n.order.sort(key=place.__getitem__)
         n.order0 = n.order
     return nodes, missing
 
@@ -386,9 +390,9 @@ def choose(n, nodes, W, esize, launch_bound=False):
     xoff = X.off
     yoff = Y.off if Y is not None else {}
     # shared range in X's memory order, lowest first
-    ks = sorted(n.ksum, key=lambda v: (xoff.get(v, 1 << 40), yoff.get(v, 0), v))
+    ks = sorted(n.ksum, key=lambda v: (xoff.get(v, 1 << 40), yoff.get(v, 0), v)) if len(n.ksum) > 1 else list(n.ksum)
     s = len(ks)
-    if Y is not None and all(v in xoff and v in yoff for v in ks):
+    if Y is not None and n.rank >= 2 * schedule.GEMM_MIN_FREE and all(v in xoff and v in yoff for v in ks):
         kept = [v for v in n.order if v in xoff and v in yoff]
         xo = [v for v in n.order if v in xoff and v not in yoff]
         yo = [v for v in n.order if v in yoff and v not in xoff]
@@ -423,7 +427,7 @@ def choose(n, nodes, W, esize, launch_bound=False):
     # the 16-byte form, streaming the operand that has the outputs' two lowest variables as its
     # own: the larger one, else the other (2^16 by 2^16 over 2^3 to 2^20, 4096 slices: 6.4 ms as
     # a register tile with 4-byte stores, 5.7 here)
-    for x, y in ((X, Y), (Y, X)) if Y is not None else ():
+    for x, y in ((X, Y), (Y, X)) if Y is not None and nc >= 10 else ():
         v = _vec_form(x.off, y.off, x.rank, y.rank, out, n.off, n.ksum, nb, launch_bound)
         if v is not None:
             n.geom = dict(fx=nc - v["fy"], fy=v["fy"], s=s, X=x.idx, Y=y.idx, var=v)
@@ -432,7 +436,7 @@ def choose(n, nodes, W, esize, launch_bound=False):
     g = dict(fx=nc - len(yonly), fy=len(yonly), s=s, X=X.idx, Y=Y.idx if Y is not None else -1)
     # register tile: outputs enough to fill the chip without the tile's bits
     xonly = [v for v in out if v not in yoff]
-    for na, nbits in REG_TILES if Y is not None else ():
+    for na, nbits in REG_TILES if Y is not None and nc >= 10 else ():
         if len(xonly) < na or len(yonly) < nbits or nc - na - nbits < 8 or lognb + nc - na - nbits < REG_MIN_LOG:
             continue
         # the tile's variables: the highest bits of the result, so that the lanes keep low ones
@@ -662,24 +666,34 @@ def tree_programs(nodes, W, esize, scaled, lds=None):
         while k < len(joins):
             n = joins[k]
             i, cut = n.idx, n.idx in full
-            below = [c for c in (n.left, n.right) if c in depth and nodes[c].batched == n.batched]
-            # a block reads a large tensor of another launch at the latency of L2: fewer products
-            far = any(c >= 0 and nodes[c].rank > TREE_FAR_RANK and
-                      (cut or c not in stage or nodes[c].batched != n.batched) for c in (n.left, n.right))
+            below, far, deep = [], False, 0
+            for c in (n.left, n.right):
+                if c >= 0:
+                    near = nodes[c].batched == n.batched
+                    # a block reads a large tensor of another launch at the latency of L2: fewer products
+                    far = far or nodes[c].rank > TREE_FAR_RANK and (cut or not near or c not in stage)
+                    if near and c in depth:
+                        below.append(c)
+                        deep = max(deep, depth[c])
             small = n.geom["var"]["kind"] == "fold" and n.rank <= TREE_RANK and \
                 len(n.ksum) + n.rank <= (TREE_FAR_BITS if far else TREE_BITS)
-            depth[i] = max([depth[c] for c in below], default=0) + (cut or not small)
-            stage.pop(i, None)
+            if cut or not small:
+                deep += 1
+            depth[i] = deep
             k += 1
             if not small:
+                stage.pop(i, None)
                 continue
-            stage[i] = (n.batched, depth[i])
-            mine = [c for c in below if stage.get(c) == stage[i]]
-            size[i] = 1 + sum(size[c] for c in mine)
-            sure[i] = max([sure[c] for c in mine], default=1)
+            stage[i] = mine = (n.batched, deep)
+            held, known = 1, 1
+            for c in below:
+                if stage.get(c) == mine:
+                    held += size[c]
+                    known = max(known, sure[c])
+            size[i], sure[i] = held, known
             # (long ones are checked where they have doubled, so that a join is looked at a few
             # times in all; the others where they end)
-            if size[i] > max(TREE_LONG, 2 * sure[i]) and fits(i) is None:
+            if held > TREE_LONG and held > 2 * known and fits(i) is None:
                 j = first_full(i)
                 full.add(j)
                 k = at[j]
@@ -703,7 +717,7 @@ def _tree_task(n, ksum, operands):
     def key(v):
         return tuple(t.off.get(v, 1 << 40) for t in operands) + (v,)
 
-    ks = sorted(ksum, key=key)
+    ks = sorted(ksum, key=key) if len(ksum) > 1 else list(ksum)
     nc, s = n.rank, len(ks)
     lo = min(nc, 6)
     lk = max(0, min(s - 2, 6 - lo))

@@ -319,8 +319,10 @@ def leaf_spec_table(tensor, lookup, ngroups):
     (``tensor.py:95-119``); None for other leaves."""
     from .network import OrTensor, VariableTensor
 
+    copy = None
     if isinstance(tensor, VariableTensor):
         w_neg, w_pos = tensor.weights
+        copy = (w_neg, w_pos, tensor.rank > 0)
         kind, kw = _lib.TO_LEAF_VAR, dict(w_neg=w_neg, w_pos=w_pos)
     elif isinstance(tensor, OrTensor):
         kind, kw = _lib.TO_LEAF_OR, dict(positive=tensor.literals_positive, output_index=tensor.output_index)
@@ -335,7 +337,7 @@ def leaf_spec_table(tensor, lookup, ngroups):
         coef[lookup[i]] += offset
         offset *= 2
     spec = schedule.LeafSpec(kind, rank, sliced + unsliced, **kw)
-    return schedule.LeafTable(None, coef, len(unsliced), spec, copy=copy_weights(tensor))
+    return schedule.LeafTable(None, coef, len(unsliced), spec, copy=copy)
 
 
 class HipAPI(BaseTensorAPI):

@@ -770,12 +770,15 @@ def analyse(tree, tables, regroup=True):
 def peak_bound(tree, esize):
     """An upper bound of the arena peak of one slice: every tensor and every join's scratch
     (permuted operands, partial sums) at once."""
-    total = 0
-    for t in tree.iterate_postorder():
+    total, nodes, todo = 0, tree.context.nodes, [tree.node_id]
+    while todo:
+        t = nodes[todo.pop()]
+        rank = len(t.free_edges)
         # the tensor itself and, as an operand, its permuted copy
-        total += 2 * max(ALIGN, esize << len(t.free_edges))
+        total += 2 * max(ALIGN, esize << rank)
         if not t.is_leaf:  # partial sums: at most 4096, or one per output
-            total += 8 * max(4096, 1 << len(t.free_edges))
+            total += 8 * max(4096, 1 << rank)
+            todo += (t.left, t.right)
     return total
 
 
