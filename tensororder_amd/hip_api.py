@@ -179,7 +179,7 @@ class Executable:
             if not self._whole:
                 raise RuntimeError("the last run was cut short while it was queued")
             acc = self._host_sum()
-            if self._lent:  # (launches that a caller runs count in the word too)
+            if self._lent or not self._sums:  # (launches that a caller runs count in the word too)
                 api.synchronize()
             elif self._queued:
                 _lib.check(api._lib.to_wait(ctypes.c_void_p(ctypes.addressof(acc) + _lib.Accum.pad.offset),

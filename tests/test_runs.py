@@ -67,6 +67,14 @@ def test_runs_between_launches_of_a_caller(et, tol):
     assert exe.result().value == pytest.approx(want, rel=tol)
 
 
+def test_runs_of_no_slices():
+    # no sum ends such a run: its prologue is waited for
+    plan, _ = _plan()
+    api = EmulatedAPI()
+    exe = api.prepare(plan, 0)
+    assert exe.nwaves == 0 and exe.run().value == 0.0 and api.waits == 1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("graph", [True, False])
 def test_runs_after_one_cut_short_on_the_device(graph, monkeypatch):
