@@ -130,6 +130,7 @@ class CostModel:
         self.grad = torch.zeros_like(self.params)
         # the loss of a step, in host memory that the device writes, for each calling thread
         self.losses = threading.local()
+        self._loss_word()
         self.step = 0
         self.x_mean = np.zeros(16, np.float32)
         self.x_std = np.ones(16, np.float32)
@@ -141,6 +142,12 @@ class CostModel:
 
     def _stream(self):
         return ctypes.c_void_p(self.api._stream.cuda_stream)
+
+    def _loss_word(self):
+        loss = getattr(self.losses, "word", None)
+        if loss is None:
+            loss = self.losses.word = self.torch.zeros(1, dtype=self.torch.float32, pin_memory=True)
+        return loss
 
     def _buffers(self, n):
         torch, dev = self.torch, self.api._device
@@ -161,9 +168,7 @@ class CostModel:
         """(loss, gradient) on device data (normalised)."""
         n = xdev.shape[0]
         (h1, h2, y), (dh1, dh2, dy) = self._buffers(n), self._buffers(n)
-        loss = getattr(self.losses, "word", None)
-        if loss is None:
-            loss = self.losses.word = self.torch.zeros(1, dtype=self.torch.float32, pin_memory=True)
+        loss = self._loss_word()
         rc = self.lib.to_mlp_gradient(*map(self._ptr, (self.params, xdev, tdev)), n,
                                       *map(self._ptr, (h1, h2, y, dy, dh2, dh1, self.grad, loss)), self._stream())
         _lib.check(rc, "to_mlp_gradient")

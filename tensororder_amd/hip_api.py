@@ -716,8 +716,11 @@ class HipAPI(BaseTensorAPI):
         for t in (a, b):
             if any(d != 2 for d in (t.shape if isinstance(t, DeviceTensor) else np.shape(t))):
                 raise ValueError("HipAPI tensors must have all dimensions 2")
-        with self._settled():
+        try:
             return self._tensordot(self._to_device(a), self._to_device(b), list(axes[0]), list(axes[1]))
+        except BaseException:
+            self.synchronize()  # (see _settled, which would take 2 us of a small join)
+            raise
 
     def _tensordot(self, A, B, lmap, rmap):
         g = schedule.join_geometry(A.rank, B.rank, lmap, rmap)
