@@ -108,10 +108,13 @@ class FoldDesc:
 
 class TooWide(ValueError):
     """A join over more variables, or of a larger tensor, than a descriptor holds (offsets are
-    32 bits): the plan runs edge by edge."""
+    32 bits), or more exponents than a program adds up: the plan runs edge by edge."""
 
 
 OFFSET_BITS = 32
+# nodes of an FP32-scaled plan: a program keeps its tensors' exponents in 32 bits, and a node adds
+# less than 2^11 to them (a leaf's table lies between 2^-1074 and 2^1024)
+EXPONENT_NODES = 1 << 20
 
 
 class FNode:
@@ -479,6 +482,8 @@ def choose(n, nodes, W, esize, launch_bound=False):
 
 def choose_all(nodes, W, esize, launch_bound=False):
     nodes[-1].layout = None
+    if esize == 4 and len(nodes) > EXPONENT_NODES:
+        raise TooWide("more than %d nodes" % EXPONENT_NODES)
     for n in nodes:
         n.want = None
     for n in nodes:

@@ -108,3 +108,20 @@ def test_tensors_beyond_32_bit_offsets_run_edge_by_edge(esize):
                     for record in fold.join_records(t, nodes, 1, esize, False, 0, scratch, lambda n: 0, (0, 0)):
                         assert bytes(record[4])
     assert 32 in seen and max(seen) > 32
+
+
+def test_exponents_of_programs_fit(monkeypatch):
+    # a program's records hold 32-bit exponents, to which a node adds less than 2^11
+    assert fold.EXPONENT_NODES * 2 ** 11 <= 2 ** 31
+    plan = _plan(12, 0)
+    want = numpy_oracle.contract_sliced(plan_io.plan_to_dict(plan))
+    for et, folds in ((_lib.TO_F64, True), (_lib.TO_F32S, False)):
+        api = EmulatedAPI(et)
+        _, tree, tables, _ = api._plan_inputs(plan, None)
+        nodes = fold.analyse(tree, tables, api._esize)[0]
+        for most, fits in ((len(nodes), True), (len(nodes) - 1, folds)):
+            monkeypatch.setattr(fold, "EXPONENT_NODES", most)
+            assert (fold.analyse_batch([(tree, tables)], api._esize) is not None) == fits
+            exe = api.prepare(plan)
+            assert (exe.prog.host_accum is not None) == fits  # (the walk's sums stay on the device)
+            assert exe.run().value == pytest.approx(want, rel=1e-6)
