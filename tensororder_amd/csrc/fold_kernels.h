@@ -221,9 +221,10 @@ __global__ __launch_bounds__(kBlock) void k_fold_any(const to_fold_desc* __restr
 // Register tile: a thread owns the 2^A by 2^B outputs of A variables only X has and B only Y
 // has, and loads 2^A + 2^B entries for their products; the lanes run along the lowest other
 // variables of the result.  For the joins of two mid-sized tensors each of which has one of the
-// result's two lowest variables alone, so that neither streams in the 16-byte form: the
-// one-output form loads two entries a product (4096 slices of 2^16 by 2^16 over 2^3 to 2^20:
-// 42 ms, 6.2 as tiles, 5.7 in the 16-byte form, which takes that join).
+// result's two lowest variables alone, so that neither streams in the 16-byte form, where the
+// one-output form loads two entries a product.  Scaled floats, one-output form / tile: 4096 slices
+// of 2^8 by 2^6 over 2 to 2^12 95 / 19 us; 64 of 2^16 by 2^13 over 2^2 to 2^20 631 / 84; 1024 of
+// 2^14 by 2^11 over 2^3 to 2^16 544 / 112; 256 of 2^16 by 2^14 over 2^8 to 2^13 181 / 73.
 template <typename T, bool SCALED, int A, int B>
 __global__ __launch_bounds__(kBlock) void k_fold_reg(const to_fold_desc* __restrict__ descs, int ndesc, const int32_t* __restrict__ bmap) {
     constexpr int NX = 1 << A, NY = 1 << B;
@@ -574,7 +575,8 @@ __global__ __launch_bounds__(kBlock) void k_fold_pair(const to_pair_desc* __rest
 // fetched while the wave works on the join before it, and the joins that need no more than one
 // round of four products per lane (nearly all) run straight through: 0.7 us per level in
 // float64, 1.1 us scaled (a chain of 64 joins; 1.2 and 1.6 us at 2^10 outputs), against 3-5 us
-// for a launch.  The n = 90 vertex cover's 224 joins are 10 levels of one block, 32 us where
+// for a launch; a product of 3 or 4 tensors, scaled by its own maximum, 0.07 us more (2 x 2
+// matrices in a chain: 1.35 -> 1.43 us a level).  The n = 90 vertex cover's 224 joins are 10 levels of one block, 32 us where
 // their launches took 450.  Tried: deposits computed per join instead of fetched lane offsets
 // (twice the time of a level), one generic-pointer loop for every sum (long sums 1.6x), the
 // maximum by LDS atomics of all lanes (+2 us per level of 64 outputs).
