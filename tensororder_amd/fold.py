@@ -218,19 +218,18 @@ def analyse(tree, tables, esize, regroup=True):
     # weight vectors (and scalars) multiply one leaf that holds their variable: an unsliced
     # one where possible, so that the product is not repeated per slice
     attach, placed = {}, set()
-
-    def host_key(i):
-        return (len(offs[i]), i)
-
-    by_var = {}
+    by_var, best = {}, {}  # leaves by variable; the one taken, by variable (None: any) and slicing
     for h in hosts:
         for v in offs[h]:
             by_var.setdefault(v, []).append(h)
     for w in weights:
-        cand = by_var.get(next(iter(offs[w])), []) if offs[w] else hosts
+        v = next(iter(offs[w]), None)
+        cand = hosts if v is None else by_var.get(v)
         if cand:
-            h = min(cand, key=lambda i: (sliced[i] != sliced[w], host_key(i)))
-            attach.setdefault(h, []).append(w)
+            key = v, sliced[w]
+            if key not in best:
+                best[key] = min(cand, key=lambda i: (sliced[i] != sliced[w], len(offs[i]), i))
+            attach.setdefault(best[key], []).append(w)
             placed.add(w)
 
     total = {}

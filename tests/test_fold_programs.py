@@ -149,3 +149,23 @@ def test_the_layout_of_the_accepted_batch_is_compiled(et, tol, monkeypatch):
     made.clear()
     assert api.contract_sliced(plan) == pytest.approx(want, rel=tol, abs=0)
     assert made == [64, 64]
+
+
+def test_analysis_of_many_weights_is_linear(monkeypatch):
+    # weights of variables that no clause holds are scalars, and multiply one leaf: which one is
+    # looked for once, not among all leaves for each
+    n = 1200
+    lines = ["p cnf %d %d" % (2 * n, n - 1)] + ["%d %d 0" % (i, i + 1) for i in range(1, n)]
+    lines += ["w %d 0.25" % i for i in range(1, 2 * n + 1)]
+    net = network.cnf_count(parse_dimacs_text("\n".join(lines) + "\n", "cachet"))
+    tree, tables = test_fold.plan_inputs(planners.best_plan(net, "line", solver=None, seed=0))[1:3]
+    compared = [0]
+
+    def counted(values, *args, **kw):
+        values = list(values)
+        compared[0] += len(values)
+        return min(values, *args, **kw)
+
+    monkeypatch.setattr(fold, "min", counted, raising=False)
+    nodes, _ = fold.analyse(tree, tables, 8)
+    assert len(nodes) > 2 * n and compared[0] < 40 * len(nodes)
