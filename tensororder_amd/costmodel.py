@@ -198,7 +198,8 @@ class CostModel:
             tot, cnt = 0.0, 0
             for s in range(0, n, batch):
                 idx = order[s:s + batch]
-                xb, yb = xd.index_select(0, idx).contiguous(), yd.index_select(0, idx).contiguous()
+                with torch.cuda.stream(self.api._stream):  # (the kernels that read them run there)
+                    xb, yb = xd.index_select(0, idx).contiguous(), yd.index_select(0, idx).contiguous()
                 loss, _ = self.gradient(xb, yb)
                 self.adam_step(lr)
                 tot += loss * len(idx)

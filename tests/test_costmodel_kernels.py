@@ -60,6 +60,40 @@ def test_rows_and_alignment(n, shift):
                                    atol=1e-6 * float(ref[shift:].abs().max()))
 
 
+def test_training_rows_are_there_when_they_are_read():
+    # the rows of a batch are gathered where the kernels that read them run, not on the caller's
+    # stream, which may be busy
+    import torch
+
+    from tensororder_amd import costmodel
+    from tensororder_amd.hip_api import HipAPI
+
+    rng = np.random.default_rng(1)
+    x = rng.standard_normal((600, 16))
+    y = np.stack([x[:, 0] + x[:, 1], x[:, 2]], axis=1)
+    got = []
+    for busy in (False, True):
+        model = costmodel.CostModel(HipAPI(), seed=5)
+        print("case training, caller's stream busy:", busy, flush=True)
+        a = torch.rand((4096, 4096), device="cuda")
+        pending = []
+        select = torch.Tensor.index_select
+
+        def after_work(t, *args):  # a product before every gather, on the stream it runs on
+            if busy:
+                with torch.cuda.stream(torch.cuda.default_stream()):
+                    pending.append(a @ a)
+            return select(t, *args)
+
+        torch.Tensor.index_select = after_work
+        try:
+            got.append(model.fit(x, y, epochs=3, batch=128))
+        finally:
+            torch.Tensor.index_select = select
+        torch.cuda.synchronize()
+    assert got[0] == got[1]
+
+
 def test_rows_beyond_one_launch():
     # 2^27 rows and some: more threads, at 32 a row, than a launch counts
     import torch
