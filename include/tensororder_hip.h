@@ -303,7 +303,8 @@ typedef struct to_pair_desc {
  * connected part of the tree whose intermediate tensors fit LDS.  A join of a program is a
  * product of up to 4 tensors, summed over the k bits; one of 3 or 4 is stored scaled by the power
  * of two that brings its largest entry to [0.5, 1), which its record's exponent carries
- * (TO_F32S).  Each wave of the block walks its own stream of ntask words, tasks[wave * ntask + i]: bits 0-15 the join, bits 16-22 its first
+ * (TO_F32S).  Each wave of the block walks its own stream of ntask words,
+ * tasks[wave * ntask + i]: bits 0-15 the join, bits 16-22 its first
  * chunk of 64 outputs-times-shares and bits 23-26 log2 of the step to the next one, bit 30:
  * nothing to do, bit 31: all waves meet after this entry (in the same entries of every
  * stream).  A join is TO_TREE_WORDS words, ops[join * TO_TREE_WORDS + i]:
