@@ -104,6 +104,13 @@ class Executable:
         # a plan that runs once only pays for capturing waves that repeat
         captured = {}
         self._runs = []
+        # the sum in host memory, and its word (None: the sum stays on the device, and a run's
+        # first launch resets what it needs)
+        self._sum = self._sum_word = None
+        if prog.host_accum is not None:
+            self._sum = _lib.Accum.from_address(prog.host_accum.data_ptr())
+            self._sum_word = ctypes.c_void_p(prog.host_accum.data_ptr() + _lib.Accum.pad.offset)
+        self._stream = ctypes.c_void_p(api._stream.cuda_stream)
         # runs queued since the last wait, and the value of the sum's word that ends them
         self._queued, self._word = 0, 0
         # whether the device's wave counter stands at the first slice once what is queued is
@@ -129,8 +136,7 @@ class Executable:
         return graph
 
     def _launch_graph(self, graph):
-        _lib.check(self.api._lib.to_graph_launch(graph, ctypes.c_void_p(self.api._stream.cuda_stream)),
-                   "to_graph_launch")
+        _lib.check(self.api._lib.to_graph_launch(graph, self._stream), "to_graph_launch")
 
     @property
     def step_launches(self):
@@ -146,24 +152,25 @@ class Executable:
 
     def enqueue(self):
         """Queue one full contraction on the API's stream (no synchronisation)."""
-        own = self.prog.host_accum is not None  # (else the run's first launch resets what it needs)
-        if own and not self._whole:
-            # an earlier run was cut short (a failed launch, an interrupt): nothing of it is
-            # counted, and the device's counter may stand between its waves
-            self.api.synchronize()
-            self._queued = 0
-        if own and (self._lent or not self._whole):
-            self.api._upload(self.prog.params, self.counters(self.total))
-        if own and not self._queued:
-            self._word = self._host_sum().pad
+        if self._sum is not None:
+            if not self._whole:
+                # an earlier run was cut short (a failed launch, an interrupt): nothing of it is
+                # counted, and the device's counter may stand between its waves
+                self.api.synchronize()
+                self._queued = 0
+            if self._lent or not self._whole:
+                self.api._upload(self.prog.params, self.counters(self.total))
+            if not self._queued:
+                self._word = self._sum.pad
         self._whole = False
         for graph, launches in self._runs:
             if graph is not None:
                 self._launch_graph(graph)
             else:
                 self.api._run(launches)
-        self._queued += own
-        self._word += self._sums
+        if self._sum is not None:
+            self._queued += 1
+            self._word += self._sums
         self._whole = True
 
     @staticmethod
@@ -175,20 +182,18 @@ class Executable:
     def result(self):
         """Synchronise and read the (mantissa, exponent) slice sum."""
         api = self.api
-        if self.prog.host_accum is not None:
+        acc = self._sum
+        if acc is not None:
             if not self._whole:
                 raise RuntimeError("the last run was cut short while it was queued")
-            acc = self._host_sum()
             if self._lent or not self._sums:  # (launches that a caller runs count in the word too)
                 api.synchronize()
             elif self._queued:
-                _lib.check(api._lib.to_wait(ctypes.c_void_p(ctypes.addressof(acc) + _lib.Accum.pad.offset),
-                                            self._word, ctypes.c_void_p(api._stream.cuda_stream)), "to_wait")
+                _lib.check(api._lib.to_wait(self._sum_word, self._word, self._stream), "to_wait")
                 if acc.pad < self._word:
                     raise RuntimeError("the device is idle and has not written the sum")
             if self._queued or self._lent:
                 self._queued, self._fresh = 0, False
-            acc = _lib.Accum.from_buffer_copy(acc)
         else:
             api.synchronize()
             self._fresh = False
@@ -200,9 +205,6 @@ class Executable:
         api.last_result = res
         api.last_stats = dict(self.prog.stats, nbatch=self.prog.nbatch, waves=self.nwaves, slices=self.total)
         return res
-
-    def _host_sum(self):
-        return _lib.Accum.from_address(self.prog.host_accum.data_ptr())
 
     def run(self):
         self.enqueue()
