@@ -174,7 +174,7 @@ def _join_cost(left, right, union, out, batched, esize):
 
 def analyse(tree, tables, esize, regroup=True):
     """(post-order FNode list, number of variables no remaining leaf holds -- each doubles the
-    count) of a plan, or None when no leaf would remain."""
+    count) of a plan, or None when no leaf would remain, or none of those that slicing changes."""
     # the tree's nodes, children before parents
     flat, inner, todo = [], tree.context.nodes, [tree.node_id]
     while todo:  # (each after what is to its right, then turned round)
@@ -202,7 +202,7 @@ def analyse(tree, tables, esize, regroup=True):
 
     # leaves: variable -> offset mask in the leaf's own table
     offs, weights, hosts = {}, [], []
-    seen, sliced = set(), {}
+    seen, sliced, changes = set(), {}, False
     for i, t, free in leaves:
         off, bit = {}, 1 << len(free)
         for e in free:
@@ -210,11 +210,14 @@ def analyse(tree, tables, esize, regroup=True):
             v = find(e)
             off[v] = off.get(v, 0) | bit
         seen.update(off)
+        changes = changes or t.batched
         if t.copy is not None and t.copy[2] and t.copy[0] == 1 and t.copy[1] == 1:
             continue  # a vector of ones
         offs[i] = off
         sliced[i] = t.batched
         (weights if len(off) <= 1 else hosts).append(i)
+    if changes and not any(sliced.values()):
+        return None  # every slice counts, though what is left is the same in all of them
     # weight vectors (and scalars) multiply one leaf that holds their variable: an unsliced
     # one where possible, so that the product is not repeated per slice
     attach, placed = {}, set()

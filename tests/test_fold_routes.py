@@ -44,6 +44,27 @@ def test_copies_sliced_on_a_part_of_their_edges(seed, et, tol):
         assert api.contract_sliced(got) == pytest.approx(want, rel=tol)
 
 
+@pytest.mark.parametrize("et", [_lib.TO_F64, _lib.TO_F32S])
+def test_groups_that_only_ones_hold(et):
+    # two unweighted COPY tensors that share an edge, beside two that a weight is on: slicing the
+    # first edge changes no value, but each slice counts
+    net = TensorNetwork()
+    ends = [net.add_node(VariableTensor(1, *w)) for w in ((1, 1), (1, 1), (0.3, 0.6), (1, 1))]
+    net.connect(*ends[0][0], *ends[1][0])
+    net.connect(*ends[2][0], *ends[3][0])
+    ctx, tree = TreeContext(), None
+    for end in ends:
+        leaf = ctx.leaf(net, end[0][0])
+        tree = leaf if tree is None else ctx.join(tree, leaf)
+    plan = SlicedExecutionPlan(ctx.get_tree(tree), net)
+    for groups, limit, want in (([], None, 1.8), ([{0}], None, 1.8), ([{0}], 1, 0.9), ([{1}], None, 1.8),
+                                ([{1}], 1, 1.2), ([{0}, {1}], None, 1.8), ([{0}, {1}], 2, 0.9)):
+        plan.groups_to_slice = groups
+        exe = EmulatedAPI(et).prepare(plan, limit)
+        got = exe.run()
+        assert got.value == pytest.approx(want, rel=1e-6) and got.slices == exe.total == (limit or 2 ** len(groups))
+
+
 def _star(n):
     """A plan of dense tensors and COPY tensors that opens 2 n variables before it sums any."""
     net, first, second = TensorNetwork(), [], []
