@@ -253,21 +253,9 @@ def analyse(tree, tables, esize, regroup=True):
     def leaf(i):
         return _T(i, {v: 1 for v in offs[i]}, batched=sliced[i])
 
-    stack = []
-    for i, n in enumerate(flat):
-        if n.is_leaf:
-            if i not in offs or i in placed:
-                stack.append(None)
-                continue
-            t = leaf(i)
-            for w in sorted(attach.get(i, []), key=lambda i: (sliced[i], i)):
-                t = join(t, leaf(w))
-            stack.append(t)
-            continue
-        right, left = stack.pop(), stack.pop()
-        if left is None or right is None:
-            stack.append(left or right)
-            continue
+    def absorb(left, right):
+        """Their join; where one operand is a large tensor's join with a small one, the small ones
+        are joined first if that costs less."""
         t = join(left, right)
         while regroup:
             big, small = (t.left, t.right) if len(t.left.open) >= len(t.right.open) else (t.right, t.left)
@@ -283,7 +271,24 @@ def analyse(tree, tables, esize, regroup=True):
             if nt.cost + m.cost >= t.cost + big.cost:
                 break
             t = nt
-        stack.append(t)
+        return t
+
+    stack = []
+    for i, n in enumerate(flat):
+        if n.is_leaf:
+            if i not in offs or i in placed:
+                stack.append(None)
+                continue
+            t = leaf(i)
+            for w in sorted(attach.get(i, []), key=lambda i: (sliced[i], i)):
+                t = absorb(t, leaf(w))
+            stack.append(t)
+            continue
+        right, left = stack.pop(), stack.pop()
+        if left is None or right is None:
+            stack.append(left or right)
+            continue
+        stack.append(absorb(left, right))
     top = stack[0]
     if top is None:
         return None

@@ -169,3 +169,24 @@ def test_analysis_of_many_weights_is_linear(monkeypatch):
     monkeypatch.setattr(fold, "min", counted, raising=False)
     nodes, _ = fold.analyse(tree, tables, 8)
     assert len(nodes) > 2 * n and compared[0] < 40 * len(nodes)
+
+
+@pytest.mark.parametrize("et,tol", [(_lib.TO_F64, 1e-12), (_lib.TO_F32S, 1e-6)])
+def test_weights_reach_a_wide_clause_together(et, tol):
+    # two clauses of 14 literals over 24 variables, and variables that none holds: a leaf takes the
+    # weights of all its variables in few joins, no more than the walk takes
+    first, second = range(1, 15), range(11, 25)
+    lines = ["p cnf 30 2"] + [" ".join(str(v * (-1) ** (v % 3)) for v in c) + " 0" for c in (first, second)]
+    lines += ["w %d %r" % (v, 0.2 + v / 60) for v in range(1, 31)]
+    net = network.cnf_count(parse_dimacs_text("\n".join(lines) + "\n", "cachet"))
+    for planner in ("line", "factor"):
+        plan = planners.best_plan(net, planner, solver=None, seed=0)
+        tree, tables = test_fold.plan_inputs(plan)[1:3]
+
+        def large(nodes):
+            return sum(max(nodes[n.left].rank, nodes[n.right].rank) >= fold.BIG_RANK for n in nodes if not n.is_leaf)
+
+        esize = 8 if et == _lib.TO_F64 else 4
+        assert large(fold.analyse(tree, tables, esize)[0]) <= max(6, large(schedule.analyse(tree, tables)))
+        want = numpy_oracle.contract_sliced(plan_io.plan_to_dict(plan))
+        assert EmulatedAPI(et).contract_sliced(plan) == pytest.approx(want, rel=tol)
